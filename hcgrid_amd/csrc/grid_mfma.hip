@@ -127,11 +127,11 @@ __device__ inline Window block_cell_window(const GridParams& P, const GridBuffer
 __device__ inline void ring_cell_window(const GridParams& P, const GridBuffers& B, const hcg_ring_meta& m,
                                         const Window& win, uint32_t r, uint32_t& lp, uint32_t& rp) {
   const uint32_t kr = r - m.firstring;
-  uint64_t a64 = 1, b64 = 0;
+  uint32_t a = 1, b = 0;
   const bool act =
-      r >= win.uring && r <= win.dring && ring_window(P, win, r, B.ring_z[kr], B.ring_s[kr], a64, b64) && a64 <= b64;
-  lp = act ? (uint32_t)a64 : 1u;
-  rp = act ? (uint32_t)b64 : 0u;
+      r >= win.uring && r <= win.dring && ring_window(P, win, r, B.ring_z[kr], B.ring_s[kr], a, b) && a <= b;
+  lp = act ? a : 1u;
+  rp = act ? b : 0u;
 }
 
 // The sorted range of the union of the wave's windows within [start, end)

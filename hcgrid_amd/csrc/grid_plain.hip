@@ -201,10 +201,10 @@ __global__ void __launch_bounds__(64 * kRowWaves) k_grid_rows(GridParams P, Grid
     const uint32_t kr = r - m.firstring;
     const uint32_t start = B.lut[kr], end = B.lut[kr + 1];
     if (start == end) continue;  // uniform: empty ring
-    uint64_t a = 1, b = 0;
+    uint32_t a = 1, b = 0;
     const bool act =
         r >= win.uring && r <= win.dring && ring_window(P, win, r, B.ring_z[kr], B.ring_s[kr], a, b) && a <= b;
-    const uint32_t lp = act ? (uint32_t)a : 1u, rp = act ? (uint32_t)b : 0u;
+    const uint32_t lp = act ? a : 1u, rp = act ? b : 0u;
     {
       const uint32_t wl = wave_min_u32(act ? lp : 0xFFFFFFFFu);
       const uint32_t wr = wave_max_u32(act ? rp : 0u);

@@ -103,10 +103,16 @@ __device__ inline Window window_of(const GridParams& P, uint32_t firstring, uint
   const double disc_theta = kHalfPi - b1;
   double utheta = disc_theta - P.disc_size;
   if (utheta * kRad2Deg < 0) utheta = 0;
-  uint64_t uring = pix2ring(P.hp, ang2pix(P.hp, utheta, l1));
+  const Hpx32 hx = hpx32(P.hp);
+  // a ring of kNoRing (theta outside [0, pi]) is past every used ring, as the
+  // reference's ring of its MAX_Y key is
+  constexpr uint32_t kNoRing = 0x7FFFFFFFu;
+  uint32_t pix = ang2pix32(hx, utheta, l1);
+  uint32_t uring = pix < hx.npix ? pix2ring32(hx, pix) : kNoRing;
   utheta = disc_theta + P.disc_size;
   if (P.selection == HCG_SELECT_DISC && utheta > kPi) utheta = kPi;  // the reference's MAX_Y key
-  uint64_t dring = pix2ring(P.hp, ang2pix(P.hp, utheta, l1));
+  pix = ang2pix32(hx, utheta, l1);
+  uint32_t dring = pix < hx.npix ? pix2ring32(hx, pix) : kNoRing;
   if (P.selection == HCG_SELECT_DISC) {
     // a point lies in one of the two rings whose centres bracket it, so two
     // rings either side cover every sample with |ts - tc| < R <= disc_size
@@ -116,10 +122,8 @@ __device__ inline Window window_of(const GridParams& P, uint32_t firstring, uint
   } else {
     w.mode = ((disc_theta * kRad2Deg <= kNorthB) || (disc_theta * kRad2Deg >= kSouthB)) ? kWinPolar : kWinCompat;
   }
-  if (uring < firstring) uring = firstring;
-  if (dring >= (uint64_t)firstring + usedrings) dring = (uint64_t)firstring + usedrings - 1;
-  w.uring = (uint32_t)uring;
-  w.dring = (uint32_t)dring;
+  w.uring = uring < firstring ? firstring : uring;
+  w.dring = dring >= firstring + usedrings ? firstring + usedrings - 1 : dring;
   if (w.mode == kWinCompat)
     w.phi = l1;
   else
@@ -134,10 +138,11 @@ __device__ inline bool skips_first_ring(const GridParams& P) { return P.selectio
 // lpix/rpix of ring r (HCGrid/gridding.cu:336-360).  Returns false where the
 // reference would `continue` without advancing (an endless loop there); the
 // ring is skipped here instead.  ang2pix(theta_r, phi) == loc2pix(cos theta_r, ...).
-__device__ inline bool ring_window(const GridParams& P, const Window& w, uint64_t ring, double rz, double rs,
-                                   uint64_t& lpix, uint64_t& rpix) {
-  uint64_t sp, npr;
-  ring_info(P.hp, ring, sp, npr);
+__device__ inline bool ring_window(const GridParams& P, const Window& w, uint32_t ring, double rz, double rs,
+                                   uint32_t& lpix, uint32_t& rpix) {
+  const Hpx32 hx = hpx32(P.hp);
+  uint32_t sp, npr;
+  ring_info32(hx, ring, sp, npr);
   if (w.mode != kWinCompat) {
     lpix = sp;
     rpix = sp + npr - 1;
@@ -147,25 +152,25 @@ __device__ inline bool ring_window(const GridParams& P, const Window& w, uint64_
     // the cap rings only (ring < nside or > 3 nside), with one pixel of
     // margin; disc windows narrow every ring, with two.  (float: tt npr / 4
     // < 32768 is good to 0.004 pixel.)
-    const bool cap = ring < P.hp.nside || ring > 3 * (uint64_t)P.hp.nside;
+    const bool cap = ring < hx.nside || ring > 3 * hx.nside;
     if (w.range.tlo <= w.range.thi && (cap || w.mode == kWinDisc)) {
       const int32_t m = w.mode == kWinDisc ? 2 : 1;
-      const float q = (float)(uint32_t)(npr >> 2);
+      const float q = (float)(npr >> 2);
       const int32_t lo = (int32_t)floorf(w.range.tlo * q) - m;
       const int32_t hi = (int32_t)floorf(w.range.thi * q) + m;
       if (lo >= 0 && hi < (int32_t)npr) {
-        lpix = sp + (uint64_t)lo;
-        rpix = sp + (uint64_t)hi;
+        lpix = sp + (uint32_t)lo;
+        rpix = sp + (uint32_t)hi;
       }
     }
     return true;
   }
   const bool have = rs >= 0.0;
-  lpix = loc2pix(P.hp, rz, w.phi - P.disc_size, have ? rs : 0., have);
-  if (!(lpix >= sp && lpix < sp + npr)) return false;
-  rpix = loc2pix(P.hp, rz, w.phi + P.disc_size, have ? rs : 0., have);
-  if (!(rpix >= sp && rpix < sp + npr)) return false;
-  return true;
+  const double s = have ? rs : 0.;
+  lpix = loc2pix32(hx, rz, fmodulo4((w.phi - P.disc_size) * kInvHalfPi), s, have);
+  if (lpix - sp >= npr) return false;
+  rpix = loc2pix32(hx, rz, fmodulo4((w.phi + P.disc_size) * kInvHalfPi), s, have);
+  return rpix - sp < npr;
 }
 
 // ---- out-of-line slow paths (rare; kept out of the inner loop's registers) ----

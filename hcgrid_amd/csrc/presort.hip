@@ -34,13 +34,14 @@ constexpr int kSortWaves = kSortThreads / 64;
 __global__ void __launch_bounds__(256) k_keys(hcg_healpix hp, uint32_t n, const double* __restrict__ lon,
                                               const double* __restrict__ lat, uint32_t* __restrict__ keys,
                                               uint32_t* __restrict__ idx) {
+  const Hpx32 hx = hpx32(hp);
   // 64-bit index: with a 32-bit one, i + stride wraps below n for n close to 2^32
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     // HCGrid/gridding.cu:78-80
     const double theta = kHalfPi - kDeg2Rad * lat[i];
     const double phi = kDeg2Rad * lon[i];
-    keys[i] = (uint32_t)ang2pix(hp, theta, phi);
+    keys[i] = ang2pix32(hx, theta, phi);
     idx[i] = (uint32_t)i;
   }
 }
