@@ -6,8 +6,9 @@
 // Here a geometry (one map's sorted samples, ring LUT and target
 // coordinates) is built once and kept in HBM; a batch names any number of
 // (geometry, channel values, output cube) jobs of uneven sizes and grids
-// them all with one launch of k_grid_mfma_batch, whose workgroups pull
-// (job, tile, channel group) items from a device queue.  Everything a batch
+// them with one launch of k_grid_mfma_batch, whose workgroups pull (job,
+// tile, channel group) items from a device queue, and one launch per tile
+// route (one- and few-channel jobs).  Everything a batch
 // enqueues is kernels only (no memsets, no host copies), so the sequence
 // can be captured into a graph and replayed.
 #include <hip/hip_runtime.h>
@@ -58,12 +59,15 @@ struct hcg_batch {
   PrepRange* d_ranges;   // the prep launch: every job's channel gather and tile plan
   PrepJob* d_prep;
   uint32_t nranges, prep_blocks;
+  TileRange* d_tiles;    // the tile-route jobs: every route's ranges, route after route
+  uint32_t tile_first[kRoutes + 1], tile_blocks[kRoutes];
   std::vector<hcg_batch_job> jobs;
   std::vector<void*> values_sorted;
   std::vector<MfmaJob> host_jobs;     // upload sources, alive until destroy
   std::vector<MfmaItem> host_items;
   std::vector<PrepRange> host_ranges;
   std::vector<PrepJob> host_prep;
+  std::vector<TileRange> host_tiles;
   // optional kernel timing (hcg_batch_timing): start, after the prep launch, after the gridding launches
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   bool timed = false;  // the events of the last eager enqueue were recorded
@@ -256,7 +260,9 @@ struct BatchPlan {
   uint32_t waves = 0, chunk = 0;
   uint32_t n_dense = 0;  // the first n_dense items belong to the dense launch
   std::vector<MfmaItem> items;
-  std::vector<uint32_t> tiles, tcols, tpi, tstreams;  // tile-path jobs: tiles per item, streams; else 0
+  std::vector<uint32_t> tiles, tcols, route;
+  std::vector<TileRange> tile_ranges;                 // tile-route jobs, route after route
+  uint32_t tile_first[kRoutes + 1] = {}, tile_blocks[kRoutes] = {};
   std::vector<size_t> voff, poff;
   size_t bytes = 0;
 };
@@ -286,10 +292,7 @@ int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32
   std::vector<double> cost(njobs);
   p.tiles.assign(njobs, 0);
   p.tcols.assign(njobs, 0);
-  p.tpi.assign(njobs, 0);
-  p.tstreams.assign(njobs, 0);
-  const uint32_t tile_tpi = tile_items_per_block(chunk, waves, kTileLdsBytes);
-  const uint32_t few_tpi = tile_items_per_block(chunk, waves, kFewTileLdsBytes);
+  p.route.assign(njobs, kRouteMfma);
   uint64_t nitems = 0;
   for (uint32_t j = 0; j < njobs; ++j) {
     const hcg_batch_job& b = jobs[j];
@@ -297,26 +300,12 @@ int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32
     const uint32_t side = g->side;
     order[j] = j;
     const GridParams P = make_grid_params(&g->hp, &g->kern, side);
-    if (one_channel_tiles(P, g->kern.kernel_type, false, b.nchan)) {
-      // one channel: FP64 tile path, tile_tpi tiles of 64 cells per item (one
-      // per wave), or on small maps one tile per item over its ring streams;
-      // the tile loop weighs a pair roughly 8x faster than the MFMA stage
+    p.route[j] = route_of(P, g->kern.kernel_type, false, b.nchan, g->n);
+    if (p.route[j] != kRouteMfma) {  // FP64 tile loop: a workgroup per tile, in its route's own launch
       p.tcols[j] = kTileCols;
       p.tiles[j] = side ? tile_count_of(side) : 0;
-      p.tstreams[j] = one_channel_streams(side);
-      p.tpi[j] = p.tstreams[j] > 1 ? 1u : tile_tpi;
       groups[j] = 1;
-      units[j] = ceil_div_u32(p.tiles[j], p.tpi[j]);
-      cost[j] = item_cost(g, kTileCols, 1) * p.tpi[j] / 8.0;
-    } else if (few_channel_tiles(P, g->kern.kernel_type, false, b.nchan, g->n)) {
-      // few channels on a large map: FP64 tile path, one tile per wave
-      p.tcols[j] = kTileCols;
-      p.tiles[j] = tile_count_of(side);
-      p.tstreams[j] = 1;
-      p.tpi[j] = few_tpi;
-      groups[j] = 1;
-      units[j] = ceil_div_u32(p.tiles[j], few_tpi);
-      cost[j] = item_cost(g, kTileCols, b.nchan) * few_tpi / 4.0;
+      units[j] = 0;
     } else {
       const uint32_t tc = b.tile_cols ? b.tile_cols : kMcDefaultTileCols;
       p.tcols[j] = tc;
@@ -333,6 +322,18 @@ int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32
     nitems += (uint64_t)units[j] * groups[j];
   }
   if (nitems >= 0xFFFFFFFFull) return set_error(HCG_ERR_INVALID, "hcg_batch_create: too many work items");
+  for (uint32_t r = kRouteMfma + 1; r < kRoutes; ++r) {
+    p.tile_first[r] = (uint32_t)p.tile_ranges.size();
+    uint64_t blocks = 0;
+    for (uint32_t j = 0; j < njobs; ++j)
+      if (p.route[j] == r && p.tiles[j]) {
+        p.tile_ranges.push_back(TileRange{(uint32_t)blocks, j});
+        blocks += p.tiles[j];
+      }
+    if (blocks >= 0x7FFFFFFFull) return set_error(HCG_ERR_INVALID, "hcg_batch_create: too many tiles");
+    p.tile_blocks[r] = (uint32_t)blocks;
+  }
+  p.tile_first[kRoutes] = (uint32_t)p.tile_ranges.size();
   std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return cost[a] > cost[b]; });
   p.items.clear();
   p.items.reserve(nitems);
@@ -351,13 +352,14 @@ int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32
   c.take<uint32_t>(2 + njobs);
   c.take<PrepRange>(2 * (size_t)njobs + 1);
   c.take<PrepJob>(njobs ? njobs : 1);
+  c.take<TileRange>(njobs ? njobs : 1);
   p.voff.assign(njobs, 0);
   p.poff.assign(njobs, 0);
   for (uint32_t j = 0; j < njobs; ++j) {
     p.voff[j] = c.off;
     c.off += hcg_batch_job_bytes(jobs[j].geometry, jobs[j].nchan);
     p.poff[j] = c.off;
-    if (!p.tpi[j]) c.off = align_up(c.off + (size_t)p.tiles[j] * kPlanTileWords * sizeof(uint32_t));
+    if (p.route[j] == kRouteMfma) c.off = align_up(c.off + (size_t)p.tiles[j] * kPlanTileWords * sizeof(uint32_t));
   }
   p.bytes = c.off;
   return HCG_OK;
@@ -385,6 +387,10 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
   bt->d_counters = d.take<uint32_t>(2 + njobs);
   bt->d_ranges = d.take<PrepRange>(2 * (size_t)njobs + 1);
   bt->d_prep = d.take<PrepJob>(njobs ? njobs : 1);
+  bt->d_tiles = d.take<TileRange>(njobs ? njobs : 1);
+  bt->host_tiles = p.tile_ranges;
+  std::copy(std::begin(p.tile_first), std::end(p.tile_first), bt->tile_first);
+  std::copy(std::begin(p.tile_blocks), std::end(p.tile_blocks), bt->tile_blocks);
   bt->values_sorted.resize(njobs);
   std::vector<MfmaJob>& hj = bt->host_jobs;
   hj.resize(njobs);
@@ -409,9 +415,9 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
                     ceil_div_u32(g->side, p.tcols[j]),
                     p.tiles[j],
                     (uint32_t)(b.normalize ? 1 : 0),
-                    p.tpi[j] ? nullptr : reinterpret_cast<uint32_t*>(static_cast<char*>(bt->base) + p.poff[j]),
-                    p.tpi[j],
-                    p.tstreams[j]};
+                    p.route[j] != kRouteMfma
+                        ? nullptr
+                        : reinterpret_cast<uint32_t*>(static_cast<char*>(bt->base) + p.poff[j])};
   }
   // the prep launch: gathers (channel-major values) and plans of every job
   bt->host_prep.resize(njobs);
@@ -428,6 +434,7 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
   hipError_t e = hipSuccess;
   const size_t jb = njobs * sizeof(MfmaJob), ib = p.items.size() * sizeof(MfmaItem);
   const size_t rb = bt->host_ranges.size() * sizeof(PrepRange), pb = njobs * sizeof(PrepJob);
+  const size_t tb = bt->host_tiles.size() * sizeof(TileRange);
   if (upload_async) {
     // ordered on `stream`; the host sources live in the batch until destroy
     if (jb) e = hipMemcpyAsync(bt->d_jobs, hj.data(), jb, hipMemcpyHostToDevice, stream);
@@ -436,11 +443,14 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
     if (e == hipSuccess && rb)
       e = hipMemcpyAsync(bt->d_ranges, bt->host_ranges.data(), rb, hipMemcpyHostToDevice, stream);
     if (e == hipSuccess && pb) e = hipMemcpyAsync(bt->d_prep, bt->host_prep.data(), pb, hipMemcpyHostToDevice, stream);
+    if (e == hipSuccess && tb)
+      e = hipMemcpyAsync(bt->d_tiles, bt->host_tiles.data(), tb, hipMemcpyHostToDevice, stream);
   } else {
     if (jb) e = hipMemcpy(bt->d_jobs, hj.data(), jb, hipMemcpyHostToDevice);
     if (e == hipSuccess && ib) e = hipMemcpy(bt->d_items, p.items.data(), ib, hipMemcpyHostToDevice);
     if (e == hipSuccess && rb) e = hipMemcpy(bt->d_ranges, bt->host_ranges.data(), rb, hipMemcpyHostToDevice);
     if (e == hipSuccess && pb) e = hipMemcpy(bt->d_prep, bt->host_prep.data(), pb, hipMemcpyHostToDevice);
+    if (e == hipSuccess && tb) e = hipMemcpy(bt->d_tiles, bt->host_tiles.data(), tb, hipMemcpyHostToDevice);
   }
   int rc = HCG_OK;
   if (e != hipSuccess) rc = set_error(HCG_ERR_HIP, std::string("hcg_batch_create: ") + hipGetErrorString(e));
@@ -511,6 +521,11 @@ extern "C" int hcg_batch_enqueue(hcg_batch* b, void* stream) {
   int rc = launch_batch_prep(b->d_ranges, b->nranges, b->prep_blocks, b->d_prep, b->d_jobs, s);
   if (rc != HCG_OK) return rc;
   if (timing) HCG_CHECK_HIP(hipEventRecord(b->ev[1], s));
+  for (uint32_t r = kRouteMfma + 1; r < kRoutes; ++r) {
+    rc = launch_batch_tiles(r, b->d_tiles + b->tile_first[r], b->tile_first[r + 1] - b->tile_first[r],
+                            b->tile_blocks[r], b->d_jobs, s);
+    if (rc != HCG_OK) return rc;
+  }
   // the dense jobs' launch (its own queue head after the job counters), then the rest
   if (b->nitems_dense) {
     rc = launch_mfma_batch(kDenseChunk, kDenseWaves, b->blocks_dense, b->d_jobs, b->d_items, b->nitems_dense,
@@ -556,6 +571,7 @@ extern "C" int hcg_batch_info(const hcg_batch* b, hcg_batch_stats* st) {
   HCG_REQUIRE(b && st, "hcg_batch_info: NULL argument");
   st->njobs = b->njobs;
   st->nitems = b->nitems;
+  for (uint32_t t : b->tile_blocks) st->nitems += t;
   st->blocks = b->blocks;
   st->waves = b->waves;
   st->chunk = b->chunk;

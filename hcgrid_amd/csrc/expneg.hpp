@@ -38,8 +38,20 @@ __device__ __constant__ const double kExp2Table[64] = {
     0x1.d5818dcfba487p+0, 0x1.da9e603db3285p+0, 0x1.dfc97337b9b5fp+0, 0x1.e502ee78b3ff6p+0,
     0x1.ea4afa2a490dap+0, 0x1.efa1bee615a27p+0, 0x1.f50765b6e4540p+0, 0x1.fa7c1819e90d8p+0};
 
-// Copies the table into a 64-entry LDS array (one element per lane of the wave).
-__device__ inline void exp_table_load(double* lds_table) { lds_table[__lane_id()] = kExp2Table[__lane_id()]; }
+// Copies the table into a 64-entry LDS array (one element per lane of the
+// wave), entry j less j 2^14 in its high word: 2^(n/64) of n = 64 m + j is
+// then the entry plus n 2^14 there (n 2^14 = m 2^20 + j 2^14, and 2^20 is
+// one step of the exponent field), which gauss_weight_lean uses; exp_tab
+// gives the plain 2^(j/64).
+constexpr int kExpTabShift = 14;
+__device__ inline void exp_table_load(double* lds_table) {
+  const uint32_t j = __lane_id();
+  lds_table[j] = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, kExp2Table[j]) -
+                                                ((uint64_t)j << (32 + kExpTabShift)));
+}
+__device__ inline double exp_tab(const double* lds_table, int j) {
+  return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, lds_table[j]) + ((uint64_t)j << (32 + kExpTabShift)));
+}
 
 // exp(y * ln2/64) for y <= 0 given pre-scaled: n = rint(y), y - n is exact,
 // r = (y - n) ln2/64 with |r| <= ln2/128, degree-5 Taylor polynomial
@@ -56,7 +68,7 @@ __device__ inline double exp_scaled_neg(double y, const double* lds_table) {
   q = fma(r, q, 0.5);
   q = fma(r, q, 1.0);
   const double p = r * q;  // exp(r) - 1
-  const double t = lds_table[j];
+  const double t = exp_tab(lds_table, j);
   return ldexp(fma(t, p, t), m);
 }
 
@@ -73,7 +85,7 @@ __device__ inline double exp_scaled_neg_nc(double y, const double* lds_table) {
   q = fma(r, q, 0.5);
   q = fma(r, q, 1.0);
   const double p = r * q;
-  const double t = lds_table[j];
+  const double t = exp_tab(lds_table, j);
   return ldexp(fma(t, p, t), m);
 }
 
@@ -108,7 +120,7 @@ __device__ inline double exp_scaled_neg_fold(double y, const double* lds_table) 
   q = fma_vvs(u, q, c2);
   q = fma_vvs(u, q, c1);
   const double p = u * q;
-  const double t = lds_table[j];
+  const double t = exp_tab(lds_table, j);
   return ldexp(fma(t, p, t), m);
 }
 
@@ -125,7 +137,7 @@ __device__ inline double exp_neg(double x, const double* lds_table) {
   q = fma(r, q, 0.5);
   q = fma(r, q, 1.0);
   const double p = r * q;  // exp(r) - 1
-  const double t = lds_table[j];
+  const double t = exp_tab(lds_table, j);
   return ldexp(fma(t, p, t), m);
 }
 

@@ -138,8 +138,15 @@ __device__ inline bool skips_first_ring(const GridParams& P) { return P.selectio
 // lpix/rpix of ring r (HCGrid/gridding.cu:336-360).  Returns false where the
 // reference would `continue` without advancing (an endless loop there); the
 // ring is skipped here instead.  ang2pix(theta_r, phi) == loc2pix(cos theta_r, ...).
-__device__ inline bool ring_window(const GridParams& P, const Window& w, uint32_t ring, double rz, double rs,
-                                   uint32_t& lpix, uint32_t& rpix) {
+// The longitude edges of a compat window do not depend on the ring:
+// compat_edges gives them once, ring_window_at takes them.
+__device__ inline void compat_edges(const GridParams& P, const Window& w, double& tl, double& tr) {
+  tl = fmodulo4((w.phi - P.disc_size) * kInvHalfPi);
+  tr = fmodulo4((w.phi + P.disc_size) * kInvHalfPi);
+}
+
+__device__ inline bool ring_window_at(const GridParams& P, const Window& w, double tl, double tr, uint32_t ring,
+                                      double rz, double rs, uint32_t& lpix, uint32_t& rpix) {
   const Hpx32 hx = hpx32(P.hp);
   uint32_t sp, npr;
   ring_info32(hx, ring, sp, npr);
@@ -167,24 +174,37 @@ __device__ inline bool ring_window(const GridParams& P, const Window& w, uint32_
   }
   const bool have = rs >= 0.0;
   const double s = have ? rs : 0.;
-  lpix = loc2pix32(hx, rz, fmodulo4((w.phi - P.disc_size) * kInvHalfPi), s, have);
+  lpix = loc2pix32(hx, rz, tl, s, have);
   if (lpix - sp >= npr) return false;
-  rpix = loc2pix32(hx, rz, fmodulo4((w.phi + P.disc_size) * kInvHalfPi), s, have);
+  rpix = loc2pix32(hx, rz, tr, s, have);
   return rpix - sp < npr;
+}
+
+__device__ inline bool ring_window(const GridParams& P, const Window& w, uint32_t ring, double rz, double rs,
+                                   uint32_t& lpix, uint32_t& rpix) {
+  double tl = 0.0, tr = 0.0;
+  if (w.mode == kWinCompat) compat_edges(P, w, tl, tr);
+  return ring_window_at(P, w, tl, tr, ring, rz, rs, lpix, rpix);
 }
 
 // ---- out-of-line slow paths (rare; kept out of the inner loop's registers) ----
 
 // The reference's radius test (HCGrid/helpers.cu:128-130, gridding.cu:381-386)
 // for a pair inside the guard band.
-[[maybe_unused]] static __device__ __noinline__ bool radius_test_ref(const double* xwcs, const double* ywcs, const double* lon_s,
-                                             const double* lat_s, uint32_t cell, uint32_t i, double radius) {
+__device__ __forceinline__ bool radius_test_inline(const double* xwcs, const double* ywcs, const double* lon_s,
+                                                   const double* lat_s, uint32_t cell, uint32_t i, double radius) {
   const double l1 = xwcs[cell] * kDeg2Rad, b1 = ywcs[cell] * kDeg2Rad;
   const double l2 = lon_s[i] * kDeg2Rad, b2 = lat_s[i] * kDeg2Rad;
   const double a = sin((b1 - b2) / 2.);
   const double c = sin((l1 - l2) / 2.);
   const double d = 2 * asin(sqrt(a * a + cos(b1) * cos(b2) * (c * c))) * kRad2Deg;
   return d < radius;
+}
+
+[[maybe_unused]] static __device__ __noinline__ bool radius_test_ref(const double* xwcs, const double* ywcs,
+                                                                     const double* lon_s, const double* lat_s,
+                                                                     uint32_t cell, uint32_t i, double radius) {
+  return radius_test_inline(xwcs, ywcs, lon_s, lat_s, cell, i, radius);
 }
 
 [[maybe_unused]] static __device__ __noinline__ double asin2_direct(double h) {
@@ -246,6 +266,12 @@ inline bool dot_distance_ok(const GridParams& P) { return P.c_hi >= 1e-7; }
 // term, (4/560) c2^3 relative to the leading one, is below 6e-17 (host side).
 inline bool gauss_tiny_radius(const GridParams& P) { return gauss_small_radius(P) && P.c_hi < 2e-5; }
 
+// gauss_weight_lean's range: gauss_tiny_radius, dot_distance_ok, and every
+// selected weight a normal number (2^-937 and up; 36 sigma).
+inline bool lean_weight_ok(const GridParams& P) {
+  return gauss_tiny_radius(P) && dot_distance_ok(P) && P.c_hi * (P.k0 + P.c_hi * P.k1) > -60000.0;
+}
+
 // The GAUSS1D weight of a selected pair from the exponent's series (W = 1:
 // four terms, gauss_small_radius; W = 2: three terms, gauss_tiny_radius) and
 // exp_scaled_neg_fold; steps with a parameter as one v_fma_f64 each.
@@ -269,6 +295,14 @@ __device__ inline double in_vgprs(double x) {
   return v;
 }
 
+// (a << SHIFT) + b as the one instruction it is.
+template <int SHIFT>
+__device__ inline uint32_t lshl_add_u32(uint32_t a, uint32_t b) {
+  uint32_t d;
+  asm("v_lshl_add_u32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "n"(SHIFT), "v"(b));
+  return d;
+}
+
 // Degree-3 coefficient of exp(u ln2/64) - 1 = u (e1 + u (e2 + u e3)).
 constexpr double kExpE1 = 0x1.62e42fefa39efp-7;  // ln2 / 64
 constexpr double kExpE2 = kExpE1 * kExpE1 / 2.0;
@@ -284,16 +318,26 @@ constexpr double kExpE3 = kExpE2 * kExpE1 / 3.0;
 // and b = 4 k1 (y = h (a + b h) is the same value: every scaling is by a
 // power of two); bv and e3v hold b and kExpE3 in vector registers
 // (in_vgprs), so every step is one v_fma_f64.
+//
+// rint(y) comes from adding 1.5 2^52 (the sum's low word is the integer, so
+// no conversion), u = y - rint(y) is one FMA of the unrounded product, and
+// 2^(n/64) is assembled by adding n 2^14 to the high word of the table entry,
+// which holds 2^(j/64) less j 2^14 (exp_table_load): one integer instruction
+// instead of a shift and an ldexp.  That needs a normal result, which
+// lean_weight_ok ensures.
 __device__ inline double gauss_weight_lean(double h, double a, double bv, double e3v, const double* s_exp) {
-  const double y = h * fma(h, bv, a);
-  const double n = rint(y);
-  const int ni = (int)n;
-  const double u = y - n;
+  constexpr double kRound = 0x1.8p+52;
+  const double t = fma(h, bv, a);
+  const double s = fma_vvs(h, t, kRound);
+  const double u = fma(h, t, kRound - s);  // s - kRound is exact, and so is its negative
   double q = fma_vvs(u, e3v, kExpE2);  // three-operand v_fma_f64: no copy of a constant register
   q = fma_vvs(u, q, kExpE1);
-  const double p = u * q;
-  const double t = s_exp[ni & 63];
-  return ldexp(fma(t, p, t), ni >> 6);
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const uint32_t ni = __builtin_bit_cast(u32x2, s).x;
+  u32x2 tab = __builtin_bit_cast(u32x2, s_exp[ni & 63u]);
+  tab.y = lshl_add_u32<kExpTabShift>(ni, tab.y);
+  const double w = __builtin_bit_cast(double, tab);
+  return fma(w, u * q, w);
 }
 
 // GAUSS2D / TAPERED_SINC weights (HCGrid/gridding.cu:242-256).
@@ -354,22 +398,46 @@ __device__ inline uint32_t wave_search(const uint32_t* __restrict__ keys, uint32
   return m ? lo + (uint32_t)__ffsll((unsigned long long)m) - 1 : hi;
 }
 
+// Wave reductions by DPP (row shifts by 1, 2, 4, 8, then the row broadcasts:
+// lane 63 holds the result), returned wave-uniform.  A lane whose source is
+// outside the row keeps `id`.
+template <int CTRL, int ROWS>
+__device__ inline uint32_t dpp_u32(uint32_t id, uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, CTRL, ROWS, 0xF, false);
+}
+template <int CTRL, int ROWS>
+__device__ inline double dpp_f64(double id, double v) {
+  const uint64_t i = __builtin_bit_cast(uint64_t, id), u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t)dpp_u32<CTRL, ROWS>((uint32_t)i, (uint32_t)u) |
+                                        ((uint64_t)dpp_u32<CTRL, ROWS>((uint32_t)(i >> 32), (uint32_t)(u >> 32)) << 32));
+}
+constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
+constexpr int kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+
 __device__ inline uint32_t wave_min_u32(uint32_t v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const uint32_t o = __shfl_xor(v, off, 64);
-    v = o < v ? o : v;
-  }
-  return v;
+  constexpr uint32_t id = 0xFFFFFFFFu;
+  v = min(v, dpp_u32<kRowShr1, 0xF>(id, v));
+  v = min(v, dpp_u32<kRowShr2, 0xF>(id, v));
+  v = min(v, dpp_u32<kRowShr4, 0xF>(id, v));
+  v = min(v, dpp_u32<kRowShr8, 0xF>(id, v));
+  v = min(v, dpp_u32<kRowBcast15, 0xA>(id, v));
+  v = min(v, dpp_u32<kRowBcast31, 0xC>(id, v));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-__device__ inline uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const uint32_t o = __shfl_xor(v, off, 64);
-    v = o > v ? o : v;
-  }
-  return v;
+__device__ inline uint32_t wave_max_u32(uint32_t v) { return ~wave_min_u32(~v); }
+
+__device__ inline double wave_min_f64(double v) {
+  constexpr double id = 1e308;
+  v = fmin(v, dpp_f64<kRowShr1, 0xF>(id, v));
+  v = fmin(v, dpp_f64<kRowShr2, 0xF>(id, v));
+  v = fmin(v, dpp_f64<kRowShr4, 0xF>(id, v));
+  v = fmin(v, dpp_f64<kRowShr8, 0xF>(id, v));
+  v = fmin(v, dpp_f64<kRowBcast15, 0xA>(id, v));
+  v = fmin(v, dpp_f64<kRowBcast31, 0xC>(id, v));
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, 63) |
+                                        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(u >> 32), 63) << 32));
 }
 
 // Kernel-argument form of the set-up (host side).

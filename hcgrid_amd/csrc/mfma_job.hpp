@@ -35,14 +35,14 @@ static_assert(sizeof(Window) % 8 == 0 && kPlanHeadWords % 2 == 0 && kPlanTileWor
 // The weight form of a job (MfmaJob::kt): the kernel type, or
 // kKtGaussSmall (GAUSS1D whose radius rules out the exponent's asin branch
 // and the exp clamp, gauss_small_radius), or kKtGaussLean (also
-// gauss_tiny_radius and dot_distance_ok: the p.q candidate test and
-// gauss_weight_lean of the tile loop).
+// lean_weight_ok: the p.q candidate test and gauss_weight_lean of the tile
+// loop).
 constexpr uint32_t kKtGaussSmall = HCG_GAUSS1D + 16u;
 constexpr uint32_t kKtGaussLean = HCG_GAUSS1D + 32u;
 
 inline uint32_t mfma_weight_form(const GridParams& P, int kernel_type) {
   if (kernel_type != HCG_GAUSS1D || !gauss_small_radius(P)) return (uint32_t)kernel_type;
-  return gauss_tiny_radius(P) && dot_distance_ok(P) ? kKtGaussLean : kKtGaussSmall;
+  return lean_weight_ok(P) ? kKtGaussLean : kKtGaussSmall;
 }
 
 // One multi-channel job: geometry, sorted channel values and outputs, with
@@ -56,14 +56,28 @@ struct MfmaJob {
   uint32_t kt, n_pad, nchan, dtype;  // kt: mfma_weight_form
   uint32_t tc_shift, tiles_x, ntiles, normalize;
   uint32_t* plan;     // [ntiles][kPlanTileWords], or NULL (windows and searches in the gridding kernel)
-  // 0: the MFMA contraction; else a one-channel job on the FP64 tile path
-  // (one_channel_tiles) with tiles_x and ntiles counting kTileCols x
-  // kTileRows tiles: this many tiles per work item, one per wave, when
-  // tile_streams is 1; one tile per item split over tile_streams partial
-  // ring streams otherwise (one_channel_streams)
-  uint32_t tiles_per_item;
-  uint32_t tile_streams;
 };
+
+// The routes of a job: the MFMA contraction, or the FP64 tile loop (tiles_x
+// and ntiles then count kTileCols x kTileRows tiles): one channel with four
+// ring streams per tile (one_channel_streams) or one, or few channels.
+enum : uint32_t { kRouteMfma = 0, kRouteOne4 = 1, kRouteOne1 = 2, kRouteFew = 3, kRoutes = 4 };
+inline uint32_t route_of(const GridParams& P, uint32_t kernel_type, bool weighted, uint32_t nchan, uint32_t n) {
+  if (one_channel_tiles(P, kernel_type, weighted, nchan))
+    return one_channel_streams(P.side) == kOneChannelStreams ? kRouteOne4 : kRouteOne1;
+  return few_channel_tiles(P, kernel_type, weighted, nchan, n) ? kRouteFew : kRouteMfma;
+}
+
+// The tile-route jobs of a batch: job `job`'s tiles are workgroups first,
+// first + 1, ... of its route's launch.
+struct TileRange {
+  uint32_t first, job;
+};
+// Launches one tile route's workgroups (`blocks` of them over `nranges`
+// ranges): the same tile bodies as the one-job launches, so a job's cube is
+// the same alone or batched.
+int launch_batch_tiles(uint32_t route, const TileRange* ranges, uint32_t nranges, uint32_t blocks,
+                       const MfmaJob* jobs, hipStream_t s);
 
 // One unit of the persistent launch: a tile of one job, one channel group.
 struct MfmaItem {
@@ -96,11 +110,6 @@ int launch_batch_prep(const PrepRange* ranges, uint32_t nranges, uint32_t blocks
 
 // Enqueues the tile-plan kernel of a job into J.plan (non-NULL).
 int launch_mfma_plan(const MfmaJob& J, hipStream_t s);
-
-// Tiles per work item of a tile-path job in the persistent kernel of (chunk,
-// waves): one per wave, as many as the workgroup's LDS holds at tile_bytes
-// per tile.
-uint32_t tile_items_per_block(uint32_t chunk, uint32_t waves, size_t tile_bytes);
 
 // Grid size of the persistent kernel: CUs x resident workgroups per CU.
 int mfma_batch_blocks(uint32_t chunk, uint32_t waves, uint32_t* blocks);

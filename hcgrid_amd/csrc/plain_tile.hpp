@@ -1,34 +1,50 @@
 // plain_tile.hpp -- one tile of the single-channel gather-convolution, the
 // body of k_grid_tiles (grid_plain.hip), shared with the one- and
 // few-channel jobs of the multi-channel entry points (grid_plain.hip's
-// k_grid_tiles_1ch / k_grid_tiles_few, and the persistent batch kernel in
-// grid_mfma.hip).
+// k_grid_tiles_1ch / k_grid_tiles_few, and k_batch_tiles for the jobs of a
+// batch).
 //
-// A tile is kTileCols x kTileRows map cells worked by one wave: lane l owns
-// column l / kLaneRows and, in it, kCellsPerLane vertically adjacent cells
-// from lane row l % kLaneRows.  Column-major lanes put the four cells of a
-// column (whose sample bands in a ring are nearly the same) next to each
-// other: the 16 lanes an LDS read serves at once then fetch from four bands
-// instead of sixteen, which cut LDS bank conflicts from 0.46 to 0.18 of
-// LDS-active cycles and the 20M-sample 2048^2 map from 4.92 to 4.65 ms
-// (row-major lanes; the sums are the same bit for bit, since each cell's
-// accumulation order does not depend on its lane).  The selection,
-// distance, weight and accumulation order are the ones described in
-// grid_plain.hip.  Instantiations:
-//  * BATCH false (k_grid_tiles): FP64 values from the sample records,
-//    sums accumulated in place into the FP64 data and weight cubes (the
-//    reference's datacube/weightscube), workgroup barriers (one wave per
-//    workgroup);
+// A tile is kTileCols x kTileRows (16 x 4) map cells worked by one wave, in
+// three steps:
+//   1. lane = cell (column lane / 4, row lane % 4): the cell's window and
+//      unit vector;
+//   2. lane = ring: the sorted range of each of the tile's rings (up to 64
+//      at once), a superset of the union of its cells' windows, by a binary
+//      search per lane.  One such round of dependent loads per tile replaces
+//      two cooperative searches per ring;
+//   3. the ranges are staged in LDS (as many rings as fit at a time), and
+//      ring by ring the four lanes of a column take the samples between the
+//      column's window edges four at a time (lane phase p: samples p, p + 4,
+//      ...) and test each against the column's four cells: its window (one
+//      integer compare in half-pixel units, belt_window) and the radius.
+// A sample is read from LDS once for four cells, and the four rows are
+// separate branches: at a given step the sixteen columns stand at the same
+// place of their bands, so a row whose disc does not reach the ring, or no
+// longer reaches this far along it, is skipped by the whole wave.  The loop
+// is bound by FP64 issue (a candidate costs three FMAs and the compares, a
+// selected pair thirteen more), so what counts is that the lanes of a weight
+// evaluation are nearly all selected: with lane = cell and one band per lane
+// 44% of the lane slots did selected pairs on the 20M-sample raster (rows
+// outside a ring's reach and the window's corners outside the disc idled
+// through the weight): 1.97e9 vector instructions and 4.40 ms then, 1.34e9
+// and 3.42 ms now.  On sparse maps the per-ring chain of searches, loads and
+// window arithmetic is what counts (160k samples onto 1024^2: 199 us).
+//
+// The selection, distance and weight are the ones described in
+// grid_plain.hip; a cell's sum is the sum of its four phases' partial sums
+// (and of its ring streams'), each in ring and sorted order.
+// Instantiations:
+//  * BATCH false (k_grid_tiles): FP64 values from the sample records, sums
+//    added to the FP64 data and weight cubes (the reference's
+//    datacube/weightscube);
 //  * BATCH true (a one-channel job of the multi-channel entry points): the
-//    job's sorted 16-bit values, one partial stream of the tile's rings
-//    (every stride-th ring from the phase-th), sums from zero returned to
-//    the caller, which adds the streams in stream order and writes the FP32
-//    cube (divided by the weight sum when the job normalises; NaN where no
-//    sample contributes) and FP32 weight sum (tile_write); wave-level
-//    synchronisation only, since the other waves of the workgroup work
-//    other tiles or streams;
-//  * NC > 0 (few-channel jobs): as BATCH true, with one FP32 sum per channel
-//    and the outputs written by the tile itself.
+//    job's sorted 16-bit values; the caller adds the streams in stream order
+//    and writes the FP32 cube (divided by the weight sum when the job
+//    normalises; NaN where no sample contributes) and FP32 weight sum
+//    (tile_write);
+//  * NC > 0 (few-channel jobs): as BATCH true, with one FP32 sum per channel.
+// All synchronisation is within the wave, so the waves of a workgroup may
+// work other tiles or streams.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -36,32 +52,6 @@
 #include "common.hpp"
 #include "expneg.hpp"
 #include "healpix.hpp"
-
-#ifndef HCG_GRID_TILE_COLS
-#define HCG_GRID_TILE_COLS 16
-#endif
-#ifndef HCG_GRID_CELLS_PER_LANE
-#define HCG_GRID_CELLS_PER_LANE 1
-#endif
-#ifndef HCG_GRID_STAGE_CAP
-#define HCG_GRID_STAGE_CAP 256
-#endif
-#ifndef HCG_GRID_WAVES_PER_EU
-#define HCG_GRID_WAVES_PER_EU 4
-#endif
-#ifndef HCG_GRID_LANE_LOOP
-// 0: the wave walks the union of its lanes' bands (broadcast LDS reads; lanes
-// outside their band only evaluate the distance); 1: each lane walks its own
-// band (per-lane LDS addresses).  Measured on the 20M raster: 6.69 ms vs 7.14.
-#define HCG_GRID_LANE_LOOP 0
-#endif
-#ifndef HCG_GRID_SMALLR
-#define HCG_GRID_SMALLR 1  // GAUSS1D at R < ~1.1 deg: no series/asin switch, no exp clamp in the inner loop
-#endif
-#ifndef HCG_GRID_TABLE_EXP
-#define HCG_GRID_TABLE_EXP 1
-#endif
-
 
 namespace hcg {
 
@@ -71,12 +61,12 @@ namespace hcg {
 // one block row, and the MFMA path packs ring ranges at this granularity.
 constexpr uint32_t kVB = 8;
 
-constexpr int kTileCols = HCG_GRID_TILE_COLS;
-constexpr int kLaneRows = 64 / kTileCols;
-constexpr int kCellsPerLane = HCG_GRID_CELLS_PER_LANE;
-constexpr int kTileRows = kLaneRows * kCellsPerLane;
-constexpr uint32_t kStageCap = HCG_GRID_STAGE_CAP;
-static_assert(kTileCols * kLaneRows == 64, "tile columns must divide 64");
+constexpr int kTileCols = 16;
+constexpr int kTileRows = 4;
+constexpr uint32_t kPhases = 4;      // lanes that share a column's band
+constexpr uint32_t kStageCap = 256;  // staged samples
+constexpr uint32_t kShortRing = 12;  // a ring's staged samples up to which every column takes them all
+static_assert(kTileCols * kTileRows == 64 && kTileCols * kPhases == 64, "one wave per tile");
 
 }  // namespace hcg
 
@@ -86,21 +76,16 @@ namespace hcg {
 
 // LDS ordering among the lanes of one wave: its LDS instructions execute in
 // issue order, so a compiler fence at wavefront scope is enough.
-template <bool WAVE>
 __device__ inline void tile_sync() {
-  if constexpr (WAVE) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  } else {
-    __syncthreads();
-  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // A one-channel job's values and outputs (BATCH true).
 struct TileOut {
-  const uint16_t* vs;  // sorted values, BF16 or FP16: [n_pad] (one channel), or 32-sample blocked
-                       // [n_pad / 32][nchan][32] (few channels)
+  const uint16_t* vs;  // sorted values, BF16 or FP16: [n_pad] (one channel), or 8-sample blocked
+                       // [n_pad / 8][nchan][8] (few channels)
   float* cube;         // [nchan][side * side]
   float* wsum;         // [side * side] or NULL
   uint32_t bf16;       // vs holds BF16 (else FP16)
@@ -108,14 +93,17 @@ struct TileOut {
   uint32_t nchan;      // channels (few-channel tiles)
 };
 
-// The part of a tile's rings one call of grid_tile walks: rings r_begin +
-// phase, + phase + stride, ... (the whole range: phase 0, stride 1).
+// The part of a tile's non-empty rings one call of grid_tile walks: the
+// phase-th, the phase + stride-th, ... in ascending order (all of them:
+// phase 0, stride 1; stride a power of two).
 struct RingStream {
   uint32_t phase, stride;
 };
 
-// Per-wave LDS of a tile: staged x, y, z, value columns and keys.
-constexpr size_t kTileLdsBytes = (size_t)kStageCap * (4 * sizeof(double) + sizeof(uint32_t));
+// Per-wave LDS of a one-channel tile: staged x, y, z, value columns and keys
+// (of a size that lets four four-wave workgroups share a CU).
+constexpr uint32_t kOneCap = 192;
+constexpr size_t kTileLdsBytes = (size_t)kOneCap * (4 * sizeof(double) + sizeof(uint32_t));
 
 // Tiles of the kTileCols x kTileRows tiling of a side x side map.
 inline uint32_t tile_cols_of(uint32_t side) { return (side + kTileCols - 1) / kTileCols; }
@@ -173,304 +161,629 @@ int launch_tiles_one_channel(const GridParams& P, const GridBuffers& B, const Ti
 // Launches the tile path for one few-channel job: one wave per tile.
 int launch_tiles_few_channels(const GridParams& P, const GridBuffers& B, const TileOut& O, hipStream_t s);
 
-// WMODE (GAUSS1D): 0 general exponent and exp; 1 gauss_small_radius; 2 gauss_tiny_radius; 3 as 2,
-// with the candidate test on p.q (dot_distance_ok).
-// s_exp: the 64-entry exponential table (exp_table_load), visible to the wave.
-//
-// NC > 0 (few-channel tiles, BATCH true): up to NC channels of 16-bit values
-// staged per sample in s_c ([CAP][NC]; s_v unused), one FP32 accumulator per
-// channel and lane, and the cube, weight sum and normalisation written here
-// (no ring streams: S must be {0, 1}).
-template <int KT, bool HAS_W, int WMODE, bool BATCH, int NC = 0, uint32_t CAP = kStageCap>
-__device__ __forceinline__ void grid_tile(const GridParams P, const GridBuffers B, uint32_t tile,
-                                          uint32_t tiles_x, double* __restrict__ s_x, double* __restrict__ s_y,
-                                          double* __restrict__ s_z, double* __restrict__ s_v,
-                                          uint32_t* __restrict__ s_key, const double* __restrict__ s_exp,
-                                          const TileOut& O, RingStream S, double* sum_d, double* sum_w,
-                                          uint16_t* __restrict__ s_c = nullptr) {
-  static_assert(!BATCH || kCellsPerLane == 1, "the one-channel path keeps one cell per lane");
-  static_assert(WMODE != 3 || (kCellsPerLane == 1 && !HCG_GRID_LANE_LOOP && KT == HCG_GAUSS1D),
-                "the p.q candidate test is written for the one-cell-per-lane GAUSS1D loop");
-  static_assert(NC == 0 || (BATCH && NC % 2 == 0), "few-channel tiles: an even channel count, batch outputs");
-  // the p.q loop with one value per sample: the lean weight and the guard
-  // band handled after it (below)
-  constexpr bool kLean = WMODE == 3 && NC == 0;
-  float acc_c[NC > 0 ? NC : 1];
-#pragma unroll
-  for (int ch = 0; ch < (NC > 0 ? NC : 1); ++ch) acc_c[ch] = 0.0f;
-  const hcg_ring_meta m = *B.meta;
-  if constexpr (!BATCH) {
-    if (m.usedrings == 0) return;
+// ---- the quad of lanes that share a column (DPP, no LDS traffic) ----
+
+template <int CTRL>
+__device__ inline uint32_t quad_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ inline double quad_f64(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t)quad_u32<CTRL>((uint32_t)u) |
+                                        ((uint64_t)quad_u32<CTRL>((uint32_t)(u >> 32)) << 32));
+}
+template <int CTRL>
+__device__ inline float quad_f32(float v) {
+  return __builtin_bit_cast(float, quad_u32<CTRL>(__builtin_bit_cast(uint32_t, v)));
+}
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int quad_bcast(int r) { return r * 0x55; }
+// v[r] = x of the quad's lane r, r < ROWS
+template <int ROWS>
+__device__ inline void quad_all(uint32_t x, uint32_t (&v)[ROWS]) {
+  v[0] = ROWS == 1 ? x : quad_u32<quad_bcast(0)>(x);
+  if constexpr (ROWS > 1) v[1] = quad_u32<quad_bcast(1)>(x);
+  if constexpr (ROWS > 2) {
+    v[2] = quad_u32<quad_bcast(2)>(x);
+    v[3] = quad_u32<quad_bcast(3)>(x);
   }
+}
+template <int ROWS>
+__device__ inline void quad_all(double x, double (&v)[ROWS]) {
+  v[0] = ROWS == 1 ? x : quad_f64<quad_bcast(0)>(x);
+  if constexpr (ROWS > 1) v[1] = quad_f64<quad_bcast(1)>(x);
+  if constexpr (ROWS > 2) {
+    v[2] = quad_f64<quad_bcast(2)>(x);
+    v[3] = quad_f64<quad_bcast(3)>(x);
+  }
+}
+// row `row`'s sum over the quad
+template <int ROWS>
+__device__ inline double quad_rows_sum(const double (&v)[ROWS], uint32_t row) {
+  double out = 0.0;
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    double t = v[r] + quad_f64<kQuadXor1>(v[r]);
+    t += quad_f64<kQuadXor2>(t);
+    if (r == 0 || row == (uint32_t)r) out = t;
+  }
+  return out;
+}
+template <int ROWS>
+__device__ inline float quad_rows_sum(const float (&v)[ROWS], uint32_t row) {
+  float out = 0.f;
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    float t = v[r] + quad_f32<kQuadXor1>(v[r]);
+    t += quad_f32<kQuadXor2>(t);
+    if (r == 0 || row == (uint32_t)r) out = t;
+  }
+  return out;
+}
+
+// The windows of a tile taken together, for the ring ranges: the span of the
+// longitudes (compat) and of the longitude ranges (polar, disc) of its cells.
+struct TileSpan {
+  uint32_t r_begin, r_end;     // rings (r_begin > r_end: none)
+  bool any_compat, any_range;  // some cell has a window of that kind
+  bool whole;                  // some cell takes whole rings, or longitudes are not in [0, 2 pi)
+  double tl, tr;               // the outermost compat window edges (units of pi/2, not reduced)
+  float tlo, thi;              // outermost ranges
+  bool disc;                   // HCG_SELECT_DISC
+};
+
+__device__ inline TileSpan tile_span(const GridParams& P, const Window& w, uint32_t firstring) {
+  TileSpan t;
+  const bool has = w.uring <= w.dring;
+  t.r_begin = wave_min_u32(has ? w.uring : 0xFFFFFFFFu);
+  t.r_end = wave_max_u32(has ? w.dring : 0u);
+  if (t.r_begin == firstring && skips_first_ring(P)) ++t.r_begin;  // the first used ring contributes nothing
+  const bool compat = has && w.mode == kWinCompat, range = has && w.mode != kWinCompat;
+  t.any_compat = __ballot(compat) != 0;
+  t.any_range = __ballot(range) != 0;
+  t.disc = P.selection == HCG_SELECT_DISC;
+  t.whole = false;
+  t.tl = t.tr = 0.0;
+  t.tlo = 1.f;
+  t.thi = 0.f;
+  if (t.any_compat) {
+    const double lo = wave_min_f64(compat ? w.phi : 1e300);
+    const double hi = -wave_min_f64(compat ? -w.phi : 1e300);
+    t.whole = !(lo >= 0.0 && hi < 2.0 * kPi);
+    t.tl = (lo - P.disc_size) * kInvHalfPi;
+    t.tr = (hi + P.disc_size) * kInvHalfPi;
+  }
+  if (t.any_range) {
+    t.whole = t.whole || __ballot(range && !(w.range.tlo <= w.range.thi)) != 0;
+    t.tlo = (float)wave_min_f64(range ? (double)w.range.tlo : 1e300);
+    t.thi = (float)-wave_min_f64(range ? -(double)w.range.thi : 1e300);
+  }
+  return t;
+}
+
+// A pixel range of ring r that holds every cell's window in it (ring_window):
+// a ring's pixel index grows with the longitude, so the outermost edges bound
+// the others; two pixels of margin.  Within three pixels of longitude 0 an
+// edge opens to the ring's end (a cell whose own window wraps through 0
+// selects nothing, since its lpix is then past its rpix), and whole rings
+// are taken where the reasoning ends.
+__device__ inline void span_pixels(const GridParams& P, const TileSpan& t, uint32_t ring, double rz, double rs,
+                                   uint32_t& lp, uint32_t& rp) {
+  const Hpx32 hx = hpx32(P.hp);
+  uint32_t sp, npr;
+  ring_info32(hx, ring, sp, npr);
+  const uint32_t last = sp + npr - 1;
+  lp = sp;
+  rp = last;
+  const bool cap = ring < hx.nside || ring > 3 * hx.nside;
+  if (t.whole || (t.any_range && !cap && !t.disc)) return;
+  uint32_t a = last, b = sp;
+  if (t.any_compat) {
+    const bool have = rs >= 0.0;
+    const double q = (double)(npr >> 2);
+    a = sp;
+    b = last;
+    if (t.tl * q > 3.0) {
+      const uint32_t l = loc2pix32(hx, rz, t.tl, have ? rs : 0., have);
+      if (l - sp >= npr) return;
+      a = l - sp < 2 ? sp : l - 2;
+    }
+    if (t.tr * q < (double)npr - 3.0) {
+      const uint32_t r = loc2pix32(hx, rz, t.tr, have ? rs : 0., have);
+      if (r - sp >= npr) return;
+      b = last - r < 2 ? last : r + 2;
+    }
+  }
+  if (t.any_range) {
+    const float q = (float)(npr >> 2);
+    const int32_t m = t.disc ? 4 : 3;
+    const int32_t lo = (int32_t)floorf(t.tlo * q) - m;
+    const int32_t hi = (int32_t)floorf(t.thi * q) + m;
+    if (lo < 0 || hi >= (int32_t)npr) return;
+    a = min(a, sp + (uint32_t)lo);
+    b = max(b, sp + (uint32_t)hi);
+  }
+  lp = a;
+  rp = b;
+}
+
+// The sorted range of ring rb + lane's part of the tile (lo_l >= hi_l: none).
+__device__ inline void ring_ranges(const GridParams& P, const GridBuffers& B, const TileSpan& T, const hcg_ring_meta& m,
+                                   uint32_t rb, uint32_t& lo_l, uint32_t& hi_l) {
+  lo_l = hi_l = 0;
   const uint32_t lane = __lane_id();
-  const uint32_t col = (tile % tiles_x) * kTileCols + lane / kLaneRows;
-  const uint32_t row0 = (tile / tiles_x) * kTileRows + (lane % kLaneRows) * kCellsPerLane;
-
-  uint32_t cell[kCellsPerLane];
-  double px[kCellsPerLane], py[kCellsPerLane], pz[kCellsPerLane];
-  double acc_d[kCellsPerLane], acc_w[kCellsPerLane];
-  Window win[kCellsPerLane];
-  uint32_t lane_ur = 0xFFFFFFFFu, lane_dr = 0;
-#pragma unroll
-  for (int k = 0; k < kCellsPerLane; ++k) {
-    const uint32_t row = row0 + k;
-    const bool live = (col < P.side) && (row < P.side);
-    const uint32_t rr = live ? row : 0, cc = live ? col : 0;
-    cell[k] = rr * P.side + cc;
-    const uint32_t anchor = rr * P.side + (cc / P.factor) * P.factor;
-    win[k] = window_of(P, m.firstring, m.usedrings, B.xwcs[anchor], B.ywcs[anchor]);
-    if (!live || (BATCH && m.usedrings == 0)) {  // an empty ring range: never active
-      win[k].uring = 1;
-      win[k].dring = 0;
-    }
-    double sb, cb, sl, cl;
-    sincos(B.ywcs[cell[k]] * kDeg2Rad, &sb, &cb);
-    sincos(B.xwcs[cell[k]] * kDeg2Rad, &sl, &cl);
-    px[k] = cb * cl;
-    py[k] = cb * sl;
-    pz[k] = sb;
-    if constexpr (BATCH) {
-      acc_d[k] = 0.0;
-      acc_w[k] = 0.0;
-    } else {
-      acc_d[k] = live ? B.dc[cell[k]] : 0.0;
-      acc_w[k] = live ? B.wc[cell[k]] : 0.0;
-    }
-    if (win[k].uring <= win[k].dring) {
-      lane_ur = min(lane_ur, win[k].uring);
-      lane_dr = max(lane_dr, win[k].dring);
+  if (T.r_begin <= T.r_end && rb + lane <= T.r_end) {
+    const uint32_t kr = rb + lane - m.firstring;
+    const uint32_t start = B.lut[kr], end = B.lut[kr + 1];
+    if (start < end) {
+      uint32_t lp, rp;
+      span_pixels(P, T, rb + lane, B.ring_z[kr], B.ring_s[kr], lp, rp);
+      // both bounds in one loop, three probes each a step: a step is one
+      // round of dependent loads, and the range falls to a quarter
+      uint32_t a0 = start, a1 = end, b0 = start, b1 = end;
+      while (a0 < a1 || b0 < b1) {
+        const uint32_t da = (a1 - a0) >> 2, db = (b1 - b0) >> 2;
+        // a0 <= pa0 <= pa1 <= pa2 < a1 while the range is not empty; index
+        // `end` of an empty one can be read (keys[n] is the sentinel)
+        const uint32_t pa0 = a0 + da, pa1 = a0 + ((a1 - a0) >> 1), pa2 = pa1 + da;
+        const uint32_t pb0 = b0 + db, pb1 = b0 + ((b1 - b0) >> 1), pb2 = pb1 + db;
+        const uint32_t ka0 = B.keys[pa0], ka1 = B.keys[pa1], ka2 = B.keys[min(pa2, end)];
+        const uint32_t kb0 = B.keys[pb0], kb1 = B.keys[pb1], kb2 = B.keys[min(pb2, end)];
+        if (a0 < a1) {
+          if (pa2 < a1 && ka2 < lp)
+            a0 = pa2 + 1;
+          else if (ka1 < lp)
+            a0 = pa1 + 1, a1 = min(a1, pa2);
+          else if (ka0 < lp)
+            a0 = pa0 + 1, a1 = pa1;
+          else
+            a1 = pa0;
+        }
+        if (b0 < b1) {
+          if (pb2 < b1 && kb2 <= rp)
+            b0 = pb2 + 1;
+          else if (kb1 <= rp)
+            b0 = pb1 + 1, b1 = min(b1, pb2);
+          else if (kb0 <= rp)
+            b0 = pb0 + 1, b1 = pb1;
+          else
+            b1 = pb0;
+        }
+      }
+      lo_l = a0;
+      hi_l = b0;
     }
   }
-  uint32_t r_begin = wave_min_u32(lane_ur);
-  const uint32_t r_end = wave_max_u32(lane_dr);
-  if (r_begin == m.firstring && skips_first_ring(P)) ++r_begin;  // the first used ring contributes nothing
+}
 
-  for (uint32_t r = r_begin + S.phase; r <= r_end && r_begin <= r_end; r += S.stride) {
-    const uint32_t kr = r - m.firstring;
-    const uint32_t start = B.lut[kr], end = B.lut[kr + 1];
-    if (start == end) continue;
-    const double rz = B.ring_z[kr], rs = B.ring_s[kr];
-    uint32_t lp[kCellsPerLane], rp[kCellsPerLane];
-    uint32_t lane_lp = 0xFFFFFFFFu, lane_rp = 0;
+// First index in [from, from + cnt) with g >= x (from + cnt if none), in
+// halving steps that are uniform over the wave (cnt > 0).
+__device__ inline uint32_t band_search(const uint32_t* __restrict__ g, uint32_t from, uint32_t cnt, uint32_t x) {
+  uint32_t a = 0;
+  for (uint32_t s = 1u << (31 - __builtin_clz(cnt)); s; s >>= 1) {
+    const uint32_t i = a + s;
+    const uint32_t v = g[from + min(i, cnt) - 1];
+    if (i <= cnt && v < x) a = i;
+  }
+  return from + a;
+}
+
+// Inclusive maximum over the lanes up to this one.
+__device__ inline uint32_t wave_scan_max_u32(uint32_t v) {
+  v = max(v, dpp_u32<kRowShr1, 0xF>(0u, v));
+  v = max(v, dpp_u32<kRowShr2, 0xF>(0u, v));
+  v = max(v, dpp_u32<kRowShr4, 0xF>(0u, v));
+  v = max(v, dpp_u32<kRowShr8, 0xF>(0u, v));
+  v = max(v, dpp_u32<kRowBcast15, 0xA>(0u, v));
+  return max(v, dpp_u32<kRowBcast31, 0xC>(0u, v));
+}
+
+// A cell's window in a ring, in half pixels: sample (pixel p of ring r, p
+// counted from the ring's first) is in it when g - lo <= hi - lo (unsigned),
+// g = 2 p + 1 - (r odd).
+//
+// In a belt ring (nside < r < 3 nside) pixel boundaries lie at longitudes tt
+// (units of pi/2) whose nside tt is an integer for even r and a half-integer
+// for odd r: the formulas of HCGrid/healpix.cu:126-205 at the ring's centre
+// give p = floor(nside tt) and floor(nside tt + 1/2).  With h = floor(2 nside
+// tt), an edge at tt lies in pixel floor(h / 2) or floor((h + 1) / 2), and a
+// window from tl to tr holds the samples with hl <= g <= hr + 1 whatever the
+// ring's parity.  So a compat window is one pair of numbers for every belt
+// ring.  Exact unless an edge is within rounding of a boundary (2 nside tt
+// within 1e-6 of an integer; the formulas' own error is below 1e-10), or the
+// window meets longitude 0: then (returns false) the tile evaluates its
+// windows ring by ring.
+constexpr uint32_t kNoWindow = 0x80000001u;  // lo of a cell outside the ring's range: no g reaches it
+__device__ inline bool belt_window(const GridParams& P, double tl, double tr, uint32_t& lo, uint32_t& hi) {
+  const uint32_t ns = (uint32_t)P.hp.nside;
+  const double xl = 2.0 * (double)ns * tl, xr = 2.0 * (double)ns * tr;
+  const double fl = floor(xl), fr = floor(xr);
+  lo = (uint32_t)fl;
+  hi = (uint32_t)fr + 1;
+  const double gl = xl - fl, gr = xr - fr;
+  return ns >= 2 && gl > 1e-6 && gl < 1.0 - 1e-6 && gr > 1e-6 && gr < 1.0 - 1e-6 && xl < xr &&
+         xr < 8.0 * (double)ns - 2.0;
+}
+
+__device__ inline float high_f32(double x) {
+  return __builtin_bit_cast(float, (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32));
+}
+
+// A tile's sums, one cell per lane (column lane / 4, row lane % 4).
+template <int NC>
+struct TileSums {
+  double d, w;
+  float c[NC > 0 ? NC : 1];
+};
+
+// Step 1 and 2 of a tile, for the other waves of its workgroup.
+struct TileShared {
+  Window win[64];
+  double tl[64], tr[64], p[3][64];
+  uint32_t lo[64], hi[64];
+  TileSpan T;
+};
+
+// WMODE (GAUSS1D): 0 general exponent and exp; 1 gauss_small_radius; 2
+// gauss_tiny_radius; 3 also lean_weight_ok (the candidate test on p.q and
+// the lean weight).
+// lds: CAP x (x, y, z, v doubles, key), with HAS_W then CAP weights; with NC
+// > 0 CAP x (x, y, z doubles, key, NC 16-bit values).
+// s_exp: the 64-entry exponential table (exp_table_load), visible to the wave.
+// ROWS: map rows of the tile (4; fewer on small maps, for more tiles).
+// SHARED: the waves of the workgroup walk streams of the same tile; wave 0
+// works out the windows and ring ranges and the others take them from `sh`
+// (holds a workgroup barrier).
+template <int KT, bool HAS_W, int WMODE, bool BATCH, int NC, uint32_t CAP, int ROWS = kTileRows, bool SHARED = false>
+__device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers& B, uint32_t tile, uint32_t tiles_x,
+                                          char* __restrict__ lds, const double* __restrict__ s_exp, const TileOut& O,
+                                          RingStream S, TileSums<NC>& out, TileShared* sh = nullptr) {
+  static_assert(NC == 0 || (BATCH && NC % 2 == 0 && WMODE == 3), "few-channel tiles: even counts, the lean weight");
+  static_assert(WMODE != 3 || KT == HCG_GAUSS1D, "the lean weight is GAUSS1D's");
+  static_assert(!(HAS_W && BATCH), "batch jobs carry no sample weights");
+  double* const s_x = reinterpret_cast<double*>(lds);
+  double* const s_y = s_x + CAP;
+  double* const s_z = s_y + CAP;
+  double* const s_v = s_z + CAP;                                   // NC == 0
+  double* const s_w = s_v + CAP;                                   // HAS_W
+  uint32_t* const s_g = reinterpret_cast<uint32_t*>(NC > 0 ? s_v : HAS_W ? s_w + CAP : s_w);
+  uint16_t* const s_c = reinterpret_cast<uint16_t*>(s_g + CAP);  // NC > 0
+
+  const hcg_ring_meta m = *B.meta;
+  const uint32_t lane = __lane_id();
+  const uint32_t row = lane & (ROWS - 1u);  // this lane's row as a cell
+  const uint32_t phase = lane & 3u;         // and its phase in the sample loop
+  const uint32_t col = (tile % tiles_x) * kTileCols + (lane >> 2);
+  const uint32_t row0 = (tile / tiles_x) * ROWS;
+
+  double npx[ROWS], npy[ROWS], npz[ROWS], acc_d[ROWS], acc_w[ROWS];
+  float acc_c[ROWS][NC > 0 ? NC : 1];
 #pragma unroll
-    for (int k = 0; k < kCellsPerLane; ++k) {
-      uint32_t a = 1, b = 0;
-      const bool act = r >= win[k].uring && r <= win[k].dring && ring_window(P, win[k], r, rz, rs, a, b) && a <= b;
-      lp[k] = act ? a : 1u;  // inactive: the empty window [1, 0]
-      rp[k] = act ? b : 0u;
-      if (act) {
-        lane_lp = min(lane_lp, lp[k]);
-        lane_rp = max(lane_rp, rp[k]);
+  for (int r = 0; r < ROWS; ++r) {
+    acc_d[r] = acc_w[r] = 0.0;
+#pragma unroll
+    for (int c = 0; c < (NC > 0 ? NC : 1); ++c) acc_c[r][c] = 0.f;
+  }
+  Window win;
+  double tl = 0.0, tr = 0.0;  // compat: the window's edges, fmodulo4 in units of pi/2
+  TileSpan T;
+  uint32_t lo_r, hi_r;  // lane = ring: the ranges of the first 64 rings
+  {
+    double px, py, pz;
+    if (!SHARED || threadIdx.x < 64) {
+      const bool live = col < P.side && row0 + row < P.side;
+      const uint32_t rr = live ? row0 + row : 0, cc = live ? col : 0;
+      const uint32_t cell = rr * P.side + cc;
+      const uint32_t anchor = rr * P.side + (cc / P.factor) * P.factor;
+      win = window_of(P, m.firstring, m.usedrings, B.xwcs[anchor], B.ywcs[anchor]);
+      if (!live || m.usedrings == 0) {  // an empty ring range: never active
+        win.uring = 1;
+        win.dring = 0;
+      }
+      if (win.mode == kWinCompat) compat_edges(P, win, tl, tr);
+      double sb, cb, sl, cl;
+      sincos(B.ywcs[cell] * kDeg2Rad, &sb, &cb);
+      sincos(B.xwcs[cell] * kDeg2Rad, &sl, &cl);
+      px = cb * cl;
+      py = cb * sl;
+      pz = sb;
+      T = tile_span(P, win, m.firstring);
+      ring_ranges(P, B, T, m, T.r_begin, lo_r, hi_r);
+    }
+    if constexpr (SHARED) {
+      TileShared& H = *sh;
+      if (threadIdx.x < 64) {
+        H.win[lane] = win;
+        H.tl[lane] = tl;
+        H.tr[lane] = tr;
+        H.p[0][lane] = px;
+        H.p[1][lane] = py;
+        H.p[2][lane] = pz;
+        H.lo[lane] = lo_r;
+        H.hi[lane] = hi_r;
+        if (lane == 0) H.T = T;
+      }
+      __syncthreads();
+      if (threadIdx.x >= 64) {
+        win = H.win[lane];
+        tl = H.tl[lane];
+        tr = H.tr[lane];
+        px = H.p[0][lane];
+        py = H.p[1][lane];
+        pz = H.p[2][lane];
+        lo_r = H.lo[lane];
+        hi_r = H.hi[lane];
+        T = H.T;
+        T.r_begin = __builtin_amdgcn_readfirstlane(T.r_begin);
+        T.r_end = __builtin_amdgcn_readfirstlane(T.r_end);
       }
     }
-    const uint32_t LP = wave_min_u32(lane_lp), RP = wave_max_u32(lane_rp);
-    if (LP > RP) continue;
-    const uint32_t lo_u = wave_search<false>(B.keys, start, end, LP);
-    const uint32_t hi_u = wave_search<true>(B.keys, lo_u, end, RP);
-    for (uint32_t cb = lo_u; cb < hi_u; cb += CAP) {
-      const uint32_t cnt = min(CAP, hi_u - cb);
-      tile_sync<BATCH>();  // previous chunk fully consumed
-      for (uint32_t j = lane; j < cnt; j += 64) {
-        const hcg_sample q = B.rec[cb + j];
-        s_x[j] = q.x;
-        s_y[j] = q.y;
-        s_z[j] = q.z;
-        if constexpr (NC > 0)
-          ;  // channel values below
-        else if constexpr (BATCH)
-          s_v[j] = (double)widen16(O.vs[cb + j], O.bf16 != 0);
-        else
-          s_v[j] = q.v;
-        s_key[j] = B.keys[cb + j];
+    // -p: h = 1 - p.q is three FMAs from 1
+    quad_all(-px, npx);
+    quad_all(-py, npy);
+    quad_all(-pz, npz);
+  }
+  uint32_t hl0 = 0, hh0 = 0;  // the cell's window in every belt ring (belt_window)
+  const bool has = win.uring <= win.dring;
+  const bool belt_ok = __ballot(has && !(win.mode == kWinCompat && belt_window(P, tl, tr, hl0, hh0))) == 0;
+  const uint32_t ns = (uint32_t)P.hp.nside;
+  // WMODE 3: the tests on h = 1 - p.q = c2 / 2 (halving is exact, so
+  // h < c_hi / 2 <=> c2 < c_hi)
+  const double t_hi = WMODE == 3 ? 0.5 * P.c_hi : P.c_hi, t_lo = WMODE == 3 ? 0.5 * P.c_lo : P.c_lo;
+  // With sample weights the pairs are tested on the high words of the
+  // distances, compared as floats (a double's high word is its order, NaN
+  // included): below t_lo32 selected, above t_hi32 not, and a lane between the
+  // two (a relative 1e-6 of the radius around the guard band) is decided
+  // exactly.  The 347^2 map with weights took 1160 us with these compares and
+  // 1282 us with 64-bit ones; without weights the 64-bit ones are the faster
+  // (20M samples: 3421 against 3527 us).
+  constexpr bool kHigh = HAS_W;
+  const float t_lo32 = high_f32(t_lo), t_hi32 = high_f32(t_hi);
+  // the lean weight's constants for y = h (2 k0 + 4 k1 h), which equals
+  // c2 (k0 + k1 c2); k1 and kExpE3 in vector registers (hoisted out of the loops)
+  const double k0h = 2.0 * P.k0;
+  const double k1v = WMODE == 3 ? in_vgprs(4.0 * P.k1) : 0.0, e3v = WMODE == 3 ? in_vgprs(kExpE3) : 0.0;
+  uint32_t seen = 0;  // non-empty rings before this round
+
+  for (uint32_t rb = T.r_begin; rb <= T.r_end && T.r_begin <= T.r_end; rb += 64) {
+    // lane = ring
+    uint32_t lo_l = lo_r, hi_l = hi_r;
+    if (rb != T.r_begin) ring_ranges(P, B, T, m, rb, lo_l, hi_l);  // (more than 64 rings)
+    const uint64_t ne = __ballot(lo_l < hi_l);
+    const uint32_t rank = seen + (uint32_t)__popcll(ne & lanemask_lt());
+    uint64_t mine = __ballot(lo_l < hi_l && (rank & (S.stride - 1u)) == S.phase);
+    seen += (uint32_t)__popcll(ne);
+    // of this lane's ring: g = 2 key + gc
+    uint32_t gc;
+    {
+      uint32_t sp, npr;
+      ring_info32(hpx32(P.hp), rb + lane, sp, npr);
+      gc = 1u - ((rb + lane) & 1u) - 2u * sp;
+    }
+    while (mine) {  // uniform
+      // A chunk: whole rings while they fit in CAP, or a piece of a longer
+      // one.  On sparse maps it holds many rings, and one round of loads
+      // serves them all.
+      uint32_t cnt = 0, first = 0;
+      uint32_t seg_off = 0, seg_len = 0, seg_src = 0;  // this lane's ring in the chunk
+      uint64_t in = 0;                                 // the chunk's rings
+      while (mine) {
+        const uint32_t k = (uint32_t)__ffsll((unsigned long long)mine) - 1u;
+        const uint32_t lo_u = __builtin_amdgcn_readlane(lo_l, k), hi_u = __builtin_amdgcn_readlane(hi_l, k);
+        if (cnt != 0 && hi_u - lo_u > CAP - cnt) break;
+        const uint32_t take = min(hi_u - lo_u, CAP);
+        if (lane == k) {
+          seg_off = cnt;
+          seg_len = take;
+          seg_src = lo_u;
+          lo_l = lo_u + take;
+        }
+        if (cnt == 0) first = k;
+        in |= 1ull << k;
+        cnt += take;
+        if (take < hi_u - lo_u) break;
+        mine &= mine - 1;
       }
-      if constexpr (NC > 0) {
-        // channel by channel: lanes read consecutive samples of one channel
-        // (contiguous within a kVB-sample block); slots past nchan hold 0
-        for (uint32_t ch = 0; ch < (uint32_t)NC; ++ch) {
-          const bool have = ch < O.nchan;
-          for (uint32_t j = lane; j < cnt; j += 64) {
-            const uint32_t i = cb + j;
-            s_c[j * NC + ch] = have ? O.vs[((size_t)(i / kVB) * O.nchan + ch) * kVB + (i % kVB)] : (uint16_t)0;
+      const bool one_ring = (in & (in - 1)) == 0;
+      tile_sync();  // previous chunk fully consumed
+      if (!one_ring) {
+        // each ring marks its first position; a position's ring is the last mark at or before it
+        for (uint32_t p = lane; p < cnt; p += 64) s_g[p] = 0;
+        tile_sync();
+        if (in >> lane & 1u) s_g[seg_off] = lane + 1;
+        tile_sync();
+      }
+      const uint32_t base1 = __builtin_amdgcn_readlane(seg_src, first), gc1 = __builtin_amdgcn_readlane(gc, first);
+      uint32_t carry = 0;
+      for (uint32_t p0 = 0; p0 < cnt; p0 += 128) {  // uniform; two positions per lane in flight
+        uint32_t src[2], sgc[2];
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+          const uint32_t p = p0 + 64 * i + lane;
+          src[i] = base1 + min(p, cnt - 1);
+          sgc[i] = gc1;
+          if (!one_ring && p0 + 64 * i < cnt) {  // uniform
+            const uint32_t k1 = max(carry, wave_scan_max_u32(p < cnt ? s_g[p] : 0u));
+            carry = (uint32_t)__builtin_amdgcn_readlane((int)k1, 63);
+            const int from = (int)((k1 - 1) * 4);
+            src[i] = min(p, cnt - 1) + (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)(seg_src - seg_off));
+            sgc[i] = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)gc);
+          }
+        }
+        hcg_sample q[2];
+        uint32_t key[2];
+        double ws[2];
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i)
+          if (p0 + 64 * i < cnt) {  // uniform
+            q[i] = B.rec[src[i]];
+            key[i] = B.keys[src[i]];
+            if constexpr (BATCH && NC == 0) q[i].v = (double)widen16(O.vs[src[i]], O.bf16 != 0);
+            if constexpr (HAS_W) ws[i] = B.w_s[src[i]];
+          }
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+          const uint32_t j = p0 + 64 * i + lane;
+          if (j < cnt) {
+            s_x[j] = q[i].x;
+            s_y[j] = q[i].y;
+            s_z[j] = q[i].z;
+            if constexpr (HAS_W) {  // the value times its weight, and the weight: one FMA each per pair
+              s_v[j] = q[i].v * ws[i];
+              s_w[j] = ws[i];
+            } else if constexpr (NC == 0) {
+              s_v[j] = q[i].v;
+            }
+            s_g[j] = 2 * key[i] + sgc[i];
+            if constexpr (NC > 0) {
+              // a sample's channels are kVB values apart; slots past nchan hold 0
+              const uint16_t* v = O.vs + (size_t)(src[i] / kVB) * O.nchan * kVB + (src[i] % kVB);
+#pragma unroll
+              for (uint32_t ch = 0; ch < (uint32_t)NC; ++ch) s_c[j * NC + ch] = ch < O.nchan ? v[ch * kVB] : (uint16_t)0;
+            }
           }
         }
       }
-      tile_sync<BATCH>();
-      uint32_t lo[kCellsPerLane], len[kCellsPerLane];
-      uint32_t jb = 0xFFFFFFFFu, je = 0;
-#pragma unroll
-      for (int k = 0; k < kCellsPerLane; ++k) {
-        const uint32_t a = lower_bound_u32(s_key, 0, cnt, lp[k]);
-        const uint32_t b = (lp[k] <= rp[k]) ? upper_bound_u32(s_key, a, cnt, rp[k]) : a;
-        lo[k] = a;
-        len[k] = b - a;
-        if (b > a) {
-          jb = min(jb, a);
-          je = max(je, b);
+      tile_sync();
+      for (; in; in &= in - 1) {  // the chunk's rings, uniform
+        const uint32_t k = (uint32_t)__ffsll((unsigned long long)in) - 1u;
+        const uint32_t r = rb + k;
+        const uint32_t off = __builtin_amdgcn_readlane(seg_off, k), n_r = __builtin_amdgcn_readlane(seg_len, k);
+        // this lane's cell's window in the ring
+        bool act = r >= win.uring && r <= win.dring;
+        uint32_t wl = hl0, wh = hh0;
+        if (!(belt_ok && r > ns && r < 3 * ns)) {  // uniform
+          const uint32_t kr = r - m.firstring;
+          uint32_t a = 0, b = 0;
+          act = act && ring_window_at(P, win, tl, tr, r, B.ring_z[kr], B.ring_s[kr], a, b) && a <= b;
+          wl = 2 * a + (uint32_t)__builtin_amdgcn_readlane(gc, k);
+          wh = 2 * b + (uint32_t)__builtin_amdgcn_readlane(gc, k);
         }
-      }
-#if HCG_GRID_LANE_LOOP
-      // each lane walks its own band: the trip count is the wave's longest
-      // band, not the bands' union (over half of which a lane would skip);
-      // per cell the samples are still taken in sorted order
-      uint32_t tmax = 0;
+        const uint64_t live = __ballot(act);
+        if (live == 0) continue;  // uniform
+        uint32_t hl[ROWS], hw[ROWS];
+        quad_all(act ? wl : kNoWindow, hl);
+        quad_all(act ? wh - wl : 0u, hw);
+        // the column's samples: all of a short segment, else from the first
+        // lower edge to the last upper edge of its four cells (lanes 0 and 1
+        // of the quad search the one, 2 and 3 the other)
+        uint32_t jb = off, je = off + n_r;
+        if (n_r > kShortRing) {
+          uint32_t lo = act ? wl : 0xFFFFFFFFu, hi = act ? wh + 1 : 0u;
+          lo = min(lo, quad_u32<kQuadXor1>(lo));
+          lo = min(lo, quad_u32<kQuadXor2>(lo));
+          hi = max(hi, quad_u32<kQuadXor1>(hi));
+          hi = max(hi, quad_u32<kQuadXor2>(hi));
+          const uint32_t at = band_search(s_g, off, n_r, phase < 2 ? lo : hi);
+          jb = quad_u32<quad_bcast(0)>(at);
+          je = quad_u32<quad_bcast(2)>(at);
+        }
+        constexpr uint64_t kRow = ROWS == 1 ? ~0ull : ROWS == 2 ? 0x5555555555555555ull : 0x1111111111111111ull;
+        const uint32_t src0 = (uint32_t)__builtin_amdgcn_readlane(seg_src, k) - off;  // sorted index of position 0
+        for (uint32_t j = jb + phase; j < je; j += kPhases) {
+          const double qx = s_x[j], qy = s_y[j], qz = s_z[j];
+          const uint32_t qg = s_g[j];
+          double qv = 0.0, qw = 1.0;
+          if constexpr (NC == 0) qv = s_v[j];
+          if constexpr (HAS_W) qw = s_w[j];
+          float cv[NC > 0 ? NC : 1];
+          if constexpr (NC > 0) {
+            // two channels per 32-bit LDS word; the value type is the job's (a uniform branch)
+            const uint32_t* w2 = reinterpret_cast<const uint32_t*>(s_c + j * NC);
 #pragma unroll
-      for (int k = 0; k < kCellsPerLane; ++k) tmax = max(tmax, len[k]);
-      tmax = wave_max_u32(tmax);
-      (void)jb;
-      (void)je;
-      for (uint32_t t = 0; t < tmax; ++t) {
-#pragma unroll
-        for (int k = 0; k < kCellsPerLane; ++k) {
-          if (t >= len[k]) continue;
-          const uint32_t j = lo[k] + t;
-          const double qx = s_x[j], qy = s_y[j], qz = s_z[j], qv = s_v[j];
-          const double dx = px[k] - qx, dy = py[k] - qy, dz = pz[k] - qz;
-          const double c2 = fma(dx, dx, fma(dy, dy, dz * dz));
-          if (c2 < P.c_hi) {
-            const double gq = c2, glo = P.c_lo;
-#elif HCG_GRID_CELLS_PER_LANE == 1
-      // one cell per lane: its band is exactly [lo, lo + len)
-      (void)jb;
-      (void)je;
-      // WMODE 3: the tests on h = 1 - p.q = c2 / 2 (halving is exact, so
-      // h < c_hi / 2 <=> c2 < c_hi); -p in registers, so h is three FMAs
-      const double h_hi = 0.5 * P.c_hi, h_lo = 0.5 * P.c_lo;
-      const double npx = -px[0], npy = -py[0], npz = -pz[0];
-      (void)h_hi;
-      (void)npx;
-      (void)npy;
-      (void)npz;
-      // the lean weight's constants for y = h (2 k0 + 4 k1 h), which equals
-      // c2 (k0 + k1 c2) bit for bit: k1 and kExpE3 in vector registers
-      // (hoisted out of the loops)
-      const double k0h = 2.0 * P.k0;
-      const double k1v = WMODE == 3 ? in_vgprs(4.0 * P.k1) : 0.0, e3v = WMODE == 3 ? in_vgprs(kExpE3) : 0.0;
-      (void)k0h;
-      (void)k1v;
-      (void)e3v;
-      for (uint32_t t = 0; t < len[0]; ++t) {
-        const uint32_t j = lo[0] + t;
-        const double qx = s_x[j], qy = s_y[j], qz = s_z[j], qv = NC > 0 ? 0.0 : s_v[j];
-        {
-          constexpr int k = 0;
-          // WMODE 3: the candidate test on h = 1 - p.q (three FP64
-          // operations instead of seven); otherwise c2 = |p - q|^2
-          double c2, h = 0.0;
-          if constexpr (WMODE == 3) {
-            h = fma(npx, qx, fma(npy, qy, fma(npz, qz, 1.0)));
-          } else {
-            const double dx = px[k] - qx, dy = py[k] - qy, dz = pz[k] - qz;
-            c2 = fma(dx, dx, fma(dy, dy, dz * dz));
-          }
-          if (WMODE == 3 ? h < h_hi : c2 < P.c_hi) {
-            if constexpr (WMODE == 3) c2 = 2.0 * h;
-            const double gq = WMODE == 3 ? h : c2, glo = WMODE == 3 ? h_lo : P.c_lo;
-#else
-      for (uint32_t j = jb; j < je; ++j) {
-        const double qx = s_x[j], qy = s_y[j], qz = s_z[j], qv = s_v[j];
-#pragma unroll
-        for (int k = 0; k < kCellsPerLane; ++k) {
-          const double dx = px[k] - qx, dy = py[k] - qy, dz = pz[k] - qz;
-          const double c2 = fma(dx, dx, fma(dy, dy, dz * dz));
-          if ((j - lo[k]) < len[k] && c2 < P.c_hi) {
-            const double gq = c2, glo = P.c_lo;
-#endif
-            if constexpr (kLean) {
-              // every candidate's weight; a lane in the guard band (rare, and
-              // wave-uniformly skipped) that the reference's test rejects then
-              // adds zero: one compare and no lane mask in the common case
-              double wt = gauss_weight_lean(h, k0h, k1v, e3v, s_exp);
-              double qw = qv;
-              if constexpr (HAS_W) wt = B.w_s[cb + j] * wt;
-              if (__builtin_amdgcn_ballot_w64(!(gq < glo))) {
-                // (a block of its own, so the branch above stays a scalar one)
-                asm volatile("; guard band" ::);
-                if (!(gq < glo) &&
-                    !radius_test_ref(B.xwcs, B.ywcs, B.lon_s, B.lat_s, cell[k], cb + j, P.sphere_radius)) {
-                  wt = 0.0;
-                  qw = 0.0;
-                }
+            for (int h = 0; h < NC / 2; ++h) {
+              const uint32_t u = w2[h];
+              if (O.bf16) {
+                cv[2 * h] = __uint_as_float(u << 16);
+                cv[2 * h + 1] = __uint_as_float(u & 0xFFFF0000u);
+              } else {
+                cv[2 * h] = (float)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xFFFFu));
+                cv[2 * h + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(u >> 16));
               }
-              acc_d[k] = fma(qw, wt, acc_d[k]);
-              acc_w[k] += wt;
-            } else if (gq < glo ||
-                       radius_test_ref(B.xwcs, B.ywcs, B.lon_s, B.lat_s, cell[k], cb + j, P.sphere_radius)) {
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < ROWS; ++k) {
+            if ((live & (kRow << k)) == 0) continue;  // uniform: the ring is out of this row's reach
+            double t;  // the tested distance: h = 1 - p.q (WMODE 3) or c2 = |p - q|^2
+            if constexpr (WMODE == 3) {
+              t = fma(npx[k], qx, fma(npy[k], qy, fma(npz[k], qz, 1.0)));
+            } else {
+              const double dx = npx[k] + qx, dy = npy[k] + qy, dz = npz[k] + qz;
+              t = fma(dx, dx, fma(dy, dy, dz * dz));
+            }
+            if (qg - hl[k] <= hw[k] && (kHigh ? high_f32(t) <= t_hi32 : t < t_hi)) {
+              const uint32_t cell = (row0 + (uint32_t)k) * P.side + col, isrc = src0 + j;
               double wt;
-              if constexpr (KT == HCG_GAUSS1D && WMODE > 0)
-                wt = gauss_weight_series<WMODE == 3 ? 2 : WMODE>(P, c2, s_exp);
+              if constexpr (WMODE == 3)
+                wt = gauss_weight_lean(t, k0h, k1v, e3v, s_exp);
+              else if constexpr (KT == HCG_GAUSS1D && WMODE > 0)
+                wt = gauss_weight_series<WMODE>(P, t, s_exp);
               else if constexpr (KT == HCG_GAUSS1D)
-                wt = HCG_GRID_TABLE_EXP ? exp_scaled_neg(gauss_exponent_scaled(P, c2), s_exp)
-                                        : exp(gauss_exponent_scaled(P, c2) * 0x1.62e42fefa39efp-7);
+                wt = exp_scaled_neg(gauss_exponent_scaled(P, t), s_exp);
               else
                 wt = weight_general<KT>(P.params[0], P.params[1], P.params[2], B.xwcs, B.ywcs, B.lon_s, B.lat_s,
-                                        0.25 * c2, cell[k], cb + j);
-              if constexpr (HAS_W) wt = B.w_s[cb + j] * wt;
-              if constexpr (NC > 0) {
-                // two channels per 32-bit LDS word; the value type is the
-                // job's (a uniform branch)
-                const float wf = (float)wt;
-                const uint32_t* cv = reinterpret_cast<const uint32_t*>(s_c + j * NC);
-                if (O.bf16) {
-#pragma unroll
-                  for (int h = 0; h < NC / 2; ++h) {
-                    const uint32_t u = cv[h];
-                    acc_c[2 * h] = fmaf(wf, __uint_as_float(u << 16), acc_c[2 * h]);
-                    acc_c[2 * h + 1] = fmaf(wf, __uint_as_float(u & 0xFFFF0000u), acc_c[2 * h + 1]);
-                  }
-                } else {
-#pragma unroll
-                  for (int h = 0; h < NC / 2; ++h) {
-                    const uint32_t u = cv[h];
-                    acc_c[2 * h] = fmaf(wf, (float)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xFFFFu)),
-                                        acc_c[2 * h]);
-                    acc_c[2 * h + 1] = fmaf(wf, (float)__builtin_bit_cast(_Float16, (uint16_t)(u >> 16)),
-                                            acc_c[2 * h + 1]);
-                  }
+                                        0.25 * t, cell, isrc);
+              // a lane near the radius (rare, and wave-uniformly skipped)
+              // that the reference's test rejects adds zero: one compare
+              // and no lane mask in the common case
+              double vv = qv;
+              if (__builtin_amdgcn_ballot_w64(!(kHigh ? high_f32(t) < t_lo32 : t < t_lo))) {
+                // (a block of its own, so the branch above stays a scalar one)
+                asm volatile("; guard band" ::);
+                if (!(t < t_lo) && !(t < t_hi && radius_test_ref(B.xwcs, B.ywcs, B.lon_s, B.lat_s, cell, isrc,
+                                                                 P.sphere_radius))) {
+                  wt = 0.0;
+                  vv = 0.0;
                 }
-                (void)qv;
-              } else {
-                acc_d[k] = fma(qv, wt, acc_d[k]);
               }
-              acc_w[k] += wt;
+              if constexpr (NC > 0) {
+                const float wf = (float)wt;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) acc_c[k][c] = fmaf(wf, cv[c], acc_c[k][c]);
+              } else {
+                acc_d[k] = fma(vv, wt, acc_d[k]);
+              }
+              if constexpr (HAS_W)
+                acc_w[k] = fma(qw, wt, acc_w[k]);
+              else
+                acc_w[k] += wt;
             }
           }
         }
       }
     }
   }
+  out.w = quad_rows_sum(acc_w, row);
   if constexpr (NC > 0) {
-    if (col < P.side && row0 < P.side) {
-      const size_t M = (size_t)P.side * P.side;
-      const uint32_t c0 = cell[0];
 #pragma unroll
-      for (int ch = 0; ch < NC; ++ch)
-        if ((uint32_t)ch < O.nchan)
-          O.cube[(size_t)ch * M + c0] =
-              O.normalize ? (float)((double)acc_c[ch] / acc_w[0]) : acc_c[ch];
-      if (O.wsum) O.wsum[c0] = (float)acc_w[0];
-    }
-    return;
-  }
+    for (int c = 0; c < NC; ++c) {
+      float v[ROWS];
 #pragma unroll
-  for (int k = 0; k < kCellsPerLane; ++k) {
-    if constexpr (BATCH) {
-      sum_d[k] = acc_d[k];
-      sum_w[k] = acc_w[k];
-    } else if (col < P.side && row0 + k < P.side) {
-      B.dc[cell[k]] = acc_d[k];
-      B.wc[cell[k]] = acc_w[k];
+      for (int r = 0; r < ROWS; ++r) v[r] = acc_c[r][c];
+      out.c[c] = quad_rows_sum(v, row);
     }
+  } else {
+    out.d = quad_rows_sum(acc_d, row);
   }
+}
+
+// The map cell whose sums this lane holds; false for none.
+template <int ROWS = kTileRows>
+__device__ inline bool tile_cell(uint32_t side, uint32_t tile, uint32_t tiles_x, uint32_t& cell) {
+  const uint32_t lane = __lane_id();
+  const uint32_t col = (tile % tiles_x) * kTileCols + (lane >> 2);
+  const uint32_t row = (tile / tiles_x) * ROWS + (lane & 3u);
+  cell = row * side + col;
+  return col < side && row < side && (lane & 3u) < (uint32_t)ROWS;
 }
 
 // The FP32 outputs of one one-channel tile cell (lane) from its sums.
 __device__ inline void tile_write(const GridParams& P, uint32_t tile, uint32_t tiles_x, const TileOut& O, double d,
                                   double w) {
-  const uint32_t lane = __lane_id();
-  const uint32_t col = (tile % tiles_x) * kTileCols + lane / kLaneRows;
-  const uint32_t row = (tile / tiles_x) * kTileRows + lane % kLaneRows;
-  if (col < P.side && row < P.side) {
-    const uint32_t cell = row * P.side + col;
+  uint32_t cell;
+  if (tile_cell(P.side, tile, tiles_x, cell)) {
     O.cube[cell] = O.normalize ? (float)(d / w) : (float)d;
     if (O.wsum) O.wsum[cell] = (float)w;
   }
@@ -487,64 +800,53 @@ constexpr size_t one_channel_lds_bytes(uint32_t active, uint32_t streams) {
 // slice of `lds`; the streams' sums meet after the slices and wave 0 adds
 // them in stream order and writes the cells.  Every wave of the workgroup
 // calls this (it holds a workgroup barrier when streams > 1).
+template <int WMODE>
 __device__ __forceinline__ void one_channel_tile(const GridParams& P, const GridBuffers& B, const TileOut& O,
                                                  uint32_t tile, uint32_t tiles_x, uint32_t streams, uint32_t active,
                                                  char* lds, const double* s_exp) {
   const uint32_t wave = threadIdx.x >> 6, lane = __lane_id();
   double* red = reinterpret_cast<double*>(lds + active * kTileLdsBytes);
-  double d = 0.0, w = 0.0;
+  TileSums<0> s{};
   if (wave < active) {
-    double* s_x = reinterpret_cast<double*>(lds + wave * kTileLdsBytes);
-    double* s_y = s_x + kStageCap;
-    double* s_z = s_y + kStageCap;
-    double* s_v = s_z + kStageCap;
-    uint32_t* s_key = reinterpret_cast<uint32_t*>(s_v + kStageCap);
     for (uint32_t q = wave; q < streams; q += active) {
-      grid_tile<HCG_GAUSS1D, false, 2, true>(P, B, tile, tiles_x, s_x, s_y, s_z, s_v, s_key, s_exp, O,
-                                             RingStream{q, streams}, &d, &w);
+      grid_tile<HCG_GAUSS1D, false, WMODE, true, 0, kOneCap>(P, B, tile, tiles_x, lds + wave * kTileLdsBytes, s_exp,
+                                                               O, RingStream{q, streams}, s);
       if (streams > 1) {
-        red[(q * 64 + lane) * 2] = d;
-        red[(q * 64 + lane) * 2 + 1] = w;
+        red[(q * 64 + lane) * 2] = s.d;
+        red[(q * 64 + lane) * 2 + 1] = s.w;
       }
     }
   }
   if (streams > 1) {
     __syncthreads();
     if (wave == 0) {
-      d = red[lane * 2];
-      w = red[lane * 2 + 1];
+      s.d = red[lane * 2];
+      s.w = red[lane * 2 + 1];
       for (uint32_t q = 1; q < streams; ++q) {
-        d += red[(q * 64 + lane) * 2];
-        w += red[(q * 64 + lane) * 2 + 1];
+        s.d += red[(q * 64 + lane) * 2];
+        s.w += red[(q * 64 + lane) * 2 + 1];
       }
     }
   }
-  if (wave == 0) tile_write(P, tile, tiles_x, O, d, w);
+  if (wave == 0) tile_write(P, tile, tiles_x, O, s.d, s.w);
 }
 
 // One few-channel tile in a kFewTileLdsBytes slice of LDS (one wave).
 __device__ __forceinline__ void few_channel_tile_body(const GridParams& P, const GridBuffers& B, const TileOut& O,
                                                       uint32_t tile, uint32_t tiles_x, char* lds,
                                                       const double* s_exp) {
-  double* s_x = reinterpret_cast<double*>(lds);
-  double* s_y = s_x + kFewCap;
-  double* s_z = s_y + kFewCap;
-  uint32_t* s_key = reinterpret_cast<uint32_t*>(s_z + kFewCap);
-  uint16_t* s_c = reinterpret_cast<uint16_t*>(s_key + kFewCap);
-  grid_tile<HCG_GAUSS1D, false, 3, true, kFewChannels, kFewCap>(P, B, tile, tiles_x, s_x, s_y, s_z, nullptr, s_key,
-                                                                s_exp, O, RingStream{0, 1}, nullptr, nullptr, s_c);
-}
-
-// The same, out of line, for the persistent batch kernel: inlined there as
-// a third copy of the tile body, it raised that kernel's register spills
-// and slowed its MFMA and one-channel items by 1-10%; the call costs a
-// few-channel tile ~4%.  (The one-job kernel inlines the body: a called
-// function takes the register budget of its widest caller.)
-[[maybe_unused]] static __device__ __noinline__ void few_channel_tile(const GridParams& P, const GridBuffers& B,
-                                                                    const TileOut& O, uint32_t tile,
-                                                                    uint32_t tiles_x, char* lds,
-                                                                    const double* s_exp) {
-  few_channel_tile_body(P, B, O, tile, tiles_x, lds, s_exp);
+  TileSums<kFewChannels> s;
+  grid_tile<HCG_GAUSS1D, false, 3, true, kFewChannels, kFewCap>(P, B, tile, tiles_x, lds, s_exp, O, RingStream{0, 1},
+                                                                s);
+  uint32_t cell;
+  if (tile_cell(P.side, tile, tiles_x, cell)) {
+    const size_t M = (size_t)P.side * P.side;
+#pragma unroll
+    for (int ch = 0; ch < kFewChannels; ++ch)
+      if ((uint32_t)ch < O.nchan)
+        O.cube[(size_t)ch * M + cell] = O.normalize ? (float)((double)s.c[ch] / s.w) : s.c[ch];
+    if (O.wsum) O.wsum[cell] = (float)s.w;
+  }
 }
 
 }  // namespace hcg
