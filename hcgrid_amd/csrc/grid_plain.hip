@@ -216,11 +216,13 @@ static void launch_tiles_as(const GridParams& P, const GridBuffers& B, hipStream
 // 400^2 at 100 (1, 4) 106, (4, 4) 139; 512^2 at 980 (1, 4) 739, (4, 4) 921.
 template <int KT, bool HAS_W, int WMODE>
 static void launch_tiles(const GridParams& P, const GridBuffers& B, uint32_t n, hipStream_t s) {
+  // GAUSS2D's tangent frames take twelve registers a row: two rows
+  constexpr int R = KT == HCG_GAUSS2D && WMODE == 4 ? 2 : 4;
   const uint32_t tiles = tile_count_of(P.side);
   if (tiles >= 4096 || (tiles >= 2048 && n < 256 * tiles))
-    launch_tiles_as<KT, HAS_W, WMODE, 1, 4>(P, B, s);
+    launch_tiles_as<KT, HAS_W, WMODE, 1, R>(P, B, s);
   else if (tiles >= 512)
-    launch_tiles_as<KT, HAS_W, WMODE, 4, 4>(P, B, s);
+    launch_tiles_as<KT, HAS_W, WMODE, 4, R>(P, B, s);
   else if (tiles >= 128)
     launch_tiles_as<KT, HAS_W, WMODE, 4, 1>(P, B, s);
   else
@@ -240,6 +242,8 @@ int launch_grid(const GridParams& P, const GridBuffers& B, uint32_t n, hipStream
       launch_tiles<KT, HAS_W, 1>(P, B, n, s);
     else
       launch_tiles<KT, HAS_W, 0>(P, B, n, s);
+  } else if (frame_weight_ok(P, KT)) {
+    launch_tiles<KT, HAS_W, 4>(P, B, n, s);
   } else {
     launch_tiles<KT, HAS_W, 0>(P, B, n, s);
   }

@@ -427,7 +427,7 @@ struct TileShared {
 
 // WMODE (GAUSS1D): 0 general exponent and exp; 1 gauss_small_radius; 2
 // gauss_tiny_radius; 3 also lean_weight_ok (the candidate test on p.q and
-// the lean weight).
+// the lean weight).  The other kernels: 0 general, 4 frame_weight_ok.
 // lds: CAP x (x, y, z, v doubles, key), with HAS_W then CAP weights; with NC
 // > 0 CAP x (x, y, z doubles, key, NC 16-bit values).
 // s_exp: the 64-entry exponential table (exp_table_load), visible to the wave.
@@ -465,6 +465,9 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
 #pragma unroll
     for (int c = 0; c < (NC > 0 ? NC : 1); ++c) acc_c[r][c] = 0.f;
   }
+  // GAUSS2D's tangent frames (WMODE 4): east and north turned by the position angle
+  constexpr bool kFrame = WMODE == 4 && KT == HCG_GAUSS2D;
+  double fu[kFrame ? ROWS : 1][3], fv[kFrame ? ROWS : 1][3];
   Window win;
   double tl = 0.0, tr = 0.0;  // compat: the window's edges, fmodulo4 in units of pi/2
   TileSpan T;
@@ -517,6 +520,24 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
         T = H.T;
         T.r_begin = __builtin_amdgcn_readfirstlane(T.r_begin);
         T.r_end = __builtin_amdgcn_readfirstlane(T.r_end);
+      }
+    }
+    if constexpr (kFrame) {
+      const uint32_t rr = min(row0 + row, P.side - 1), cc = min(col, P.side - 1);
+      double sl, cl;
+      sincos(B.xwcs[rr * P.side + cc] * kDeg2Rad, &sl, &cl);
+      const double cb = cos(B.ywcs[rr * P.side + cc] * kDeg2Rad);
+      const double e[3] = {-sl, cl, 0.0}, nn[3] = {-pz * cl, -pz * sl, cb};
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        double u[ROWS], v[ROWS];
+        quad_all(fma(e[i], P.f[2], -(nn[i] * P.f[3])), u);
+        quad_all(fma(nn[i], P.f[2], e[i] * P.f[3]), v);
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+          fu[r][i] = u[r];
+          fv[r][i] = v[r];
+        }
       }
     }
     // -p: h = 1 - p.q is three FMAs from 1
@@ -707,10 +728,11 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
           for (int k = 0; k < ROWS; ++k) {
             if ((live & (kRow << k)) == 0) continue;  // uniform: the ring is out of this row's reach
             double t;  // the tested distance: h = 1 - p.q (WMODE 3) or c2 = |p - q|^2
+            double dx = 0.0, dy = 0.0, dz = 0.0;
             if constexpr (WMODE == 3) {
               t = fma(npx[k], qx, fma(npy[k], qy, fma(npz[k], qz, 1.0)));
             } else {
-              const double dx = npx[k] + qx, dy = npy[k] + qy, dz = npz[k] + qz;
+              dx = npx[k] + qx, dy = npy[k] + qy, dz = npz[k] + qz;
               t = fma(dx, dx, fma(dy, dy, dz * dz));
             }
             if (qg - hl[k] <= hw[k] && (kHigh ? high_f32(t) <= t_hi32 : t < t_hi)) {
@@ -718,6 +740,11 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
               double wt;
               if constexpr (WMODE == 3)
                 wt = gauss_weight_lean(t, k0h, k1v, e3v, s_exp);
+              else if constexpr (kFrame)
+                wt = gauss2d_frame_weight(P, t, fma(dx, fu[k][0], fma(dy, fu[k][1], dz * fu[k][2])),
+                                          fma(dx, fv[k][0], fma(dy, fv[k][1], dz * fv[k][2])), s_exp);
+              else if constexpr (WMODE == 4)
+                wt = sinc_frame_weight(P, t, s_exp);
               else if constexpr (KT == HCG_GAUSS1D && WMODE > 0)
                 wt = gauss_weight_series<WMODE>(P, t, s_exp);
               else if constexpr (KT == HCG_GAUSS1D)
