@@ -6,17 +6,24 @@
 // host, gathers lon/lat/data through the permutation and builds the ring
 // LUT with a sequential binary-search loop.  Here all of it stays in HBM:
 //
-//   k_keys        ang2pix per sample -> (key u32, index u32)
-//   k_rs_upsweep  per-tile 8-bit digit histograms           } 4 passes of a
-//   k_rs_scan     per-digit scan over tiles + digit offsets } stable LSD radix
-//   k_rs_downsweep stable in-tile ranking, scatter          } sort
-//   k_gather      permutation gather fused with the unit-vector records
-//   k_ring_meta / k_ring_lut  firstring, usedrings, LUT and per-ring cos/sin
+//   k_keys         ang2pix per sample -> key, and the first digit's counts per tile
+//   k_rs_upsweep   a later digit's counts per tile        } two or three passes of
+//   k_rs_scan      per digit, scan over the tiles         } a stable LSD radix sort
+//   k_rs_downsweep stable in-tile ranking, scatter        } on up to ten bits each
+//   k_gather       permutation gather fused with the unit-vector records
+//   k_ring_lut     firstring, usedrings, LUT and per-ring cos/sin
 //
-// The radix sort is reduce-then-scan (no inter-workgroup waiting), stable by
-// construction: tiles keep input order, and inside a tile items are ranked
-// in index order with wave ballots.  Keys are < 2^31 (npix(8192) < 2^30 and
-// MAX_Y = 2^30), so 4 passes of 8 bits order them completely.
+// The radix sort is reduce-then-scan (no inter-workgroup waiting) and stable
+// by construction: tiles keep input order, a wave of a tile owns a contiguous
+// part of it, and within a wave items are ranked in index order with ballots.
+// Keys are < npix <= 12 8192^2 < 2^30, or MAX_Y, which sorts as npix: at most
+// 30 bits, three digits of ten (two digits up to nside 256).
+//
+// What it costs: on small inputs the launches (a dependent launch takes about
+// 4.5 us whatever it does), on large ones the scatter, whose 4-byte stores of
+// a wave go to as many lines as it has digits.  Four 8-bit passes of four
+// launches each, ranked with three workgroup barriers per 256 items, took
+// 142 us for 250k samples and 760 us for 20M.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -26,77 +33,133 @@
 
 namespace hcg {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortItems = 16;
-constexpr uint32_t kSortTile = kSortThreads * kSortItems;  // 4096 keys per workgroup
-constexpr int kSortWaves = kSortThreads / 64;
+// Keys per sort tile: small tiles fill the chip's 256 CUs from few samples on,
+// large ones have fewer counts to write and scan (1024 digits a tile).
+// Presort: 1M samples 111 us with small tiles, 1.2M 123 us with large ones and
+// 112 with middle ones, 2M 150 us with middle and 138 with large ones.
+constexpr uint32_t kSmallTile = 256 * 4, kMidTile = 256 * 8, kLargeTile = 512 * 16;
+constexpr uint32_t kSmallTiles = 512, kMidTiles = 768;
+constexpr int kMaxDigitBits = 10;
+constexpr uint32_t kMaxDigits = 1u << kMaxDigitBits;
 
-__global__ void __launch_bounds__(256) k_keys(hcg_healpix hp, uint32_t n, const double* __restrict__ lon,
-                                              const double* __restrict__ lat, uint32_t* __restrict__ keys,
-                                              uint32_t* __restrict__ idx) {
+// A pass: digit = (min(key, top) >> shift) & (2^bits - 1).
+struct Digit {
+  uint32_t top;  // npix: MAX_Y keys sort as it
+  int shift, bits;
+};
+
+__device__ inline uint32_t digit_of(uint32_t key, const Digit& g) {
+  return (min(key, g.top) >> g.shift) & ((1u << g.bits) - 1u);
+}
+
+// The tile of this workgroup: neighbouring tiles, whose counts share cache
+// lines, on one XCD (block b runs on XCD b % 8).  sort_blocks(tiles)
+// workgroups; tile >= tiles has nothing to do.
+__device__ inline uint32_t sort_tile(uint32_t tiles) {
+  return (blockIdx.x & 7u) * ((tiles + 7u) >> 3) + (blockIdx.x >> 3);
+}
+inline uint32_t sort_blocks(uint32_t tiles) { return (tiles + 7u) & ~7u; }
+
+// Adds each valid lane's digit to the workgroup's LDS counts: one add for a
+// wave whose digits are all equal (nearly sorted input), else one per lane.
+__device__ inline void count_digit(uint32_t* h, uint32_t d, bool valid) {
+  const uint64_t vm = __ballot(valid);
+  if (vm == 0) return;
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)d, (int)__ffsll((unsigned long long)vm) - 1);
+  if (__ballot(valid && d == first) == vm) {
+    if (__lane_id() == 0) atomicAdd(&h[first], (uint32_t)__popcll(vm));
+  } else if (valid) {
+    atomicAdd(&h[d], 1u);
+  }
+}
+
+// Keys of one tile and its counts of the first digit, hist[d * tiles + tile].
+// Workgroup 0 writes the npix sentinel (HCGrid/gridding.cu:100).
+template <uint32_t THREADS, uint32_t ITEMS>
+__global__ void __launch_bounds__(THREADS) k_keys(hcg_healpix hp, uint32_t n, const double* __restrict__ lon,
+                                                  const double* __restrict__ lat, uint32_t* __restrict__ keys,
+                                                  uint32_t* __restrict__ sentinel, Digit g, uint32_t tiles,
+                                                  uint32_t* __restrict__ hist) {
+  __shared__ uint32_t h[kMaxDigits];
   const Hpx32 hx = hpx32(hp);
-  // 64-bit index: with a 32-bit one, i + stride wraps below n for n close to 2^32
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    // HCGrid/gridding.cu:78-80
-    const double theta = kHalfPi - kDeg2Rad * lat[i];
-    const double phi = kDeg2Rad * lon[i];
-    keys[i] = ang2pix32(hx, theta, phi);
-    idx[i] = (uint32_t)i;
+  const uint32_t digits = 1u << g.bits, tile = sort_tile(tiles);
+  if (tile >= tiles) return;
+  for (uint32_t d = threadIdx.x; d < digits; d += THREADS) h[d] = 0;
+  __syncthreads();
+  // 64-bit index: a 32-bit one wraps for n close to 2^32
+  const uint64_t base = (uint64_t)tile * (THREADS * ITEMS);
+#pragma unroll 2
+  for (uint32_t j = 0; j < ITEMS; ++j) {
+    const uint64_t i = base + j * THREADS + threadIdx.x;
+    uint32_t key = 0;
+    if (i < n) {
+      // HCGrid/gridding.cu:78-80
+      key = ang2pix32(hx, kHalfPi - kDeg2Rad * lat[i], kDeg2Rad * lon[i]);
+      keys[i] = key;
+    }
+    count_digit(h, digit_of(key, g), i < n);
   }
+  __syncthreads();
+  for (uint32_t d = threadIdx.x; d < digits; d += THREADS) hist[(size_t)d * tiles + tile] = h[d];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *sentinel = hx.npix;
 }
 
-// Digit histogram of one 4096-key tile, written digit-major: hist[d * tiles + t].
-__global__ void __launch_bounds__(256) k_rs_upsweep(const uint32_t* __restrict__ keys, uint32_t n, int shift,
-                                                    uint32_t tiles, uint32_t* __restrict__ hist) {
-  __shared__ uint32_t h[256];
-  const uint32_t tid = threadIdx.x;
-  h[tid] = 0;
+// Digit counts of one tile, hist[d * tiles + tile].
+template <uint32_t THREADS, uint32_t ITEMS>
+__global__ void __launch_bounds__(THREADS) k_rs_upsweep(const uint32_t* __restrict__ keys, uint32_t n, Digit g,
+                                                        uint32_t tiles, uint32_t* __restrict__ hist) {
+  __shared__ uint32_t h[kMaxDigits];
+  const uint32_t digits = 1u << g.bits, tile = sort_tile(tiles);
+  if (tile >= tiles) return;
+  for (uint32_t d = threadIdx.x; d < digits; d += THREADS) h[d] = 0;
   __syncthreads();
-  const uint32_t base = blockIdx.x * kSortTile;
-  const uint64_t lt = lanemask_lt();
+  const uint64_t base = (uint64_t)tile * (THREADS * ITEMS);
 #pragma unroll 4
-  for (int j = 0; j < kSortItems; ++j) {
-    const uint32_t i = base + j * kSortThreads + tid;
+  for (uint32_t j = 0; j < ITEMS; ++j) {
+    const uint64_t i = base + j * THREADS + threadIdx.x;
     const bool valid = i < n;
-    const uint32_t d = valid ? ((keys[i] >> shift) & 0xFFu) : 0u;
-    const uint64_t peers = match_digit8(d, valid);
-    // the lowest lane of each peer group adds the group's count
-    if (valid && (peers & lt) == 0) atomicAdd(&h[d], (uint32_t)__popcll(peers));
+    count_digit(h, digit_of(valid ? keys[i] : 0u, g), valid);
   }
   __syncthreads();
-  hist[tid * tiles + blockIdx.x] = h[tid];
+  for (uint32_t d = threadIdx.x; d < digits; d += THREADS) hist[(size_t)d * tiles + tile] = h[d];
 }
 
-// Exclusive scan of 256 values held one per thread (block of 256).
-__device__ inline uint32_t block_exclusive_scan256(uint32_t v, uint32_t* lds_waves, uint32_t& total) {
-  const uint32_t lane = __lane_id();
-  const uint32_t wave = threadIdx.x >> 6;
+// Orders this wave's LDS operations (they execute in issue order: a fence for
+// the compiler).
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Exclusive scan of one value per thread over the workgroup (a multiple of
+// 64 threads, at most 1024); lds holds one word per wave.
+__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* lds, uint32_t& total) {
+  const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   uint32_t x = v;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
     const uint32_t y = __shfl_up(x, off, 64);
     if (lane >= (uint32_t)off) x += y;
   }
-  if (lane == 63) lds_waves[wave] = x;
+  if (lane == 63) lds[wave] = x;
   __syncthreads();
-  uint32_t wave_off = 0;
+  uint32_t before = 0;
   total = 0;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const uint32_t s = lds_waves[w];
-    if (w < (int)wave) wave_off += s;
+  for (uint32_t w = 0; w < nw; ++w) {
+    const uint32_t s = lds[w];
+    if (w < wave) before += s;
     total += s;
   }
   __syncthreads();
-  return wave_off + x - v;
+  return before + x - v;
 }
 
 // One workgroup per digit: exclusive scan of its row of tile counts; the row
 // total goes to digit_tot[d].
-__global__ void __launch_bounds__(256) k_rs_scan_rows(uint32_t* __restrict__ hist, uint32_t tiles,
-                                                      uint32_t* __restrict__ digit_tot) {
-  __shared__ uint32_t waves[4];
+__global__ void __launch_bounds__(256) k_rs_scan(uint32_t* __restrict__ hist, uint32_t tiles,
+                                                 uint32_t* __restrict__ digit_tot) {
+  __shared__ uint32_t lds[4];
   uint32_t* row = hist + (size_t)blockIdx.x * tiles;
   uint32_t running = 0;
   for (uint32_t base = 0; base < tiles; base += 256 * 4) {
@@ -109,7 +172,7 @@ __global__ void __launch_bounds__(256) k_rs_scan_rows(uint32_t* __restrict__ his
       s += v[q];
     }
     uint32_t total;
-    uint32_t pre = block_exclusive_scan256(s, waves, total) + running;
+    uint32_t pre = block_exclusive_scan(s, lds, total) + running;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const uint32_t i = base + threadIdx.x * 4 + q;
@@ -121,55 +184,92 @@ __global__ void __launch_bounds__(256) k_rs_scan_rows(uint32_t* __restrict__ his
   if (threadIdx.x == 0) digit_tot[blockIdx.x] = running;
 }
 
-__global__ void __launch_bounds__(256) k_rs_scan_digits(uint32_t* __restrict__ digit_tot) {
-  __shared__ uint32_t waves[4];
-  uint32_t total;
-  const uint32_t v = digit_tot[threadIdx.x];
-  const uint32_t ex = block_exclusive_scan256(v, waves, total);
-  digit_tot[threadIdx.x] = ex;
-}
-
-// Stable scatter of one tile.  Items are visited in index order (round j,
-// thread t -> index tile*4096 + j*256 + t); within a round an item's rank
-// among equal digits is (items of earlier waves) + (earlier lanes of its wave).
-__global__ void __launch_bounds__(256) k_rs_downsweep(const uint32_t* __restrict__ kin,
-                                                      const uint32_t* __restrict__ vin,
-                                                      uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                      uint32_t n, int shift, uint32_t tiles,
-                                                      const uint32_t* __restrict__ hist,
-                                                      const uint32_t* __restrict__ digit_off) {
-  __shared__ uint32_t base_off[256];
-  __shared__ uint32_t wave_cnt[kSortWaves][256];
-  const uint32_t tid = threadIdx.x;
-  const uint32_t lane = __lane_id();
-  const uint32_t wave = tid >> 6;
-  base_off[tid] = digit_off[tid] + hist[tid * tiles + blockIdx.x];
-  const uint64_t lt = lanemask_lt();
-  const uint32_t tile_base = blockIdx.x * kSortTile;
-  __syncthreads();
-  for (int j = 0; j < kSortItems; ++j) {
-    const uint32_t i = tile_base + j * kSortThreads + tid;
-    const bool valid = i < n;
-    const uint32_t key = valid ? kin[i] : 0u;
-    const uint32_t val = valid ? vin[i] : 0u;
-    const uint32_t d = (key >> shift) & 0xFFu;
-    const uint64_t peers = match_digit8(d, valid);
-    const uint32_t rank = (uint32_t)__popcll(peers & lt);
-    const uint32_t cnt = (uint32_t)__popcll(peers);
+// Stable scatter of one tile.  Wave w owns the tile's items w * ITEMS * 64 ..
+// and ranks them in index order against its own counts in LDS (its LDS
+// operations execute in order, so this needs no barrier); the waves' counts
+// then become offsets in wave order.  FIRST: the values are the indexes.
+template <uint32_t THREADS, uint32_t ITEMS, bool FIRST>
+__global__ void __launch_bounds__(THREADS) k_rs_downsweep(const uint32_t* __restrict__ kin,
+                                                          const uint32_t* __restrict__ vin,
+                                                          uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
+                                                          uint32_t n, Digit g, uint32_t tiles,
+                                                          const uint32_t* __restrict__ hist,
+                                                          const uint32_t* __restrict__ digit_tot) {
+  constexpr uint32_t W = THREADS / 64;
+  constexpr uint32_t PER = kMaxDigits / THREADS;  // digits per thread
+  __shared__ uint32_t cnt[W][kMaxDigits];
+  __shared__ uint32_t lds[W];
+  const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
+  const uint32_t digits = 1u << g.bits, tile = sort_tile(tiles);
+  if (tile >= tiles) return;
+  for (uint32_t d = lane; d < digits; d += 64) cnt[wave][d] = 0;  // (its own wave's: no barrier)
+  wave_fence();
+  // this tile's first position of each digit: the digits before it, and the tiles before it
+  uint32_t off[PER];
+  {
+    uint32_t tot[PER], s = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) wave_cnt[wave][lane + 64 * q] = 0;
-    if (valid && rank == cnt - 1) wave_cnt[wave][d] = cnt;
-    __syncthreads();
-    uint32_t pos = base_off[d] + rank;
-    for (uint32_t w = 0; w < wave; ++w) pos += wave_cnt[w][d];
-    __syncthreads();
-    base_off[tid] += wave_cnt[0][tid] + wave_cnt[1][tid] + wave_cnt[2][tid] + wave_cnt[3][tid];
-    if (valid) {
-      kout[pos] = key;
-      vout[pos] = val;
+    for (uint32_t q = 0; q < PER; ++q) {
+      const uint32_t d = threadIdx.x * PER + q;
+      tot[q] = d < digits ? digit_tot[d] : 0u;
+      off[q] = d < digits ? hist[(size_t)d * tiles + tile] : 0u;
+      s += tot[q];
     }
-    __syncthreads();
+    uint32_t total;
+    uint32_t pre = block_exclusive_scan(s, lds, total);
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q) {
+      off[q] += pre;
+      pre += tot[q];
+    }
   }
+  const uint64_t base = (uint64_t)tile * (THREADS * ITEMS) + (uint64_t)wave * (ITEMS * 64) + lane;
+  uint32_t key[ITEMS], val[ITEMS];
+#pragma unroll
+  for (uint32_t j = 0; j < ITEMS; ++j) {
+    const uint64_t i = base + j * 64;
+    key[j] = i < n ? kin[i] : 0u;
+    val[j] = FIRST ? (uint32_t)i : (i < n ? vin[i] : 0u);
+  }
+  const uint64_t lt = lanemask_lt();
+  uint32_t rank[ITEMS];
+#pragma unroll
+  for (uint32_t j = 0; j < ITEMS; ++j) {
+    const bool valid = base + j * 64 < n;
+    const uint32_t d = digit_of(key[j], g);
+    uint64_t peers = __ballot(valid);
+    for (int b = 0; b < g.bits; ++b) {  // uniform
+      const uint64_t vote = __ballot((d >> b) & 1u);
+      peers &= ((d >> b) & 1u) ? vote : ~vote;
+    }
+    const uint32_t before = valid ? cnt[wave][d] : 0u;
+    rank[j] = before + (uint32_t)__popcll(peers & lt);
+    wave_fence();
+    if (valid && (peers & lt) == 0) cnt[wave][d] = before + (uint32_t)__popcll(peers);
+    wave_fence();
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t q = 0; q < PER; ++q) {
+    const uint32_t d = threadIdx.x * PER + q;
+    if (d < digits) {
+      uint32_t at = off[q];
+#pragma unroll
+      for (uint32_t w = 0; w < W; ++w) {
+        const uint32_t c = cnt[w][d];
+        cnt[w][d] = at;
+        at += c;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t j = 0; j < ITEMS; ++j)
+    if (base + j * 64 < n) {
+      const uint32_t pos = cnt[wave][digit_of(key[j], g)] + rank[j];
+      kout[pos] = key[j];
+      vout[pos] = val[j];
+    }
 }
 
 __global__ void __launch_bounds__(64) k_set_sentinel(uint32_t* keys, uint32_t n, uint32_t npix) {
@@ -208,38 +308,54 @@ __global__ void __launch_bounds__(256) k_gather(uint32_t n, const uint32_t* __re
   }
 }
 
+// First index of n keys with key >= x (n if none), three probes a step: a
+// step is one round of dependent loads and quarters the range.
+__device__ inline uint32_t lower_bound_4(const uint32_t* __restrict__ keys, uint32_t n, uint32_t x) {
+  uint32_t a = 0, b = n;
+  while (a < b) {
+    const uint32_t d = (b - a) >> 2, p0 = a + d, p1 = a + ((b - a) >> 1), p2 = min(p1 + d, b - 1);
+    const uint32_t k0 = keys[p0], k1 = keys[p1], k2 = keys[p2];
+    if (k2 < x)
+      a = p2 + 1;
+    else if (k1 < x)
+      a = p1 + 1, b = p2;
+    else if (k0 < x)
+      a = p0 + 1, b = p1;
+    else
+      b = p0;
+  }
+  return a;
+}
+
 // firstring / usedrings / n_valid (HCGrid/gridding.cu:118-121).  Samples
 // whose key is >= npix (theta outside [0, pi]) sort last and are left out of
 // the ring span; the reference would take pix2ring of MAX_Y there.
-__global__ void __launch_bounds__(64) k_ring_meta(hcg_healpix hp, uint32_t n, const uint32_t* __restrict__ keys,
-                                                  hcg_ring_meta* __restrict__ meta) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const uint32_t nv = lower_bound_u32(keys, 0, n, (uint32_t)hp.npix);
+__device__ inline hcg_ring_meta ring_meta(const hcg_healpix& hp, uint32_t n, const uint32_t* __restrict__ keys) {
+  const Hpx32 hx = hpx32(hp);
   hcg_ring_meta m;
   m.n = n;
-  m.n_valid = nv;
-  if (nv == 0) {
-    m.firstring = 0;
-    m.usedrings = 0;
-  } else {
-    const uint64_t first = pix2ring(hp, keys[0]);
-    const uint64_t last = pix2ring(hp, keys[nv - 1]);
-    m.firstring = (uint32_t)first;
-    m.usedrings = (uint32_t)(1 + last - first);
+  m.firstring = m.usedrings = 0;
+  m.n_valid = n == 0 || keys[n - 1] < hx.npix ? n : lower_bound_4(keys, n, hx.npix);
+  if (m.n_valid) {
+    m.firstring = pix2ring32(hx, keys[0]);
+    m.usedrings = 1 + pix2ring32(hx, keys[m.n_valid - 1]) - m.firstring;
   }
-  *meta = m;
+  return m;
 }
 
 // Level-1 LUT (HCGrid/gridding.cu:122-136): lut[k] = first index with key >=
 // startpix(firstring + k).  The reference's incremental searchLastPosLessThan
 // walk returns exactly this lower bound.  Also the per-ring cos/sin of the
 // ring-centre colatitude (HCGrid/gridding.cu:332-334); ring_s < 0 marks rings
-// where the reference's ang2pix takes the cos-only branch.
-__global__ void __launch_bounds__(256) k_ring_lut(hcg_healpix hp, const uint32_t* __restrict__ keys,
-                                                  const hcg_ring_meta* __restrict__ meta, uint32_t* __restrict__ lut,
+// where the reference's ang2pix takes the cos-only branch.  Every thread
+// works out the ring span (three loads) rather than wait for a launch that
+// does; the first writes it.
+__global__ void __launch_bounds__(256) k_ring_lut(hcg_healpix hp, uint32_t n, const uint32_t* __restrict__ keys,
+                                                  hcg_ring_meta* __restrict__ meta, uint32_t* __restrict__ lut,
                                                   double* __restrict__ ring_z, double* __restrict__ ring_s) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  const hcg_ring_meta m = *meta;
+  const hcg_ring_meta m = ring_meta(hp, n, keys);
+  if (k == 0) *meta = m;
   if (k > m.usedrings) return;
   if (k == 0) {
     lut[0] = 0;
@@ -248,7 +364,7 @@ __global__ void __launch_bounds__(256) k_ring_lut(hcg_healpix hp, const uint32_t
   } else {
     uint64_t sp, npr;
     ring_info(hp, (uint64_t)m.firstring + k, sp, npr);
-    lut[k] = lower_bound_u32(keys, 0, m.n, (uint32_t)sp);
+    lut[k] = lower_bound_4(keys, m.n, (uint32_t)sp);
   }
   if (k < m.usedrings) {
     const RingGeom g = ring_geom(hp, (uint64_t)m.firstring + k);
@@ -272,16 +388,23 @@ struct SortWorkspace {
 
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+constexpr uint32_t sort_tile_of(uint32_t n) {
+  return n <= kSmallTile * kSmallTiles ? kSmallTile : n <= kMidTile * kMidTiles ? kMidTile : kLargeTile;
+}
+constexpr uint32_t sort_tiles_of(uint32_t n) {
+  return n ? (uint32_t)(((uint64_t)n + sort_tile_of(n) - 1) / sort_tile_of(n)) : 1u;
+}
+
 // Sort scratch for n keys: ping-pong keys and values, per-tile digit
 // counts, per-digit totals.  Every byte of it is written before it is read.
 constexpr size_t sort_ws_bytes(uint32_t n) {
-  return 2 * align256((size_t)n * 4) + align256((size_t)((n ? n : 1) + kSortTile - 1) / kSortTile * 256 * 4) +
-         align256(256 * 4);
+  return 2 * align256((size_t)n * 4) + align256((size_t)sort_tiles_of(n) * kMaxDigits * 4) +
+         align256(kMaxDigits * 4);
 }
 
 size_t sort_ws_layout(uint32_t n, void* base, SortWorkspace* ws) {
-  const uint32_t tiles = ceil_div_u32(n ? n : 1, kSortTile);
-  const size_t kb = align256((size_t)n * 4), hb = align256((size_t)tiles * 256 * 4);
+  const uint32_t tiles = sort_tiles_of(n);
+  const size_t kb = align256((size_t)n * 4), hb = align256((size_t)tiles * kMaxDigits * 4);
   if (ws) {
     char* p = static_cast<char*>(base);
     ws->keys_b = reinterpret_cast<uint32_t*>(p);
@@ -306,34 +429,51 @@ int presort_args(const hcg_healpix* hp, uint32_t n, const double* lon_deg, const
   return HCG_OK;
 }
 
-// Keys, the four radix passes and the sentinel, on workspace `ws` (n > 0).
-int presort_enqueue(const hcg_healpix* hp, uint32_t n, const double* lon_deg, const double* lat_deg,
-                    uint32_t* keys_sorted, uint32_t* perm, const SortWorkspace& ws, hipStream_t s) {
-  const uint32_t blocks = std::min<uint32_t>(ceil_div_u32(n, 256), 8192);
-  k_keys<<<blocks, 256, 0, s>>>(*hp, n, lon_deg, lat_deg, keys_sorted, perm);
-  HCG_CHECK_LAUNCH("k_keys");
-
-  uint32_t* kin = keys_sorted;
-  uint32_t* vin = perm;
-  uint32_t* kout = ws.keys_b;
-  uint32_t* vout = ws.vals_b;
-  for (int pass = 0; pass < 4; ++pass) {
-    const int shift = 8 * pass;
-    k_rs_upsweep<<<ws.tiles, 256, 0, s>>>(kin, n, shift, ws.tiles, ws.hist);
-    HCG_CHECK_LAUNCH("k_rs_upsweep");
-    k_rs_scan_rows<<<256, 256, 0, s>>>(ws.hist, ws.tiles, ws.digit);
-    HCG_CHECK_LAUNCH("k_rs_scan_rows");
-    k_rs_scan_digits<<<1, 256, 0, s>>>(ws.digit);
-    HCG_CHECK_LAUNCH("k_rs_scan_digits");
-    k_rs_downsweep<<<ws.tiles, 256, 0, s>>>(kin, vin, kout, vout, n, shift, ws.tiles, ws.hist, ws.digit);
+// Keys, the radix passes and the sentinel, on workspace `ws` (n > 0).
+template <uint32_t THREADS, uint32_t ITEMS>
+int presort_enqueue_as(const hcg_healpix* hp, uint32_t n, const double* lon_deg, const double* lat_deg,
+                       uint32_t* keys_sorted, uint32_t* perm, const SortWorkspace& ws, hipStream_t s) {
+  const uint32_t npix = (uint32_t)hp->npix, tiles = ws.tiles;
+  int bits = 1;
+  while ((npix >> bits) != 0) ++bits;  // keys sort as 0 .. npix
+  const int passes = bits <= 2 * kMaxDigitBits ? 2 : 3;
+  // the last pass writes keys_sorted and perm
+  uint32_t *kin = passes == 2 ? keys_sorted : ws.keys_b, *vin = passes == 2 ? perm : ws.vals_b;
+  uint32_t *kout = passes == 2 ? ws.keys_b : keys_sorted, *vout = passes == 2 ? ws.vals_b : perm;
+  Digit g{npix, 0, 0};
+  for (int pass = 0; pass < passes; ++pass) {
+    g.shift += g.bits;
+    g.bits = (bits - g.shift + passes - pass - 1) / (passes - pass);
+    if (pass == 0) {
+      k_keys<THREADS, ITEMS>
+          <<<sort_blocks(tiles), THREADS, 0, s>>>(*hp, n, lon_deg, lat_deg, kin, keys_sorted + n, g, tiles, ws.hist);
+      HCG_CHECK_LAUNCH("k_keys");
+    } else {
+      k_rs_upsweep<THREADS, ITEMS><<<sort_blocks(tiles), THREADS, 0, s>>>(kin, n, g, tiles, ws.hist);
+      HCG_CHECK_LAUNCH("k_rs_upsweep");
+    }
+    k_rs_scan<<<1u << g.bits, 256, 0, s>>>(ws.hist, tiles, ws.digit);
+    HCG_CHECK_LAUNCH("k_rs_scan");
+    if (pass == 0)
+      k_rs_downsweep<THREADS, ITEMS, true>
+          <<<sort_blocks(tiles), THREADS, 0, s>>>(kin, vin, kout, vout, n, g, tiles, ws.hist, ws.digit);
+    else
+      k_rs_downsweep<THREADS, ITEMS, false>
+          <<<sort_blocks(tiles), THREADS, 0, s>>>(kin, vin, kout, vout, n, g, tiles, ws.hist, ws.digit);
     HCG_CHECK_LAUNCH("k_rs_downsweep");
     std::swap(kin, kout);
     std::swap(vin, vout);
   }
-  // four passes: the result is back in keys_sorted / perm
-  k_set_sentinel<<<1, 64, 0, s>>>(keys_sorted, n, (uint32_t)hp->npix);
-  HCG_CHECK_LAUNCH("k_set_sentinel");
   return HCG_OK;
+}
+
+int presort_enqueue(const hcg_healpix* hp, uint32_t n, const double* lon_deg, const double* lat_deg,
+                    uint32_t* keys_sorted, uint32_t* perm, const SortWorkspace& ws, hipStream_t s) {
+  switch (sort_tile_of(n)) {
+    case kSmallTile: return presort_enqueue_as<256, 4>(hp, n, lon_deg, lat_deg, keys_sorted, perm, ws, s);
+    case kMidTile: return presort_enqueue_as<256, 8>(hp, n, lon_deg, lat_deg, keys_sorted, perm, ws, s);
+    default: return presort_enqueue_as<512, 16>(hp, n, lon_deg, lat_deg, keys_sorted, perm, ws, s);
+  }
 }
 
 // The no-allocation variant's scratch: one sort workspace for up to
@@ -428,10 +568,8 @@ extern "C" int hcg_ring_lut(const hcg_healpix* hp, uint32_t n, const uint32_t* k
   if (hp->nside == 0 || hp->nside > HCG_MAX_NSIDE)
     return set_error(HCG_ERR_UNSUPPORTED, "hcg_ring_lut: nside must be <= 8192");
   hipStream_t s = as_stream(stream);
-  k_ring_meta<<<1, 64, 0, s>>>(*hp, n, keys_sorted, meta);
-  HCG_CHECK_LAUNCH("k_ring_meta");
   const uint32_t threads = (uint32_t)hp->nrings + 1;
-  k_ring_lut<<<ceil_div_u32(threads, 256), 256, 0, s>>>(*hp, keys_sorted, meta, lut, ring_z, ring_s);
+  k_ring_lut<<<ceil_div_u32(threads, 256), 256, 0, s>>>(*hp, n, keys_sorted, meta, lut, ring_z, ring_s);
   HCG_CHECK_LAUNCH("k_ring_lut");
   return HCG_OK;
 }

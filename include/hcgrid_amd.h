@@ -144,7 +144,7 @@ int hcg_presort(const hcg_healpix *hp, uint32_t n, const double *lon_deg, const 
  * hipMalloc, hipFree or allocating library call): no counterpart in the
  * reference; for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid it).  The
- * sort's scratch is a static device array of the library (66 MiB per GPU,
+ * sort's scratch is a static device array of the library (68 MiB per GPU,
  * held until the process ends), so n <= HCG_PRESORT_NOALLOC_MAX_N
  * (2^23 = 8388608 samples); larger n is rejected with
  * HCG_ERR_UNSUPPORTED.  Results equal hcg_presort's bit for bit.  Every
