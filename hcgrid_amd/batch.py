@@ -4,8 +4,8 @@
 A Geometry is one map's sorted samples, ring LUT and target coordinates in
 HBM; building it is the pre-sort of the reference's init_input_with_cpu
 (HCGrid/gridding.cu:70-147) done on the device.  A Batch grids many
-(geometry, channel values, cube) jobs of uneven sizes in one persistent
-launch.  A Graph captures any sequence of these on a stream and replays it.
+(geometry, channel values, cube) jobs of uneven sizes in a few
+launches.  A Graph captures any sequence of these on a stream and replays it.
 torch only allocates device memory and provides streams.
 """
 from __future__ import annotations

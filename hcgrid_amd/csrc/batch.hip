@@ -1,16 +1,16 @@
-// batch.hip -- resident geometries, batched multi-channel gridding in one
-// persistent launch, and HIP graph capture of the whole sequence.
+// batch.hip -- resident geometries, batched multi-channel gridding, and HIP
+// graph capture of the whole sequence.
 //
 // The reference grids one map per process run (HCGrid/HCGrid.cpp:38-197;
 // HCGrid+ loops over channels of one map, HCGrid+/gridding-omp.cu:552-678).
 // Here a geometry (one map's sorted samples, ring LUT and target
 // coordinates) is built once and kept in HBM; a batch names any number of
 // (geometry, channel values, output cube) jobs of uneven sizes and grids
-// them with one launch of k_grid_mfma_batch, whose workgroups pull (job,
-// tile, channel group) items from a device queue, and one launch per tile
-// route (one- and few-channel jobs).  Everything a batch
-// enqueues is kernels only (no memsets, no host copies), so the sequence
-// can be captured into a graph and replayed.
+// them with one launch per kind of job in it (kernel instance of the
+// contraction by value type and channel count, or tile route of one- and
+// few-channel jobs).  Everything a batch enqueues is kernels only (no
+// memsets, no host copies), so the sequence can be captured into a graph and
+// replayed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -49,22 +49,19 @@ struct hcg_geometry {
 struct hcg_batch {
   int device;
   bool owns;             // base was allocated here (freed by destroy)
-  uint32_t njobs, nitems, waves, chunk, blocks;
-  uint32_t nitems_dense, blocks_dense;  // the dense jobs' launch (kDenseWaves, kDenseChunk), run first
+  uint32_t njobs, waves, chunk;
   size_t bytes;
   void* base;
   MfmaJob* d_jobs;
-  MfmaItem* d_items;
-  uint32_t* d_counters;  // [0] queue head, [1 + j] non-finite values of job j, [1 + njobs] dense queue head
-  PrepRange* d_ranges;   // the prep launch: every job's channel gather and tile plan
+  uint32_t* d_counters;  // [j] non-finite values of job j
+  PrepRange* d_ranges;   // the prep launch: every job's channel gather
   PrepJob* d_prep;
   uint32_t nranges, prep_blocks;
-  TileRange* d_tiles;    // the tile-route jobs: every route's ranges, route after route
+  TileRange* d_tiles;    // every route's ranges, route after route
   uint32_t tile_first[kRoutes + 1], tile_blocks[kRoutes];
   std::vector<hcg_batch_job> jobs;
   std::vector<void*> values_sorted;
   std::vector<MfmaJob> host_jobs;     // upload sources, alive until destroy
-  std::vector<MfmaItem> host_items;
   std::vector<PrepRange> host_ranges;
   std::vector<PrepJob> host_prep;
   std::vector<TileRange> host_tiles;
@@ -115,9 +112,9 @@ __global__ void __launch_bounds__(256) k_fill_u32(uint32_t* p, uint32_t count, u
   if (i < count) p[i] = v;
 }
 
-// Rough cost of one work item of a job: samples in a tile's neighbourhood
-// times (channels in the item + a fixed weight-evaluation share).
-double item_cost(const hcg_geometry* g, uint32_t tile_cols, uint32_t chans) {
+// Rough cost of one workgroup of a job: samples in a block's neighbourhood
+// times (channels in the group + a fixed weight-evaluation share).
+double group_cost(const hcg_geometry* g, uint32_t tile_cols, uint32_t chans) {
   const double side = g->side, tc = tile_cols, tr = 64.0 / tile_cols;
   const double cell_deg = 0.01;  // only the ratio between jobs matters
   const double d = 2.0 * g->kern.sphere_radius / cell_deg;
@@ -243,29 +240,20 @@ extern "C" size_t hcg_batch_job_bytes(const hcg_geometry* g, uint32_t nchan) {
 
 namespace {
 
-// A batch's plan: work items and the layout of its one device allocation.
-// Dense MFMA jobs (at least kDenseSamplesPerCell samples per map cell), and
-// jobs with more channels than one channel group of the batch's shape
-// holds, run in a persistent launch of their own at 8 waves and 512-sample
-// chunks, the shape that suits them (one workgroup per CU sharing each
-// block's weights over 512 channels): a 3.9M-sample 128^2 x 512-channel job
-// takes 18.2 ms there against 26.7 ms at 4 waves / 256, a 3.2M-sample
-// 2048^2 x 512-channel one 21.6 against 24.5, while sparse jobs with one
-// channel group run up to 1.8x slower at 8 waves.  Results do not depend on
-// the launch shape.
-constexpr double kDenseSamplesPerCell = 32.0;
-constexpr uint32_t kDenseWaves = 8, kDenseChunk = 512;
-
+// A batch's plan: its launches and the layout of its one device allocation.
 struct BatchPlan {
   uint32_t waves = 0, chunk = 0;
-  uint32_t n_dense = 0;  // the first n_dense items belong to the dense launch
-  std::vector<MfmaItem> items;
   std::vector<uint32_t> tiles, tcols, route;
-  std::vector<TileRange> tile_ranges;                 // tile-route jobs, route after route
+  std::vector<TileRange> tile_ranges;                 // route after route
   uint32_t tile_first[kRoutes + 1] = {}, tile_blocks[kRoutes] = {};
-  std::vector<size_t> voff, poff;
+  std::vector<size_t> voff, poff;  // sorted channel values; plans
   size_t bytes = 0;
 };
+
+GridBuffers buffers_of(const hcg_geometry* g) {
+  return GridBuffers{g->rec,    g->keys, g->lon_s, g->lat_s, nullptr, g->lut, g->ring_z,
+                     g->ring_s, g->meta, g->xwcs,  g->ywcs,  nullptr, nullptr};
+}
 
 int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32_t chunk, BatchPlan& p) {
   HCG_REQUIRE(njobs == 0 || jobs, "hcg_batch_create: NULL jobs");
@@ -285,15 +273,12 @@ int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32
   }
   p.waves = waves;
   p.chunk = chunk;
-  // work items: jobs longest item first, each job's tiles in order, a
-  // tile's channel groups adjacent (they share the tile's samples in L2)
-  std::vector<uint32_t> order(njobs), groups(njobs), units(njobs);
-  std::vector<char> dense(njobs, 0);
-  std::vector<double> cost(njobs);
+  std::vector<uint32_t> order(njobs);
+  std::vector<uint64_t> blocks(njobs, 0);
+  std::vector<double> cost(njobs, 0.0);
   p.tiles.assign(njobs, 0);
   p.tcols.assign(njobs, 0);
   p.route.assign(njobs, kRouteMfma);
-  uint64_t nitems = 0;
   for (uint32_t j = 0; j < njobs; ++j) {
     const hcg_batch_job& b = jobs[j];
     const hcg_geometry* g = b.geometry;
@@ -301,55 +286,41 @@ int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32
     order[j] = j;
     const GridParams P = make_grid_params(&g->hp, &g->kern, side);
     p.route[j] = route_of(P, g->kern.kernel_type, false, b.nchan, g->n);
-    if (p.route[j] != kRouteMfma) {  // FP64 tile loop: a workgroup per tile, in its route's own launch
+    if (p.route[j] != kRouteMfma) {  // FP64 tile loop: a workgroup per tile
       p.tcols[j] = kTileCols;
-      p.tiles[j] = side ? tile_count_of(side) : 0;
-      groups[j] = 1;
-      units[j] = 0;
+      blocks[j] = p.tiles[j] = side ? tile_count_of(side) : 0;
     } else {
       const uint32_t tc = b.tile_cols ? b.tile_cols : kMcDefaultTileCols;
       p.tcols[j] = tc;
       p.tiles[j] = (b.nchan && side) ? ceil_div_u32(side, tc) * ceil_div_u32(side, 64 / tc) : 0;
-      // dense, or more channels than one channel group at the batch's shape
-      // covers (each group recomputes the block's weights)
-      dense[j] = waves != kDenseWaves && side &&
-                 ((double)g->n >= kDenseSamplesPerCell * side * side || b.nchan > waves * kMcChanPerWave);
-      const uint32_t w = dense[j] ? kDenseWaves : waves;
-      groups[j] = ceil_div_u32(ceil_div_u32(b.nchan, kMcChanPerWave), w);
-      units[j] = p.tiles[j];
-      cost[j] = item_cost(g, tc, std::min<uint32_t>(b.nchan, w * kMcChanPerWave));
+      MfmaJob J{};
+      J.kt = mfma_weight_form(P, g->kern.kernel_type);
+      J.nchan = b.nchan;
+      J.dtype = (uint32_t)b.dtype;
+      J.ntiles = p.tiles[j];
+      p.route[j] = kRouteMfma + mfma_instance(J);
+      blocks[j] = p.tiles[j] ? mfma_blocks(J) : 0;
+      cost[j] = group_cost(g, tc, std::min<uint32_t>(b.nchan, 256u));
     }
-    nitems += (uint64_t)units[j] * groups[j];
   }
-  if (nitems >= 0xFFFFFFFFull) return set_error(HCG_ERR_INVALID, "hcg_batch_create: too many work items");
-  for (uint32_t r = kRouteMfma + 1; r < kRoutes; ++r) {
+  // a launch's workgroups start in order: its jobs with the longest ones first
+  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return cost[a] > cost[b]; });
+  for (uint32_t r = 0; r < kRoutes; ++r) {
     p.tile_first[r] = (uint32_t)p.tile_ranges.size();
-    uint64_t blocks = 0;
-    for (uint32_t j = 0; j < njobs; ++j)
-      if (p.route[j] == r && p.tiles[j]) {
-        p.tile_ranges.push_back(TileRange{(uint32_t)blocks, j});
-        blocks += p.tiles[j];
+    uint64_t total = 0;
+    for (uint32_t j : order)
+      if (p.route[j] == r && blocks[j]) {
+        p.tile_ranges.push_back(TileRange{(uint32_t)total, j});
+        total += blocks[j];
+        if (total >= 0x7FFFFFFFull) return set_error(HCG_ERR_INVALID, "hcg_batch_create: too many tiles");
       }
-    if (blocks >= 0x7FFFFFFFull) return set_error(HCG_ERR_INVALID, "hcg_batch_create: too many tiles");
-    p.tile_blocks[r] = (uint32_t)blocks;
+    p.tile_blocks[r] = (uint32_t)total;
   }
   p.tile_first[kRoutes] = (uint32_t)p.tile_ranges.size();
-  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return cost[a] > cost[b]; });
-  p.items.clear();
-  p.items.reserve(nitems);
-  for (int pass = 0; pass < 2; ++pass) {  // the dense launch's items first
-    for (uint32_t j : order) {
-      if (dense[j] != (pass == 0)) continue;
-      for (uint32_t t = 0; t < units[j]; ++t)
-        for (uint32_t g = 0; g < groups[j]; ++g) p.items.push_back(MfmaItem{j, t, g, 0});
-    }
-    if (pass == 0) p.n_dense = (uint32_t)p.items.size();
-  }
-  // one allocation: job table, items, counters, sorted channel values
+  // one allocation: job table, counters, ranges, sorted channel values
   Carver c{nullptr};
   c.take<MfmaJob>(njobs ? njobs : 1);
-  c.take<MfmaItem>(p.items.empty() ? 1 : p.items.size());
-  c.take<uint32_t>(2 + njobs);
+  c.take<uint32_t>(njobs ? njobs : 1);
   c.take<PrepRange>(2 * (size_t)njobs + 1);
   c.take<PrepJob>(njobs ? njobs : 1);
   c.take<TileRange>(njobs ? njobs : 1);
@@ -359,13 +330,14 @@ int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32
     p.voff[j] = c.off;
     c.off += hcg_batch_job_bytes(jobs[j].geometry, jobs[j].nchan);
     p.poff[j] = c.off;
-    if (p.route[j] == kRouteMfma) c.off = align_up(c.off + (size_t)p.tiles[j] * kPlanTileWords * sizeof(uint32_t));
+    if (p.route[j] >= kRouteMfma && mfma_uses_plan(p.route[j] - kRouteMfma))
+      c.off = align_up(c.off + p.tiles[j] * kPlanBytes);
   }
   p.bytes = c.off;
   return HCG_OK;
 }
 
-// Lays the batch out in `mem` and uploads the job table and work list:
+// Lays the batch out in `mem` and uploads the job table and ranges:
 // asynchronously on `stream` when upload_async, else synchronously.
 int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, void* mem, bool owns,
                bool upload_async, hipStream_t stream, hcg_batch** out) {
@@ -374,8 +346,6 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
   bt->njobs = njobs;
   bt->waves = p.waves;
   bt->chunk = p.chunk;
-  bt->nitems = (uint32_t)p.items.size();
-  bt->nitems_dense = p.n_dense;
   bt->bytes = p.bytes;
   bt->base = mem;
   bt->owns = owns;
@@ -383,8 +353,7 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
   (void)hipGetDevice(&bt->device);
   Carver d{static_cast<char*>(bt->base)};
   bt->d_jobs = d.take<MfmaJob>(njobs ? njobs : 1);
-  bt->d_items = d.take<MfmaItem>(p.items.empty() ? 1 : p.items.size());
-  bt->d_counters = d.take<uint32_t>(2 + njobs);
+  bt->d_counters = d.take<uint32_t>(njobs ? njobs : 1);
   bt->d_ranges = d.take<PrepRange>(2 * (size_t)njobs + 1);
   bt->d_prep = d.take<PrepJob>(njobs ? njobs : 1);
   bt->d_tiles = d.take<TileRange>(njobs ? njobs : 1);
@@ -394,16 +363,13 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
   bt->values_sorted.resize(njobs);
   std::vector<MfmaJob>& hj = bt->host_jobs;
   hj.resize(njobs);
-  bt->host_items = p.items;
   for (uint32_t j = 0; j < njobs; ++j) {
     const hcg_batch_job& b = jobs[j];
     const hcg_geometry* g = b.geometry;
     bt->values_sorted[j] = static_cast<char*>(bt->base) + p.voff[j];
-    GridBuffers B{g->rec,  g->keys, g->lon_s, g->lat_s, nullptr, g->lut, g->ring_z,
-                  g->ring_s, g->meta, g->xwcs,  g->ywcs,  nullptr, nullptr};
     const GridParams P = make_grid_params(&g->hp, &g->kern, g->side);
     hj[j] = MfmaJob{P,
-                    B,
+                    buffers_of(g),
                     bt->values_sorted[j],
                     b.cube,
                     b.wsum,
@@ -415,15 +381,15 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
                     ceil_div_u32(g->side, p.tcols[j]),
                     p.tiles[j],
                     (uint32_t)(b.normalize ? 1 : 0),
-                    p.route[j] != kRouteMfma
-                        ? nullptr
-                        : reinterpret_cast<uint32_t*>(static_cast<char*>(bt->base) + p.poff[j])};
+                    p.route[j] >= kRouteMfma && mfma_uses_plan(p.route[j] - kRouteMfma)
+                        ? static_cast<char*>(bt->base) + p.poff[j]
+                        : nullptr};
   }
   // the prep launch: gathers (channel-major values) and plans of every job
   bt->host_prep.resize(njobs);
   std::vector<uint32_t> layouts(njobs, 0u);
   for (uint32_t j = 0; j < njobs; ++j)
-    bt->host_prep[j] = PrepJob{jobs[j].values, jobs[j].geometry->perm, bt->d_counters + 1 + j, jobs[j].geometry->n, 0u};
+    bt->host_prep[j] = PrepJob{jobs[j].values, jobs[j].geometry->perm, bt->d_counters + j, jobs[j].geometry->n, 0u};
   int prc = prep_ranges(njobs, hj.data(), layouts.data(), bt->host_ranges, &bt->prep_blocks);
   if (prc != HCG_OK) {
     if (owns) (void)hipFree(bt->base);
@@ -432,14 +398,12 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
   }
   bt->nranges = (uint32_t)bt->host_ranges.size();
   hipError_t e = hipSuccess;
-  const size_t jb = njobs * sizeof(MfmaJob), ib = p.items.size() * sizeof(MfmaItem);
+  const size_t jb = njobs * sizeof(MfmaJob);
   const size_t rb = bt->host_ranges.size() * sizeof(PrepRange), pb = njobs * sizeof(PrepJob);
   const size_t tb = bt->host_tiles.size() * sizeof(TileRange);
   if (upload_async) {
     // ordered on `stream`; the host sources live in the batch until destroy
     if (jb) e = hipMemcpyAsync(bt->d_jobs, hj.data(), jb, hipMemcpyHostToDevice, stream);
-    if (e == hipSuccess && ib)
-      e = hipMemcpyAsync(bt->d_items, bt->host_items.data(), ib, hipMemcpyHostToDevice, stream);
     if (e == hipSuccess && rb)
       e = hipMemcpyAsync(bt->d_ranges, bt->host_ranges.data(), rb, hipMemcpyHostToDevice, stream);
     if (e == hipSuccess && pb) e = hipMemcpyAsync(bt->d_prep, bt->host_prep.data(), pb, hipMemcpyHostToDevice, stream);
@@ -447,16 +411,12 @@ int batch_init(uint32_t njobs, const hcg_batch_job* jobs, const BatchPlan& p, vo
       e = hipMemcpyAsync(bt->d_tiles, bt->host_tiles.data(), tb, hipMemcpyHostToDevice, stream);
   } else {
     if (jb) e = hipMemcpy(bt->d_jobs, hj.data(), jb, hipMemcpyHostToDevice);
-    if (e == hipSuccess && ib) e = hipMemcpy(bt->d_items, p.items.data(), ib, hipMemcpyHostToDevice);
     if (e == hipSuccess && rb) e = hipMemcpy(bt->d_ranges, bt->host_ranges.data(), rb, hipMemcpyHostToDevice);
     if (e == hipSuccess && pb) e = hipMemcpy(bt->d_prep, bt->host_prep.data(), pb, hipMemcpyHostToDevice);
     if (e == hipSuccess && tb) e = hipMemcpy(bt->d_tiles, bt->host_tiles.data(), tb, hipMemcpyHostToDevice);
   }
   int rc = HCG_OK;
   if (e != hipSuccess) rc = set_error(HCG_ERR_HIP, std::string("hcg_batch_create: ") + hipGetErrorString(e));
-  // grid size of the persistent launch, fixed here so that enqueueing makes no queries
-  if (rc == HCG_OK) rc = mfma_batch_blocks(p.chunk, p.waves, &bt->blocks);
-  if (rc == HCG_OK && bt->nitems_dense) rc = mfma_batch_blocks(kDenseChunk, kDenseWaves, &bt->blocks_dense);
   if (rc != HCG_OK) {
     if (owns) (void)hipFree(bt->base);
     delete bt;
@@ -514,27 +474,19 @@ extern "C" int hcg_batch_enqueue(hcg_batch* b, void* stream) {
     timing = cs == hipStreamCaptureStatusNone;
   }
   if (timing) HCG_CHECK_HIP(hipEventRecord(b->ev[0], s));
-  const uint32_t nc = 2 + b->njobs;
-  k_fill_u32<<<ceil_div_u32(nc, 256), 256, 0, s>>>(b->d_counters, nc, 0u);
-  HCG_CHECK_LAUNCH("k_fill_u32");
-  // every job's channel gather and tile plan, one launch
+  if (b->njobs) {
+    k_fill_u32<<<ceil_div_u32(b->njobs, 256), 256, 0, s>>>(b->d_counters, b->njobs, 0u);
+    HCG_CHECK_LAUNCH("k_fill_u32");
+  }
+  // every job's channel gather, one launch
   int rc = launch_batch_prep(b->d_ranges, b->nranges, b->prep_blocks, b->d_prep, b->d_jobs, s);
   if (rc != HCG_OK) return rc;
   if (timing) HCG_CHECK_HIP(hipEventRecord(b->ev[1], s));
-  for (uint32_t r = kRouteMfma + 1; r < kRoutes; ++r) {
-    rc = launch_batch_tiles(r, b->d_tiles + b->tile_first[r], b->tile_first[r + 1] - b->tile_first[r],
-                            b->tile_blocks[r], b->d_jobs, s);
-    if (rc != HCG_OK) return rc;
-  }
-  // the dense jobs' launch (its own queue head after the job counters), then the rest
-  if (b->nitems_dense) {
-    rc = launch_mfma_batch(kDenseChunk, kDenseWaves, b->blocks_dense, b->d_jobs, b->d_items, b->nitems_dense,
-                           b->d_counters + 1 + b->njobs, s);
-    if (rc != HCG_OK) return rc;
-  }
-  if (b->nitems != b->nitems_dense) {
-    rc = launch_mfma_batch(b->chunk, b->waves, b->blocks, b->d_jobs, b->d_items + b->nitems_dense,
-                           b->nitems - b->nitems_dense, b->d_counters, s);
+  for (uint32_t r = 0; r < kRoutes; ++r) {
+    const TileRange* ranges = b->d_tiles + b->tile_first[r];
+    const uint32_t nr = b->tile_first[r + 1] - b->tile_first[r];
+    rc = r < kRouteMfma ? launch_batch_tiles(r, ranges, nr, b->tile_blocks[r], b->d_jobs, s)
+                        : launch_mfma_batch(r - kRouteMfma, ranges, nr, b->tile_blocks[r], b->d_jobs, s);
     if (rc != HCG_OK) return rc;
   }
   if (timing) {
@@ -570,9 +522,9 @@ extern "C" int hcg_batch_last_times(hcg_batch* b, float* prep_ms, float* grid_ms
 extern "C" int hcg_batch_info(const hcg_batch* b, hcg_batch_stats* st) {
   HCG_REQUIRE(b && st, "hcg_batch_info: NULL argument");
   st->njobs = b->njobs;
-  st->nitems = b->nitems;
+  st->nitems = 0;
   for (uint32_t t : b->tile_blocks) st->nitems += t;
-  st->blocks = b->blocks;
+  st->blocks = st->nitems;
   st->waves = b->waves;
   st->chunk = b->chunk;
   st->reserved = 0;
@@ -584,7 +536,7 @@ extern "C" int hcg_batch_nonfinite(const hcg_batch* b, uint32_t* counts, void* s
   HCG_REQUIRE(b && counts, "hcg_batch_nonfinite: NULL argument");
   if (b->njobs == 0) return HCG_OK;
   hipStream_t s = as_stream(stream);
-  HCG_CHECK_HIP(hipMemcpyAsync(counts, b->d_counters + 1, b->njobs * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  HCG_CHECK_HIP(hipMemcpyAsync(counts, b->d_counters, b->njobs * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   HCG_CHECK_HIP(hipStreamSynchronize(s));
   return HCG_OK;
 }

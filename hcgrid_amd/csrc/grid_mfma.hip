@@ -6,28 +6,33 @@
 // The selection and weights do not depend on the channel, so here they are
 // computed once per (cell, sample) pair in FP64 and the channel sums become
 //     cube[ch][cell] = sum_s W[cell][s] * V[ch][s]   (FP32 accumulation)
-// evaluated with v_mfma_f32_16x16x32_{bf16,f16}: W (cells x samples) in LDS,
-// V (channels x sorted samples) streamed from HBM.  Each FP64 weight is
-// carried as hi + lo, two values of the channel type (hi = round(w),
-// lo = round(w - hi)), and both are contracted: the weight keeps ~2x the
-// type's significand (relative error ~2^-17 for BF16) at twice the MFMA
-// count, which the kernel's HBM/L2 stream of V hides.
+// evaluated with v_mfma_f32_16x16x32_{bf16,f16}.  Each FP64 weight is carried
+// as hi + lo, two values of the channel type (hi = round(w), lo = round(w -
+// hi)), and both are contracted: the weight keeps ~2x the type's significand
+// (relative error ~2^-17 for BF16) at twice the MFMA count.
 //
-// Work decomposition: a workgroup owns a block of 64 cells (TR rows x TC
-// columns; 4 MFMA row blocks of 16 cells) and up to 8 x 64 channels (wave
-// w: 4 blocks of 16 channels; 4 row blocks x 4 channel blocks x 4 = 64 FP32
-// accumulators per lane).  Wider channel ranges take more workgroups along
-// grid.y.  For every non-empty ring of the block's ring range:
-//   1. each cell's [lpix, rpix] window (the reference's compat selection);
-//   2. the union window's sorted range by a 64-way cooperative key search;
-//   3. per chunk of <= CHUNK samples: stage unit vectors and keys in LDS,
-//      zero the weight tiles, let every cell's threads fill its band with
-//      the FP64-decided weights (as hi + lo; the sum of the rounded pairs is
-//      the normalisation, so numerator and denominator use the same
-//      weights), record each row block's k-block span;
-//   4. MFMA over the union's 32-sample k-blocks: B (16 channels x 32
-//      samples) is loaded once per k-block and applied to every row block
-//      whose span covers it.
+// A workgroup owns a block of 64 cells, four squares of 16.  A square's
+// samples are the 8-sample blocks of its rings' sorted ranges, each ring
+// narrowed to its windows and to what the radius reaches; 32 at a time
+// (a k-block) they are staged in LDS, and lane l evaluates the weights of
+// cell l % 16 and samples 8 (l / 16) .. + 7: exactly its A operand, in
+// registers, every pair of the 16 x 32 (45% of them selected on rasters of
+// two and more samples per cell).  mfma_tile is a wave per square, without
+// barriers, for up to 256 channels; mfma_wide shares a block's weights over
+// 512 channels through LDS.
+//
+// What counts is vector instructions (FP64 weights), then the latency of the
+// LDS reads and weight chains at two to four waves per SIMD.  Before, weights
+// went through a row-major LDS tile (cleared, each cell's band searched and
+// filled by lane = cell, 44% of the lanes on selected pairs) between four
+// workgroup barriers per 128-512 samples, one wave contracting while the
+// rest waited on small jobs.  A pass before and now: 195k samples x 3
+// channels onto 500^2 911 -> 194 us; 482k x 67 onto 511^2 1316 -> 495 us;
+// 300k x 16 onto 2048^2 3337 -> 1395 us; 1.2M x 64 onto 512^2 (new
+// coordinates) 2697 -> 1511 us; 2M x 1024 onto 1024^2 9526 -> 8716 us (this
+// kernel 7.40 -> 6.64 ms: 1.39e9 vector and 2.0e8 MFMA instructions, 64% of
+// the wave cycles waiting at two waves per SIMD).
+//
 // Selection, FP64 distance and weight follow the single-channel kernel
 // exactly; only the products with channel values run in BF16/FP16.
 #include <hip/hip_runtime.h>
@@ -42,22 +47,17 @@ namespace hcg {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 
 typedef short s16x8_t __attribute__((ext_vector_type(8)));  // a raw 16-byte MFMA operand
 
-// Channel type of a kernel instance: fixed at compile time (one-job
-// launches) or read from the job descriptor (the batched launch, whose jobs
-// may mix BF16 and FP16).  Values and weights are kept as raw 16-bit words;
-// the type matters only where a weight is rounded and where the MFMA issues.
-enum : int { kDtBf16 = 0, kDtF16 = 1, kDtAny = 2 };
-
-template <int DT>
-__device__ inline bool dt_is_bf16(uint32_t dtype) {
-  if constexpr (DT == kDtBf16) return true;
-  else if constexpr (DT == kDtF16) return false;
-  else return dtype == HCG_DTYPE_BF16;
-}
+// Channel type of a kernel instance.  Values and weights are kept as raw
+// 16-bit words; the type matters only where a weight is rounded and where
+// the MFMA issues.
+enum : int { kDtBf16 = 0, kDtF16 = 1 };
 
 __device__ inline f32x4_t mfma16(bool bf, s16x8_t a, s16x8_t b, f32x4_t c) {
   if (bf)
@@ -65,17 +65,6 @@ __device__ inline f32x4_t mfma16(bool bf, s16x8_t a, s16x8_t b, f32x4_t c) {
                                                    c, 0, 0, 0);
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
                                                 0, 0, 0);
-}
-
-// One k-block of B for kMcNB channel blocks, 16 bytes per lane per block.
-// The sorted channel values are blocked by kVB = 8 samples ([nchan][8] per
-// block): lane l's operand is 8 samples of one channel, a row of the value
-// block of its k-group (l / 16) in the k-block, so `blk` points at that
-// value block and lofs[nb] = 16 x the lane's channel; the 16 lanes of a
-// k-group read one contiguous 256-byte piece per channel block.
-__device__ inline void load_b_rows(s16x8_t* b, const char* blk, const uint32_t* lofs) {
-#pragma unroll
-  for (int nb = 0; nb < kMcNB; ++nb) b[nb] = *reinterpret_cast<const s16x8_t*>(blk + lofs[nb]);
 }
 
 // FP64 weight of a selected pair (the single-channel kernel's evaluation).
@@ -92,816 +81,1070 @@ __device__ inline double pair_weight_any(const GridParams& P, const GridBuffers&
                                           B.lat_s, 0.25 * c2, cell, i);
 }
 
-// Block geometry, lane l = cell l of a (64 >> tc_shift) x (1 << tc_shift)
-// block at (y0, x0): the cell's window (its anchor's, HCGrid/gridding.cu:306-323)
-// and unit vector q, and the block's ring span [ur, dr] (a wave reduction;
-// ur > dr when no cell has rings), first used ring excluded.
-__device__ inline Window block_cell_window(const GridParams& P, const GridBuffers& B, const hcg_ring_meta& m,
-                                           uint32_t y0, uint32_t x0, uint32_t tc_shift, uint32_t lane, double q[3],
-                                           uint32_t& ur, uint32_t& dr) {
-  const uint32_t tc_mask = (1u << tc_shift) - 1u;
-  const uint32_t rl = y0 + (lane >> tc_shift), cl = x0 + (lane & tc_mask);
-  const bool lv = cl < P.side && rl < P.side;
-  const uint32_t celll = lv ? rl * P.side + cl : 0;
-  const uint32_t anchor = lv ? rl * P.side + (cl / P.factor) * P.factor : 0;
-  Window win = window_of(P, m.firstring, m.usedrings, B.xwcs[anchor], B.ywcs[anchor]);
-  if (!lv || m.usedrings == 0) {
-    win.uring = 1;
-    win.dring = 0;
-  }
-  double sb, cb0, sn, cs;
-  sincos(B.ywcs[celll] * kDeg2Rad, &sb, &cb0);
-  sincos(B.xwcs[celll] * kDeg2Rad, &sn, &cs);
-  q[0] = cb0 * cs;
-  q[1] = cb0 * sn;
-  q[2] = sb;
-  const bool has = win.uring <= win.dring;
-  ur = wave_min_u32(has ? win.uring : 0xFFFFFFFFu);
-  dr = wave_max_u32(has ? win.dring : 0u);
-  if (ur == m.firstring && skips_first_ring(P)) ++ur;  // the first used ring contributes nothing (start_int - 1 wraps)
-  return win;
+// The tested distance of a pair: h = 1 - p.q (LEAN), or c2 = |p - q|^2 (np = -p).
+template <bool LEAN>
+__device__ inline double pair_distance(double npx, double npy, double npz, double x, double y, double z) {
+  if constexpr (LEAN) return fma(npx, x, fma(npy, y, fma(npz, z, 1.0)));
+  const double dx = npx + x, dy = npy + y, dz = npz + z;
+  return fma(dx, dx, fma(dy, dy, dz * dz));
 }
 
-// A cell's [lpix, rpix] in ring r (HCGrid/gridding.cu:334-360); (1, 0) when
-// the cell takes no samples from the ring.
-__device__ inline void ring_cell_window(const GridParams& P, const GridBuffers& B, const hcg_ring_meta& m,
-                                        const Window& win, uint32_t r, uint32_t& lp, uint32_t& rp) {
-  const uint32_t kr = r - m.firstring;
+// Four consecutive doubles (32-byte aligned), two 16-byte reads.
+__device__ inline void lds_read4(const double* p, double (&v)[4]) {
+  const double2 a = *reinterpret_cast<const double2*>(p), b = *reinterpret_cast<const double2*>(p + 2);
+  v[0] = a.x;
+  v[1] = a.y;
+  v[2] = b.x;
+  v[3] = b.y;
+}
+
+// Two FP32 values rounded to 16 bits (nearest even) in one word, and back.
+template <bool BF>
+__device__ inline uint32_t round16x2(f32x2_t v) {
+  if constexpr (BF)
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+  else
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
+}
+template <bool BF>
+__device__ inline f32x2_t widen16x2(uint32_t w) {
+  if constexpr (BF)
+    return f32x2_t{__uint_as_float(w << 16), __uint_as_float(w & 0xFFFF0000u)};
+  else
+    return __builtin_convertvector(__builtin_bit_cast(f16x2_t, w), f32x2_t);
+}
+
+// The cells of a wave's square: their extent in latitude and longitude, for
+// narrowing each ring to what the radius reaches (block_ring_range).
+struct BlockSpan {
+  TileSpan T;
+  bool simple;          // every window is one pair of half-pixel numbers (belt_window), every ring a belt ring
+  uint32_t hlo, hhi;    // simple: the outermost of them
+  bool chord;           // the extents below hold
+  double bmin, bmax;    // latitudes, radians
+  double tmin, tmax;    // longitudes, units of pi/2 in [0, 4)
+  double cmin;          // the smallest cos latitude
+};
+
+constexpr uint32_t kNoRingLane = 255;        // the ring lane of a block list's padding
+constexpr uint32_t kNoSample = 0x40000000u;  // half-pixel position that no window holds
+
+// NS staged samples.
+template <uint32_t NS>
+struct Staged {
+  __attribute__((aligned(16))) double x[NS], y[NS], z[NS];
+  __attribute__((aligned(16))) uint32_t g[NS];  // half-pixel positions
+};
+
+// The value blocks that a set of cells looks at, for 64 rings (lane = ring),
+// listed NL (a multiple of 4) at a time.
+template <uint32_t NL>
+struct BlockList {
+  uint32_t lb[NL];         // listed block: its index among the sorted 8-sample blocks
+  double rz[64], rs[64];   // ring_z, ring_s
+  uint32_t gc[64];         // half-pixel position of a sample: 2 key + gc
+  uint32_t b0[64], ex[64], nb[64];  // the ring's first value block, their place in the sequence, their number
+  BlockSpan span;
+  uint8_t lr[NL];          // listed block: its ring's lane
+};
+
+// A block's 64 cells, row by row.
+struct MfmaCells {
+  Window win[kMcCols];
+  double tl[kMcCols], tr[kMcCols];  // compat: the window's edges (compat_edges)
+  double p[3][kMcCols];
+  double lat[kMcCols], coslat[kMcCols], tt[kMcCols];  // latitude (radians) and its cos; longitude (units of pi/2)
+  uint32_t wlo[kMcCols], wwid[kMcCols];           // the window in every belt ring (belt_window)
+  uint8_t belt[kMcCols];                          // it holds
+};
+
+// One wave's LDS: a staged k-block and its list.
+struct MfmaWave {
+  Staged<32> st;
+  BlockList<128> bl;
+};
+union MfmaLds {
+  struct {
+    MfmaWave w[kMcWaves];
+    MfmaCells c;
+  } s;
+  float t[kMcCols * 64];  // the epilogue's 64 channels x 64 cells
+};
+
+// The square's set-up runs once per 64 rings and the windows of general rings
+// once per k-block, both next to the sample loop: out of line, so that their
+// constants and temporaries do not live in its registers (230 of them inline
+// against 100).  Ranges come back as first | last << 32, 1 | 0 for none.
+constexpr uint64_t kNoRange = 1;
+__device__ inline uint64_t pack_range(uint32_t lp, uint32_t rp) { return (uint64_t)rp << 32 | lp; }
+
+static __device__ __noinline__ uint64_t span_pixels_call(Hpx32 hx, TileSpan t, uint32_t ring, double rz, double rs) {
+  uint32_t lp, rp;
+  span_pixels(hx, t, ring, rz, rs, lp, rp);
+  return pack_range(lp, rp);
+}
+
+static __device__ __noinline__ uint64_t ring_window_call(Hpx32 hx, const MfmaCells* C, uint32_t cb, uint32_t ring,
+                                                         double rz, double rs) {
   uint32_t a = 1, b = 0;
-  const bool act =
-      r >= win.uring && r <= win.dring && ring_window(P, win, r, B.ring_z[kr], B.ring_s[kr], a, b) && a <= b;
-  lp = act ? a : 1u;
-  rp = act ? b : 0u;
+  if (!ring_window_at(hx, C->win[cb], C->tl[cb], C->tr[cb], ring, rz, rs, a, b)) return kNoRange;
+  return pack_range(a, b);
 }
 
-// The sorted range of the union of the wave's windows within [start, end)
-// (a 64-way cooperative search of the keys); lo >= hi when empty.
-__device__ inline void ring_union_range(const GridBuffers& B, uint32_t lp, uint32_t rp, uint32_t start, uint32_t end,
-                                        uint32_t& lo, uint32_t& hi) {
-  const bool act = lp <= rp;
-  const uint32_t LP = wave_min_u32(act ? lp : 0xFFFFFFFFu);
-  const uint32_t RP = wave_max_u32(act ? rp : 0u);
-  lo = hi = 0;
-  if (LP <= RP) {  // uniform
-    lo = wave_search<false>(B.keys, start, end, LP);
-    hi = wave_search<true>(B.keys, lo, end, RP);
+// The keys lp..rp of a ring (first pixel sp, npr pixels), narrowed to what the
+// radius reaches from a square's cells.  A sample at latitude bs within R of
+// a cell at bc has hav R > hav(bs - bc) + cos bs cos bc hav(dl); ring r's
+// pixels lie between the centre latitudes of rings r - 1 and r + 1 (z = zu,
+// zd), so |bs - bc| >= d, the gap between that band and the cells' latitudes,
+// and
+//   sin^2(dl / 2) <= (sin^2(R / 2) - sin^2(d / 2)) / (cos bs cos bc).
+// The pixel of longitude tt (units of pi/2) is floor(tt npr / 4) or the next
+// one.  half = sin(R' / 2), R' = R (1 + 1e-6).  The windows span the disc's
+// whole width in every ring; a quarter of what a 4 x 4 square would look at
+// is outside the radius.
+static __device__ __noinline__ uint64_t chord_range(uint32_t lp, uint32_t rp, uint32_t sp, uint32_t npr, double zu,
+                                                    double zd, double bmin, double bmax, double tmin, double tmax,
+                                                    double cmin, double half) {
+  const double d = fmax(0.0, fmax(asin(zd) - bmax, bmin - asin(zu)));
+  const double sd = sin(0.5 * d);
+  const double num = half * half - sd * sd;
+  if (!(num > 0.0)) return kNoRange;
+  const double cs = sqrt(fmin((1.0 - zu) * (1.0 + zu), (1.0 - zd) * (1.0 + zd)));
+  const double s2 = num / (cs * cmin);
+  if (s2 < 0.25) {
+    const double dt = (4.0 / kPi) * sqrt(s2 / (1.0 - s2)) * (1.0 + 1e-9) + 1e-12;  // asin s <= s / sqrt(1 - s^2)
+    const double tl = tmin - dt, tr = tmax + dt, q = 0.25 * (double)npr;
+    if (tl >= 0.0 && tr * q < (double)npr - 2.0) {
+      lp = max(lp, sp + (uint32_t)fmax(tl * q - 1e-6, 0.0));
+      rp = min(rp, sp + (uint32_t)(tr * q + 1e-6) + 1u);
+    }
+  }
+  return pack_range(lp, rp);
+}
+
+// The keys of ring `ring` that a square's cells can take samples from: a
+// superset of the samples both in a cell's window and within its radius.
+__device__ inline uint64_t block_ring_range(const GridParams& P, const GridBuffers& B, const BlockSpan& S,
+                                            const hcg_ring_meta& m, uint32_t ring) {
+  const uint32_t kr = ring - m.firstring;
+  const Hpx32 hx = hpx32(P.hp);
+  uint32_t sp, npr;
+  ring_info32(hx, ring, sp, npr);
+  uint64_t range;
+  if (S.simple) {  // g = 2 p + 1 - odd in [hlo, hhi]
+    const uint32_t odd = ring & 1u;
+    range = pack_range(sp + ((S.hlo + odd) >> 1), sp + ((S.hhi - 1u + odd) >> 1));
+  } else {
+    range = span_pixels_call(hx, S.T, ring, B.ring_z[kr], B.ring_s[kr]);
+  }
+  if (!S.chord || kr == 0 || kr + 1 >= m.usedrings) return range;
+  return chord_range((uint32_t)range, (uint32_t)(range >> 32), sp, npr, B.ring_z[kr - 1], B.ring_z[kr + 1], S.bmin,
+                     S.bmax, S.tmin, S.tmax, S.cmin, P.polar_half);
+}
+
+// A cell (a lane's) of a block.
+struct CellGeom {
+  Window win;
+  double tl, tr;              // compat: the window's edges (compat_edges)
+  double px, py, pz;          // unit vector
+  double lat, coslat, tt;     // latitude (radians) and its cos; longitude (units of pi/2)
+  uint32_t wlo, wwid;         // the window in every belt ring (belt_window)
+  bool belt;                  // it holds
+};
+
+// Lane = cell of the block at (y0, x0), row by row.
+__device__ __forceinline__ CellGeom block_cell(const GridParams& P, const GridBuffers& B, const hcg_ring_meta& m,
+                                               uint32_t y0, uint32_t x0, uint32_t tc_shift, bool& live) {
+  const uint32_t lane = __lane_id();
+  const uint32_t row = y0 + (lane >> tc_shift), col = x0 + (lane & ((1u << tc_shift) - 1u));
+  live = row < P.side && col < P.side;
+  const uint32_t cell = live ? row * P.side + col : 0;
+  const uint32_t anchor = live ? row * P.side + (col / P.factor) * P.factor : 0;
+  const double xc = B.xwcs[cell] * kDeg2Rad, yc = B.ywcs[cell] * kDeg2Rad;
+  CellGeom g;
+  g.win = window_of(P, m.firstring, m.usedrings, B.xwcs[anchor], B.ywcs[anchor]);
+  if (!live || m.usedrings == 0) {
+    g.win.uring = 1;
+    g.win.dring = 0;
+  }
+  double cb, sl, cl;
+  sincos(yc, &g.pz, &cb);
+  sincos(xc, &sl, &cl);
+  g.px = cb * cl;
+  g.py = cb * sl;
+  g.tl = g.tr = 0.0;
+  uint32_t whi = 0;
+  g.wlo = 0;
+  g.belt = false;
+  if (g.win.mode == kWinCompat) {
+    compat_edges(P, g.win, g.tl, g.tr);
+    g.belt = belt_window(P, g.tl, g.tr, g.wlo, whi);
+  }
+  g.wwid = whi - g.wlo;
+  g.lat = yc;
+  g.coslat = cb;
+  g.tt = fmodulo4(xc * kInvHalfPi);
+  return g;
+}
+
+__device__ __forceinline__ void put_cell(MfmaCells& C, uint32_t i, const CellGeom& g) {
+  C.win[i] = g.win;
+  C.tl[i] = g.tl;
+  C.tr[i] = g.tr;
+  C.p[0][i] = g.px;
+  C.p[1][i] = g.py;
+  C.p[2][i] = g.pz;
+  C.lat[i] = g.lat;
+  C.coslat[i] = g.coslat;
+  C.tt[i] = g.tt;
+  C.wlo[i] = g.wlo;
+  C.wwid[i] = g.wwid;
+  C.belt[i] = g.belt;
+}
+
+// The span of the wave's cells (live: on the map).
+__device__ __forceinline__ BlockSpan cells_span(const GridParams& P, const hcg_ring_meta& m, const CellGeom& g,
+                                                bool live) {
+  BlockSpan S;
+  S.T = tile_span(P, g.win, m.firstring);
+  const bool has = g.win.uring <= g.win.dring;
+  const uint32_t ns = (uint32_t)P.hp.nside;
+  const bool belt_ok = __ballot(has && !g.belt) == 0;
+  S.simple = belt_ok && S.T.r_begin > ns && S.T.r_end < 3 * ns;  // uniform
+  S.hlo = wave_min_u32(has ? g.wlo : 0xFFFFFFFFu);
+  S.hhi = wave_max_u32(has ? g.wlo + g.wwid : 1u);
+  S.bmin = wave_min_f64(live ? g.lat : 1e300);
+  S.bmax = -wave_min_f64(live ? -g.lat : 1e300);
+  S.tmin = wave_min_f64(live ? g.tt : 1e300);
+  S.tmax = -wave_min_f64(live ? -g.tt : 1e300);
+  S.cmin = wave_min_f64(live ? g.coslat : 1e300);
+  // (a cell outside the projection, NaN, leaves the chord out)
+  S.chord = __ballot(live && !(g.lat > -2.0 && g.lat < 2.0 && g.tt >= 0.0)) == 0 && S.cmin > 0.05 &&
+            S.tmax - S.tmin < 1.0;
+  return S;
+}
+
+// The value blocks [b0, b0 + nblk) of ring r of a span (lane = ring).
+__device__ __forceinline__ void ring_block_range(const GridParams& P, const GridBuffers& B, const hcg_ring_meta& m,
+                                                 const BlockSpan& S, uint32_t r, uint32_t& b0, uint32_t& nblk) {
+  b0 = nblk = 0;
+  if (r > S.T.r_end) return;
+  const uint32_t kr = r - m.firstring;
+  const uint32_t start = B.lut[kr], end = B.lut[kr + 1];
+  if (start >= end) return;
+  const uint64_t range = block_ring_range(P, B, S, m, r);
+  const uint32_t lp = (uint32_t)range, rp = (uint32_t)(range >> 32);
+  uint32_t lo = 0, hi = 0;
+  if (lp <= rp) key_range(B.keys, start, end, lp, rp, lo, hi);
+  if (lo < hi) {
+    b0 = lo / kVB;
+    nblk = (hi + kVB - 1) / kVB - b0;
   }
 }
 
-// The tile plan: one wave per tile, lane = cell.  Many small workgroups per
-// CU hide the latency of the per-ring searches that the gridding kernel,
-// with one or two large workgroups per CU, cannot.
-__device__ inline void plan_tile(const MfmaJob& J, uint32_t tile) {
+__device__ __forceinline__ uint32_t wave_scan_sum_u32(uint32_t v) {  // inclusive
+  const uint32_t lane = __lane_id();
+#pragma unroll
+  for (uint32_t off = 1; off < 64; off <<= 1) {
+    const uint32_t t = __shfl_up(v, off, 64);
+    if (lane >= off) v += t;
+  }
+  return v;
+}
+
+// Rings rb .. rb + 63 of the list's span (lane = ring, one wave) with their
+// value blocks; the blocks' number.
+template <uint32_t NL>
+__device__ __forceinline__ uint32_t put_rings(const GridParams& P, BlockList<NL>& L, uint32_t rb, uint32_t b0,
+                                              uint32_t nblk) {
+  const uint32_t lane = __lane_id(), r = rb + lane;
+  uint32_t sp, npr;
+  ring_info32(hpx32(P.hp), r, sp, npr);
+  L.gc[lane] = 1u - (r & 1u) - 2u * sp;
+  const uint32_t in = wave_scan_sum_u32(nblk);
+  L.b0[lane] = b0;
+  L.ex[lane] = in - nblk;
+  L.nb[lane] = nblk;
+  return (uint32_t)__builtin_amdgcn_readlane((int)in, 63);
+}
+template <uint32_t NL>
+__device__ __forceinline__ uint32_t ring_blocks(const GridParams& P, const GridBuffers& B, const hcg_ring_meta& m,
+                                                uint32_t rb, BlockList<NL>& L) {
+  const uint32_t lane = __lane_id(), r = rb + lane;
+  uint32_t b0, nblk;
+  ring_block_range(P, B, m, L.span, r, b0, nblk);
+  if (r <= L.span.T.r_end) {
+    L.rz[lane] = B.ring_z[r - m.firstring];
+    L.rs[lane] = B.ring_s[r - m.firstring];
+  }
+  return put_rings(P, L, rb, b0, nblk);
+}
+
+// The plan of a block for mfma_wide: what its set-up works out, in one
+// coalesced read (set up in the kernel, one wave at work and seven waiting,
+// the 2M x 1024 cube's 32768 blocks took 0.8 ms more).  ok: the span is
+// simple and has at most 64 rings; otherwise the kernel does the set-up.
+struct MfmaPlan {
+  double p[3][kMcCols];
+  uint32_t uring[kMcCols], dring[kMcCols], wlo[kMcCols], wwid[kMcCols];  // cell by cell
+  uint32_t b0[64], nb[64];                                              // ring by ring
+  uint32_t ok, r_begin, r_end, pad;
+};
+static_assert(sizeof(MfmaPlan) <= kPlanBytes && kPlanBytes % 8 == 0, "plan layout");
+__device__ __forceinline__ void plan_tile(const MfmaJob& J, uint32_t tile) {  // one wave
   const uint32_t lane = __lane_id();
   const hcg_ring_meta m = *J.B.meta;
-  const uint32_t tc_shift = J.tc_shift;
-  const uint32_t y0 = (tile / J.tiles_x) << (6u - tc_shift);
-  const uint32_t x0 = (tile % J.tiles_x) << tc_shift;
-  double q[3];
-  uint32_t r_begin, r_end;
-  const Window win = block_cell_window(J.P, J.B, m, y0, x0, tc_shift, lane, q, r_begin, r_end);
-  uint32_t* out = J.plan + (size_t)tile * kPlanTileWords;
+  bool live;
+  const CellGeom g = block_cell(J.P, J.B, m, (tile / J.tiles_x) << (6u - J.tc_shift),
+                                (tile % J.tiles_x) << J.tc_shift, J.tc_shift, live);
+  const BlockSpan S = cells_span(J.P, m, g, live);
+  MfmaPlan& L = *reinterpret_cast<MfmaPlan*>(static_cast<char*>(J.plan) + tile * kPlanBytes);
+  const bool none = S.T.r_begin > S.T.r_end, ok = none || (S.simple && S.T.r_end - S.T.r_begin < 64);
   if (lane == 0) {
-    out[0] = r_begin;
-    out[1] = r_end;
+    L.ok = ok;
+    L.r_begin = none ? 1 : S.T.r_begin;
+    L.r_end = none ? 0 : S.T.r_end;
   }
-  reinterpret_cast<Window*>(out + kPlanHeadWords)[lane] = win;
-  double* pq = reinterpret_cast<double*>(out + kPlanHeadWords + kPlanWinWords);
-  pq[lane] = q[0];
-  pq[kMcCols + lane] = q[1];
-  pq[2 * kMcCols + lane] = q[2];
-  for (uint32_t k = 0; k < kPlanRings; ++k) {
-    const uint32_t r = r_begin + k;
-    uint32_t lo = 0, hi = 0;
-    if (r_begin <= r_end && r <= r_end) {  // uniform
-      const uint32_t kr = r - m.firstring;
-      const uint32_t start = J.B.lut[kr], end = J.B.lut[kr + 1];
-      if (start != end) {
-        uint32_t lp, rp;
-        ring_cell_window(J.P, J.B, m, win, r, lp, rp);
-        ring_union_range(J.B, lp, rp, start, end, lo, hi);
-      }
-    }
-    if (lane == 0) {
-      out[2 + 2 * k] = lo;
-      out[3 + 2 * k] = hi;
-    }
-  }
+  if (!ok) return;  // uniform
+  L.p[0][lane] = g.px;
+  L.p[1][lane] = g.py;
+  L.p[2][lane] = g.pz;
+  L.uring[lane] = g.win.uring;
+  L.dring[lane] = g.win.dring;
+  L.wlo[lane] = g.wlo;
+  L.wwid[lane] = g.wwid;
+  uint32_t b0 = 0, nblk = 0;
+  if (!none) ring_block_range(J.P, J.B, m, S, S.T.r_begin + lane, b0, nblk);
+  L.b0[lane] = b0;
+  L.nb[lane] = nblk;
 }
 
 __global__ void __launch_bounds__(64) k_mfma_plan(MfmaJob J) { plan_tile(J, blockIdx.x); }
 
-int launch_mfma_plan(const MfmaJob& J, hipStream_t s) {
-  if (J.ntiles == 0) return HCG_OK;
-  k_mfma_plan<<<J.ntiles, 64, 0, s>>>(J);
-  HCG_CHECK_LAUNCH("k_mfma_plan");
-  return HCG_OK;
+// Lists blocks q0 .. q0 + cnt - 1 (one wave), then the last one again up to
+// the k-block boundary, as padding without samples.
+template <uint32_t NL>
+__device__ __forceinline__ void list_blocks(BlockList<NL>& L, uint32_t q0, uint32_t cnt) {
+  const uint32_t lane = __lane_id();
+  const uint32_t ex = L.ex[lane], in = ex + L.nb[lane], b = L.b0[lane] - ex;
+  for (uint32_t t = max(ex, q0); t < min(in, q0 + cnt); ++t) {
+    L.lb[t - q0] = b + t;
+    L.lr[t - q0] = (uint8_t)lane;
+    if (t - q0 == cnt - 1)
+      for (uint32_t p = cnt; p < (cnt + 3) / 4 * 4; ++p) {
+        L.lb[p] = b + t;
+        L.lr[p] = (uint8_t)kNoRingLane;
+      }
+  }
 }
 
-// LDS of one workgroup (the weight tiles as raw 16-bit storage).
-template <uint32_t CHUNK>
-struct MfmaLds {
-  // first, so one address and immediate offsets reach a sample's x, y, z
-  double x[CHUNK], y[CHUNK], z[CHUNK];
-  uint32_t key[CHUNK];
-  // the weight tiles, row-interleaved: cell c's hi weights at c * RS, its lo
-  // weights at c * RS + CHUNK (elements; RS = 2 CHUNK + 8), so one address
-  // and an immediate offset reach both; RS is an odd multiple of 16 bytes,
-  // so the 16 rows of an MFMA operand read start in 16 distinct groups of 4
-  // banks
-  __attribute__((aligned(16))) uint16_t w[kMcCols * (2 * CHUNK + 8)];
-  uint32_t mb[2][4][2];  // row blocks' k-block spans, by chunk parity
-  double inv[kMcCols];  // per cell: 1 / its weight sum (1 without normalisation)
-  double p[kMcCols][3];          // cell unit vectors
-  uint32_t span[2];              // the block's ring span
-  uint32_t plan[kPlanStride];    // the tile's plan (when the job has one)
-  // chunk descriptors (double-buffered): blocks and segments; per block its
-  // sorted 32-sample block index, per segment its ring, first block, blocks
-  uint32_t dn[2][3];                   // k-blocks, segments, value blocks
-  uint32_t dgb[2][CHUNK / kVB];        // per value block of the chunk: its sorted block index
-  uint32_t dring[2][CHUNK / 32];       // per segment (at most CHUNK / 32 per chunk): its ring,
-  uint16_t du0[2][CHUNK / 32], dnb[2][CHUNK / 32];  // first value block, value blocks
-  uint32_t band[CHUNK / 32][kMcCols];  // each cell's band per segment: ja | jb << 16
-  // a planned tile's rings (the wave-parallel descriptor builder), slot l =
-  // ring r_begin + l, written and read by lane l of wave 0 only: first value
-  // block, the ring's offset in the tile's block sequence, its block count
-  uint32_t rl_b0[kPlanRings], rl_ex[kPlanRings], rl_nb[kPlanRings];
-  Window win[kMcCols];                 // each cell's window
+// Sample s of k-block u of the list, half of it a lane: half 0 its x and y,
+// half 1 its z and position; in flight from fetch to store.
+struct StageRegs {
+  double v0, v1;
+  uint32_t pos;
+  template <uint32_t NL>
+  __device__ __forceinline__ void fetch(const GridBuffers& B, const hcg_ring_meta& m, const BlockList<NL>& L,
+                                        uint32_t u, uint32_t s, uint32_t half) {
+    const uint32_t q = u * 4 + (s >> 3);
+    const uint32_t i = L.lb[q] * kVB + (s & 7u), rl = L.lr[q];
+    v0 = v1 = 0.0;
+    pos = kNoSample;
+    if (rl != kNoRingLane && i < m.n) {
+      const double* r = &B.rec[i].x + 2 * half;
+      v0 = r[0];
+      v1 = r[1];
+      if (half) pos = 2u * B.keys[i] + L.gc[rl];
+    }
+  }
+  template <uint32_t NS>
+  __device__ __forceinline__ void store(Staged<NS>& S, uint32_t p, uint32_t half) const {
+    if (half) {
+      S.z[p] = v0;
+      S.g[p] = pos;
+    } else {
+      S.x[p] = v0;
+      S.y[p] = v1;
+    }
+  }
 };
 
-// CHUNK = staged samples per chunk.  LDS: the weight tiles (64 rows of
-// 2 CHUNK + 8 elements) + CHUNK unit vectors and keys + the chunk
-// descriptors and bands: 156 KB at 512 (one workgroup per CU), 79 KB at 256
-// (two per CU), 46 KB at 128.
-//
-// The 64 cells of a workgroup form a TR x TC block of the map (TC = 1 <<
-// tc_shift columns, TR = 64 / TC rows); cell c of the block is (c / TC,
-// c % TC) and MFMA row block mb holds cells 16 mb .. 16 mb + 15.  Square-ish
-// blocks share more of their neighbourhood, so each channel value is
-// re-read by fewer workgroups: (TR + d)(TC + d) / 64 reads per value for a
-// support of d cells, 16.8 for 1 x 64 and 7.7 for 4 x 16 at d = 13.
-// STAGED: the cube stores go through LDS (the one-job kernel, where they
-// took the 2M x 1024 cube from 7.29 to 7.08 ms; in the persistent kernel,
-// whose register budget is tighter, the 64-job batch measured 159.4 ms
-// with them against 158.9 without).
-template <int DT, uint32_t CHUNK, bool STAGED>
-__device__ __forceinline__ void mfma_block(const MfmaJob& J, uint32_t tile, uint32_t group, MfmaLds<CHUNK>& L,
-                                           const double* s_exp) {
-  typedef s16x8_t vec;
-  constexpr uint32_t WS = CHUNK;       // hi -> lo offset within a weight row (elements)
-  constexpr uint32_t RS = 2 * WS + 8;  // weight row stride (elements)
-  static_assert((WS * 2) % 16 == 0 && (RS * 2) % 16 == 0 && (RS / 2) % 8 == 4, "weight tile layout");
-  uint16_t* s_wh = L.w;
-  uint16_t* s_wl = L.w + WS;
-  const bool bf = dt_is_bf16<DT>(J.dtype);
-  double* s_x = L.x;
-  double* s_y = L.y;
-  double* s_z = L.z;
-  uint32_t* s_key = L.key;
-  auto& s_mb = L.mb;
-  double* s_inv = L.inv;
+// One lane's cell of a square, and the constants of the weights.
+template <bool LEAN>
+struct SquareCell {
+  double npx, npy, npz;
+  uint32_t uring, dring, wlo, wwid;
+  double h_hi, h_lo, k0h, k1v, e3v;
+  double wsum;
+  uint32_t cb;  // its place in the block
+  bool simple;
+  __device__ __forceinline__ void init(const GridParams& P, const MfmaCells& C, uint32_t cell_in_block, bool smp) {
+    cb = cell_in_block;
+    simple = smp;
+    npx = -C.p[0][cb];
+    npy = -C.p[1][cb];
+    npz = -C.p[2][cb];
+    uring = C.win[cb].uring;
+    dring = C.win[cb].dring;
+    wlo = C.wlo[cb];
+    wwid = C.wwid[cb];
+    h_hi = LEAN ? 0.5 * P.c_hi : P.c_hi;
+    h_lo = LEAN ? 0.5 * P.c_lo : P.c_lo;
+    k0h = 2.0 * P.k0;
+    k1v = LEAN ? in_vgprs(4.0 * P.k1) : 0.0;
+    e3v = LEAN ? in_vgprs(kExpE3) : 0.0;
+    wsum = 0.0;
+  }
+  // the window in ring lane rl of the list, in half pixels
+  template <uint32_t NL>
+  __device__ __forceinline__ void window(const GridParams& P, const MfmaCells& C, const BlockList<NL>& L, uint32_t rb,
+                                         uint32_t rl, uint32_t& wl, uint32_t& ww) const {
+    const uint32_t r = rb + rl;
+    bool act = rl != kNoRingLane && r >= uring && r <= dring;
+    wl = wlo;
+    ww = wwid;
+    if (!simple) {  // uniform
+      const uint64_t range = ring_window_call(hpx32(P.hp), &C, cb, r, L.rz[rl & 63u], L.rs[rl & 63u]);
+      const uint32_t a = (uint32_t)range, b = (uint32_t)(range >> 32);
+      act = act && a <= b;
+      wl = 2u * a + L.gc[rl & 63u];
+      ww = 2u * (b - a);
+    }
+    if (!act) {
+      wl = kNoWindow;
+      ww = 0;
+    }
+  }
+};
+
+// One lane's A operand: the weights of 8 samples, hi and lo.
+struct WeightOperand {
+  union {
+    uint32_t d[4];
+    s16x8_t v;
+  } h, l;
+};
+
+// The weights of a wave's 16 cells and the 32 samples at S[at ..]: lane l
+// takes cell l % 16 and samples 8 (l / 16) .. + 7 (of value block blk), which
+// is the layout of an MFMA operand.  Returns the lanes with a selected pair;
+// guard: those with one within rounding of the radius (kept here).
+template <int DT, bool LEAN, uint32_t NS>
+__device__ __forceinline__ uint64_t weigh_kblock(const MfmaJob& J, SquareCell<LEAN>& Q, const Staged<NS>& S,
+                                                 uint32_t at, uint32_t wl, uint32_t ww, uint32_t cell, uint32_t blk,
+                                                 const double* s_exp, WeightOperand& A, uint64_t& guard) {
+  constexpr bool bf = DT == kDtBf16;
+  uint64_t any = 0;
+  guard = 0;
+#pragma unroll
+  for (uint32_t hf = 0; hf < 2; ++hf) {  // four samples at a time
+    const uint32_t j0 = at + (__lane_id() >> 4) * 8 + hf * 4;
+    double qx[4], qy[4], qz[4], t[4];
+    uint32_t qg[4];
+    lds_read4(&S.x[j0], qx);
+    lds_read4(&S.y[j0], qy);
+    lds_read4(&S.z[j0], qz);
+    *reinterpret_cast<uint4*>(qg) = *reinterpret_cast<const uint4*>(&S.g[j0]);
+    uint64_t sel[4];
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) {
+      t[e] = pair_distance<LEAN>(Q.npx, Q.npy, Q.npz, qx[e], qy[e], qz[e]);
+      sel[e] = __builtin_amdgcn_ballot_w64(t[e] < Q.h_hi) & __builtin_amdgcn_ballot_w64(qg[e] - wl <= ww);
+      guard |= sel[e] & __builtin_amdgcn_ballot_w64(!(t[e] < Q.h_lo));
+    }
+    any |= (sel[0] | sel[1]) | (sel[2] | sel[3]);
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+      const uint32_t jj = hf * 2 + k;
+      A.h.d[jj] = A.l.d[jj] = 0;
+      if ((sel[2 * k] | sel[2 * k + 1]) == 0) continue;  // uniform
+      // both weights at once, every lane's (two chains of FP64 steps and
+      // table reads hide each other's latency), then the selected ones
+      double wt[2] = {0.0, 0.0};
+      if constexpr (LEAN) {
+        gauss_weight_lean2(t[2 * k], t[2 * k + 1], Q.k0h, Q.k1v, Q.e3v, s_exp, wt);
+      } else {
+#pragma unroll
+        for (uint32_t e = 0; e < 2; ++e)
+          if (__builtin_amdgcn_inverse_ballot_w64(sel[2 * k + e])) {
+            const uint32_t isrc = blk * kVB + jj * 2 + e;
+            wt[e] = pair_weight_any(J.P, J.B, J.kt, t[2 * k + e], s_exp, cell, isrc);
+            if (J.B.w_s) wt[e] *= J.B.w_s[isrc];
+          }
+      }
+      const f32x2_t wf = {__builtin_amdgcn_inverse_ballot_w64(sel[2 * k]) ? (float)wt[0] : 0.f,
+                          __builtin_amdgcn_inverse_ballot_w64(sel[2 * k + 1]) ? (float)wt[1] : 0.f};
+      // the weight as hi + lo in the value type (~2x its significand): wf -
+      // hi is exact (Sterbenz), and hi + lo is exact in FP32 (at most 2 x 11
+      // significant bits, the second ~2^-8 below the first)
+      A.h.d[jj] = round16x2<bf>(wf);
+      const f32x2_t fh = widen16x2<bf>(A.h.d[jj]);
+      A.l.d[jj] = round16x2<bf>(f32x2_t{wf.x - fh.x, wf.y - fh.y});
+      const f32x2_t fl = widen16x2<bf>(A.l.d[jj]);
+      Q.wsum += (double)(fh.x + fl.x);
+      Q.wsum += (double)(fh.y + fl.y);
+    }
+  }
+  return any;
+}
+
+// The pairs within rounding of the radius: the reference's test decides, and
+// a pair that it rejects is taken out again.
+template <int DT, bool LEAN, uint32_t NS>
+__device__ __forceinline__ void guard_kblock(const MfmaJob& J, SquareCell<LEAN>& Q, const Staged<NS>& S, uint32_t at,
+                                             uint32_t wl, uint32_t ww, uint32_t cell, uint32_t blk, WeightOperand& A) {
+  constexpr bool bf = DT == kDtBf16;
+#pragma unroll 1
+  for (uint32_t e = 0; e < 8; ++e) {
+    const uint32_t j = at + (__lane_id() >> 4) * 8 + e;
+    const double t = pair_distance<LEAN>(Q.npx, Q.npy, Q.npz, S.x[j], S.y[j], S.z[j]);
+    if (t < Q.h_hi && S.g[j] - wl <= ww && !(t < Q.h_lo) &&
+        !radius_test_ref(J.B.xwcs, J.B.ywcs, J.B.lon_s, J.B.lat_s, cell, blk * kVB + e, J.P.sphere_radius)) {
+      const uint32_t sh = (e & 1u) * 16u, keep = 0xFFFF0000u >> sh;
+      uint32_t hw = 0, lw = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i)
+        if (i == e >> 1) {
+          hw = A.h.d[i] >> sh;
+          lw = A.l.d[i] >> sh;
+          A.h.d[i] &= keep;
+          A.l.d[i] &= keep;
+        }
+      Q.wsum -= (double)(widen16((uint16_t)hw, bf) + widen16((uint16_t)lw, bf));
+    }
+  }
+}
+
+// The squares of a block: 4 x 4 cells (2 x 8 and 1 x 16 in blocks of 32 and
+// 64 columns); MFMA row i of square mb is cell (i / width, i % width) of it.
+struct Squares {
+  uint32_t w_shift, x_shift, tc_shift;  // a square's width; squares side by side; the block's width
+  __device__ __forceinline__ explicit Squares(uint32_t tc)
+      : w_shift(tc <= 4 ? 2u : tc - 2u), x_shift(tc - (tc <= 4 ? 2u : tc - 2u)), tc_shift(tc) {}
+  __device__ __forceinline__ uint32_t cell(uint32_t mb, uint32_t i) const {  // its place in the block
+    const uint32_t mx = (mb & ((1u << x_shift) - 1u)) << w_shift, my = (mb >> x_shift) << (4u - w_shift);
+    return ((my + (i >> w_shift)) << tc_shift) + mx + (i & ((1u << w_shift) - 1u));
+  }
+};
+
+// Four cells of a map row (quad q of the block at (y0, x0)) of channel ch.
+__device__ __forceinline__ void store_quad(const MfmaJob& J, uint32_t y0, uint32_t x0, uint32_t q, uint32_t ch,
+                                           const float4& v) {
+  const uint32_t side = J.P.side, c0 = q * 4;
+  const uint32_t row = y0 + (c0 >> J.tc_shift), col = x0 + (c0 & ((1u << J.tc_shift) - 1u));
+  if (row >= side || col >= side || ch >= J.nchan) return;
+  float* dst = J.cube + (size_t)ch * side * side + (size_t)row * side + col;
+  if ((side & 3u) == 0) {  // uniform; aligned then
+    *reinterpret_cast<float4*>(dst) = v;
+  } else {
+    dst[0] = v.x;
+    if (col + 1 < side) dst[1] = v.y;
+    if (col + 2 < side) dst[2] = v.z;
+    if (col + 3 < side) dst[3] = v.w;
+  }
+}
+
+// The lane's row of the channel values (MFMA B operand): row ch_base + l % 16
+// of a value block, 16 bytes; the 16 lanes of a k-group read one contiguous
+// 256-byte piece.  Rows past the last channel fill columns that nothing
+// reads: they are the following blocks' (with one channel every lane reads
+// row 0; else there are fewer of them than eight blocks hold, and eight
+// blocks of padding follow the last sample's).
+__device__ __forceinline__ const char* value_rows(const MfmaJob& J, uint32_t ch_base) {
+  return static_cast<const char*>(J.vs) +
+         (size_t)(ch_base + (J.nchan > 1 ? __lane_id() & 15u : 0u)) * (kVB * 2u);
+}
+
+// One block of 64 cells and up to 16 NB channels (group `group` of them): a
+// wave takes a square of 16 cells, on its own but for the set-up and the
+// stores.  LEAN: GAUSS1D at lean_weight_ok radii without sample weights.
+template <int DT, int NB, bool LEAN>
+__device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint32_t group, MfmaLds& lds,
+                                          const double* s_exp) {
+  constexpr bool bf = DT == kDtBf16;
   const GridParams& P = J.P;
   const GridBuffers& B = J.B;
-  const uint16_t* __restrict__ vs = static_cast<const uint16_t*>(J.vs);
-  const uint32_t kt = J.kt, nchan = J.nchan, tc_shift = J.tc_shift, tiles_x = J.tiles_x;
-  const size_t blk = (size_t)nchan * kVB;  // elements per value block
-  float* __restrict__ cube = J.cube;
-  float* __restrict__ wsum_out = J.wsum;
-  const int normalize = J.normalize;
-
+  const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6, kg = lane >> 4;
   const hcg_ring_meta m = *B.meta;
-  const uint32_t nthreads = blockDim.x;
-  const uint32_t nw = nthreads >> 6;       // waves in this workgroup
-  const uint32_t S = nw;                   // threads per cell (one per wave)
-  const uint32_t tid = threadIdx.x;
-  const uint32_t lane = __lane_id();
-  const uint32_t wave = tid >> 6;
+  const uint32_t y0 = (tile / J.tiles_x) << (6u - J.tc_shift), x0 = (tile % J.tiles_x) << J.tc_shift;
+  MfmaCells& C = lds.s.c;
+  MfmaWave& W = lds.s.w[wave];
+  const Squares sq(J.tc_shift);
 
-  const uint32_t tc_mask = (1u << tc_shift) - 1u;
-  const uint32_t y0 = (tile / tiles_x) << (6u - tc_shift);
-  const uint32_t x0 = (tile % tiles_x) << tc_shift;
-  const uint32_t M = P.side * P.side;
+  if (wave == 0) {
+    bool lv;
+    const CellGeom g = block_cell(P, B, m, y0, x0, J.tc_shift, lv);
+    put_cell(C, lane, g);
+  }
+  __syncthreads();
+  const uint32_t cb = sq.cell(wave, lane & 15u);
+  const uint32_t crow = y0 + (cb >> J.tc_shift), ccol = x0 + (cb & ((1u << J.tc_shift) - 1u));
+  const bool live = crow < P.side && ccol < P.side;
+  const uint32_t cell = live ? crow * P.side + ccol : 0;
+  uint32_t r_begin, r_end;
+  SquareCell<LEAN> Q;
+  {
+    CellGeom g;
+    g.win = C.win[cb];
+    g.lat = C.lat[cb];
+    g.coslat = C.coslat[cb];
+    g.tt = C.tt[cb];
+    g.wlo = C.wlo[cb];
+    g.wwid = C.wwid[cb];
+    g.belt = C.belt[cb] != 0;
+    const BlockSpan S = cells_span(P, m, g, live);
+    r_begin = S.T.r_begin;
+    r_end = S.T.r_end;
+    Q.init(P, C, cb, S.simple);
+    if (lane == 0) W.bl.span = S;
+  }
+  const uint32_t ch_base = group * (NB * 16u);
+  const char* const vs = value_rows(J, ch_base);
+  const size_t blk_bytes = (size_t)J.nchan * kVB * 2u;
+  f32x4_t acc[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  // this thread's cell c = lane and its share sub = wave of the cell's band:
-  // every wave holds all 64 cells, so the weight work is balanced across
-  // the waves whichever rows of the block a ring reaches
-  const uint32_t c = lane, sub = wave;
-  const uint32_t row = y0 + (c >> tc_shift);
-  const uint32_t col = x0 + (c & tc_mask);
-  const bool live = col < P.side && row < P.side;
-  const uint32_t cell = live ? row * P.side + col : 0;
-
-  // Wave 0 evaluates the block's geometry, lane l = cell l: the cell's
-  // window (kept in LDS, not registers, through the chunk loop) and unit
-  // vector, the block's ring span, and per ring the cells' [lpix, rpix] and
-  // the union's sorted range, published through LDS.  The other waves only
-  // stage, weigh and contract.
-  if (J.plan) {  // the plan holds all of it (one round of coalesced loads)
-    const uint32_t* tp = J.plan + (size_t)tile * kPlanTileWords;
-    for (uint32_t i = tid; i < kPlanStride; i += nthreads) L.plan[i] = tp[i];
-    if (wave == 0) {
-      L.win[lane] = reinterpret_cast<const Window*>(tp + kPlanHeadWords)[lane];
-      const double* pq = reinterpret_cast<const double*>(tp + kPlanHeadWords + kPlanWinWords);
-      L.p[lane][0] = pq[lane];
-      L.p[lane][1] = pq[kMcCols + lane];
-      L.p[lane][2] = pq[2 * kMcCols + lane];
-      if (lane == 0) {
-        L.span[0] = tp[0];
-        L.span[1] = tp[1];
+  for (uint32_t rb = r_begin; r_begin <= r_end && rb <= r_end; rb += 64) {
+    tile_sync();
+    const uint32_t total = ring_blocks(P, B, m, rb, W.bl);
+    for (uint32_t q0 = 0; q0 < total; q0 += 128) {  // uniform
+      const uint32_t cnt = min(total - q0, 128u), nkb = (cnt + 3) / 4;
+      tile_sync();
+      list_blocks(W.bl, q0, cnt);
+      tile_sync();
+      StageRegs st;
+      st.fetch(B, m, W.bl, 0, lane & 31u, lane >> 5);
+      for (uint32_t u = 0; u < nkb; ++u) {
+        tile_sync();  // the previous k-block is consumed
+        st.store(W.st, lane & 31u, lane >> 5);
+        const uint32_t blk = W.bl.lb[u * 4 + kg];
+        uint32_t wl, ww;
+        Q.window(P, C, W.bl, rb, W.bl.lr[u * 4 + kg], wl, ww);
+        s16x8_t bn[NB];
+        auto load_b = [&]() {
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            bn[nb] = *reinterpret_cast<const s16x8_t*>(vs + blk * blk_bytes + nb * (16 * kVB * 2));
+        };
+        load_b();
+        if (u + 1 < nkb) st.fetch(B, m, W.bl, u + 1, lane & 31u, lane >> 5);
+        tile_sync();
+        WeightOperand A;
+        uint64_t guard;
+        const uint64_t any = weigh_kblock<DT>(J, Q, W.st, 0, wl, ww, cell, blk, s_exp, A, guard);
+        if (guard) {  // uniform, rare
+          // the sums wait in scratch memory meanwhile (volatile: here and only
+          // here), and the channel values are read again: across the call they
+          // would not fit the registers that it preserves, and would be
+          // spilled in every k-block
+          volatile float keep[NB * 4];
+#pragma unroll
+          for (int i = 0; i < NB * 4; ++i) keep[i] = acc[i / 4][i % 4];
+          guard_kblock<DT>(J, Q, W.st, 0, wl, ww, cell, blk, A);
+#pragma unroll
+          for (int i = 0; i < NB * 4; ++i) acc[i / 4][i % 4] = keep[i];
+          load_b();
+        }
+        if (any) {  // uniform
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            acc[nb] = mfma16(bf, A.h.v, bn[nb], acc[nb]);
+            acc[nb] = mfma16(bf, A.l.v, bn[nb], acc[nb]);
+          }
+        }
       }
+    }
+  }
+
+  // per-cell weight sums over the k-groups (exact in FP64 in any order: every
+  // weight is hi + lo of two 16-bit values).  The normalisation is one
+  // multiply per value: v * (1 / t) is within an FP64 ulp or two of v / t, so
+  // the FP32 result is the quotient's except where it lies that close to an
+  // FP32 rounding boundary (1 ulp then); t = 0 gives inf, so an empty cell is
+  // 0 * inf = NaN as 0 / 0 is.
+  double wsum = Q.wsum;
+  wsum += __shfl_xor(wsum, 16, 64);
+  wsum += __shfl_xor(wsum, 32, 64);
+  if (group == 0 && J.wsum && live && lane < 16) J.wsum[cell] = (float)wsum;
+  const double inv = J.normalize ? 1.0 / wsum : 1.0;
+  double iv[4];  // of the lane's MFMA rows 4 kg .. 4 kg + 3
+#pragma unroll
+  for (uint32_t j = 0; j < 4; ++j) iv[j] = __shfl(inv, kg * 4 + j, 64);
+  // Stores through LDS, 64 channels of the block at a time: the 16-byte quads
+  // (four cells of a map row) of a channel's 64 cells, XOR-swizzled by the
+  // channel, so that the 16 channels of a write and the 16 quads of a read
+  // fall in distinct bank groups; a store instruction then writes four
+  // channels' whole rows of the block instead of 64 scattered pieces.
+  const uint32_t q_own = sq.cell(wave, kg * 4) >> 2;
+#pragma unroll
+  for (int s = 0; s < (NB + 3) / 4; ++s) {
+    if (ch_base + s * 64 >= J.nchan) break;  // uniform
+    __syncthreads();  // the samples, or the previous channels, are done with
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int nb = s * 4 + k;
+      if (nb < NB) {
+        const uint32_t cr = k * 16 + (lane & 15u);
+        *reinterpret_cast<float4*>(&lds.t[cr * 64 + ((q_own ^ (cr & 15u)) << 2)]) =
+            make_float4((float)((double)acc[nb][0] * iv[0]), (float)((double)acc[nb][1] * iv[1]),
+                        (float)((double)acc[nb][2] * iv[2]), (float)((double)acc[nb][3] * iv[3]));
+      }
+    }
+    __syncthreads();
+    constexpr uint32_t kSteps = NB >= 4 ? 4 : NB;  // 16 channels a step of the four waves
+    const uint32_t q = lane & 15u;
+#pragma unroll
+    for (uint32_t k = 0; k < kSteps; ++k) {
+      const uint32_t cr = k * 16 + wave * 4 + kg;
+      store_quad(J, y0, x0, q, ch_base + s * 64 + cr,
+                 *reinterpret_cast<const float4*>(&lds.t[cr * 64 + ((q ^ (cr & 15u)) << 2)]));
+    }
+  }
+}
+
+// Many channels: a workgroup of eight waves takes a block of 64 cells and 512
+// channels, a wave all four squares of 64 channels, and the weights, once per
+// workgroup, go through LDS.  Four k-blocks a round, one barrier: wave w
+// evaluates the weights of square w % 4 in k-blocks w / 4 and w / 4 + 2 of the
+// round to come and contracts all squares of the present one, two k-blocks
+// after each.  Half of the waves (one on each SIMD) start with the weights and
+// half with the products, so that matrix and vector instructions overlap.  The
+// channel values of two k-blocks are read when the two before are done with,
+// and arrive while weights are evaluated.
+constexpr uint32_t kWideWaves = 8, kWideList = 256;
+union MfmaWideLds {
+  struct {
+    s16x8_t a[2][4][4][2][64];  // [round parity][k-block][square][hi, lo][lane]
+    uint32_t any[2][4][4];      // the operand holds a weight
+    Staged<128> st[2];
+    BlockList<kWideList> bl;
+    MfmaCells c;
+    double wsum[kWideWaves][16];
+    double inv[kMcCols];
+    uint32_t total;
+  } s;
+  float t[kWideWaves][16 * 64];  // the epilogue's 16 channels x 64 cells of a wave
+};
+
+template <int DT, bool LEAN>
+__device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint32_t group, MfmaWideLds& lds,
+                                          const double* s_exp) {
+  constexpr bool bf = DT == kDtBf16;
+  const GridParams& P = J.P;
+  const GridBuffers& B = J.B;
+  const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6, kg = lane >> 4;
+  const hcg_ring_meta m = *B.meta;
+  const uint32_t y0 = (tile / J.tiles_x) << (6u - J.tc_shift), x0 = (tile % J.tiles_x) << J.tc_shift;
+  MfmaCells& C = lds.s.c;
+  BlockList<kWideList>& L = lds.s.bl;
+  const Squares sq(J.tc_shift);
+  const uint32_t mb_own = wave & 3u, kb_own = wave >> 2;  // whose weights this wave evaluates
+
+  const MfmaPlan* const plan =
+      J.plan ? reinterpret_cast<const MfmaPlan*>(static_cast<const char*>(J.plan) + tile * kPlanBytes) : nullptr;
+  const bool planned = plan && __builtin_amdgcn_readfirstlane(plan->ok) != 0;  // uniform
+  if (planned) {
+    if (wave < 3) {
+      C.p[wave][lane] = plan->p[wave][lane];
+    } else if (wave == 3) {
+      C.win[lane].uring = plan->uring[lane];
+      C.win[lane].dring = plan->dring[lane];
+    } else if (wave == 4) {
+      C.wlo[lane] = plan->wlo[lane];
+      C.wwid[lane] = plan->wwid[lane];
+    } else if (wave == 5 && lane == 0) {
+      L.span.T.r_begin = plan->r_begin;
+      L.span.T.r_end = plan->r_end;
+      L.span.simple = true;
     }
   } else if (wave == 0) {
-    double q[3];
-    uint32_t ur, dr;
-    L.win[lane] = block_cell_window(P, B, m, y0, x0, tc_shift, lane, q, ur, dr);
-    L.p[lane][0] = q[0];
-    L.p[lane][1] = q[1];
-    L.p[lane][2] = q[2];
-    if (lane == 0) {
-      L.span[0] = ur;
-      L.span[1] = dr;
-    }
+    bool lv;
+    const CellGeom g = block_cell(P, B, m, y0, x0, J.tc_shift, lv);
+    put_cell(C, lane, g);
+    const BlockSpan S = cells_span(P, m, g, lv);
+    if (lane == 0) L.span = S;
   }
   __syncthreads();
-  const double px = L.p[c][0], py = L.p[c][1], pz = L.p[c][2];
-  double wsum = 0.0;
-
-  // accumulators: 4 row blocks x kMcNB channel blocks of 16x16
-  f32x4_t acc[4][kMcNB];
+  const uint32_t cb = sq.cell(mb_own, lane & 15u);
+  const uint32_t crow = y0 + (cb >> J.tc_shift), ccol = x0 + (cb & ((1u << J.tc_shift) - 1u));
+  const bool live = crow < P.side && ccol < P.side;
+  const uint32_t cell = live ? crow * P.side + ccol : 0;
+  const uint32_t r_begin = __builtin_amdgcn_readfirstlane(L.span.T.r_begin);
+  const uint32_t r_end = __builtin_amdgcn_readfirstlane(L.span.T.r_end);
+  SquareCell<LEAN> Q;
+  Q.init(P, C, cb, __builtin_amdgcn_readfirstlane((uint32_t)L.span.simple) != 0);
+  const uint32_t ch_base = (group * kWideWaves + wave) * 64u;
+  const bool mine = ch_base < J.nchan;  // uniform: the wave has channels
+  const char* const vs = value_rows(J, mine ? ch_base : 0);
+  const size_t blk_bytes = (size_t)J.nchan * kVB * 2u;
+  f32x4_t acc[4][4];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < kMcNB; ++nb) acc[mb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const uint32_t ch_base = (group * nw + wave) * kMcChanPerWave;
-  // B operand addressing: lane l reads samples 8 (l / 16) .. +7 of a
-  // k-block for channel ch_base + 16 nb + l % 16 (clamped to the last one)
-  const uint32_t kg = lane >> 4, koff = kg * 8;  // the lane's k-group: samples koff .. koff + 7 of a k-block
-  uint32_t lofs[kMcNB];
-#pragma unroll
-  for (int nb = 0; nb < kMcNB; ++nb) {
-    const uint32_t ch = ch_base + nb * 16 + (lane & 15);
-    lofs[nb] = (ch < nchan ? ch : nchan - 1) * (kVB * 2u);
-  }
-  // the lane's value block of k-block u of descriptor db
-  const char* vs_bytes = reinterpret_cast<const char*>(vs);
-  auto kblock = [&](uint32_t db, uint32_t u) {
-    return vs_bytes + (size_t)L.dgb[db][u * (32 / kVB) + kg] * (blk * 2);
-  };
+  for (int i = 0; i < 16; ++i) acc[i / 4][i % 4] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  s16x8_t bn[2][4];
 
-  const uint32_t r_begin = L.span[0], r_end = L.span[1];
-  const uint32_t n_all = m.n;       // sorted samples (records and keys beyond are not read)
-  constexpr uint32_t KV = CHUNK / kVB;    // value blocks per chunk
-  constexpr uint32_t KSEG = CHUNK / 32;   // segments per chunk
-
-  auto planned = [&](uint32_t rr) { return J.plan != nullptr && (rr - r_begin) < kPlanRings; };
-  auto plan_lo = [&](uint32_t rr) { return L.plan[2 + 2 * (rr - r_begin)]; };
-  auto plan_hi = [&](uint32_t rr) { return L.plan[3 + 2 * (rr - r_begin)]; };
-  // sorted index of chunk position p of descriptor db
-  auto gidx = [&](uint32_t db, uint32_t p) { return L.dgb[db][p / kVB] * kVB + (p % kVB); };
-
-  // ---- chunk descriptors -----------------------------------------------------
-  // A chunk packs the value blocks of consecutive rings' union ranges, at
-  // most KV blocks in at most KSEG segments: ring r's blocks [lo_r / kVB,
-  // (hi_r + kVB - 1) / kVB), in ascending ring and block order, so the
-  // staged keys are sorted and each cell's band in a ring is one interval of
-  // the chunk.  The chunk's k-blocks (32 positions) are nkb = ceil(blocks /
-  // 4); the slots past the last block repeat it (their positions are staged
-  // empty, weight 0).  Wave 0 builds them, one ahead, walking the rings from
-  // its cursor (ring cr at block offset cbo of its range [clo, chi)); a ring
-  // past the plan has its range searched here (every lane of wave 0 takes
-  // part).
-  uint32_t cr = r_begin, cbo = 0, clo = 0, chi = 0;
-  bool crange = false;
-  constexpr uint32_t VPK = 32 / kVB;  // value blocks per k-block
-  static_assert(KSEG >= VPK && KV % VPK == 0, "chunk geometry");
-  auto build_desc = [&](uint32_t db) {  // wave 0, uniform
-    uint32_t nvb = 0, nseg = 0;
-    while (nvb < KV && r_begin <= r_end && cr <= r_end) {
-      // with at most VPK - 1 segments left, only complete the current
-      // k-block, then end the chunk: every chunk but a tile's last ends on a
-      // k-block boundary, so k-block j of a tile is always value blocks
-      // VPK j .. VPK j + VPK - 1 of the tile's block sequence whatever the
-      // chunk size, and the FP32 sums do not depend on it
-      const uint32_t need = (VPK - nvb % VPK) % VPK;
-      const bool closing = nseg + (VPK - 1) >= KSEG;
-      if (closing && need == 0) break;  // uniform
-      if (!crange) {
-        clo = chi = 0;
-        if (planned(cr)) {
-          clo = plan_lo(cr);
-          chi = plan_hi(cr);
-        } else {
-          const uint32_t kr = cr - m.firstring;
-          const uint32_t start = B.lut[kr], end = B.lut[kr + 1];
-          if (start != end) {  // uniform
-            uint32_t a, b;
-            ring_cell_window(P, B, m, L.win[lane], cr, a, b);
-            ring_union_range(B, a, b, start, end, clo, chi);
-          }
-        }
-        crange = true;
-        cbo = 0;
-      }
-      if (clo >= chi) {
-        ++cr;
-        crange = false;
-        continue;
-      }
-      const uint32_t b0 = clo / kVB + cbo, b1 = (chi + kVB - 1) / kVB;
-      uint32_t take = min(KV - nvb, b1 - b0);
-      if (closing) take = min(take, need);
-      if (lane == 0) {
-        for (uint32_t t = 0; t < take; ++t) L.dgb[db][nvb + t] = b0 + t;
-        L.dring[db][nseg] = cr;
-        L.du0[db][nseg] = (uint16_t)nvb;
-        L.dnb[db][nseg] = (uint16_t)take;
-      }
-      nvb += take;
-      ++nseg;
-      if (b0 + take == b1) {
-        ++cr;
-        crange = false;
-      } else {
-        cbo += take;
-      }
-    }
-    const uint32_t nkb = (nvb + VPK - 1) / VPK;
-    if (lane == 0) {
-      for (uint32_t t = nvb; t < nkb * VPK; ++t) L.dgb[db][t] = L.dgb[db][nvb - 1];
-      L.dn[db][0] = nkb;
-      L.dn[db][1] = nseg;
-      L.dn[db][2] = nvb;
-    }
-  };
-
-  // The same packing built by the 64 lanes of wave 0 at once, for a tile
-  // whose rings are all in its plan: lane l holds ring r_begin + l (its
-  // block count nb, 0 when empty, and its offset ex in the tile's block
-  // sequence, an exclusive prefix sum), and the non-empty rings are ranked
-  // by popcount.  A chunk starting at block cpos ends at E = min(cpos + KV,
-  // the first k-block boundary at or after the end of the (KSEG - VPK +
-  // 1)-th non-empty ring from the one holding cpos) -- where the walk above
-  // stops -- and every ring overlapping [cpos, E) writes its own segment.
-  // Lanes exchange values by shuffles only: LDS slots are read back by the
-  // lane that wrote them.
-  const bool par_desc = J.plan != nullptr && r_begin <= r_end && r_end - r_begin < kPlanRings;  // uniform
-  uint32_t cpos = 0;
-  auto ring_list = [&]() {  // wave 0
-    const uint32_t r = r_begin + lane;
-    uint32_t nb = 0, b0 = 0;
-    if (r <= r_end) {
-      const uint32_t lo = plan_lo(r), hi = plan_hi(r);
-      if (lo < hi) {
-        b0 = lo / kVB;
-        nb = (hi + kVB - 1) / kVB - b0;
-      }
-    }
-    uint32_t incl = nb;  // inclusive prefix sum over the lanes
-#pragma unroll
-    for (uint32_t off = 1; off < 64; off <<= 1) {
-      const uint32_t t = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += t;
-    }
-    L.rl_b0[lane] = b0;
-    L.rl_ex[lane] = incl - nb;
-    L.rl_nb[lane] = nb;
-  };
-  auto build_desc_par = [&](uint32_t db) {  // wave 0, after ring_list
-    const uint32_t b0 = L.rl_b0[lane], ex = L.rl_ex[lane], nb = L.rl_nb[lane];  // this lane's own slots
-    const uint32_t in = ex + nb;
-    const uint32_t total = __shfl(in, 63, 64);
-    uint32_t nvb = 0, nseg = 0;
-    const uint64_t hm = __ballot(nb > 0 && ex <= cpos && cpos < in);  // the ring holding cpos
-    if (cpos < total && hm) {  // uniform (the rings' [ex, ex + nb) tile [0, total): one lane holds cpos)
-      const uint64_t ne = __ballot(nb > 0);
-      const uint32_t rank = (uint32_t)__popcll(ne & ((1ull << lane) - 1ull));
-      const uint32_t kl = (uint32_t)__ffsll((long long)hm) - 1u;
-      const uint32_t rk = __shfl(rank, kl, 64);  // the rank of the ring holding cpos
-      const uint64_t tm = __ballot(nb > 0 && rank == rk + (KSEG - (VPK - 1)) - 1u);
-      const uint32_t tl = tm ? (uint32_t)__ffsll((long long)tm) - 1u : 63u;
-      const uint32_t end_t = __shfl(in, tl, 64);
-      const uint32_t pos_s = tm ? end_t : total;
-      const uint32_t e = min(min(cpos + KV, total), (pos_s + VPK - 1) / VPK * VPK);
-      const uint32_t nkb = (e - cpos + VPK - 1) / VPK;
-      const bool seg = nb > 0 && lane >= kl && ex < e && rank - rk < KSEG;
-      if (seg) {
-        const uint32_t sg = rank - rk;
-        const uint32_t a = max(ex, cpos), b = min(in, e);
-        const uint32_t du = a - cpos, g0 = b0 + (a - ex);
-        L.dring[db][sg] = r_begin + lane;
-        L.du0[db][sg] = (uint16_t)du;
-        L.dnb[db][sg] = (uint16_t)(b - a);
-        for (uint32_t t = 0; t < b - a; ++t) L.dgb[db][du + t] = g0 + t;
-        if (b == e)  // the last segment repeats its last block up to the k-block boundary
-          for (uint32_t p = e - cpos; p < nkb * VPK; ++p) L.dgb[db][p] = g0 + (b - a - 1);
-      }
-      nseg = (uint32_t)__popcll(__ballot(seg));
-      nvb = e - cpos;
-      cpos = e;
-    }
-    if (lane == 0) {
-      L.dn[db][0] = (nvb + VPK - 1) / VPK;
-      L.dn[db][1] = nseg;
-      L.dn[db][2] = nvb;
-    }
-  };
-
-  // ---- per-chunk steps -------------------------------------------------
-  // stage chunk positions [from, 32 nkb) of descriptor db into LDS (keys past
-  // the samples and past the chunk's nvb value blocks are the empty key,
-  // beyond every window)
-  auto stage = [&](uint32_t db, uint32_t from, uint32_t nkb, uint32_t nvb) {
-    for (uint32_t p = from + tid; p < nkb * 32u; p += nthreads) {
-      const uint32_t g = gidx(db, p);
-      if (g < n_all && p < nvb * kVB) {
-        const hcg_sample q = B.rec[g];
-        s_x[p] = q.x;
-        s_y[p] = q.y;
-        s_z[p] = q.z;
-        s_key[p] = B.keys[g];
-      } else {
-        s_x[p] = s_y[p] = s_z[p] = 0.0;
-        s_key[p] = 0xFFFFFFFFu;
-      }
-    }
-  };
-  // zero the weight tiles' used width
-  auto clear = [&](uint32_t nkb) {
-    const uint32_t width8 = nkb * 4;  // 16-byte groups per row
-    for (uint32_t g = tid; g < kMcCols * width8; g += nthreads) {
-      const uint32_t rr = g / width8, cc = (g % width8) * 8;
-      *reinterpret_cast<uint4*>(&s_wh[rr * RS + cc]) = uint4{0u, 0u, 0u, 0u};
-      *reinterpret_cast<uint4*>(&s_wl[rr * RS + cc]) = uint4{0u, 0u, 0u, 0u};
-    }
-  };
-  // reset the row blocks' k-block spans of buffer db (read last by the
-  // contraction two chunks back, written by the bands of the next chunk)
-  auto reset_spans = [&](uint32_t db) {
-    if (tid < 4) {
-      s_mb[db][tid][0] = 0xFFFFFFFFu;
-      s_mb[db][tid][1] = 0u;
-    }
-  };
-  // each cell's band in each segment of the chunk (wave w: segments w, w +
-  // nw, ...), and the row blocks' k-block spans
-  auto bands = [&](uint32_t db, uint32_t nseg) {
-    for (uint32_t sg = wave; sg < nseg; sg += nw) {
-      uint32_t a, b;
-      ring_cell_window(P, B, m, L.win[lane], L.dring[db][sg], a, b);
-      uint32_t ja = 0, jb = 0;
-      if (a <= b) {
-        const uint32_t p0 = (uint32_t)L.du0[db][sg] * kVB, p1 = p0 + (uint32_t)L.dnb[db][sg] * kVB;
-        ja = lower_bound_u32(s_key, p0, p1, a);
-        jb = upper_bound_u32(s_key, ja, p1, b);
-        if (ja < jb) {
-          atomicMin(&s_mb[db][lane >> 4][0], ja >> 5);
-          atomicMax(&s_mb[db][lane >> 4][1], (jb + 31) >> 5);
-        }
-      }
-      L.band[sg][lane] = ja | (jb << 16);
-    }
-  };
-  // the lean form (kKtGaussLean): the tile loop's p.q candidate test on
-  // h = 1 - p.q and gauss_weight_lean, the guard band after the weight
-  const double npx = -px, npy = -py, npz = -pz;
-  const double h_hi = 0.5 * P.c_hi, h_lo = 0.5 * P.c_lo, k0h = 2.0 * P.k0;
-  const bool lean = kt == kKtGaussLean && B.w_s == nullptr;
-  const double k1v = in_vgprs(4.0 * P.k1), e3v = in_vgprs(kExpE3);
-  // the weight wt of pair (c, j) as hi + lo in the value type (~2x its
-  // significand), its two halves stored in the weight tiles and summed
-  auto store_weight = [&](uint32_t j, double wt) {
-    const float wf = (float)wt;
-    const uint16_t hi = round16(wf, bf);
-    const float hif = widen16(hi, bf);
-    // wf - hif is exact (Sterbenz), and hif + lof is exact in FP32 (at most
-    // 2 x 11 significant bits, the second ~2^-8 below the first)
-    const uint16_t lo = round16(wf - hif, bf);
-    s_wh[c * RS + j] = hi;
-    s_wl[c * RS + j] = lo;
-    wsum += (double)(hif + widen16(lo, bf));
-  };
-  // weights of this thread's cell over its bands in the chunk (after the
-  // bands barrier)
-  auto weigh = [&](uint32_t db, uint32_t nseg) {
-    if (lean) {  // uniform
-      for (uint32_t sg = 0; sg < nseg; ++sg) {
-        const uint32_t bd = L.band[sg][c];
-        const uint32_t ja = bd & 0xFFFFu, jb = bd >> 16;
-        for (uint32_t j = ja + sub; j < jb; j += S) {
-          const double h = fma(npx, s_x[j], fma(npy, s_y[j], fma(npz, s_z[j], 1.0)));
-          if (h < h_hi) {
-            double wt = gauss_weight_lean(h, k0h, k1v, e3v, s_exp);
-            if (__builtin_amdgcn_ballot_w64(!(h < h_lo))) {  // some lane in the guard band (rare)
-              asm volatile("; guard band" ::);                // (keeps the branch above a scalar one)
-              if (!(h < h_lo) && !radius_test_ref(B.xwcs, B.ywcs, B.lon_s, B.lat_s, cell, gidx(db, j),
-                                                  P.sphere_radius))
-                wt = 0.0;
-            }
-            store_weight(j, wt);
-          }
-        }
-      }
-      return;
-    }
-    for (uint32_t sg = 0; sg < nseg; ++sg) {
-      const uint32_t bd = L.band[sg][c];
-      const uint32_t ja = bd & 0xFFFFu, jb = bd >> 16;
-      for (uint32_t j = ja + sub; j < jb; j += S) {
-        const double dx = px - s_x[j], dy = py - s_y[j], dz = pz - s_z[j];
-        const double c2 = fma(dx, dx, fma(dy, dy, dz * dz));
-        if (c2 < P.c_hi &&
-            (c2 < P.c_lo || radius_test_ref(B.xwcs, B.ywcs, B.lon_s, B.lat_s, cell, gidx(db, j), P.sphere_radius))) {
-          // (the sample's sorted index only for the kernels that read its coordinates)
-          const bool need_i = kt == HCG_GAUSS2D || kt == HCG_TAPERED_SINC;
-          double wt = pair_weight_any(P, B, kt, c2, s_exp, cell, need_i ? gidx(db, j) : 0u);
-          if (B.w_s) wt *= B.w_s[gidx(db, j)];
-          store_weight(j, wt);
-        }
-      }
-    }
-  };
-  // the contraction over the chunk's k-blocks; bn holds block 0's channel
-  // values on entry
-  auto contract = [&](uint32_t db, uint32_t nkb, vec* b0) {
-    // the row blocks' k-block spans (wave-uniform: scalar compares)
-    uint32_t mblo[4], mbhi[4];
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-      mblo[mb] = __builtin_amdgcn_readfirstlane(s_mb[db][mb][0]);
-      mbhi[mb] = __builtin_amdgcn_readfirstlane(s_mb[db][mb][1]);
-    }
-    // block u's MFMAs on B operand b
-    auto mfmas = [&](uint32_t u, const vec* b) {
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        if (!(u >= mblo[mb] && u < mbhi[mb])) continue;
-        // A: the row block's hi and lo weights, from LDS
-        const uint32_t off = (mb * 16 + (lane & 15)) * RS + u * 32 + koff;
-        const vec ah = *reinterpret_cast<const vec*>(&s_wh[off]);
-        const vec al = *reinterpret_cast<const vec*>(&s_wl[off]);
-#pragma unroll
-        for (int nb = 0; nb < kMcNB; ++nb) {
-          acc[mb][nb] = mfma16(bf, ah, b[nb], acc[mb][nb]);
-          acc[mb][nb] = mfma16(bf, al, b[nb], acc[mb][nb]);
-        }
-      }
-    };
-    // software pipeline over two register sets (no copies): block u's
-    // MFMAs run while block u+1's channel values load.  The loads are
-    // unconditional (past the last block they repeat it, unused), so every
-    // MFMA waits only for its own operand's loads
-    vec b1[kMcNB];
-    const uint32_t last = nkb - 1;
-    for (uint32_t u = 0; u < nkb; u += 2) {
-      load_b_rows(b1, kblock(db, min(u + 1, last)), lofs);
-      mfmas(u, b0);
-      if (u + 1 >= nkb) break;
-      load_b_rows(b0, kblock(db, min(u + 2, last)), lofs);
-      mfmas(u + 1, b1);
-    }
-  };
-
-  // ---- chunks ---------------------------------------------------------------
-  // barriers per chunk: staging (B1, only when records are left to stage),
-  // bands (B2), weights (B3), contraction done (T).  The next chunk's
-  // descriptor is built by wave 0 between B2 and B3; its first nthreads
-  // records load during the contraction and go to LDS after it (the
-  // contraction reads only weight tiles and channel values), so a chunk of
-  // at most nthreads samples needs no staging of its own.
-  uint32_t db = 0, staged = 0;
-  if (wave == 0) {
-    if (par_desc) {
-      ring_list();
-      build_desc_par(0);
-    } else {
-      build_desc(0);
-    }
-  }
-  reset_spans(0);
-  __syncthreads();
-  for (;;) {
-    const uint32_t nkb = L.dn[db][0], nseg = L.dn[db][1], nvb = L.dn[db][2];
-    if (nkb == 0) break;  // uniform
-    clear(nkb);
-    reset_spans(db ^ 1u);
-    if (staged < nkb * 32u) {  // uniform
-      stage(db, staged, nkb, nvb);
-      __syncthreads();  // B1
-    }
-    bands(db, nseg);
-    __syncthreads();  // B2
-    // channel values of the chunk's first k-block, in flight while the weights are computed
-    vec bn[kMcNB];
-    if (ch_base < nchan) load_b_rows(bn, kblock(db, 0), lofs);
+  for (uint32_t rb = r_begin; r_begin <= r_end && rb <= r_end; rb += 64) {
+    __syncthreads();
     if (wave == 0) {
-      if (par_desc)
-        build_desc_par(db ^ 1u);
-      else
-        build_desc(db ^ 1u);
-    }
-    weigh(db, nseg);
-    __syncthreads();  // B3
-    const uint32_t nn = L.dn[db ^ 1u][0] * 32u, nvb_next = L.dn[db ^ 1u][2];
-    staged = min(nn, nthreads);
-    const bool pre = tid < staged;
-    hcg_sample pq{};
-    uint32_t pkey = 0xFFFFFFFFu;
-    if (pre) {
-      const uint32_t g = gidx(db ^ 1u, tid);
-      if (g < n_all && tid < nvb_next * kVB) {
-        pq = B.rec[g];
-        pkey = B.keys[g];
-      }
-    }
-    if (ch_base < nchan) contract(db, nkb, bn);
-    if (pre) {
-      s_x[tid] = pq.x;
-      s_y[tid] = pq.y;
-      s_z[tid] = pq.z;
-      s_key[tid] = pkey;
-    }
-    db ^= 1u;
-    __syncthreads();  // T
-  }
-
-  // per-cell weight sums over the waves (exact in FP64 in any order: every
-  // weight is hi + lo of two 16-bit values); the weight tiles are free now
-  __syncthreads();
-  double* wpart = reinterpret_cast<double*>(L.w);
-  wpart[wave * kMcCols + lane] = wsum;
-  __syncthreads();
-  if (wave == 0) {
-    double t = 0.0;
-    for (uint32_t w = 0; w < nw; ++w) t += wpart[w * kMcCols + lane];
-    // the normalisation as one multiply per value: v * (1 / t) is within an
-    // FP64 ulp or two of v / t, so the FP32 result is the quotient's except
-    // where it lies that close to an FP32 rounding boundary (1 ulp then);
-    // t = 0 gives inf, so an empty cell is 0 * inf = NaN as 0 / 0 is
-    s_inv[lane] = normalize ? 1.0 / t : 1.0;
-    if (group == 0 && wsum_out && live) wsum_out[cell] = (float)t;
-  }
-  __syncthreads();
-  // lane l holds cells 16 mb + 4 (l / 16) + j, j = 0..3: four consecutive
-  // cells of one map row (tile widths are multiples of 4), stored as one
-  // 16-byte piece when the map side is a multiple of 4 (then aligned)
-  auto value = [&](int mb, int nb, int j, uint32_t cl0) {
-    return (float)((double)acc[mb][nb][j] * s_inv[cl0 + j]);
-  };
-  constexpr uint32_t kEpiFloats = kMcCols * 64;  // one wave's 64 cells x 64 channels
-  if (STAGED && (P.side & 3u) == 0 && nw * kEpiFloats * sizeof(float) <= sizeof(L.w)) {  // uniform
-    // Through LDS: each wave stages its cells x channels by channel (the
-    // 16-byte quads of a channel's row XOR-swizzled by the channel, so the
-    // 16 channels of a write, and the 16 quads of a read, fall in 16
-    // distinct bank groups), then stores four channels per instruction, a
-    // channel's 64 cells as 16 pieces of 4 consecutive cells of a map row.
-    // An instruction then spans 4 channel planes instead of 16 (each plane
-    // its own pages: 4 MB at 1024^2), so it needs fewer address
-    // translations.  The weight tiles are free: the last chunk's
-    // contraction and the weight-sum reduction are behind barriers.
-    float* T = reinterpret_cast<float*>(L.w) + (size_t)wave * kEpiFloats;
-    if (ch_base < nchan) {
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const uint32_t q = mb * 4 + (lane >> 4), cl0 = q * 4;
-#pragma unroll
-        for (int nb = 0; nb < kMcNB; ++nb) {
-          const uint32_t cr = nb * 16 + (lane & 15);
-          *reinterpret_cast<float4*>(&T[cr * 64 + ((q ^ (cr & 15u)) << 2)]) =
-              make_float4(value(mb, nb, 0, cl0), value(mb, nb, 1, cl0), value(mb, nb, 2, cl0), value(mb, nb, 3, cl0));
-        }
-      }
+      const uint32_t t =
+          planned ? put_rings(P, L, rb, plan->b0[lane], plan->nb[lane]) : ring_blocks(P, B, m, rb, L);
+      if (lane == 0) lds.s.total = t;
     }
     __syncthreads();
-    if (ch_base < nchan) {
-      const uint32_t q = lane & 15, cl0 = q * 4;
-      const uint32_t rowj = y0 + (cl0 >> tc_shift), col0 = x0 + (cl0 & tc_mask);
-      const bool in_map = col0 < P.side && rowj < P.side;
+    const uint32_t total = __builtin_amdgcn_readfirstlane(lds.s.total);
+    for (uint32_t q0 = 0; q0 < total; q0 += kWideList) {  // uniform
+      const uint32_t cnt = min(total - q0, kWideList), nkb = (cnt + 3) / 4, nr = (nkb + 3) / 4;
+      __syncthreads();
+      if (wave == 0) list_blocks(L, q0, cnt);
+      __syncthreads();
+      // waves 0 to 3 stage the 128 samples of round r (a k-block past the
+      // last is neither staged nor weighed)
+      StageRegs st;
+      const uint32_t ssp = (wave & 1u) * 64 + lane;  // sample of a round
+      auto fetch = [&](uint32_t r) {
+        if (wave < 4 && 4 * r + (ssp >> 5) < nkb) st.fetch(B, m, L, 4 * r + (ssp >> 5), ssp & 31u, wave >> 1);
+      };
+      auto stage = [&](uint32_t r) {
+        if (wave < 4 && 4 * r + (ssp >> 5) < nkb) st.store(lds.s.st[r & 1u], ssp, wave >> 1);
+      };
+      auto load_b = [&](uint32_t u) {  // of k-blocks u and u + 1
+        if (!mine) return;
 #pragma unroll
-      for (uint32_t k = 0; k < 16; ++k) {
-        const uint32_t cr = k * 4 + (lane >> 4), ch = ch_base + cr;
-        const float4 v = *reinterpret_cast<const float4*>(&T[cr * 64 + ((q ^ (cr & 15u)) << 2)]);
-        if (in_map && ch < nchan)
-          *reinterpret_cast<float4*>(cube + (size_t)ch * M + (size_t)rowj * P.side + col0) = v;
+        for (uint32_t kb = 0; kb < 2; ++kb) {
+          const uint32_t blk = L.lb[min(u + kb, nkb - 1) * 4 + kg];
+#pragma unroll
+          for (int nb = 0; nb < 4; ++nb)
+            bn[kb][nb] = *reinterpret_cast<const s16x8_t*>(vs + blk * blk_bytes + nb * (16 * kVB * 2));
+        }
+      };
+      auto weigh = [&](uint32_t r, uint32_t h) {  // k-block kb_own + 2 h of round r
+        const uint32_t k = kb_own + 2 * h, u = 4 * r + k, par = r & 1u;
+        uint64_t any = 0;
+        if (u < nkb) {  // uniform
+          const uint32_t blk = L.lb[u * 4 + kg];
+          uint32_t wl, ww;
+          Q.window(P, C, L, rb, L.lr[u * 4 + kg], wl, ww);
+          WeightOperand A;
+          uint64_t guard;
+          any = weigh_kblock<DT>(J, Q, lds.s.st[par], k * 32, wl, ww, cell, blk, s_exp, A, guard);
+          if (guard) {  // uniform, rare; the sums wait in scratch memory (see mfma_tile)
+            volatile float keep[64];
+#pragma unroll
+            for (int i = 0; i < 64; ++i) keep[i] = acc[i / 16][i / 4 % 4][i % 4];
+            guard_kblock<DT>(J, Q, lds.s.st[par], k * 32, wl, ww, cell, blk, A);
+#pragma unroll
+            for (int i = 0; i < 64; ++i) acc[i / 16][i / 4 % 4][i % 4] = keep[i];
+          }
+          if (any) {
+            lds.s.a[par][k][mb_own][0][lane] = A.h.v;
+            lds.s.a[par][k][mb_own][1][lane] = A.l.v;
+          }
+        }
+        if (lane == 0) lds.s.any[par][k][mb_own] = any != 0;
+      };
+      auto contract = [&](uint32_t r, uint32_t h) {  // k-blocks 2 h and 2 h + 1 of round r
+        if (!mine) return;
+        const uint32_t par = r & 1u;
+        uint32_t some[2][4];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) some[i / 4][i % 4] = lds.s.any[par][2 * h + i / 4][i % 4];
+#pragma unroll
+        for (uint32_t kb = 0; kb < 2; ++kb) {
+          s16x8_t ah[4], al[4];  // (stale where a square has no weight, and unused)
+#pragma unroll
+          for (uint32_t mb = 0; mb < 4; ++mb) {
+            ah[mb] = lds.s.a[par][2 * h + kb][mb][0][lane];
+            al[mb] = lds.s.a[par][2 * h + kb][mb][1][lane];
+          }
+#pragma unroll
+          for (uint32_t mb = 0; mb < 4; ++mb) {
+            if (!__builtin_amdgcn_readfirstlane(some[kb][mb])) continue;  // uniform
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+              acc[mb][nb] = mfma16(bf, ah[mb], bn[kb][nb], acc[mb][nb]);
+              acc[mb][nb] = mfma16(bf, al[mb], bn[kb][nb], acc[mb][nb]);
+            }
+          }
+        }
+      };
+      fetch(0);
+      stage(0);
+      load_b(0);
+      fetch(1);
+      __syncthreads();
+      weigh(0, 0);
+      weigh(0, 1);
+      stage(1);
+      __syncthreads();
+      for (uint32_t r = 0; r < nr; ++r) {
+        fetch(r + 2);
+        const bool more = r + 1 < nr;
+#pragma unroll 1
+        for (uint32_t h = 0; h < 2; ++h) {
+          if (wave < kWideWaves / 2 && more) weigh(r + 1, h);
+          contract(r, h);
+          load_b(4 * r + 2 * h + 2);
+          if (wave >= kWideWaves / 2 && more) weigh(r + 1, h);
+        }
+        stage(r + 2);
+        __syncthreads();
       }
     }
-    return;
   }
-  if (ch_base < nchan) {
-    if ((P.side & 3u) == 0) {  // uniform
+
+  // the weight sums of a square's two waves (see mfma_tile)
+  double wsum = Q.wsum;
+  wsum += __shfl_xor(wsum, 16, 64);
+  wsum += __shfl_xor(wsum, 32, 64);
+  if (lane < 16) lds.s.wsum[wave][lane] = wsum;
+  __syncthreads();
+  if (wave < 4 && lane < 16) {
+    const double t = lds.s.wsum[wave][lane] + lds.s.wsum[wave + 4][lane];
+    if (group == 0 && J.wsum && live) J.wsum[cell] = (float)t;
+    lds.s.inv[cb] = J.normalize ? 1.0 / t : 1.0;
+  }
+  __syncthreads();
+  double iv[4][4];
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const uint32_t cl0 = mb * 16 + (lane >> 4) * 4;
-        const uint32_t rowj = y0 + (cl0 >> tc_shift), col0 = x0 + (cl0 & tc_mask);
-        if (col0 >= P.side || rowj >= P.side) continue;
+  for (uint32_t mb = 0; mb < 4; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < kMcNB; ++nb) {
-          const uint32_t ch = ch_base + nb * 16 + (lane & 15);
-          if (ch >= nchan) continue;
-          float* dst = cube + (size_t)ch * M + (size_t)rowj * P.side + col0;
-          *reinterpret_cast<float4*>(dst) =
-              make_float4(value(mb, nb, 0, cl0), value(mb, nb, 1, cl0), value(mb, nb, 2, cl0), value(mb, nb, 3, cl0));
-        }
-      }
-    } else {
+    for (uint32_t j = 0; j < 4; ++j) iv[mb][j] = lds.s.inv[sq.cell(mb, kg * 4 + j)];
+  __syncthreads();
+  // stores as in mfma_tile, 16 channels of the wave's own at a time
+  float* const T = lds.t[wave];
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const uint32_t cl0 = mb * 16 + (lane >> 4) * 4;
-        const uint32_t rowj = y0 + (cl0 >> tc_shift), col0 = x0 + (cl0 & tc_mask);
-        if (col0 >= P.side || rowj >= P.side) continue;
+  for (int nb = 0; nb < 4; ++nb) {
+    tile_sync();
 #pragma unroll
-        for (int nb = 0; nb < kMcNB; ++nb) {
-          const uint32_t ch = ch_base + nb * 16 + (lane & 15);
-          if (ch >= nchan) continue;
-          float* dst = cube + (size_t)ch * M + (size_t)rowj * P.side + col0;
+    for (uint32_t mb = 0; mb < 4; ++mb)
+      *reinterpret_cast<float4*>(&T[(lane & 15u) * 64 + (((sq.cell(mb, kg * 4) >> 2) ^ (lane & 15u)) << 2)]) =
+          make_float4((float)((double)acc[mb][nb][0] * iv[mb][0]), (float)((double)acc[mb][nb][1] * iv[mb][1]),
+                      (float)((double)acc[mb][nb][2] * iv[mb][2]), (float)((double)acc[mb][nb][3] * iv[mb][3]));
+    tile_sync();
+    const uint32_t q = lane & 15u;
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (col0 + j < P.side) dst[j] = value(mb, nb, j, cl0);
-        }
-      }
+    for (uint32_t k = 0; k < 4; ++k) {
+      const uint32_t cr = k * 4 + kg;
+      store_quad(J, y0, x0, q, ch_base + nb * 16 + cr,
+                 *reinterpret_cast<const float4*>(&T[cr * 64 + ((q ^ cr) << 2)]));
     }
   }
 }
 
+// Block b of a launch of 8 xcd_run(tiles) runs on XCD b % 8: each XCD takes a
+// contiguous run of tiles, so neighbouring tiles share an L2.
+__host__ __device__ inline uint32_t xcd_run(uint32_t ntiles) { return (ntiles + 7u) / 8u; }
+__device__ inline uint32_t xcd_tile(uint32_t b, uint32_t ntiles) { return (b & 7u) * xcd_run(ntiles) + (b >> 3); }
 
-// One job, one launch: grid = (tiles, channel groups), tiles in XCD-contiguous
-// runs (block b runs on XCD b % 8, so neighbouring tiles share an L2).
-template <int DT, uint32_t CHUNK>
-__global__ void __launch_bounds__(64 * kMcMaxWaves) k_grid_mfma(MfmaJob J) {
-  __shared__ MfmaLds<CHUNK> L;
+// The kernel instances: NB 16-channel blocks per wave (mfma_tile), or 0: mfma_wide.
+constexpr int mfma_waves_per_simd(int nb, bool lean) {
+  return !lean || nb == 0 ? 2 : nb <= 2 ? 4 : nb <= 6 ? 3 : 2;
+}
+constexpr uint32_t mfma_threads(int nb) { return 64 * (nb == 0 ? kWideWaves : (uint32_t)kMcWaves); }
+template <int NB>
+struct InstanceLds {
+  typedef MfmaLds type;
+};
+template <>
+struct InstanceLds<0> {
+  typedef MfmaWideLds type;
+};
+template <int DT, int NB, bool LEAN>
+__device__ __forceinline__ void mfma_work(const MfmaJob& J, uint32_t tile, uint32_t group) {
+  __shared__ typename InstanceLds<NB>::type lds;
   __shared__ double s_exp[64];
   if (threadIdx.x < 64) exp_table_load(s_exp);
-  uint32_t tile = blockIdx.x;
-  const uint32_t ntiles = J.ntiles;
-  if ((ntiles & 7u) == 0) tile = (blockIdx.x & 7u) * (ntiles >> 3) + (blockIdx.x >> 3);
-  mfma_block<DT, CHUNK, true>(J, tile, blockIdx.y, L, s_exp);
+  if constexpr (NB == 0)
+    mfma_wide<DT, LEAN>(J, tile, group, lds, s_exp);
+  else
+    mfma_tile<DT, NB, LEAN>(J, tile, group, lds, s_exp);
 }
 
-// Many jobs, one launch: a persistent grid pulls work items (job, tile,
-// channel group) from a device queue in list order until the list is
-// exhausted; every workgroup exits when its pull passes nitems.  The list
-// is ordered longest-first by the host, so the tail holds the short items.
-// two 256-sample workgroups (with the exp table and the queue slot) share a
-// CU's 160 KB of LDS; one 512-sample workgroup fills it
-static_assert(2 * (sizeof(MfmaLds<256>) + 64 * sizeof(double) + 16) <= 160 * 1024, "two CHUNK-256 workgroups per CU");
-static_assert(sizeof(MfmaLds<512>) + 64 * sizeof(double) + 16 <= 160 * 1024, "one CHUNK-512 workgroup per CU");
+// One job: grid = (8 xcd_run(tiles), channel groups).
+template <int DT, int NB, bool LEAN>
+__global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, LEAN))))
+    k_grid_mfma(MfmaJob J) {
+  const uint32_t tile = xcd_tile(blockIdx.x, J.ntiles);
+  if (tile >= J.ntiles) return;  // uniform
+  mfma_work<DT, NB, LEAN>(J, tile, blockIdx.y);
+}
 
-template <uint32_t CHUNK>
-__global__ void __launch_bounds__(64 * kMcMaxWaves)
-    k_grid_mfma_batch(const MfmaJob* __restrict__ jobs, const MfmaItem* __restrict__ items, uint32_t nitems,
-                      uint32_t* __restrict__ head) {
-  __shared__ MfmaLds<CHUNK> L;
-  __shared__ double s_exp[64];
-  __shared__ uint32_t s_item;
-  if (threadIdx.x < 64) exp_table_load(s_exp);
-  for (;;) {
-    if (threadIdx.x == 0) s_item = atomicAdd(head, 1u);
-    __syncthreads();
-    const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
-    if (it >= nitems) break;  // uniform: every thread read the same value
-    const uint32_t jb = __builtin_amdgcn_readfirstlane(items[it].job);
-    const uint32_t tile = __builtin_amdgcn_readfirstlane(items[it].tile);
-    const uint32_t group = __builtin_amdgcn_readfirstlane(items[it].group);
-    // one copy of the block per value type: with the type known at compile
-    // time the contraction issues its MFMAs back to back (a type tested at
-    // run time inside the block made the 2M x 1024 cube 15% slower)
-    if (__builtin_amdgcn_readfirstlane(jobs[jb].dtype) == HCG_DTYPE_F16)
-      mfma_block<kDtF16, CHUNK, false>(jobs[jb], tile, group, L, s_exp);
+// The jobs of a batch that one instance serves, in one launch: a workgroup
+// finds its job by binary search over the range starts (multiples of 8).
+template <int DT, int NB, bool LEAN>
+__global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, LEAN))))
+    k_grid_mfma_batch(const TileRange* __restrict__ ranges, uint32_t nranges, const MfmaJob* __restrict__ jobs) {
+  uint32_t lo = 0, hi = nranges;  // last range with first <= blockIdx.x
+  while (hi - lo > 1) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (ranges[mid].first <= blockIdx.x)
+      lo = mid;
     else
-      mfma_block<kDtBf16, CHUNK, false>(jobs[jb], tile, group, L, s_exp);
-    __syncthreads();  // LDS and s_item are free for the next item
+      hi = mid;
   }
+  const MfmaJob& J = jobs[ranges[lo].job];
+  const uint32_t lb = blockIdx.x - ranges[lo].first, per = 8u * xcd_run(J.ntiles);
+  const uint32_t tile = xcd_tile(lb % per, J.ntiles), group = lb / per;
+  if (tile >= J.ntiles) return;  // uniform
+  mfma_work<DT, NB, LEAN>(J, tile, group);
 }
 
-int mfma_batch_blocks(uint32_t chunk, uint32_t waves, uint32_t* blocks) {
-  if (!(waves == 1 || waves == 2 || waves == 4 || waves == 8))
-    return set_error(HCG_ERR_INVALID, "batch: waves must be 1, 2, 4 or 8");
-  if (!(chunk == 128 || chunk == 256 || chunk == 512))
-    return set_error(HCG_ERR_INVALID, "batch: chunk must be 128, 256 or 512");
-  const void* fn = chunk == 512 ? reinterpret_cast<const void*>(&k_grid_mfma_batch<512>)
-                   : chunk == 256 ? reinterpret_cast<const void*>(&k_grid_mfma_batch<256>)
-                                  : reinterpret_cast<const void*>(&k_grid_mfma_batch<128>);
-  int dev = 0, cus = 0, per_cu = 0;
-  HCG_CHECK_HIP(hipGetDevice(&dev));
-  HCG_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  HCG_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * waves, 0));
-  if (per_cu < 1) per_cu = 1;
-  *blocks = (uint32_t)(cus * per_cu);
+// The instance of a job: value type, channel blocks per wave and weight form.
+// A wave's registers grow with its channel blocks, so its SIMD holds fewer
+// waves; more than kNarrow blocks of 16 channels take mfma_wide.
+constexpr uint32_t kNbs = 8, kNbOf[kNbs] = {1, 2, 4, 6, 8, 12, 16, 0};
+constexpr uint32_t kNarrow = 16, kNarrowGeneral = 4;
+constexpr uint32_t kGeneral[2] = {2, 7};  // the general weights' instances, as kNbOf
+static_assert(kMfmaInstances == 2 * (kNbs + 2), "instances");
+static uint32_t nb_of_instance(uint32_t inst) {
+  return kNbOf[inst / 2 < kNbs ? inst / 2 : kGeneral[inst / 2 - kNbs]];
+}
+bool mfma_uses_plan(uint32_t inst) { return nb_of_instance(inst) == 0; }
+uint32_t mfma_instance(const MfmaJob& J) {
+  const uint32_t d = J.dtype == HCG_DTYPE_BF16 ? 0u : 1u, blocks = ceil_div_u32(J.nchan, 16);
+  if (J.kt != kKtGaussLean || J.B.w_s) return 2 * (kNbs + (blocks > kNarrowGeneral ? 1 : 0)) + d;
+  if (blocks > kNarrow) return 2 * (kNbs - 1) + d;
+  uint32_t i = 0;
+  while (kNbOf[i] < blocks) ++i;
+  return 2 * i + d;
+}
+static uint32_t mfma_groups(const MfmaJob& J, uint32_t inst) {
+  const uint32_t nb = nb_of_instance(inst);
+  return ceil_div_u32(J.nchan, nb ? 16u * nb : 64u * kWideWaves);
+}
+uint64_t mfma_blocks(const MfmaJob& J) {
+  return (uint64_t)8u * xcd_run(J.ntiles) * mfma_groups(J, mfma_instance(J));
+}
+
+#define HCG_MFMA_PAIR(X, I, NB, LEAN) X(2 * (I), kDtBf16, NB, LEAN) X(2 * (I) + 1, kDtF16, NB, LEAN)
+#define HCG_MFMA_INSTANCES(X)                                                                               \
+  HCG_MFMA_PAIR(X, 0, kNbOf[0], true) HCG_MFMA_PAIR(X, 1, kNbOf[1], true) HCG_MFMA_PAIR(X, 2, kNbOf[2], true) \
+  HCG_MFMA_PAIR(X, 3, kNbOf[3], true) HCG_MFMA_PAIR(X, 4, kNbOf[4], true) HCG_MFMA_PAIR(X, 5, kNbOf[5], true) \
+  HCG_MFMA_PAIR(X, 6, kNbOf[6], true) HCG_MFMA_PAIR(X, 7, kNbOf[7], true)                                     \
+  HCG_MFMA_PAIR(X, kNbs, kNbOf[kGeneral[0]], false) HCG_MFMA_PAIR(X, kNbs + 1, kNbOf[kGeneral[1]], false)
+
+static int launch_mfma_job(const MfmaJob& J, hipStream_t s) {
+  const uint32_t inst = mfma_instance(J);
+  const dim3 grid(8u * xcd_run(J.ntiles), mfma_groups(J, inst));
+  if (J.plan) {
+    k_mfma_plan<<<J.ntiles, 64, 0, s>>>(J);
+    HCG_CHECK_LAUNCH("k_mfma_plan");
+  }
+#define HCG_CASE(I, DT, NB, LEAN) \
+  case I: k_grid_mfma<DT, NB, LEAN><<<grid, mfma_threads(NB), 0, s>>>(J); break;
+  switch (inst) { HCG_MFMA_INSTANCES(HCG_CASE) }
+#undef HCG_CASE
+  HCG_CHECK_LAUNCH("k_grid_mfma");
   return HCG_OK;
 }
 
-int launch_mfma_batch(uint32_t chunk, uint32_t waves, uint32_t blocks, const MfmaJob* jobs, const MfmaItem* items,
-                      uint32_t nitems, uint32_t* head, hipStream_t s) {
-  if (!(waves == 1 || waves == 2 || waves == 4 || waves == 8))
-    return set_error(HCG_ERR_INVALID, "batch: waves must be 1, 2, 4 or 8");
-  if (!(chunk == 128 || chunk == 256 || chunk == 512))
-    return set_error(HCG_ERR_INVALID, "batch: chunk must be 128, 256 or 512");
-  if (blocks == 0) return set_error(HCG_ERR_INVALID, "batch: zero blocks");
-  if (chunk == 512)
-    k_grid_mfma_batch<512><<<blocks, 64 * waves, 0, s>>>(jobs, items, nitems, head);
-  else if (chunk == 256)
-    k_grid_mfma_batch<256><<<blocks, 64 * waves, 0, s>>>(jobs, items, nitems, head);
-  else
-    k_grid_mfma_batch<128><<<blocks, 64 * waves, 0, s>>>(jobs, items, nitems, head);
+int launch_mfma_batch(uint32_t inst, const TileRange* ranges, uint32_t nranges, uint32_t blocks, const MfmaJob* jobs,
+                      hipStream_t s) {
+  if (nranges == 0 || blocks == 0) return HCG_OK;
+#define HCG_CASE(I, DT, NB, LEAN) \
+  case I: k_grid_mfma_batch<DT, NB, LEAN><<<blocks, mfma_threads(NB), 0, s>>>(ranges, nranges, jobs); break;
+  switch (inst) { HCG_MFMA_INSTANCES(HCG_CASE) }
+#undef HCG_CASE
   HCG_CHECK_LAUNCH("k_grid_mfma_batch");
   return HCG_OK;
 }
@@ -1020,9 +1263,9 @@ __global__ void __launch_bounds__(256) k_gather_channels_sm(uint32_t n, uint32_t
   gather_sm_block<T>(blockIdx.x, blockIdx.y, n, n_pad, nchan, perm, in, out, nonfinite, tile);
 }
 
-// Every job's channel gather and tile plan of a batch in one launch
-// (prep_ranges): the plans' dependent key searches are latency-bound and
-// the gathers bandwidth-bound, so sharing the chip lets each hide the
+// Every job's channel gather and block plan (mfma_wide) of a batch in one
+// launch (prep_ranges): the plans' dependent key searches are latency-bound
+// and the gathers bandwidth-bound, so sharing the chip lets each hide the
 // other.  A range is a run of workgroups of one kind for one job; each
 // workgroup finds its range by binary search over the range starts.
 __global__ void __launch_bounds__(256) k_batch_prep(const PrepRange* __restrict__ ranges, uint32_t nranges,
@@ -1046,7 +1289,7 @@ __global__ void __launch_bounds__(256) k_batch_prep(const PrepRange* __restrict_
   const uint32_t bx = lb % R.gx, by = lb / R.gx;
   switch (R.kind) {
     case kPrepPlan: {
-      const uint32_t t = lb * 4 + (threadIdx.x >> 6);  // a wave per tile
+      const uint32_t t = lb * 4 + (threadIdx.x >> 6);  // a wave per block
       if (t < J.ntiles) plan_tile(J, t);
       break;
     }
@@ -1148,7 +1391,7 @@ extern "C" size_t hcg_grid_mfma_workspace_size(uint32_t side, const hcg_mfma_sha
   const uint32_t tc = (shape && shape->tile_cols) ? shape->tile_cols : kMcDefaultTileCols;
   if (!(tc == 8 || tc == 16 || tc == 32 || tc == 64)) return 0;
   const size_t ntiles = (size_t)ceil_div_u32(side, tc) * ceil_div_u32(side, 64u / tc);
-  return ntiles * kPlanTileWords * sizeof(uint32_t);
+  return ntiles * kPlanBytes;
 }
 
 extern "C" int hcg_grid_mfma_ex(const hcg_healpix* hp, const hcg_kernel* kern, uint32_t side, uint32_t n,
@@ -1191,53 +1434,15 @@ extern "C" int hcg_grid_mfma_ex(const hcg_healpix* hp, const hcg_kernel* kern, u
                     (uint32_t)(normalize ? 1 : 0), nchan};
     return route == kRouteFew ? launch_tiles_few_channels(P, B, O, s) : launch_tiles_one_channel(P, B, O, s);
   }
-  const uint32_t n_pad = hcg_channels_padded_len(n);
-  const uint32_t groups_total = ceil_div_u32(nchan, kMcChanPerWave);  // waves needed
-  // waves per workgroup: a power of two (each cell's nw threads are aligned
-  // consecutive lanes, reduced with xor shuffles); surplus waves only help
-  // with the weights
-  uint32_t nw = sh.waves;
-  if (nw == 0) {
-    // default: the fewest waves that cover the channels, at most 8 (chunk
-    // 512, one workgroup per CU): with several rings packed per chunk the
-    // 8-wave shape is the fastest on the 2M x 1024 raster (13.5 ms, against
-    // 15.5 for 4 waves at chunk 256, two workgroups per CU)
-    nw = 1;
-    while (nw < groups_total && nw < 8u) nw <<= 1;
-  }
-  const uint32_t ngroups = ceil_div_u32(groups_total, nw);
   const uint32_t tc = sh.tile_cols ? sh.tile_cols : kMcDefaultTileCols;
-  const uint32_t tc_shift = tc == 8 ? 3u : tc == 16 ? 4u : tc == 32 ? 5u : 6u;
-  const uint32_t tr = 64u / tc;
-  const uint32_t tiles_x = ceil_div_u32(side, tc);
-  const uint32_t ntiles = tiles_x * ceil_div_u32(side, tr);
-  const dim3 grid(ntiles, ngroups);
-  // chunk size by workgroup width: 8 waves fill a CU alone (VGPR-limited);
-  // narrower workgroups take smaller tiles so several share a CU
-  const uint32_t chunk = sh.chunk ? sh.chunk : (nw >= 8 ? 512u : (nw >= 4 ? 256u : 128u));
-  const uint32_t ktc = mfma_weight_form(P, kern->kernel_type);
-  MfmaJob J{P,        B,       values_sorted, cube,   wsum, ktc, n_pad, nchan, (uint32_t)dtype,
-            tc_shift, tiles_x, ntiles,        (uint32_t)(normalize ? 1 : 0), nullptr};
-  if (workspace) {
-    if (workspace_bytes < (size_t)ntiles * kPlanTileWords * sizeof(uint32_t))
-      return set_error(HCG_ERR_WORKSPACE, "hcg_grid_mfma_ex: workspace smaller than hcg_grid_mfma_workspace_size");
-    J.plan = static_cast<uint32_t*>(workspace);
-    const int rc = launch_mfma_plan(J, s);
-    if (rc != HCG_OK) return rc;
-  }
-#define HCG_LAUNCH_MFMA(TT, CH) k_grid_mfma<TT, CH><<<grid, 64 * nw, 0, s>>>(J)
-  if (dtype == HCG_DTYPE_BF16) {
-    if (chunk == 512) HCG_LAUNCH_MFMA(kDtBf16, 512);
-    else if (chunk == 256) HCG_LAUNCH_MFMA(kDtBf16, 256);
-    else HCG_LAUNCH_MFMA(kDtBf16, 128);
-  } else {
-    if (chunk == 512) HCG_LAUNCH_MFMA(kDtF16, 512);
-    else if (chunk == 256) HCG_LAUNCH_MFMA(kDtF16, 256);
-    else HCG_LAUNCH_MFMA(kDtF16, 128);
-  }
-#undef HCG_LAUNCH_MFMA
-  HCG_CHECK_LAUNCH("k_grid_mfma");
-  return HCG_OK;
+  const uint32_t tiles_x = ceil_div_u32(side, tc), ntiles = tiles_x * ceil_div_u32(side, 64u / tc);
+  if (workspace && workspace_bytes < hcg_grid_mfma_workspace_size(side, &sh))
+    return set_error(HCG_ERR_WORKSPACE, "hcg_grid_mfma_ex: workspace smaller than hcg_grid_mfma_workspace_size");
+  MfmaJob J{P,     B,    values_sorted,   cube,    wsum,   mfma_weight_form(P, kern->kernel_type),
+                  hcg_channels_padded_len(n), nchan, (uint32_t)dtype, tile_shift_of(tc), tiles_x, ntiles,
+                  (uint32_t)(normalize ? 1 : 0), nullptr};
+  if (workspace && mfma_uses_plan(mfma_instance(J))) J.plan = workspace;
+  return launch_mfma_job(J, s);
 }
 
 extern "C" int hcg_grid_mfma(const hcg_healpix* hp, const hcg_kernel* kern, uint32_t side, uint32_t n, uint32_t nchan,

@@ -150,9 +150,8 @@ __device__ inline void compat_edges(const GridParams& P, const Window& w, double
   tr = fmodulo4((w.phi + P.disc_size) * kInvHalfPi);
 }
 
-__device__ inline bool ring_window_at(const GridParams& P, const Window& w, double tl, double tr, uint32_t ring,
+__device__ inline bool ring_window_at(const Hpx32& hx, const Window& w, double tl, double tr, uint32_t ring,
                                       double rz, double rs, uint32_t& lpix, uint32_t& rpix) {
-  const Hpx32 hx = hpx32(P.hp);
   uint32_t sp, npr;
   ring_info32(hx, ring, sp, npr);
   if (w.mode != kWinCompat) {
@@ -183,13 +182,6 @@ __device__ inline bool ring_window_at(const GridParams& P, const Window& w, doub
   if (lpix - sp >= npr) return false;
   rpix = loc2pix32(hx, rz, tr, s, have);
   return rpix - sp < npr;
-}
-
-__device__ inline bool ring_window(const GridParams& P, const Window& w, uint32_t ring, double rz, double rs,
-                                   uint32_t& lpix, uint32_t& rpix) {
-  double tl = 0.0, tr = 0.0;
-  if (w.mode == kWinCompat) compat_edges(P, w, tl, tr);
-  return ring_window_at(P, w, tl, tr, ring, rz, rs, lpix, rpix);
 }
 
 // ---- out-of-line slow paths (rare; kept out of the inner loop's registers) ----
@@ -343,6 +335,30 @@ __device__ inline double gauss_weight_lean(double h, double a, double bv, double
   tab.y = lshl_add_u32<kExpTabShift>(ni, tab.y);
   const double w = __builtin_bit_cast(double, tab);
   return fma(w, u * q, w);
+}
+
+// Two of them, step by step side by side.
+__device__ inline void gauss_weight_lean2(double h0, double h1, double a, double bv, double e3v, const double* s_exp,
+                                          double (&w)[2]) {
+  constexpr double kRound = 0x1.8p+52;
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const double t0 = fma(h0, bv, a), t1 = fma(h1, bv, a);
+  const double s0 = fma_vvs(h0, t0, kRound), s1 = fma_vvs(h1, t1, kRound);
+  const uint32_t n0 = __builtin_bit_cast(u32x2, s0).x, n1 = __builtin_bit_cast(u32x2, s1).x;
+  u32x2 b0 = __builtin_bit_cast(u32x2, s_exp[n0 & 63u]), b1 = __builtin_bit_cast(u32x2, s_exp[n1 & 63u]);
+  __builtin_amdgcn_sched_barrier(0);  // both reads are issued before either is waited for
+  const double u0 = fma(h0, t0, kRound - s0), u1 = fma(h1, t1, kRound - s1);
+  double q0 = fma_vvs(u0, e3v, kExpE2), q1 = fma_vvs(u1, e3v, kExpE2);
+  q0 = fma_vvs(u0, q0, kExpE1);
+  q1 = fma_vvs(u1, q1, kExpE1);
+  q0 *= u0;
+  q1 *= u1;
+  __builtin_amdgcn_sched_barrier(0);
+  b0.y = lshl_add_u32<kExpTabShift>(n0, b0.y);
+  b1.y = lshl_add_u32<kExpTabShift>(n1, b1.y);
+  const double w0 = __builtin_bit_cast(double, b0), w1 = __builtin_bit_cast(double, b1);
+  w[0] = fma(w0, q0, w0);
+  w[1] = fma(w1, q1, w1);
 }
 
 // exp(y ln2/64) of a y with |y| < 60000 (a normal result): exp_scaled_neg's

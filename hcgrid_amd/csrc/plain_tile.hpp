@@ -268,9 +268,8 @@ __device__ inline TileSpan tile_span(const GridParams& P, const Window& w, uint3
 // edge opens to the ring's end (a cell whose own window wraps through 0
 // selects nothing, since its lpix is then past its rpix), and whole rings
 // are taken where the reasoning ends.
-__device__ inline void span_pixels(const GridParams& P, const TileSpan& t, uint32_t ring, double rz, double rs,
+__device__ inline void span_pixels(const Hpx32& hx, const TileSpan& t, uint32_t ring, double rz, double rs,
                                    uint32_t& lp, uint32_t& rp) {
-  const Hpx32 hx = hpx32(P.hp);
   uint32_t sp, npr;
   ring_info32(hx, ring, sp, npr);
   const uint32_t last = sp + npr - 1;
@@ -308,6 +307,45 @@ __device__ inline void span_pixels(const GridParams& P, const TileSpan& t, uint3
   rp = b;
 }
 
+// The sorted range [lo, hi) of the keys lp..rp within [start, end) (start < end).
+// Both bounds in one loop, three probes each a step: a step is one round of
+// dependent loads, and the range falls to a quarter.
+__device__ inline void key_range(const uint32_t* __restrict__ keys, uint32_t start, uint32_t end, uint32_t lp,
+                                 uint32_t rp, uint32_t& lo, uint32_t& hi) {
+  uint32_t a0 = start, a1 = end, b0 = start, b1 = end;
+  while (a0 < a1 || b0 < b1) {
+    const uint32_t da = (a1 - a0) >> 2, db = (b1 - b0) >> 2;
+    // a0 <= pa0 <= pa1 <= pa2 < a1 while the range is not empty; index
+    // `end` of an empty one can be read (keys[n] is the sentinel)
+    const uint32_t pa0 = a0 + da, pa1 = a0 + ((a1 - a0) >> 1), pa2 = pa1 + da;
+    const uint32_t pb0 = b0 + db, pb1 = b0 + ((b1 - b0) >> 1), pb2 = pb1 + db;
+    const uint32_t ka0 = keys[pa0], ka1 = keys[pa1], ka2 = keys[min(pa2, end)];
+    const uint32_t kb0 = keys[pb0], kb1 = keys[pb1], kb2 = keys[min(pb2, end)];
+    if (a0 < a1) {
+      if (pa2 < a1 && ka2 < lp)
+        a0 = pa2 + 1;
+      else if (ka1 < lp)
+        a0 = pa1 + 1, a1 = min(a1, pa2);
+      else if (ka0 < lp)
+        a0 = pa0 + 1, a1 = pa1;
+      else
+        a1 = pa0;
+    }
+    if (b0 < b1) {
+      if (pb2 < b1 && kb2 <= rp)
+        b0 = pb2 + 1;
+      else if (kb1 <= rp)
+        b0 = pb1 + 1, b1 = min(b1, pb2);
+      else if (kb0 <= rp)
+        b0 = pb0 + 1, b1 = pb1;
+      else
+        b1 = pb0;
+    }
+  }
+  lo = a0;
+  hi = b0;
+}
+
 // The sorted range of ring rb + lane's part of the tile (lo_l >= hi_l: none).
 __device__ inline void ring_ranges(const GridParams& P, const GridBuffers& B, const TileSpan& T, const hcg_ring_meta& m,
                                    uint32_t rb, uint32_t& lo_l, uint32_t& hi_l) {
@@ -318,41 +356,8 @@ __device__ inline void ring_ranges(const GridParams& P, const GridBuffers& B, co
     const uint32_t start = B.lut[kr], end = B.lut[kr + 1];
     if (start < end) {
       uint32_t lp, rp;
-      span_pixels(P, T, rb + lane, B.ring_z[kr], B.ring_s[kr], lp, rp);
-      // both bounds in one loop, three probes each a step: a step is one
-      // round of dependent loads, and the range falls to a quarter
-      uint32_t a0 = start, a1 = end, b0 = start, b1 = end;
-      while (a0 < a1 || b0 < b1) {
-        const uint32_t da = (a1 - a0) >> 2, db = (b1 - b0) >> 2;
-        // a0 <= pa0 <= pa1 <= pa2 < a1 while the range is not empty; index
-        // `end` of an empty one can be read (keys[n] is the sentinel)
-        const uint32_t pa0 = a0 + da, pa1 = a0 + ((a1 - a0) >> 1), pa2 = pa1 + da;
-        const uint32_t pb0 = b0 + db, pb1 = b0 + ((b1 - b0) >> 1), pb2 = pb1 + db;
-        const uint32_t ka0 = B.keys[pa0], ka1 = B.keys[pa1], ka2 = B.keys[min(pa2, end)];
-        const uint32_t kb0 = B.keys[pb0], kb1 = B.keys[pb1], kb2 = B.keys[min(pb2, end)];
-        if (a0 < a1) {
-          if (pa2 < a1 && ka2 < lp)
-            a0 = pa2 + 1;
-          else if (ka1 < lp)
-            a0 = pa1 + 1, a1 = min(a1, pa2);
-          else if (ka0 < lp)
-            a0 = pa0 + 1, a1 = pa1;
-          else
-            a1 = pa0;
-        }
-        if (b0 < b1) {
-          if (pb2 < b1 && kb2 <= rp)
-            b0 = pb2 + 1;
-          else if (kb1 <= rp)
-            b0 = pb1 + 1, b1 = min(b1, pb2);
-          else if (kb0 <= rp)
-            b0 = pb0 + 1, b1 = pb1;
-          else
-            b1 = pb0;
-        }
-      }
-      lo_l = a0;
-      hi_l = b0;
+      span_pixels(hpx32(P.hp), T, rb + lane, B.ring_z[kr], B.ring_s[kr], lp, rp);
+      key_range(B.keys, start, end, lp, rp, lo_l, hi_l);
     }
   }
 }
@@ -677,7 +682,7 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
         if (!(belt_ok && r > ns && r < 3 * ns)) {  // uniform
           const uint32_t kr = r - m.firstring;
           uint32_t a = 0, b = 0;
-          act = act && ring_window_at(P, win, tl, tr, r, B.ring_z[kr], B.ring_s[kr], a, b) && a <= b;
+          act = act && ring_window_at(hpx32(P.hp), win, tl, tr, r, B.ring_z[kr], B.ring_s[kr], a, b) && a <= b;
           wl = 2 * a + (uint32_t)__builtin_amdgcn_readlane(gc, k);
           wh = 2 * b + (uint32_t)__builtin_amdgcn_readlane(gc, k);
         }

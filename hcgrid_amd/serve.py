@@ -9,7 +9,7 @@ request's slot stream, so that copy is part of the request's latency.
 The server keeps a small number of slots (streams).  Whenever a slot is
 free it forms a round from every pending request that fits the HBM budget
 (FIFO, no overtaking), enqueues the round on that slot's stream (input
-copies, geometry builds for new coordinates, one persistent batched launch)
+copies, geometry builds for new coordinates, one batch)
 and goes back to admitting, so rounds on different slots overlap on the
 device while new requests keep arriving.  A round's memory returns to the
 budget when its completion event fires.

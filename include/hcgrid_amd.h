@@ -252,11 +252,9 @@ int hcg_grid_mfma(const hcg_healpix *hp, const hcg_kernel *kern, uint32_t side, 
 
 /* Launch shape of the multi-channel kernel.  A workgroup owns 64 cells,
  * a (64 / tile_cols) x tile_cols block of the map (tile_cols 8, 16, 32 or
- * 64), with `waves` waves (1, 2, 4 or 8; 64 channels each; more channels
- * take more workgroups, each recomputing the block's weights) and stages
- * `chunk` samples at a time (128, 256 or 512).  0 in a field = the default
- * (tile_cols 16; the fewest waves that cover the channels, at most 8; chunk
- * by waves).  No counterpart in the reference: the shapes an autotuner
+ * 64; 0 = 16).  waves (0, 1, 2, 4 or 8) and chunk (0, 128, 256 or 512) are
+ * checked and have no other effect: the kernel chooses its waves by the
+ * channel count.  No counterpart in the reference: the shapes an autotuner
  * picks per workload. */
 typedef struct hcg_mfma_shape {
     uint32_t tile_cols, waves, chunk, reserved;
@@ -267,11 +265,12 @@ typedef struct hcg_mfma_shape {
 size_t hcg_grid_mfma_workspace_size(uint32_t side, const hcg_mfma_shape *shape);
 
 /* hcg_grid_mfma with a launch shape (NULL = defaults) and a workspace for
- * the tile plan (NULL = none).  With a workspace, a first small kernel (one
- * wave per tile, many per CU) computes every tile's ring span, each ring's
- * sorted range and each cell's window and unit vector, and the gridding
- * kernel reads them instead of evaluating them itself; the results are the
- * same either way. */
+ * the tile plan (NULL = none).  With a workspace and more than 256 channels
+ * (64 with weights other than GAUSS1D's at radii of 0.018 to 0.26 deg), a
+ * first small kernel (one wave per tile, many per CU) computes every tile's
+ * ring span, each ring's sorted range and each cell's window and unit vector,
+ * and the gridding kernel reads them instead of evaluating them itself; the
+ * results are the same either way. */
 int hcg_grid_mfma_ex(const hcg_healpix *hp, const hcg_kernel *kern, uint32_t side, uint32_t n,
                      uint32_t nchan, int dtype, const hcg_sample *records, const uint32_t *keys_sorted,
                      const double *lon_sorted, const double *lat_sorted, const double *weights_sorted,
@@ -344,7 +343,7 @@ int hcg_wcs_sin_p2s_device(uint32_t naxis1, uint32_t naxis2, double crpix1, doub
  * (HCGrid+/gridding-omp.cu:552-678).  A geometry holds one map's sorted
  * samples, ring LUT and target coordinates in HBM, so repeated requests on
  * the same coordinates skip the pre-sort; a batch grids many (geometry,
- * channel values, cube) jobs of uneven sizes in ONE persistent launch. */
+ * channel values, cube) jobs of uneven sizes in a few launches. */
 
 typedef struct hcg_geometry hcg_geometry;   /* opaque, device-resident */
 
@@ -401,15 +400,15 @@ typedef struct hcg_batch_job {
 typedef struct hcg_batch hcg_batch;   /* opaque */
 
 /* Device bytes of a job's sorted channel values in its batch (the batch
- * adds the job's tile plan, 520 bytes per 64-cell tile, and its work items). */
+ * adds the tile plan of a job of many channels, 3600 bytes per 64-cell tile). */
 size_t hcg_batch_job_bytes(const hcg_geometry *g, uint32_t nchan);
 
-/* Plans a batch: orders the work items (tile x channel group of every job,
- * longest items first), allocates the job table, work list, counters and
- * the sorted channel buffers, and uploads the plan (synchronously).  waves
- * per workgroup (1, 2, 4, 8; 0 = 4) and chunk (128, 256, 512; 0 = by waves)
- * fix the persistent launch's shape.  The jobs' geometries, values and
- * cubes must stay allocated while the batch is used. */
+/* Plans a batch: sorts the jobs into launches (by kernel instance or route,
+ * longest jobs first), allocates the job table, ranges, counters and the
+ * sorted channel buffers, and uploads the plan (synchronously).  waves (0, 1,
+ * 2, 4, 8) and chunk (0, 128, 256, 512) are checked and have no other effect.
+ * The jobs' geometries, values and cubes must stay allocated while the batch
+ * is used. */
 int hcg_batch_create(uint32_t njobs, const hcg_batch_job *jobs, uint32_t waves, uint32_t chunk,
                      hcg_batch **out);
 
@@ -424,12 +423,9 @@ int hcg_batch_create_in(uint32_t njobs, const hcg_batch_job *jobs, uint32_t wave
                         void *device_mem, size_t bytes, void *stream, hcg_batch **out);
 
 /* Enqueues the batch: counters cleared by a fill kernel, every job's channel
- * gather and tile plan in one launch, then the persistent launch over the
- * work items (dense jobs, 32+ samples per cell, in a persistent launch of
- * their own at 8 waves / chunk 512 first, when the batch's shape is not
- * that one).  Kernels only
- * (capturable).  Results per job equal hcg_grid_mfma_shaped's with the same
- * tile_cols, bit for bit. */
+ * gather and tile plan in one launch, then one launch per kernel instance or
+ * route that its jobs take.  Kernels only (capturable).  Results per job
+ * equal hcg_grid_mfma_shaped's with the same tile_cols, bit for bit. */
 int hcg_batch_enqueue(hcg_batch *b, void *stream);
 
 typedef struct hcg_batch_stats {
@@ -446,7 +442,7 @@ int hcg_batch_nonfinite(const hcg_batch *b, uint32_t *counts, void *stream);
  * counterpart).  enable != 0 creates three HIP events in the batch; every
  * later enqueue that is not being captured into a graph records them on its
  * stream: before the counter fill, after the prep launch (channel gathers
- * and tile plans), and after the persistent gridding launches.
+ * and tile plans), and after the gridding launches.
  * hcg_batch_last_times waits for the last such enqueue and returns the prep
  * and gridding durations in milliseconds.  enable == 0 destroys the events. */
 int hcg_batch_timing(hcg_batch *b, int enable);
