@@ -114,16 +114,11 @@ __device__ inline f32x2_t widen16x2(uint32_t w) {
     return __builtin_convertvector(__builtin_bit_cast(f16x2_t, w), f32x2_t);
 }
 
-// The cells of a wave's square: their extent in latitude and longitude, for
-// narrowing each ring to what the radius reaches (block_ring_range).
+// A set of cells taken together (block_ring_range).
 struct BlockSpan {
   TileSpan T;
   bool simple;          // every window is one pair of half-pixel numbers (belt_window), every ring a belt ring
   uint32_t hlo, hhi;    // simple: the outermost of them
-  bool chord;           // the extents below hold
-  double bmin, bmax;    // latitudes, radians
-  double tmin, tmax;    // longitudes, units of pi/2 in [0, 4)
-  double cmin;          // the smallest cos latitude
 };
 
 constexpr uint32_t kNoRingLane = 255;        // the ring lane of a block list's padding
@@ -153,7 +148,7 @@ struct MfmaCells {
   Window win[kMcCols];
   double tl[kMcCols], tr[kMcCols];  // compat: the window's edges (compat_edges)
   double p[3][kMcCols];
-  double lat[kMcCols], coslat[kMcCols], tt[kMcCols];  // latitude (radians) and its cos; longitude (units of pi/2)
+  double coslat[kMcCols], tt[kMcCols];
   uint32_t wlo[kMcCols], wwid[kMcCols];           // the window in every belt ring (belt_window)
   uint8_t belt[kMcCols];                          // it holds
 };
@@ -184,42 +179,11 @@ static __device__ __noinline__ uint64_t span_pixels_call(Hpx32 hx, TileSpan t, u
   return pack_range(lp, rp);
 }
 
-static __device__ __noinline__ uint64_t ring_window_call(Hpx32 hx, const MfmaCells* C, uint32_t cb, uint32_t ring,
+static __device__ __noinline__ uint64_t cell_window_call(Hpx32 hx, const MfmaCells* C, uint32_t cb, uint32_t ring,
                                                          double rz, double rs) {
   uint32_t a = 1, b = 0;
   if (!ring_window_at(hx, C->win[cb], C->tl[cb], C->tr[cb], ring, rz, rs, a, b)) return kNoRange;
   return pack_range(a, b);
-}
-
-// The keys lp..rp of a ring (first pixel sp, npr pixels), narrowed to what the
-// radius reaches from a square's cells.  A sample at latitude bs within R of
-// a cell at bc has hav R > hav(bs - bc) + cos bs cos bc hav(dl); ring r's
-// pixels lie between the centre latitudes of rings r - 1 and r + 1 (z = zu,
-// zd), so |bs - bc| >= d, the gap between that band and the cells' latitudes,
-// and
-//   sin^2(dl / 2) <= (sin^2(R / 2) - sin^2(d / 2)) / (cos bs cos bc).
-// The pixel of longitude tt (units of pi/2) is floor(tt npr / 4) or the next
-// one.  half = sin(R' / 2), R' = R (1 + 1e-6).  The windows span the disc's
-// whole width in every ring; a quarter of what a 4 x 4 square would look at
-// is outside the radius.
-static __device__ __noinline__ uint64_t chord_range(uint32_t lp, uint32_t rp, uint32_t sp, uint32_t npr, double zu,
-                                                    double zd, double bmin, double bmax, double tmin, double tmax,
-                                                    double cmin, double half) {
-  const double d = fmax(0.0, fmax(asin(zd) - bmax, bmin - asin(zu)));
-  const double sd = sin(0.5 * d);
-  const double num = half * half - sd * sd;
-  if (!(num > 0.0)) return kNoRange;
-  const double cs = sqrt(fmin((1.0 - zu) * (1.0 + zu), (1.0 - zd) * (1.0 + zd)));
-  const double s2 = num / (cs * cmin);
-  if (s2 < 0.25) {
-    const double dt = (4.0 / kPi) * sqrt(s2 / (1.0 - s2)) * (1.0 + 1e-9) + 1e-12;  // asin s <= s / sqrt(1 - s^2)
-    const double tl = tmin - dt, tr = tmax + dt, q = 0.25 * (double)npr;
-    if (tl >= 0.0 && tr * q < (double)npr - 2.0) {
-      lp = max(lp, sp + (uint32_t)fmax(tl * q - 1e-6, 0.0));
-      rp = min(rp, sp + (uint32_t)(tr * q + 1e-6) + 1u);
-    }
-  }
-  return pack_range(lp, rp);
 }
 
 // The keys of ring `ring` that a square's cells can take samples from: a
@@ -230,16 +194,18 @@ __device__ inline uint64_t block_ring_range(const GridParams& P, const GridBuffe
   const Hpx32 hx = hpx32(P.hp);
   uint32_t sp, npr;
   ring_info32(hx, ring, sp, npr);
-  uint64_t range;
+  uint32_t lp, rp;
   if (S.simple) {  // g = 2 p + 1 - odd in [hlo, hhi]
     const uint32_t odd = ring & 1u;
-    range = pack_range(sp + ((S.hlo + odd) >> 1), sp + ((S.hhi - 1u + odd) >> 1));
+    lp = sp + ((S.hlo + odd) >> 1);
+    rp = sp + ((S.hhi - 1u + odd) >> 1);
   } else {
-    range = span_pixels_call(hx, S.T, ring, B.ring_z[kr], B.ring_s[kr]);
+    const uint64_t range = span_pixels_call(hx, S.T, ring, B.ring_z[kr], B.ring_s[kr]);
+    lp = (uint32_t)range;
+    rp = (uint32_t)(range >> 32);
   }
-  if (!S.chord || kr == 0 || kr + 1 >= m.usedrings) return range;
-  return chord_range((uint32_t)range, (uint32_t)(range >> 32), sp, npr, B.ring_z[kr - 1], B.ring_z[kr + 1], S.bmin,
-                     S.bmax, S.tmin, S.tmax, S.cmin, P.polar_half);
+  return chord_pixels(S.T, ring_chord(P.polar_half * P.polar_half, S.T, npr, kr, m.usedrings, B.ring_z), sp, npr, lp, rp) ? pack_range(lp, rp)
+                                                                                              : kNoRange;
 }
 
 // A cell (a lane's) of a block.
@@ -247,7 +213,7 @@ struct CellGeom {
   Window win;
   double tl, tr;              // compat: the window's edges (compat_edges)
   double px, py, pz;          // unit vector
-  double lat, coslat, tt;     // latitude (radians) and its cos; longitude (units of pi/2)
+  double coslat, tt;          // cos of the latitude; longitude (units of pi/2)
   uint32_t wlo, wwid;         // the window in every belt ring (belt_window)
   bool belt;                  // it holds
 };
@@ -281,7 +247,6 @@ __device__ __forceinline__ CellGeom block_cell(const GridParams& P, const GridBu
     g.belt = belt_window(P, g.tl, g.tr, g.wlo, whi);
   }
   g.wwid = whi - g.wlo;
-  g.lat = yc;
   g.coslat = cb;
   g.tt = fmodulo4(xc * kInvHalfPi);
   return g;
@@ -294,7 +259,6 @@ __device__ __forceinline__ void put_cell(MfmaCells& C, uint32_t i, const CellGeo
   C.p[0][i] = g.px;
   C.p[1][i] = g.py;
   C.p[2][i] = g.pz;
-  C.lat[i] = g.lat;
   C.coslat[i] = g.coslat;
   C.tt[i] = g.tt;
   C.wlo[i] = g.wlo;
@@ -302,25 +266,16 @@ __device__ __forceinline__ void put_cell(MfmaCells& C, uint32_t i, const CellGeo
   C.belt[i] = g.belt;
 }
 
-// The span of the wave's cells (live: on the map).
-__device__ __forceinline__ BlockSpan cells_span(const GridParams& P, const hcg_ring_meta& m, const CellGeom& g,
-                                                bool live) {
+// The span of the wave's cells.
+__device__ __forceinline__ BlockSpan cells_span(const GridParams& P, const hcg_ring_meta& m, const CellGeom& g) {
   BlockSpan S;
-  S.T = tile_span(P, g.win, m.firstring);
+  S.T = tile_span(P, g.win, m.firstring, g.pz, g.coslat, g.tt);
   const bool has = g.win.uring <= g.win.dring;
   const uint32_t ns = (uint32_t)P.hp.nside;
   const bool belt_ok = __ballot(has && !g.belt) == 0;
   S.simple = belt_ok && S.T.r_begin > ns && S.T.r_end < 3 * ns;  // uniform
   S.hlo = wave_min_u32(has ? g.wlo : 0xFFFFFFFFu);
   S.hhi = wave_max_u32(has ? g.wlo + g.wwid : 1u);
-  S.bmin = wave_min_f64(live ? g.lat : 1e300);
-  S.bmax = -wave_min_f64(live ? -g.lat : 1e300);
-  S.tmin = wave_min_f64(live ? g.tt : 1e300);
-  S.tmax = -wave_min_f64(live ? -g.tt : 1e300);
-  S.cmin = wave_min_f64(live ? g.coslat : 1e300);
-  // (a cell outside the projection, NaN, leaves the chord out)
-  S.chord = __ballot(live && !(g.lat > -2.0 && g.lat < 2.0 && g.tt >= 0.0)) == 0 && S.cmin > 0.05 &&
-            S.tmax - S.tmin < 1.0;
   return S;
 }
 
@@ -397,7 +352,7 @@ __device__ __forceinline__ void plan_tile(const MfmaJob& J, uint32_t tile) {  //
   bool live;
   const CellGeom g = block_cell(J.P, J.B, m, (tile / J.tiles_x) << (6u - J.tc_shift),
                                 (tile % J.tiles_x) << J.tc_shift, J.tc_shift, live);
-  const BlockSpan S = cells_span(J.P, m, g, live);
+  const BlockSpan S = cells_span(J.P, m, g);
   MfmaPlan& L = *reinterpret_cast<MfmaPlan*>(static_cast<char*>(J.plan) + tile * kPlanBytes);
   const bool none = S.T.r_begin > S.T.r_end, ok = none || (S.simple && S.T.r_end - S.T.r_begin < 64);
   if (lane == 0) {
@@ -504,7 +459,7 @@ struct SquareCell {
     wl = wlo;
     ww = wwid;
     if (!simple) {  // uniform
-      const uint64_t range = ring_window_call(hpx32(P.hp), &C, cb, r, L.rz[rl & 63u], L.rs[rl & 63u]);
+      const uint64_t range = cell_window_call(hpx32(P.hp), &C, cb, r, L.rz[rl & 63u], L.rs[rl & 63u]);
       const uint32_t a = (uint32_t)range, b = (uint32_t)(range >> 32);
       act = act && a <= b;
       wl = 2u * a + L.gc[rl & 63u];
@@ -686,13 +641,13 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
   {
     CellGeom g;
     g.win = C.win[cb];
-    g.lat = C.lat[cb];
+    g.pz = C.p[2][cb];
     g.coslat = C.coslat[cb];
     g.tt = C.tt[cb];
     g.wlo = C.wlo[cb];
     g.wwid = C.wwid[cb];
     g.belt = C.belt[cb] != 0;
-    const BlockSpan S = cells_span(P, m, g, live);
+    const BlockSpan S = cells_span(P, m, g);
     r_begin = S.T.r_begin;
     r_end = S.T.r_end;
     Q.init(P, C, cb, S.simple);
@@ -862,7 +817,7 @@ __device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint3
     bool lv;
     const CellGeom g = block_cell(P, B, m, y0, x0, J.tc_shift, lv);
     put_cell(C, lane, g);
-    const BlockSpan S = cells_span(P, m, g, lv);
+    const BlockSpan S = cells_span(P, m, g);
     if (lane == 0) L.span = S;
   }
   __syncthreads();

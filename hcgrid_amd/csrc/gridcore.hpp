@@ -510,6 +510,20 @@ __device__ inline uint32_t wave_min_u32(uint32_t v) {
 
 __device__ inline uint32_t wave_max_u32(uint32_t v) { return ~wave_min_u32(~v); }
 
+// Of values above -1e30 (NaN is ignored).
+__device__ inline float wave_max_f32(float v) {
+  const auto step = [](float x, uint32_t u) { return fmaxf(x, __builtin_bit_cast(float, u)); };
+  const uint32_t id = __builtin_bit_cast(uint32_t, -1e30f);
+  v = fmaxf(v, -1e30f);
+  v = step(v, dpp_u32<kRowShr1, 0xF>(id, __builtin_bit_cast(uint32_t, v)));
+  v = step(v, dpp_u32<kRowShr2, 0xF>(id, __builtin_bit_cast(uint32_t, v)));
+  v = step(v, dpp_u32<kRowShr4, 0xF>(id, __builtin_bit_cast(uint32_t, v)));
+  v = step(v, dpp_u32<kRowShr8, 0xF>(id, __builtin_bit_cast(uint32_t, v)));
+  v = step(v, dpp_u32<kRowBcast15, 0xA>(id, __builtin_bit_cast(uint32_t, v)));
+  v = step(v, dpp_u32<kRowBcast31, 0xC>(id, __builtin_bit_cast(uint32_t, v)));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
+
 __device__ inline double wave_min_f64(double v) {
   constexpr double id = 1e308;
   v = fmin(v, dpp_f64<kRowShr1, 0xF>(id, v));
