@@ -298,6 +298,7 @@ int plan_batch(uint32_t njobs, const hcg_batch_job* jobs, uint32_t waves, uint32
       J.nchan = b.nchan;
       J.dtype = (uint32_t)b.dtype;
       J.ntiles = p.tiles[j];
+      J.tiles_x = ceil_div_u32(side, tc);
       p.route[j] = kRouteMfma + mfma_instance(J);
       blocks[j] = p.tiles[j] ? mfma_blocks(J) : 0;
       cost[j] = group_cost(g, tc, std::min<uint32_t>(b.nchan, 256u));

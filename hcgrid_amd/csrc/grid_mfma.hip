@@ -986,10 +986,31 @@ __device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint3
   }
 }
 
-// Block b of a launch of 8 xcd_run(tiles) runs on XCD b % 8: each XCD takes a
-// contiguous run of tiles, so neighbouring tiles share an L2.
-__host__ __device__ inline uint32_t xcd_run(uint32_t ntiles) { return (ntiles + 7u) / 8u; }
-__device__ inline uint32_t xcd_tile(uint32_t b, uint32_t ntiles) { return (b & 7u) * xcd_run(ntiles) + (b >> 3); }
+// The tile of workgroup b of a job.  Workgroup b runs on XCD b % 8: an XCD
+// takes a contiguous run of tiles, so neighbouring tiles share an L2.  The
+// many-channel kernel, one workgroup per CU, takes maps of 1024 tiles and more
+// in patches of 8 x 4 tiles, so that the rows of samples that vertical
+// neighbours share are read a quarter of a tile's time apart and not a row of
+// the map later: 2M x 1024 a pass 8.46 -> 8.14-8.26 ms (4 x 8 8.33, 2 x 16 8.33,
+// 2 x 8 8.28).  With fewer channels a CU holds several workgroups and patches
+// change nothing (1.2M x 64 onto 512^2 1.531 and 1.540 ms).
+constexpr uint32_t kPatchW = 8, kPatchH = 4, kPatchTiles = kPatchW * kPatchH, kPatchMinTiles = 1024;
+__host__ __device__ inline uint32_t patches_per_xcd(uint32_t ntiles, uint32_t tiles_x) {
+  return ((tiles_x + kPatchW - 1) / kPatchW * ((ntiles / tiles_x + kPatchH - 1) / kPatchH) + 7u) / 8u;
+}
+__host__ __device__ inline uint32_t tile_blocks(uint32_t ntiles, uint32_t tiles_x, bool wide) {
+  if (!wide || ntiles < kPatchMinTiles) return (ntiles + 7u) / 8u * 8u;
+  return 8u * patches_per_xcd(ntiles, tiles_x) * kPatchTiles;
+}
+// (ntiles or more: none)
+__device__ inline uint32_t block_tile(uint32_t b, uint32_t ntiles, uint32_t tiles_x, bool wide) {
+  const uint32_t xcd = b & 7u, i = b >> 3;
+  if (!wide || ntiles < kPatchMinTiles) return xcd * ((ntiles + 7u) / 8u) + i;
+  const uint32_t px = (tiles_x + kPatchW - 1) / kPatchW;
+  const uint32_t patch = xcd * patches_per_xcd(ntiles, tiles_x) + i / kPatchTiles;
+  const uint32_t x = patch % px * kPatchW + i % kPatchW, y = patch / px * kPatchH + i / kPatchW % kPatchH;
+  return x < tiles_x ? y * tiles_x + x : ntiles;  // (past the last row: past ntiles)
+}
 
 // The kernel instances: NB 16-channel blocks per wave (mfma_tile), or 0: mfma_wide.
 constexpr int mfma_waves_per_simd(int nb, bool lean) {
@@ -1015,11 +1036,11 @@ __device__ __forceinline__ void mfma_work(const MfmaJob& J, uint32_t tile, uint3
     mfma_tile<DT, NB, LEAN>(J, tile, group, lds, s_exp);
 }
 
-// One job: grid = (8 xcd_run(tiles), channel groups).
+// One job: grid = (tile_blocks, channel groups).
 template <int DT, int NB, bool LEAN>
 __global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, LEAN))))
     k_grid_mfma(MfmaJob J) {
-  const uint32_t tile = xcd_tile(blockIdx.x, J.ntiles);
+  const uint32_t tile = block_tile(blockIdx.x, J.ntiles, J.tiles_x, NB == 0);
   if (tile >= J.ntiles) return;  // uniform
   mfma_work<DT, NB, LEAN>(J, tile, blockIdx.y);
 }
@@ -1038,8 +1059,8 @@ __global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_
       hi = mid;
   }
   const MfmaJob& J = jobs[ranges[lo].job];
-  const uint32_t lb = blockIdx.x - ranges[lo].first, per = 8u * xcd_run(J.ntiles);
-  const uint32_t tile = xcd_tile(lb % per, J.ntiles), group = lb / per;
+  const uint32_t lb = blockIdx.x - ranges[lo].first, per = tile_blocks(J.ntiles, J.tiles_x, NB == 0);
+  const uint32_t tile = block_tile(lb % per, J.ntiles, J.tiles_x, NB == 0), group = lb / per;
   if (tile >= J.ntiles) return;  // uniform
   mfma_work<DT, NB, LEAN>(J, tile, group);
 }
@@ -1068,7 +1089,8 @@ static uint32_t mfma_groups(const MfmaJob& J, uint32_t inst) {
   return ceil_div_u32(J.nchan, nb ? 16u * nb : 64u * kWideWaves);
 }
 uint64_t mfma_blocks(const MfmaJob& J) {
-  return (uint64_t)8u * xcd_run(J.ntiles) * mfma_groups(J, mfma_instance(J));
+  const uint32_t inst = mfma_instance(J);
+  return (uint64_t)tile_blocks(J.ntiles, J.tiles_x, nb_of_instance(inst) == 0) * mfma_groups(J, inst);
 }
 
 #define HCG_MFMA_PAIR(X, I, NB, LEAN) X(2 * (I), kDtBf16, NB, LEAN) X(2 * (I) + 1, kDtF16, NB, LEAN)
@@ -1080,7 +1102,7 @@ uint64_t mfma_blocks(const MfmaJob& J) {
 
 static int launch_mfma_job(const MfmaJob& J, hipStream_t s) {
   const uint32_t inst = mfma_instance(J);
-  const dim3 grid(8u * xcd_run(J.ntiles), mfma_groups(J, inst));
+  const dim3 grid(tile_blocks(J.ntiles, J.tiles_x, nb_of_instance(inst) == 0), mfma_groups(J, inst));
   if (J.plan) {
     k_mfma_plan<<<J.ntiles, 64, 0, s>>>(J);
     HCG_CHECK_LAUNCH("k_mfma_plan");
