@@ -569,11 +569,18 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
   double fu[kFrame ? ROWS : 1][3], fv[kFrame ? ROWS : 1][3];
   Window win;
   double tl = 0.0, tr = 0.0;  // compat: the window's edges, fmodulo4 in units of pi/2
-  TileSpan T;
+  // the span waits in LDS: past the set-up only a tile of more than 64 rings
+  // wants it (in registers it took 25 to 70 more spills in the sample loop's
+  // surroundings; with the shared tiles' windows, passes 331 -> 296 us on the
+  // disc at dec 80, 279 -> 252 with GAUSS2D, 85 -> 79 on the 20^2 map)
+  __shared__ TileSpan spans[SHARED ? 1 : kOneChannelStreams];
+  TileSpan& far_span = SHARED ? sh->T : spans[threadIdx.x >> 6];
+  uint32_t r_begin, r_end;
   RingRange ring_r;  // lane = ring: the ranges of 64 rings
   float zf, ttf;  // the cell's place, as ring_chord wants it
   {
     double px, py, pz;
+    TileSpan T;
     if (!SHARED || threadIdx.x < 64) {
       const bool live = col < P.side && row0 + row < P.side;
       const uint32_t rr = live ? row0 + row : 0, cc = live ? col : 0;
@@ -620,8 +627,6 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
         ring_r = H.rings[lane];
         ttf = H.tt[lane];
         T = H.T;
-        T.r_begin = __builtin_amdgcn_readfirstlane(T.r_begin);
-        T.r_end = __builtin_amdgcn_readfirstlane(T.r_end);
       }
     }
     if constexpr (kFrame) {
@@ -643,6 +648,9 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
       }
     }
     zf = (float)(pz - T.zref);
+    r_begin = __builtin_amdgcn_readfirstlane(T.r_begin);
+    r_end = __builtin_amdgcn_readfirstlane(T.r_end);
+    if (!SHARED && lane == 0) far_span = T;
     // -p: h = 1 - p.q is three FMAs from 1
     quad_all(-px, npx);
     quad_all(-py, npy);
@@ -670,9 +678,12 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
   const double k1v = WMODE == 3 ? in_vgprs(4.0 * P.k1) : 0.0, e3v = WMODE == 3 ? in_vgprs(kExpE3) : 0.0;
   uint32_t seen = 0;  // non-empty rings before this round
 
-  for (uint32_t rb = T.r_begin; rb <= T.r_end && T.r_begin <= T.r_end; rb += 64) {
+  for (uint32_t rb = r_begin; rb <= r_end && r_begin <= r_end; rb += 64) {
     // lane = ring
-    if (rb != T.r_begin) ring_r = ring_range(P, B, T, m, rb + lane);  // (more than 64 rings)
+    if (rb != r_begin) {  // (more than 64 rings)
+      tile_sync();
+      ring_r = ring_range(P, B, far_span, m, rb + lane);
+    }
     uint32_t lo_l = ring_r.lo;
     const uint32_t hi_l = ring_r.hi;
     const RingChord& chord_r = ring_r.c;
@@ -781,7 +792,11 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
         uint32_t wl = hl0, wh = hh0;
         if (!(belt_ok && r > ns && r < 3 * ns)) {  // uniform
           const uint32_t kr = r - m.firstring;
-          const uint64_t ab = ring_window_call(hpx32(P.hp), win, tl, tr, r, B.ring_z[kr], B.ring_s[kr]);
+          uint64_t ab;
+          if constexpr (SHARED)  // (held there, not in registers through the sample loop)
+            ab = ring_window_call(hpx32(P.hp), sh->win[lane], sh->tl[lane], sh->tr[lane], r, B.ring_z[kr], B.ring_s[kr]);
+          else
+            ab = ring_window_call(hpx32(P.hp), win, tl, tr, r, B.ring_z[kr], B.ring_s[kr]);
           const uint32_t a = (uint32_t)ab, b = (uint32_t)(ab >> 32);
           act = act && a <= b;
           wl = 2 * a + (uint32_t)__builtin_amdgcn_readlane(gc, k);
