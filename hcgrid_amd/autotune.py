@@ -7,10 +7,9 @@ Two knobs:
     accumulation order of the contraction follows the block shape, so two
     tile_cols give cubes equal only up to FP32 summation order (both within
     the stated bound of the FP64 oracle), not bit for bit;
-  * per batch, the persistent launch's `waves` per workgroup and `chunk`
-    (samples staged per step), which fix how many channels one work item
-    carries (waves x 64) and how many workgroups share a CU.  These leave
-    every result bit-identical (the tests check it).
+  * per batch, `waves` and `chunk`, which the kernels accept and no longer
+    use (they choose their waves by the channel count); every result is
+    bit-identical.
 
 Because the tuner picks tile_cols from timings, two fresh tuning runs can
 pick different shapes and so differ in the last FP32 bits.  Persist the
@@ -109,7 +108,7 @@ class Autotuner:
         return out
 
     def launch_for(self, jobs: list, key: str) -> tuple[int, int]:
-        """(waves, chunk) of the persistent launch for this set of jobs."""
+        """(waves, chunk) for this set of jobs."""
         if key in self.launch:
             w, c = self.launch[key]
             return int(w), int(c)

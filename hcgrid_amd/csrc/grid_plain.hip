@@ -129,10 +129,7 @@ int launch_tiles_few_channels(const GridParams& P, const GridBuffers& B, const T
 }
 
 // The tile-route jobs of a batch, one route per launch: a workgroup finds its
-// job by binary search over the range starts and works one tile of it.  They
-// used to be items of the persistent MFMA kernel, at its two waves per SIMD
-// and the cost of its registers (69 VGPRs spilled with this tile body in it,
-// none without).
+// job by binary search over the range starts and works one tile of it.
 template <uint32_t ROUTE>
 __global__ void __launch_bounds__(ROUTE == kRouteOne4 ? 64 * kOneChannelStreams : 64)
     __attribute__((amdgpu_waves_per_eu(4)))
