@@ -19,7 +19,7 @@ Further legs (each on by default):
                  contraction), against the single-channel path applied
                  channel by channel to the same samples;
   batched      : 64 uneven jobs in one captured graph (geometry builds +
-                 one persistent launch), autotuned;
+                 batched launches), autotuned;
   served       : Poisson arrivals at 20 jobs/s of the batched mix through
                  the continuous-batching server.
 """
@@ -58,7 +58,7 @@ def parse():
                     help="also measure the multi-channel path (2M samples x 1024 BF16 channels)")
     ap.add_argument("--no-cube", dest="cube", action="store_false")
     ap.add_argument("--batch", dest="batch", action="store_true", default=True,
-                    help="also measure 64 uneven multi-channel jobs in one persistent launch (graph replay)")
+                    help="also measure 64 uneven multi-channel jobs in batched launches (graph replay)")
     ap.add_argument("--no-batch", dest="batch", action="store_false")
     ap.add_argument("--batch-jobs", type=int, default=64)
     ap.add_argument("--served", dest="served", action="store_true", default=True,
@@ -498,7 +498,7 @@ def bench_batch(args, log):
     """64 independent jobs (N log-uniform in [50k, 5M], map side in
     {128..2048}, channels in {1, 16, 64, 256, 512}, BF16/FP16, sigma in
     {0.015, 0.02, 0.03} deg, Dec in [-60, 80]) gridded by one graph: every
-    job's geometry build (keys, sort, records, LUT) and one persistent
+    job's geometry build (keys, sort, records, LUT) and the batched
     launch over all jobs' tiles.  Block shapes per job class and the launch
     shape are picked by the autotuner first (untimed).  Compared with the
     single-channel path applied channel by channel to the same jobs."""
@@ -562,7 +562,7 @@ def bench_batch(args, log):
     log(f"batch: {ms:.2f} ms per graph replay ({st['nitems']} work items on {st['blocks']} workgroups); "
         f"non-finite values {nonfinite}")
 
-    # the persistent gridding launches alone: HIP events recorded by the
+    # the gridding launches alone: HIP events recorded by the
     # library around them in eager enqueues of the same batch
     b.timing(True)
     prep, grid = [], []
@@ -575,7 +575,7 @@ def bench_batch(args, log):
     grid_ms = sum(grid) / len(grid)
     prep_ms = sum(prep) / len(prep)
     abytes = sum(cube_algorithmic_bytes(j["spec"].n, j["spec"].target.side ** 2, j["spec"].nchan) for j in jobs)
-    log(f"batch: eager enqueue: prep {prep_ms:.2f} ms, persistent gridding launches {grid_ms:.2f} ms")
+    log(f"batch: eager enqueue: prep {prep_ms:.2f} ms, gridding launches {grid_ms:.2f} ms")
 
     # device results of the checked bands (4 rows x every 32nd channel per job)
     checked = []
@@ -624,7 +624,7 @@ def bench_batch(args, log):
     out = {
         "workload": (f"{len(specs)} jobs: N log-uniform in [5e4, 5e6] (sum {sum(sp.n for sp in specs)}), side in "
                      "{128..2048} at 0.01 deg, channels in {1,16,64,256,512} BF16/FP16, sigma in {0.015,0.02,0.03} "
-                     "deg, Dec in [-60, 80]; one graph = every job's geometry build + one persistent launch"),
+                     "deg, Dec in [-60, 80]; one graph = every job's geometry build + batched launches"),
         "value": rate,
         "unit": UNIT,
         "ms_per_batch": ms,
@@ -636,7 +636,7 @@ def bench_batch(args, log):
         "channel_by_channel": {"value": chan_rate, "ms_total": tot_ms},
         "speedup_vs_channel_by_channel": rate / chan_rate,
         "roofline": {
-            "kernel": "k_grid_mfma_batch (+ the dense jobs' launch)",
+            "kernel": "k_grid_mfma_batch (one launch per instance) and k_batch_tiles",
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
@@ -646,7 +646,7 @@ def bench_batch(args, log):
             "avg_ms": grid_ms,
             "prep_ms": prep_ms,
             "traffic": None,
-            "note": "persistent gridding launches of eager enqueues, timed by the library's HIP events on the "
+            "note": "gridding launches of eager enqueues, timed by the library's HIP events on the "
                     "enqueue stream; the channel gathers and tile plans run before, in the prep launch",
         },
     }
@@ -729,7 +729,7 @@ def bench_served(args, log, tuner=None):
     request's coordinates and values on the device before submitting it
     (no host-to-device transfer in the latency); results stay in HBM.
     tuner: the batched leg's autotuner (block shape per job class), when
-    that leg ran; the persistent launch runs at its tuned waves/chunk."""
+    that leg ran; the launches run at its tuned waves/chunk."""
     from hcgrid_amd import serve
 
     waves, chunk = 4, 256

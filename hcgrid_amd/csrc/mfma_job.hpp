@@ -1,5 +1,5 @@
 // mfma_job.hpp -- the multi-channel job descriptor shared by the one-job
-// launch (hcg_grid_mfma) and the persistent batched launch (hcg_batch_*).
+// launch (hcg_grid_mfma) and the batched launches (hcg_batch_*).
 #pragma once
 
 #include <hip/hip_runtime.h>
