@@ -499,7 +499,7 @@ def bench_batch(args, log):
     {128..2048}, channels in {1, 16, 64, 256, 512}, BF16/FP16, sigma in
     {0.015, 0.02, 0.03} deg, Dec in [-60, 80]) gridded by one graph: every
     job's geometry build (keys, sort, records, LUT) and the batched
-    launch over all jobs' tiles.  Block shapes per job class and the launch
+    launches over all jobs' tiles.  Block shapes per job class and the launch
     shape are picked by the autotuner first (untimed).  Compared with the
     single-channel path applied channel by channel to the same jobs."""
     import torch
