@@ -50,8 +50,13 @@ __device__ inline uint32_t xcd_tile(uint32_t ntiles) {
 
 // WMODE: grid_tile.  S waves per tile, each walking every S-th non-empty
 // ring; their sums are added in stream order.
+// One-wave tiles have 168 registers at three waves per SIMD: at four (128) some
+// 70 spill around the sample loop, 3.7 GB of scratch writes on the 20M-sample
+// map (a pass 4.39 -> 4.28 ms; 250k samples onto 400^2 175 -> 160 us).  Tiles
+// of several waves, on maps that fill the chip less, are the slower for it
+// (5 sigma beam onto 347^2 1.17 -> 1.35 ms).
 template <int KT, bool HAS_W, int WMODE, uint32_t S, int ROWS>
-__global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(S == 1 ? 3 : 4)))
     k_grid_tiles(GridParams P, GridBuffers B, uint32_t tiles_x, uint32_t tiles_y) {
   constexpr uint32_t kCap = S >= 16 ? 128 : S >= 4 ? 192 : kStageCap;
   constexpr size_t kSlice = kCap * ((HAS_W ? 5 : 4) * sizeof(double) + sizeof(uint32_t));
