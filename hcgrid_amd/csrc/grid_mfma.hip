@@ -602,9 +602,8 @@ __device__ __forceinline__ void store_quad(const MfmaJob& J, uint32_t y0, uint32
 // The lane's row of the channel values (MFMA B operand): row ch_base + l % 16
 // of a value block, 16 bytes; the 16 lanes of a k-group read one contiguous
 // 256-byte piece.  Rows past the last channel fill columns that nothing
-// reads: they are the following blocks' (with one channel every lane reads
-// row 0; else there are fewer of them than eight blocks hold, and eight
-// blocks of padding follow the last sample's).
+// reads: they are the following blocks' (value_rows_read; with one channel
+// every lane reads row 0).
 __device__ __forceinline__ const char* value_rows(const MfmaJob& J, uint32_t ch_base) {
   return static_cast<const char*>(J.vs) +
          (size_t)(ch_base + (J.nchan > 1 ? __lane_id() & 15u : 0u)) * (kVB * 2u);
@@ -767,7 +766,7 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
 // half with the products, so that matrix and vector instructions overlap.  The
 // channel values of two k-blocks are read when the two before are done with,
 // and arrive while weights are evaluated.
-constexpr uint32_t kWideWaves = 8, kWideList = 256;
+constexpr uint32_t kWideList = 256;
 union MfmaWideLds {
   struct {
     s16x8_t a[2][4][4][2][64];  // [round parity][k-block][square][hi, lo][lane]
@@ -1065,24 +1064,11 @@ __global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_
   mfma_work<DT, NB, LEAN>(J, tile, group);
 }
 
-// The instance of a job: value type, channel blocks per wave and weight form.
-// A wave's registers grow with its channel blocks, so its SIMD holds fewer
-// waves; more than kNarrow blocks of 16 channels take mfma_wide.
-constexpr uint32_t kNbs = 8, kNbOf[kNbs] = {1, 2, 4, 6, 8, 12, 16, 0};
-constexpr uint32_t kNarrow = 16, kNarrowGeneral = 4;
-constexpr uint32_t kGeneral[2] = {2, 7};  // the general weights' instances, as kNbOf
-static_assert(kMfmaInstances == 2 * (kNbs + 2), "instances");
-static uint32_t nb_of_instance(uint32_t inst) {
-  return kNbOf[inst / 2 < kNbs ? inst / 2 : kGeneral[inst / 2 - kNbs]];
-}
+// The instance of a job: its form (mfma_form) and value type.
+static uint32_t nb_of_instance(uint32_t inst) { return nb_of_form(inst / 2); }
 bool mfma_uses_plan(uint32_t inst) { return nb_of_instance(inst) == 0; }
 uint32_t mfma_instance(const MfmaJob& J) {
-  const uint32_t d = J.dtype == HCG_DTYPE_BF16 ? 0u : 1u, blocks = ceil_div_u32(J.nchan, 16);
-  if (J.kt != kKtGaussLean || J.B.w_s) return 2 * (kNbs + (blocks > kNarrowGeneral ? 1 : 0)) + d;
-  if (blocks > kNarrow) return 2 * (kNbs - 1) + d;
-  uint32_t i = 0;
-  while (kNbOf[i] < blocks) ++i;
-  return 2 * i + d;
+  return 2 * mfma_form(J.nchan, J.kt == kKtGaussLean && !J.B.w_s) + (J.dtype == HCG_DTYPE_BF16 ? 0u : 1u);
 }
 static uint32_t mfma_groups(const MfmaJob& J, uint32_t inst) {
   const uint32_t nb = nb_of_instance(inst);
@@ -1098,7 +1084,8 @@ uint64_t mfma_blocks(const MfmaJob& J) {
   HCG_MFMA_PAIR(X, 0, kNbOf[0], true) HCG_MFMA_PAIR(X, 1, kNbOf[1], true) HCG_MFMA_PAIR(X, 2, kNbOf[2], true) \
   HCG_MFMA_PAIR(X, 3, kNbOf[3], true) HCG_MFMA_PAIR(X, 4, kNbOf[4], true) HCG_MFMA_PAIR(X, 5, kNbOf[5], true) \
   HCG_MFMA_PAIR(X, 6, kNbOf[6], true) HCG_MFMA_PAIR(X, 7, kNbOf[7], true)                                     \
-  HCG_MFMA_PAIR(X, kNbs, kNbOf[kGeneral[0]], false) HCG_MFMA_PAIR(X, kNbs + 1, kNbOf[kGeneral[1]], false)
+  HCG_MFMA_PAIR(X, kNbs, kNbOf[kGeneral[0]], false) HCG_MFMA_PAIR(X, kNbs + 1, kNbOf[kGeneral[1]], false)     \
+  HCG_MFMA_PAIR(X, kNbs + 2, kNbOf[kGeneral[2]], false)
 
 static int launch_mfma_job(const MfmaJob& J, hipStream_t s) {
   const uint32_t inst = mfma_instance(J);

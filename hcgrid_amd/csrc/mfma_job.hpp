@@ -48,7 +48,53 @@ struct MfmaJob {
 // batch, contraction jobs are told apart by their kernel instance too
 // (kRouteMfma + mfma_instance).
 enum : uint32_t { kRouteOne4 = 0, kRouteOne1 = 1, kRouteFew = 2, kRouteMfma = 3 };
-constexpr uint32_t kMfmaInstances = 20, kRoutes = kRouteMfma + kMfmaInstances;
+constexpr uint32_t kMfmaInstances = 22, kRoutes = kRouteMfma + kMfmaInstances;
+
+// The contraction kernel's forms: 16-channel blocks per wave (mfma_tile), or
+// 0: mfma_wide.  A wave's registers grow with its channel blocks, so its SIMD
+// holds fewer waves; more than kNarrow blocks (kNarrowGeneral with the general
+// weights) take mfma_wide.  An instance is a form for each value type: first
+// the lean weight's forms, then the general weights', kNbOf[kGeneral[...]].
+constexpr uint32_t kWideWaves = 8;  // waves of a mfma_wide workgroup, 64 channels each
+constexpr uint32_t kNbs = 8, kNbOf[kNbs] = {1, 2, 4, 6, 8, 12, 16, 0};
+constexpr uint32_t kNarrow = 16, kNarrowGeneral = 4;
+constexpr uint32_t kGenerals = 3, kGeneral[kGenerals] = {0, 2, 7};
+static_assert(kMfmaInstances == 2 * (kNbs + kGenerals), "instances");
+
+// The form of a job (index as instances count): the narrowest that holds its channels.
+constexpr uint32_t mfma_form(uint32_t nchan, bool lean) {
+  const uint32_t blocks = (nchan + 15) / 16;
+  uint32_t i = 0;
+  if (lean) {
+    while (i < kNbs - 1 && kNbOf[i] < blocks) ++i;
+    return i;
+  }
+  while (i < kGenerals - 1 && kNbOf[kGeneral[i]] < blocks) ++i;
+  return kNbs + i;
+}
+constexpr uint32_t nb_of_form(uint32_t form) { return kNbOf[form < kNbs ? form : kGeneral[form - kNbs]]; }
+
+// A lane reads whole 16-channel blocks of a value block: the rows that the
+// form of a job reads, counted from the value block's first, and those that
+// are there after the first row of the last sample's block (its own and the
+// padding's eight blocks, hcg_channels_padded_len).  Rows past the last channel
+// fill MFMA columns that nothing reads, but they have to be in the buffer.
+constexpr uint64_t value_rows_read(uint32_t nchan, bool lean) {
+  const uint64_t nb = nb_of_form(mfma_form(nchan, lean));
+  if (nchan == 1) return nb ? (nb - 1) * 16 + 1 : 49;  // (every lane reads its block's first row)
+  const uint64_t step = nb ? 16 * nb : 64;
+  return (nchan + step - 1) / step * step;
+}
+constexpr uint64_t value_rows_held(uint32_t nchan) { return 9ull * nchan; }
+// (past kNarrow blocks a form reads fewer than 64 rows beyond the last one;
+// a single channel takes the lean weight on the tile loop only)
+constexpr bool value_rows_ok() {
+  for (uint32_t c = 1; c <= 1024; ++c)
+    for (uint32_t lean = 0; lean < 2; ++lean)
+      if (value_rows_read(c, lean != 0) > value_rows_held(c)) return false;
+  return true;
+}
+static_assert(value_rows_ok(), "a form reads past the padded channel values");
 inline uint32_t route_of(const GridParams& P, uint32_t kernel_type, bool weighted, uint32_t nchan, uint32_t n) {
   if (one_channel_tiles(P, kernel_type, weighted, nchan))
     return one_channel_streams(P.side) == kOneChannelStreams ? kRouteOne4 : kRouteOne1;
