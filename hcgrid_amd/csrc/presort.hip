@@ -26,7 +26,9 @@
 // 142 us for 250k samples and 760 us for 20M.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
+#include <utility>
 
 #include "common.hpp"
 #include "healpix.hpp"
@@ -402,18 +404,22 @@ constexpr size_t sort_ws_bytes(uint32_t n) {
          align256(kMaxDigits * 4);
 }
 
-size_t sort_ws_layout(uint32_t n, void* base, SortWorkspace* ws) {
+// The largest need of up to n keys: the small tiles' counts take more than
+// those of somewhat more keys in larger tiles.
+constexpr size_t sort_ws_bytes_up_to(uint32_t n) {
+  return std::max({sort_ws_bytes(n), sort_ws_bytes(std::min(n, kSmallTile * kSmallTiles)),
+                   sort_ws_bytes(std::min(n, kMidTile * kMidTiles))});
+}
+
+void sort_ws_layout(uint32_t n, void* base, SortWorkspace& ws) {
   const uint32_t tiles = sort_tiles_of(n);
   const size_t kb = align256((size_t)n * 4), hb = align256((size_t)tiles * kMaxDigits * 4);
-  if (ws) {
-    char* p = static_cast<char*>(base);
-    ws->keys_b = reinterpret_cast<uint32_t*>(p);
-    ws->vals_b = reinterpret_cast<uint32_t*>(p + kb);
-    ws->hist = reinterpret_cast<uint32_t*>(p + 2 * kb);
-    ws->digit = reinterpret_cast<uint32_t*>(p + 2 * kb + hb);
-    ws->tiles = tiles;
-  }
-  return sort_ws_bytes(n);
+  char* p = static_cast<char*>(base);
+  ws.keys_b = reinterpret_cast<uint32_t*>(p);
+  ws.vals_b = reinterpret_cast<uint32_t*>(p + kb);
+  ws.hist = reinterpret_cast<uint32_t*>(p + 2 * kb);
+  ws.digit = reinterpret_cast<uint32_t*>(p + 2 * kb + hb);
+  ws.tiles = tiles;
 }
 
 // Argument checks shared by hcg_presort and hcg_presort_noalloc.
@@ -481,7 +487,7 @@ int presort_enqueue(const hcg_healpix* hp, uint32_t n, const double* lon_deg, co
 // `scratch` names a host-side stand-in, not a device address: its device
 // address comes from hipGetSymbolAddress, once per device (each device
 // holds its own copy of the array, at its own address).
-constexpr size_t kNoAllocScratchBytes = sort_ws_bytes(HCG_PRESORT_NOALLOC_MAX_N);
+constexpr size_t kNoAllocScratchBytes = sort_ws_bytes_up_to(HCG_PRESORT_NOALLOC_MAX_N);
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -506,7 +512,7 @@ int scratch_address(void** out) {
 }
 }  // namespace
 
-extern "C" size_t hcg_presort_workspace_size(uint32_t n) { return sort_ws_layout(n, nullptr, nullptr); }
+extern "C" size_t hcg_presort_workspace_size(uint32_t n) { return sort_ws_bytes_up_to(n); }
 
 extern "C" int hcg_presort(const hcg_healpix* hp, uint32_t n, const double* lon_deg, const double* lat_deg,
                            uint32_t* keys_sorted, uint32_t* perm, void* workspace, size_t workspace_bytes,
@@ -519,10 +525,10 @@ extern "C" int hcg_presort(const hcg_healpix* hp, uint32_t n, const double* lon_
     HCG_CHECK_LAUNCH("k_set_sentinel");
     return HCG_OK;
   }
-  if (workspace == nullptr || workspace_bytes < hcg_presort_workspace_size(n))
+  if (workspace == nullptr || workspace_bytes < sort_ws_bytes(n))
     return set_error(HCG_ERR_WORKSPACE, "hcg_presort: workspace smaller than hcg_presort_workspace_size(n)");
   SortWorkspace ws;
-  sort_ws_layout(n, workspace, &ws);
+  sort_ws_layout(n, workspace, ws);
   return presort_enqueue(hp, n, lon_deg, lat_deg, keys_sorted, perm, ws, s);
 }
 
@@ -543,7 +549,7 @@ extern "C" int hcg_presort_noalloc(const hcg_healpix* hp, uint32_t n, const doub
   rc = scratch_address(&base);
   if (rc != HCG_OK) return rc;
   SortWorkspace ws;
-  sort_ws_layout(n, base, &ws);
+  sort_ws_layout(n, base, ws);
   return presort_enqueue(hp, n, lon_deg, lat_deg, keys_sorted, perm, ws, s);
 }
 

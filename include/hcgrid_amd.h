@@ -126,7 +126,8 @@ double   hcg_host_pix2theta(const hcg_healpix *hp, uint64_t pix);
 
 /* ---- the device path ---- */
 
-/* Workspace bytes hcg_presort() needs for n samples. */
+/* Workspace bytes hcg_presort() needs for n samples or fewer (it never falls
+ * as n grows). */
 size_t hcg_presort_workspace_size(uint32_t n);
 
 /* HEALPix keys + stable sort: the ang2pix loop and sort of
