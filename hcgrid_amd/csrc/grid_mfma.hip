@@ -544,10 +544,13 @@ __device__ __forceinline__ uint64_t weigh_kblock(const MfmaJob& J, SquareCell<LE
 }
 
 // The pairs within rounding of the radius: the reference's test decides, and
-// a pair that it rejects is taken out again.
+// a pair that it rejects is taken out again.  A lean weight is subtracted from
+// the sum, exactly; with the general weights, which may be infinite or NaN by
+// the sample's, the sum starts again from wsum0, its value before the k-block.
 template <int DT, bool LEAN, uint32_t NS>
 __device__ __forceinline__ void guard_kblock(const MfmaJob& J, SquareCell<LEAN>& Q, const Staged<NS>& S, uint32_t at,
-                                             uint32_t wl, uint32_t ww, uint32_t cell, uint32_t blk, WeightOperand& A) {
+                                             uint32_t wl, uint32_t ww, uint32_t cell, uint32_t blk, double wsum0,
+                                             WeightOperand& A) {
   constexpr bool bf = DT == kDtBf16;
 #pragma unroll 1
   for (uint32_t e = 0; e < 8; ++e) {
@@ -565,7 +568,16 @@ __device__ __forceinline__ void guard_kblock(const MfmaJob& J, SquareCell<LEAN>&
           A.h.d[i] &= keep;
           A.l.d[i] &= keep;
         }
-      Q.wsum -= (double)(widen16((uint16_t)hw, bf) + widen16((uint16_t)lw, bf));
+      if constexpr (LEAN) Q.wsum -= (double)(widen16((uint16_t)hw, bf) + widen16((uint16_t)lw, bf));
+    }
+  }
+  if constexpr (!LEAN) {
+    Q.wsum = wsum0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {  // as weigh_kblock adds them
+      const f32x2_t fh = widen16x2<bf>(A.h.d[i]), fl = widen16x2<bf>(A.l.d[i]);
+      Q.wsum += (double)(fh.x + fl.x);
+      Q.wsum += (double)(fh.y + fl.y);
     }
   }
 }
@@ -686,6 +698,7 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
         tile_sync();
         WeightOperand A;
         uint64_t guard;
+        const double wsum0 = Q.wsum;
         const uint64_t any = weigh_kblock<DT>(J, Q, W.st, 0, wl, ww, cell, blk, s_exp, A, guard);
         if (guard) {  // uniform, rare
           // the sums wait in scratch memory meanwhile (volatile: here and only
@@ -695,7 +708,7 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
           volatile float keep[NB * 4];
 #pragma unroll
           for (int i = 0; i < NB * 4; ++i) keep[i] = acc[i / 4][i % 4];
-          guard_kblock<DT>(J, Q, W.st, 0, wl, ww, cell, blk, A);
+          guard_kblock<DT>(J, Q, W.st, 0, wl, ww, cell, blk, wsum0, A);
 #pragma unroll
           for (int i = 0; i < NB * 4; ++i) acc[i / 4][i % 4] = keep[i];
           load_b();
@@ -880,12 +893,13 @@ __device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint3
           Q.window(P, C, L, rb, L.lr[u * 4 + kg], wl, ww);
           WeightOperand A;
           uint64_t guard;
+          const double wsum0 = Q.wsum;
           any = weigh_kblock<DT>(J, Q, lds.s.st[par], k * 32, wl, ww, cell, blk, s_exp, A, guard);
           if (guard) {  // uniform, rare; the sums wait in scratch memory (see mfma_tile)
             volatile float keep[64];
 #pragma unroll
             for (int i = 0; i < 64; ++i) keep[i] = acc[i / 16][i / 4 % 4][i % 4];
-            guard_kblock<DT>(J, Q, lds.s.st[par], k * 32, wl, ww, cell, blk, A);
+            guard_kblock<DT>(J, Q, lds.s.st[par], k * 32, wl, ww, cell, blk, wsum0, A);
 #pragma unroll
             for (int i = 0; i < 64; ++i) acc[i / 16][i / 4 % 4][i % 4] = keep[i];
           }

@@ -79,3 +79,44 @@ def test_few_channels_values(gpu, nchan):
     cube = g.cube.cpu().numpy().reshape(nchan, -1)
     for ch in (0, nchan - 1):
         _same(cube[ch], out[ch].astype(np.float32), f"channel {ch}")
+
+
+@pytest.mark.parametrize("nchan", [3, 40, 100])
+@pytest.mark.parametrize("weight", [np.nan, np.inf])
+def test_contraction_weights(gpu, nchan, weight):
+    import ctypes as C
+
+    import torch
+    from hcgrid_amd import capi
+    side = 70
+    wl = synth.raster_small(30, 150, side, seed=53)
+    xw, yw = _target_coords(wl.target)
+    cells = np.arange(side * side // 2 + side // 2, side * side, 7 * side)[:4]
+    lon, lat = _with_edge_samples(wl, xw, yw, cells)
+    n, rng = len(lon), np.random.default_rng(7)
+    w = np.concatenate([rng.uniform(0.5, 2.0, wl.n), np.full(3 * len(cells), weight)])
+    Vt = torch.tensor(rng.uniform(0.5, 2.0, (nchan, n)).astype(np.float32)).to(torch.bfloat16).cuda()
+    print(f"case: contraction nchan={nchan} weight={weight} n={n}", flush=True)
+    kern, hp = gridder.prepare_grid_kernel(GAUSS1D, [0.02], RADIUS, RES)
+    g = gridder.CubeGridder(n, side, nchan, kern, hp)
+    d = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda")  # noqa: E731
+    x, y, lo, la, p = d(xw), d(yw), d(lon), d(lat), gridder._ptr
+    g.plain.presort(lo, la)
+    g.gather_records(lo, la)
+    g.plain.ring_lut()
+    g.gather_channels(Vt)
+    perm = g.plain.perm()
+    ws, b = d(w[perm]), g.plain.buf
+    capi.call("hcg_grid_mfma", C.byref(hp), C.byref(kern), side, n, nchan, g.dcode, p(b.records), p(b.keys),
+              p(b.lon_s), p(b.lat_s), p(ws), p(g.values_sorted), p(b.lut), p(b.ring_z), p(b.ring_s), p(b.meta),
+              p(x), p(y), p(g.cube), p(g.wsum), 0, gridder._stream_handle(None))
+    torch.cuda.synchronize()
+    Vr = Vt.float().cpu().numpy()
+    ref = oracle.pipeline(lon, lat, Vr[0], xw, yw, side, 0.02, RADIUS, RES, weights=w)
+    wsum, cube = g.wsum.cpu().numpy(), g.cube.cpu().numpy().reshape(nchan, -1)[0]
+    for dev, r in ((wsum, ref["weightscube"]), (cube, ref["datacube"])):
+        bad = ~np.isfinite(r)
+        assert np.array_equal(~np.isfinite(dev), bad) and bad.any() and not bad.all()
+        ok = ~bad
+        # weights carried to ~2^-17, FP32 sums
+        assert np.max(np.abs(dev[ok] - r[ok])) <= 1e-4 * np.max(np.abs(r[ok]))
