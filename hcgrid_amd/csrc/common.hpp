@@ -36,6 +36,17 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 
 inline uint32_t ceil_div_u32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
+// A launch counts its threads in 32 bits (HIP refuses more): work of `blocks`
+// workgroups goes as launch(first, count) over runs of at most this many, a
+// multiple of 8, so that workgroup first + b runs on XCD b % 8 as in one launch.
+constexpr uint32_t max_launch_blocks(uint32_t threads) { return 0xFFFFFFFFu / threads & ~7u; }
+template <class F>
+inline void launch_runs(uint64_t blocks, uint32_t threads, F&& launch) {
+  const uint32_t most = max_launch_blocks(threads);
+  for (uint64_t first = 0; first < blocks; first += most)
+    launch((uint32_t)first, (uint32_t)(blocks - first < most ? blocks - first : most));
+}
+
 // Lanes of the wave whose 8-bit digit equals this lane's (wave64 ballots).
 __device__ inline uint64_t match_digit8(uint32_t d, bool valid) {
   uint64_t m = __ballot(valid);

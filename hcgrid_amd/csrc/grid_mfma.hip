@@ -374,7 +374,7 @@ __device__ __forceinline__ void plan_tile(const MfmaJob& J, uint32_t tile) {  //
   L.nb[lane] = nblk;
 }
 
-__global__ void __launch_bounds__(64) k_mfma_plan(MfmaJob J) { plan_tile(J, blockIdx.x); }
+__global__ void __launch_bounds__(64) k_mfma_plan(MfmaJob J, uint32_t first) { plan_tile(J, first + blockIdx.x); }
 
 // Lists blocks q0 .. q0 + cnt - 1 (one wave), then the last one again up to
 // the k-block boundary, as padding without samples.
@@ -1049,11 +1049,11 @@ __device__ __forceinline__ void mfma_work(const MfmaJob& J, uint32_t tile, uint3
     mfma_tile<DT, NB, LEAN>(J, tile, group, lds, s_exp);
 }
 
-// One job: grid = (tile_blocks, channel groups).
+// One job: grid = (tile_blocks, or a run of them from `first` on, channel groups).
 template <int DT, int NB, bool LEAN>
 __global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, LEAN))))
-    k_grid_mfma(MfmaJob J) {
-  const uint32_t tile = block_tile(blockIdx.x, J.ntiles, J.tiles_x, NB == 0);
+    k_grid_mfma(MfmaJob J, uint32_t first) {
+  const uint32_t tile = block_tile(first + blockIdx.x, J.ntiles, J.tiles_x, NB == 0);
   if (tile >= J.ntiles) return;  // uniform
   mfma_work<DT, NB, LEAN>(J, tile, blockIdx.y);
 }
@@ -1062,17 +1062,19 @@ __global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_
 // finds its job by binary search over the range starts (multiples of 8).
 template <int DT, int NB, bool LEAN>
 __global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, LEAN))))
-    k_grid_mfma_batch(const TileRange* __restrict__ ranges, uint32_t nranges, const MfmaJob* __restrict__ jobs) {
-  uint32_t lo = 0, hi = nranges;  // last range with first <= blockIdx.x
+    k_grid_mfma_batch(const TileRange* __restrict__ ranges, uint32_t nranges, const MfmaJob* __restrict__ jobs,
+                      uint32_t first) {
+  const uint32_t block = first + blockIdx.x;
+  uint32_t lo = 0, hi = nranges;  // last range with first <= block
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (ranges[mid].first <= blockIdx.x)
+    if (ranges[mid].first <= block)
       lo = mid;
     else
       hi = mid;
   }
   const MfmaJob& J = jobs[ranges[lo].job];
-  const uint32_t lb = blockIdx.x - ranges[lo].first, per = tile_blocks(J.ntiles, J.tiles_x, NB == 0);
+  const uint32_t lb = block - ranges[lo].first, per = tile_blocks(J.ntiles, J.tiles_x, NB == 0);
   const uint32_t tile = block_tile(lb % per, J.ntiles, J.tiles_x, NB == 0), group = lb / per;
   if (tile >= J.ntiles) return;  // uniform
   mfma_work<DT, NB, LEAN>(J, tile, group);
@@ -1103,15 +1105,17 @@ uint64_t mfma_blocks(const MfmaJob& J) {
 
 static int launch_mfma_job(const MfmaJob& J, hipStream_t s) {
   const uint32_t inst = mfma_instance(J);
-  const dim3 grid(tile_blocks(J.ntiles, J.tiles_x, nb_of_instance(inst) == 0), mfma_groups(J, inst));
+  const uint32_t nb = nb_of_instance(inst), groups = mfma_groups(J, inst);
   if (J.plan) {
-    k_mfma_plan<<<J.ntiles, 64, 0, s>>>(J);
+    launch_runs(J.ntiles, 64, [&](uint32_t first, uint32_t count) { k_mfma_plan<<<count, 64, 0, s>>>(J, first); });
     HCG_CHECK_LAUNCH("k_mfma_plan");
   }
+  launch_runs(tile_blocks(J.ntiles, J.tiles_x, nb == 0), mfma_threads(nb), [&](uint32_t first, uint32_t count) {
 #define HCG_CASE(I, DT, NB, LEAN) \
-  case I: k_grid_mfma<DT, NB, LEAN><<<grid, mfma_threads(NB), 0, s>>>(J); break;
-  switch (inst) { HCG_MFMA_INSTANCES(HCG_CASE) }
+  case I: k_grid_mfma<DT, NB, LEAN><<<dim3(count, groups), mfma_threads(NB), 0, s>>>(J, first); break;
+    switch (inst) { HCG_MFMA_INSTANCES(HCG_CASE) }
 #undef HCG_CASE
+  });
   HCG_CHECK_LAUNCH("k_grid_mfma");
   return HCG_OK;
 }
@@ -1119,10 +1123,13 @@ static int launch_mfma_job(const MfmaJob& J, hipStream_t s) {
 int launch_mfma_batch(uint32_t inst, const TileRange* ranges, uint32_t nranges, uint32_t blocks, const MfmaJob* jobs,
                       hipStream_t s) {
   if (nranges == 0 || blocks == 0) return HCG_OK;
-#define HCG_CASE(I, DT, NB, LEAN) \
-  case I: k_grid_mfma_batch<DT, NB, LEAN><<<blocks, mfma_threads(NB), 0, s>>>(ranges, nranges, jobs); break;
-  switch (inst) { HCG_MFMA_INSTANCES(HCG_CASE) }
+  launch_runs(blocks, mfma_threads(nb_of_instance(inst)), [&](uint32_t first, uint32_t count) {
+#define HCG_CASE(I, DT, NB, LEAN)                                                                             \
+  case I:                                                                                                     \
+    k_grid_mfma_batch<DT, NB, LEAN><<<count, mfma_threads(NB), 0, s>>>(ranges, nranges, jobs, first); break;
+    switch (inst) { HCG_MFMA_INSTANCES(HCG_CASE) }
 #undef HCG_CASE
+  });
   HCG_CHECK_LAUNCH("k_grid_mfma_batch");
   return HCG_OK;
 }
@@ -1252,8 +1259,8 @@ template <typename T>
 __global__ void __launch_bounds__(256) k_gather_channels_sm(uint32_t n, uint32_t n_pad, uint32_t nchan,
                                                             const uint32_t* __restrict__ perm,
                                                             const T* __restrict__ in, T* __restrict__ out,
-                                                            uint32_t* __restrict__ nonfinite) {
-  gather_sm_block<T>(blockIdx.x, n, n_pad, nchan, perm, in, out, nonfinite);
+                                                            uint32_t* __restrict__ nonfinite, uint32_t first) {
+  gather_sm_block<T>(first + blockIdx.x, n, n_pad, nchan, perm, in, out, nonfinite);
 }
 
 // Every job's channel gather and block plan (mfma_wide) of a batch in one
@@ -1263,18 +1270,19 @@ __global__ void __launch_bounds__(256) k_gather_channels_sm(uint32_t n, uint32_t
 // workgroup finds its range by binary search over the range starts.
 __global__ void __launch_bounds__(256) k_batch_prep(const PrepRange* __restrict__ ranges, uint32_t nranges,
                                                     const PrepJob* __restrict__ pj,
-                                                    const MfmaJob* __restrict__ jobs) {
+                                                    const MfmaJob* __restrict__ jobs, uint32_t first) {
   __shared__ __attribute__((aligned(16))) uint16_t smem[kGatherChans * kGatherRow];
-  uint32_t lo = 0, hi = nranges;  // last range with first <= blockIdx.x
+  const uint32_t block = first + blockIdx.x;
+  uint32_t lo = 0, hi = nranges;  // last range with first <= block
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (ranges[mid].first <= blockIdx.x)
+    if (ranges[mid].first <= block)
       lo = mid;
     else
       hi = mid;
   }
   const PrepRange R = ranges[lo];
-  const uint32_t lb = blockIdx.x - R.first;
+  const uint32_t lb = block - R.first;
   const PrepJob& G = pj[R.job];
   const MfmaJob& J = jobs[R.job];
   const uint32_t bx = lb % R.gx, by = lb / R.gx;
@@ -1334,7 +1342,9 @@ int prep_ranges(uint32_t njobs, const MfmaJob* jobs, const uint32_t* layouts, st
 int launch_batch_prep(const PrepRange* ranges, uint32_t nranges, uint32_t blocks, const PrepJob* pj,
                       const MfmaJob* jobs, hipStream_t s) {
   if (nranges == 0 || blocks == 0) return HCG_OK;
-  k_batch_prep<<<blocks, 256, 0, s>>>(ranges, nranges, pj, jobs);
+  launch_runs(blocks, 256, [&](uint32_t first, uint32_t count) {
+    k_batch_prep<<<count, 256, 0, s>>>(ranges, nranges, pj, jobs, first);
+  });
   HCG_CHECK_LAUNCH("k_batch_prep");
   return HCG_OK;
 }
@@ -1363,14 +1373,15 @@ extern "C" int hcg_gather_channels(uint32_t n, uint32_t nchan, const uint32_t* p
                                                           static_cast<const _Float16*>(values),
                                                           static_cast<_Float16*>(values_sorted), nonfinite);
   } else {
-    const uint32_t grid = gather_sm_gx(n_pad, nchan);
-    if (dtype == HCG_DTYPE_BF16)
-      k_gather_channels_sm<__bf16><<<grid, 256, 0, s>>>(n, n_pad, nchan, perm, static_cast<const __bf16*>(values),
-                                                        static_cast<__bf16*>(values_sorted), nonfinite);
-    else
-      k_gather_channels_sm<_Float16><<<grid, 256, 0, s>>>(n, n_pad, nchan, perm,
-                                                          static_cast<const _Float16*>(values),
-                                                          static_cast<_Float16*>(values_sorted), nonfinite);
+    launch_runs(gather_sm_gx(n_pad, nchan), 256, [&](uint32_t first, uint32_t count) {
+      if (dtype == HCG_DTYPE_BF16)
+        k_gather_channels_sm<__bf16><<<count, 256, 0, s>>>(n, n_pad, nchan, perm, static_cast<const __bf16*>(values),
+                                                           static_cast<__bf16*>(values_sorted), nonfinite, first);
+      else
+        k_gather_channels_sm<_Float16><<<count, 256, 0, s>>>(n, n_pad, nchan, perm,
+                                                             static_cast<const _Float16*>(values),
+                                                             static_cast<_Float16*>(values_sorted), nonfinite, first);
+    });
   }
   HCG_CHECK_LAUNCH("k_gather_channels");
   return HCG_OK;

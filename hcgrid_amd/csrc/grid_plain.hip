@@ -40,12 +40,12 @@
 
 namespace hcg {
 
-// The tile of this workgroup.  XCD-aware order: workgroups are dealt
+// The tile of workgroup b.  XCD-aware order: workgroups are dealt
 // round-robin over the 8 XCDs, so block b runs on XCD b % 8; give each XCD a
 // contiguous run of tiles so neighbouring tiles (which stage overlapping
 // samples) share its L2.
-__device__ inline uint32_t xcd_tile(uint32_t ntiles) {
-  return (ntiles & 7u) == 0 ? (blockIdx.x & 7u) * (ntiles >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+__device__ inline uint32_t xcd_tile(uint32_t b, uint32_t ntiles) {
+  return (ntiles & 7u) == 0 ? (b & 7u) * (ntiles >> 3) + (b >> 3) : b;
 }
 
 // WMODE: grid_tile.  S waves per tile, each walking every S-th non-empty
@@ -57,7 +57,7 @@ __device__ inline uint32_t xcd_tile(uint32_t ntiles) {
 // (5 sigma beam onto 347^2 1.17 -> 1.35 ms).
 template <int KT, bool HAS_W, int WMODE, uint32_t S, int ROWS>
 __global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(S == 1 ? 3 : 4)))
-    k_grid_tiles(GridParams P, GridBuffers B, uint32_t tiles_x, uint32_t tiles_y) {
+    k_grid_tiles(GridParams P, GridBuffers B, uint32_t tiles_x, uint32_t tiles_y, uint32_t first) {
   constexpr uint32_t kCap = S >= 16 ? 128 : S >= 4 ? 192 : kStageCap;
   constexpr size_t kSlice = kCap * ((HAS_W ? 5 : 4) * sizeof(double) + sizeof(uint32_t));
   __shared__ __attribute__((aligned(16))) char lds[S * kSlice];
@@ -69,7 +69,7 @@ __global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(S =
   else
     tile_sync();
   if (B.meta->usedrings == 0) return;  // uniform: no samples, nothing to add
-  const uint32_t tile = xcd_tile(tiles_x * tiles_y);
+  const uint32_t tile = xcd_tile(first + blockIdx.x, tiles_x * tiles_y);
   TileSums<0> t;
   if constexpr (S == 1) {
     grid_tile<KT, HAS_W, WMODE, false, 0, kCap, ROWS>(P, B, tile, tiles_x, lds, s_exp, TileOut{}, RingStream{0, 1},
@@ -105,30 +105,32 @@ __global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(S =
 // S waves, one partial ring stream per wave (one_channel_tile).
 template <uint32_t S, int WMODE>
 __global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(4)))
-    k_grid_tiles_1ch(GridParams P, GridBuffers B, TileOut O, uint32_t tiles_x, uint32_t tiles_y) {
+    k_grid_tiles_1ch(GridParams P, GridBuffers B, TileOut O, uint32_t tiles_x, uint32_t tiles_y, uint32_t first) {
   __shared__ __attribute__((aligned(16))) char lds[one_channel_lds_bytes(S, S)];
   __shared__ double s_exp[64];
   if (threadIdx.x < 64) exp_table_load(s_exp);
   __syncthreads();
-  one_channel_tile<WMODE>(P, B, O, xcd_tile(tiles_x * tiles_y), tiles_x, S, S, lds, s_exp);
+  one_channel_tile<WMODE>(P, B, O, xcd_tile(first + blockIdx.x, tiles_x * tiles_y), tiles_x, S, S, lds, s_exp);
 }
 
 // A few-channel job of the multi-channel entry points on the tile path: one
 // wave per tile (few_channel_tile_body).
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
-    k_grid_tiles_few(GridParams P, GridBuffers B, TileOut O, uint32_t tiles_x, uint32_t tiles_y) {
+    k_grid_tiles_few(GridParams P, GridBuffers B, TileOut O, uint32_t tiles_x, uint32_t tiles_y, uint32_t first) {
   __shared__ __attribute__((aligned(16))) char lds[kFewTileLdsBytes];
   __shared__ double s_exp[64];
   exp_table_load(s_exp);
   tile_sync();
-  few_channel_tile_body(P, B, O, xcd_tile(tiles_x * tiles_y), tiles_x, lds, s_exp);
+  few_channel_tile_body(P, B, O, xcd_tile(first + blockIdx.x, tiles_x * tiles_y), tiles_x, lds, s_exp);
 }
 
 int launch_tiles_few_channels(const GridParams& P, const GridBuffers& B, const TileOut& O, hipStream_t s) {
   const uint32_t tiles_x = tile_cols_of(P.side);
   const uint32_t tiles_y = (P.side + kTileRows - 1) / kTileRows;
   if ((uint64_t)tiles_x * tiles_y == 0) return HCG_OK;
-  k_grid_tiles_few<<<tiles_x * tiles_y, 64, 0, s>>>(P, B, O, tiles_x, tiles_y);
+  launch_runs((uint64_t)tiles_x * tiles_y, 64, [&](uint32_t first, uint32_t count) {
+    k_grid_tiles_few<<<count, 64, 0, s>>>(P, B, O, tiles_x, tiles_y, first);
+  });
   HCG_CHECK_LAUNCH("k_grid_tiles_few");
   return HCG_OK;
 }
@@ -138,7 +140,8 @@ int launch_tiles_few_channels(const GridParams& P, const GridBuffers& B, const T
 template <uint32_t ROUTE>
 __global__ void __launch_bounds__(ROUTE == kRouteOne4 ? 64 * kOneChannelStreams : 64)
     __attribute__((amdgpu_waves_per_eu(4)))
-    k_batch_tiles(const TileRange* __restrict__ ranges, uint32_t nranges, const MfmaJob* __restrict__ jobs) {
+    k_batch_tiles(const TileRange* __restrict__ ranges, uint32_t nranges, const MfmaJob* __restrict__ jobs,
+                  uint32_t first) {
   constexpr uint32_t S = ROUTE == kRouteOne4 ? kOneChannelStreams : 1;
   __shared__ __attribute__((aligned(16))) char lds[ROUTE == kRouteFew ? kFewTileLdsBytes : one_channel_lds_bytes(S, S)];
   __shared__ double s_exp[64];
@@ -147,16 +150,17 @@ __global__ void __launch_bounds__(ROUTE == kRouteOne4 ? 64 * kOneChannelStreams 
     __syncthreads();
   else
     tile_sync();
-  uint32_t lo = 0, hi = nranges;  // last range with first <= blockIdx.x
+  const uint32_t block = first + blockIdx.x;
+  uint32_t lo = 0, hi = nranges;  // last range with first <= block
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (ranges[mid].first <= blockIdx.x)
+    if (ranges[mid].first <= block)
       lo = mid;
     else
       hi = mid;
   }
   const MfmaJob& J = jobs[ranges[lo].job];
-  const uint32_t tile = blockIdx.x - ranges[lo].first;
+  const uint32_t tile = block - ranges[lo].first;
   const TileOut O{static_cast<const uint16_t*>(J.vs), J.cube, J.wsum, J.dtype == HCG_DTYPE_BF16 ? 1u : 0u,
                   J.normalize, J.nchan};
   if constexpr (ROUTE == kRouteFew)
@@ -170,12 +174,15 @@ __global__ void __launch_bounds__(ROUTE == kRouteOne4 ? 64 * kOneChannelStreams 
 int launch_batch_tiles(uint32_t route, const TileRange* ranges, uint32_t nranges, uint32_t blocks,
                        const MfmaJob* jobs, hipStream_t s) {
   if (nranges == 0 || blocks == 0) return HCG_OK;
-  if (route == kRouteOne4)
-    k_batch_tiles<kRouteOne4><<<blocks, 64 * kOneChannelStreams, 0, s>>>(ranges, nranges, jobs);
-  else if (route == kRouteOne1)
-    k_batch_tiles<kRouteOne1><<<blocks, 64, 0, s>>>(ranges, nranges, jobs);
-  else
-    k_batch_tiles<kRouteFew><<<blocks, 64, 0, s>>>(ranges, nranges, jobs);
+  constexpr uint32_t kThreads4 = 64 * kOneChannelStreams;
+  launch_runs(blocks, route == kRouteOne4 ? kThreads4 : 64, [&](uint32_t first, uint32_t count) {
+    if (route == kRouteOne4)
+      k_batch_tiles<kRouteOne4><<<count, kThreads4, 0, s>>>(ranges, nranges, jobs, first);
+    else if (route == kRouteOne1)
+      k_batch_tiles<kRouteOne1><<<count, 64, 0, s>>>(ranges, nranges, jobs, first);
+    else
+      k_batch_tiles<kRouteFew><<<count, 64, 0, s>>>(ranges, nranges, jobs, first);
+  });
   HCG_CHECK_LAUNCH("k_batch_tiles");
   return HCG_OK;
 }
@@ -183,11 +190,14 @@ int launch_batch_tiles(uint32_t route, const TileRange* ranges, uint32_t nranges
 template <int WMODE>
 static void launch_1ch(const GridParams& P, const GridBuffers& B, const TileOut& O, uint32_t tiles_x,
                        uint32_t tiles_y, hipStream_t s) {
-  if (one_channel_streams(P.side) == kOneChannelStreams)
-    k_grid_tiles_1ch<kOneChannelStreams, WMODE>
-        <<<tiles_x * tiles_y, 64 * kOneChannelStreams, 0, s>>>(P, B, O, tiles_x, tiles_y);
-  else
-    k_grid_tiles_1ch<1, WMODE><<<tiles_x * tiles_y, 64, 0, s>>>(P, B, O, tiles_x, tiles_y);
+  const bool several = one_channel_streams(P.side) == kOneChannelStreams;
+  const uint32_t threads = several ? 64 * kOneChannelStreams : 64;
+  launch_runs((uint64_t)tiles_x * tiles_y, threads, [&](uint32_t first, uint32_t count) {
+    if (several)
+      k_grid_tiles_1ch<kOneChannelStreams, WMODE><<<count, threads, 0, s>>>(P, B, O, tiles_x, tiles_y, first);
+    else
+      k_grid_tiles_1ch<1, WMODE><<<count, threads, 0, s>>>(P, B, O, tiles_x, tiles_y, first);
+  });
 }
 
 int launch_tiles_one_channel(const GridParams& P, const GridBuffers& B, const TileOut& O, hipStream_t s) {
@@ -205,7 +215,9 @@ int launch_tiles_one_channel(const GridParams& P, const GridBuffers& B, const Ti
 template <int KT, bool HAS_W, int WMODE, uint32_t S, int ROWS>
 static void launch_tiles_as(const GridParams& P, const GridBuffers& B, hipStream_t s) {
   const uint32_t tiles_x = tile_cols_of(P.side), tiles_y = (P.side + ROWS - 1) / ROWS;
-  k_grid_tiles<KT, HAS_W, WMODE, S, ROWS><<<tiles_x * tiles_y, 64 * S, 0, s>>>(P, B, tiles_x, tiles_y);
+  launch_runs((uint64_t)tiles_x * tiles_y, 64 * S, [&](uint32_t first, uint32_t count) {
+    k_grid_tiles<KT, HAS_W, WMODE, S, ROWS><<<count, 64 * S, 0, s>>>(P, B, tiles_x, tiles_y, first);
+  });
 }
 
 // Rows of a tile and waves per tile (each walking its share of the rings) by
