@@ -282,14 +282,17 @@ __device__ inline TileSpan tile_span(const GridParams& P, const Window& w, uint3
 //   sin^2(dl / 2) <= (sin^2(R / 2) - (dz / (2 max cos))^2) / (min cos bs min cos bc).
 // In half pixels of the ring a sample within reach of a cell at x = q2 tt has
 // its position within k sqrt(h2 - dz^2) of x, and none is where h2 <= dz^2.
-// Single precision: dz relative to a cell of the tile, and R widened by 1e-5;
-// the position of a sample at longitude x is within [x - 2, x + 3].
+// Single precision, relative to the tile's zref: R is widened by 1e-5, which
+// covers what is relative to dz, and the band by what rounding leaves of its
+// edges and of the cells' places (tiles may be far larger than the radius) and
+// by what the keys' own rounding does (pixel edges move by ~1e-15).  The
+// position of a sample at longitude x is within [x - 2, x + 3].
 struct RingChord {
   float zu, zd;  // the band, sin of latitude relative to the tile's zref
   float h2, k, q2;
 };
 // (half2d: sin^2(R / 2))
-__device__ inline RingChord ring_chord(double half2d, const TileSpan& T, uint32_t npr, uint32_t kr,
+__host__ __device__ inline RingChord ring_chord(double half2d, const TileSpan& T, uint32_t npr, uint32_t kr,
                                        uint32_t usedrings, const double* __restrict__ ring_z) {
   RingChord c;
   c.q2 = 0.5f * (float)npr;
@@ -302,11 +305,14 @@ __device__ inline RingChord ring_chord(double half2d, const TileSpan& T, uint32_
   const double zu = ring_z[kr - 1], zd = ring_z[kr + 1];
   c.zu = (float)(zu - T.zref);
   c.zd = (float)(zd - T.zref);
+  constexpr float kEps = 1.2e-7f;  // 2^-23: half an ulp of an edge and of a cell each, twice over
+  c.zu += fmaf(kEps, fabsf(c.zu) + T.zmax, 4e-15f);
+  c.zd -= fmaf(kEps, fabsf(c.zd) + T.zmax, 4e-15f);
   const float cu = (float)((1.0 - zu) * (1.0 + zu)), cd = (float)((1.0 - zd) * (1.0 + zd));  // cos^2
-  const float zlo = (float)T.zref, zhi = (float)T.zref + T.zmax;
+  const double zlo = T.zref, zhi = T.zref + (double)T.zmax;
   // the largest cos^2 between the band and the cells: 1 if they straddle the equator
-  float cmax2 = fmaxf(fmaxf(cu, cd), 1.f - fminf(zlo * zlo, zhi * zhi));
-  if (!((zd > 0.0 && zlo > 0.f) || (zu < 0.0 && zhi < 0.f))) cmax2 = 1.f;
+  float cmax2 = fmaxf(fmaxf(cu, cd), (float)(zlo > 0.0 ? (1.0 - zlo) * (1.0 + zlo) : (1.0 - zhi) * (1.0 + zhi)));
+  if (!((zd > 0.0 && zlo > 0.0) || (zu < 0.0 && zhi < 0.0))) cmax2 = 1.f;
   cmax2 = 4.00004f * cmax2;
   const float half2 = (float)half2d * (1.f + 1e-5f);
   const float cc = sqrtf(fminf(cu, cd)) * T.cmin * (1.f - 1e-5f);
@@ -318,8 +324,8 @@ __device__ inline RingChord ring_chord(double half2d, const TileSpan& T, uint32_
 }
 // Narrows the keys lp..rp of a ring (first pixel sp, npr pixels) to what the
 // radius reaches from the tile; false: nothing.
-__device__ inline bool chord_pixels(const TileSpan& T, const RingChord& c, uint32_t sp, uint32_t npr, uint32_t& lp,
-                                    uint32_t& rp) {
+__host__ __device__ inline bool chord_pixels(const TileSpan& T, const RingChord& c, uint32_t sp, uint32_t npr,
+                                             uint32_t& lp, uint32_t& rp) {
   const float dz = fmaxf(fmaxf(c.zd - T.zmax, T.zmin - c.zu), 0.f);
   const float num = fmaf(-dz, dz, c.h2);
   if (!(num > 0.f)) return false;
@@ -330,6 +336,34 @@ __device__ inline bool chord_pixels(const TileSpan& T, const RingChord& c, uint3
     rp = min(rp, sp + ((uint32_t)xh >> 1) + 1u);
   }
   return lp <= rp;
+}
+
+// What the radius reaches of a ring from one cell (zf: sin of its latitude
+// relative to zref, ttf: its longitude in units of pi/2): half-pixel positions
+// xl to xh, all of them if not narrow.
+struct CellReach {
+  bool any, narrow;
+  float xl, xh;
+};
+// (chord(&RingChord::m): the ring's m, read where it is used: read together, one
+// after the other, 20M samples take 1% longer)
+template <class F>
+__host__ __device__ inline CellReach chord_cell(const F& chord, float zf, float ttf) {
+  CellReach r;
+  const float q2 = chord(&RingChord::q2);
+  const float dz = fmaxf(fmaxf(chord(&RingChord::zd) - zf, zf - chord(&RingChord::zu)), 0.f);
+  const float num = fmaf(-dz, dz, chord(&RingChord::h2));
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float root = __builtin_amdgcn_sqrtf(fmaxf(num, 0.f));
+#else
+  const float root = sqrtf(fmaxf(num, 0.f));
+#endif
+  const float hc = fmaf(chord(&RingChord::k), root, 2.2f);
+  r.xl = fmaf(ttf, q2, -hc);
+  r.xh = fmaf(ttf, q2, hc + 2.f);
+  r.any = !(num <= 0.f);
+  r.narrow = r.xl >= 0.f && r.xh < 4.f * q2 - 4.f;
+  return r;
 }
 
 // A pixel range of ring r that holds every cell's window in it (ring_window):
@@ -806,18 +840,14 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
         // disc in every ring): the pass of 20M samples onto 2048^2 4.45 ->
         // 4.32 ms, a 5 sigma beam with weights onto 347^2 1.27 -> 1.19
         {
-          const auto of_ring = [&](float v) {
-            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), k));
+          const auto of_ring = [&](float RingChord::*m) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, chord_r.*m), k));
           };
-          const float q2 = of_ring(chord_r.q2);
-          const float dz = fmaxf(fmaxf(of_ring(chord_r.zd) - zf, zf - of_ring(chord_r.zu)), 0.f);
-          const float num = fmaf(-dz, dz, of_ring(chord_r.h2));
-          const float hc = fmaf(of_ring(chord_r.k), __builtin_amdgcn_sqrtf(fmaxf(num, 0.f)), 2.2f);
-          const float xl = fmaf(ttf, q2, -hc), xh = fmaf(ttf, q2, hc + 2.f);
-          act = act && !(num <= 0.f);
-          if (xl >= 0.f && xh < 4.f * q2 - 4.f) {
-            wl = max(wl, (uint32_t)xl);
-            wh = min(wh, (uint32_t)xh);
+          const CellReach reach = chord_cell(of_ring, zf, ttf);
+          act = act && reach.any;
+          if (reach.narrow) {
+            wl = max(wl, (uint32_t)reach.xl);
+            wh = min(wh, (uint32_t)reach.xh);
           }
           act = act && wl <= wh;
         }
