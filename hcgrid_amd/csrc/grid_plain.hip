@@ -231,7 +231,7 @@ static void launch_tiles_as(const GridParams& P, const GridBuffers& B, hipStream
 template <int KT, bool HAS_W, int WMODE>
 static void launch_tiles(const GridParams& P, const GridBuffers& B, uint32_t n, hipStream_t s) {
   // GAUSS2D's tangent frames take twelve registers a row: two rows
-  constexpr int R = KT == HCG_GAUSS2D && WMODE == 4 ? 2 : 4;
+  constexpr int R = KT == HCG_GAUSS2D && WMODE >= 4 ? 2 : 4;
   const uint32_t tiles = tile_count_of(P.side);
   if (tiles >= 4096 || (tiles >= 2048 && n < 256 * tiles))
     launch_tiles_as<KT, HAS_W, WMODE, 1, R>(P, B, s);
@@ -257,7 +257,10 @@ int launch_grid(const GridParams& P, const GridBuffers& B, uint32_t n, hipStream
     else
       launch_tiles<KT, HAS_W, 0>(P, B, n, s);
   } else if (frame_weight_ok(P, KT)) {
-    launch_tiles<KT, HAS_W, 4>(P, B, n, s);
+    if (KT != HCG_GAUSS2D || frame_weight_short(P))
+      launch_tiles<KT, HAS_W, 4>(P, B, n, s);
+    else if constexpr (KT == HCG_GAUSS2D)
+      launch_tiles<KT, HAS_W, 5>(P, B, n, s);
   } else {
     launch_tiles<KT, HAS_W, 0>(P, B, n, s);
   }

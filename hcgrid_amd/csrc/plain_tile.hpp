@@ -560,7 +560,8 @@ struct TileShared {
 
 // WMODE (GAUSS1D): 0 general exponent and exp; 1 gauss_small_radius; 2
 // gauss_tiny_radius; 3 also lean_weight_ok (the candidate test on p.q and
-// the lean weight).  The other kernels: 0 general, 4 frame_weight_ok.
+// the lean weight).  The other kernels: 0 general, 4 frame_weight_ok (5:
+// GAUSS2D and not frame_weight_short).
 // lds: CAP x (x, y, z, v doubles, key), with HAS_W then CAP weights; with NC
 // > 0 CAP x (x, y, z doubles, key, NC 16-bit values).
 // s_exp: the 64-entry exponential table (exp_table_load), visible to the wave.
@@ -599,7 +600,7 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
     for (int c = 0; c < (NC > 0 ? NC : 1); ++c) acc_c[r][c] = 0.f;
   }
   // GAUSS2D's tangent frames (WMODE 4): east and north turned by the position angle
-  constexpr bool kFrame = WMODE == 4 && KT == HCG_GAUSS2D;
+  constexpr bool kFrame = (WMODE == 4 || WMODE == 5) && KT == HCG_GAUSS2D;
   double fu[kFrame ? ROWS : 1][3], fv[kFrame ? ROWS : 1][3];
   Window win;
   double tl = 0.0, tr = 0.0;  // compat: the window's edges, fmodulo4 in units of pi/2
@@ -911,8 +912,9 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
               if constexpr (WMODE == 3)
                 wt = gauss_weight_lean(t, k0h, k1v, e3v, s_exp);
               else if constexpr (kFrame)
-                wt = gauss2d_frame_weight(P, t, fma(dx, fu[k][0], fma(dy, fu[k][1], dz * fu[k][2])),
-                                          fma(dx, fv[k][0], fma(dy, fv[k][1], dz * fv[k][2])), s_exp);
+                wt = gauss2d_frame_weight<WMODE == 5>(
+                    P, t, fma(dx, fu[k][0], fma(dy, fu[k][1], dz * fu[k][2])),
+                    fma(dx, fv[k][0], fma(dy, fv[k][1], dz * fv[k][2])), s_exp);
               else if constexpr (WMODE == 4)
                 wt = sinc_frame_weight(P, t, s_exp);
               else if constexpr (KT == HCG_GAUSS1D && WMODE > 0)
