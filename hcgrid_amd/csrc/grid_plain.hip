@@ -114,8 +114,12 @@ __global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(4))
 }
 
 // A few-channel job of the multi-channel entry points on the tile path: one
-// wave per tile (few_channel_tile_body).
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+// wave per tile (few_channel_tile_body).  Two waves per SIMD: with its sums and
+// values of eight channels the sample loop takes 208 registers (a grid pass of
+// 300k samples x 2 onto 2048^2 677 us so, 682 at three waves, 1440 at four,
+// where 113 registers spill; 20k x 8 onto 512^2 50, 63 and 99 us).
+constexpr int kFewWaves = 2;
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kFewWaves)))
     k_grid_tiles_few(GridParams P, GridBuffers B, TileOut O, uint32_t tiles_x, uint32_t tiles_y, uint32_t first) {
   __shared__ __attribute__((aligned(16))) char lds[kFewTileLdsBytes];
   __shared__ double s_exp[64];
@@ -139,7 +143,7 @@ int launch_tiles_few_channels(const GridParams& P, const GridBuffers& B, const T
 // job by binary search over the range starts and works one tile of it.
 template <uint32_t ROUTE>
 __global__ void __launch_bounds__(ROUTE == kRouteOne4 ? 64 * kOneChannelStreams : 64)
-    __attribute__((amdgpu_waves_per_eu(4)))
+    __attribute__((amdgpu_waves_per_eu(ROUTE == kRouteFew ? kFewWaves : 4)))
     k_batch_tiles(const TileRange* __restrict__ ranges, uint32_t nranges, const MfmaJob* __restrict__ jobs,
                   uint32_t first) {
   constexpr uint32_t S = ROUTE == kRouteOne4 ? kOneChannelStreams : 1;
