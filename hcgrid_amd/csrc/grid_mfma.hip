@@ -67,18 +67,45 @@ __device__ inline f32x4_t mfma16(bool bf, s16x8_t a, s16x8_t b, f32x4_t c) {
                                                 0, 0, 0);
 }
 
-// FP64 weight of a selected pair (the single-channel kernel's evaluation).
-__device__ inline double pair_weight_any(const GridParams& P, const GridBuffers& B, uint32_t kt, double c2,
-                                         const double* s_exp, uint32_t cell, uint32_t i) {
-  // GAUSS1D whose radius rules out the exponent's asin branch and the exp
-  // clamp (gauss_small_radius): the same values
-  if (kt == kKtGaussSmall || kt == kKtGaussLean) return exp_scaled_neg_nc(gauss_exponent_series(P, c2), s_exp);
+// FP64 weight of a selected pair by calls (the single-channel kernel's general evaluation).
+__device__ inline double pair_weight_call(const GridParams& P, const GridBuffers& B, uint32_t kt, double c2,
+                                          const double* s_exp, uint32_t cell, uint32_t i) {
   if (kt == HCG_GAUSS1D) return exp_scaled_neg(gauss_exponent_scaled(P, c2), s_exp);
   if (kt == HCG_GAUSS2D)
     return weight_general<HCG_GAUSS2D>(P.params[0], P.params[1], P.params[2], B.xwcs, B.ywcs, B.lon_s, B.lat_s,
                                        0.25 * c2, cell, i);
   return weight_general<HCG_TAPERED_SINC>(P.params[0], P.params[1], P.params[2], B.xwcs, B.ywcs, B.lon_s,
                                           B.lat_s, 0.25 * c2, cell, i);
+}
+
+// FP64 weights of two pairs from series (garbage where a pair is not selected):
+// (dx, dy, dz) = q - p, fu and fv the cell's tangent frame (kWeight2d).
+template <uint32_t WK>
+__device__ __forceinline__ void pair_weights_series(const GridParams& P, const double (&c2)[2], const double (&dx)[2],
+                                                    const double (&dy)[2], const double (&dz)[2],
+                                                    const double (&fu)[3], const double (&fv)[3],
+                                                    const double* s_exp, double (&wt)[2]) {
+  double y[2], amp[2] = {1.0, 1.0};
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    if constexpr (WK == kWeightSmall) {
+      y[e] = gauss_exponent_series(P, c2[e]);
+    } else if constexpr (WK == kWeight2d) {
+      const double U = fma(dx[e], fu[0], fma(dy[e], fu[1], dz[e] * fu[2]));
+      const double V = fma(dx[e], fv[0], fma(dy[e], fv[1], dz[e] * fv[2]));
+      y[e] = distance_series<true>(c2[e]) * fma(P.f[0] * U, U, (P.f[1] * V) * V);
+    } else {
+      const double d2 = c2[e] * distance_series<false>(c2[e]);
+      y[e] = (WK == kWeightSinc ? P.f[1] : P.k0) * d2;
+      if constexpr (WK == kWeightSinc) amp[e] = sinc_triple(P.f[0] * d2);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    // (kWeightSmall's exponents are above the clamp)
+    wt[e] = WK == kWeightSmall ? exp_scaled_neg_fold(y[e], s_exp) : exp_scaled_neg(y[e], s_exp);
+    if constexpr (WK == kWeightSinc) wt[e] *= amp[e];
+  }
 }
 
 // The tested distance of a pair: h = 1 - p.q (LEAN), or c2 = |p - q|^2 (np = -p).
@@ -125,9 +152,10 @@ constexpr uint32_t kNoRingLane = 255;        // the ring lane of a block list's 
 constexpr uint32_t kNoSample = 0x40000000u;  // half-pixel position that no window holds
 
 // NS staged samples.
-template <uint32_t NS>
+template <uint32_t NS, uint32_t WK>
 struct Staged {
   __attribute__((aligned(16))) double x[NS], y[NS], z[NS];
+  __attribute__((aligned(16))) double w[WK == kWeightLean ? 2 : NS];  // sample weights
   __attribute__((aligned(16))) uint32_t g[NS];  // half-pixel positions
 };
 
@@ -153,15 +181,24 @@ struct MfmaCells {
   uint8_t belt[kMcCols];                          // it holds
 };
 
+// The cells' tangent frames (kWeight2d): east and north turned by the position angle.
+template <uint32_t WK>
+struct MfmaFrames {
+  double u[3][WK == kWeight2d ? kMcCols : 1], v[3][WK == kWeight2d ? kMcCols : 1];
+};
+
 // One wave's LDS: a staged k-block and its list.
+template <uint32_t WK>
 struct MfmaWave {
-  Staged<32> st;
+  Staged<32, WK> st;
   BlockList<128> bl;
 };
+template <uint32_t WK>
 union MfmaLds {
   struct {
-    MfmaWave w[kMcWaves];
+    MfmaWave<WK> w[kMcWaves];
     MfmaCells c;
+    MfmaFrames<WK> f;
   } s;
   float t[kMcCols * 64];  // the epilogue's 64 channels x 64 cells
 };
@@ -264,6 +301,26 @@ __device__ __forceinline__ void put_cell(MfmaCells& C, uint32_t i, const CellGeo
   C.wlo[i] = g.wlo;
   C.wwid[i] = g.wwid;
   C.belt[i] = g.belt;
+}
+
+// Lane = cell of the block, as block_cell.
+template <uint32_t WK>
+__device__ __forceinline__ void put_frames(const MfmaJob& J, MfmaFrames<WK>& F, uint32_t y0, uint32_t x0) {
+  if constexpr (WK == kWeight2d) {
+    const GridParams& P = J.P;
+    const uint32_t lane = __lane_id();
+    const uint32_t row = min(y0 + (lane >> J.tc_shift), P.side - 1);
+    const uint32_t col = min(x0 + (lane & ((1u << J.tc_shift) - 1u)), P.side - 1);
+    double sl, cl, sb, cb;
+    sincos(J.B.xwcs[row * P.side + col] * kDeg2Rad, &sl, &cl);
+    sincos(J.B.ywcs[row * P.side + col] * kDeg2Rad, &sb, &cb);
+    const double e[3] = {-sl, cl, 0.0}, nn[3] = {-sb * cl, -sb * sl, cb};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      F.u[i][lane] = fma(e[i], P.f[2], -(nn[i] * P.f[3]));
+      F.v[i][lane] = fma(nn[i], P.f[2], e[i] * P.f[3]);
+    }
+  }
 }
 
 // The span of the wave's cells.
@@ -393,40 +450,46 @@ __device__ __forceinline__ void list_blocks(BlockList<NL>& L, uint32_t q0, uint3
   }
 }
 
-// Sample s of k-block u of the list, half of it a lane: half 0 its x and y,
-// half 1 its z and position; in flight from fetch to store.
+// Sample s of k-block u of the list, half of it a lane: half 0 its x, y and
+// sample weight (if there are any), half 1 its z and position; in flight from
+// fetch to store.
+template <uint32_t WK>
 struct StageRegs {
-  double v0, v1;
+  double v0, v1, w;
   uint32_t pos;
   template <uint32_t NL>
   __device__ __forceinline__ void fetch(const GridBuffers& B, const hcg_ring_meta& m, const BlockList<NL>& L,
                                         uint32_t u, uint32_t s, uint32_t half) {
     const uint32_t q = u * 4 + (s >> 3);
     const uint32_t i = L.lb[q] * kVB + (s & 7u), rl = L.lr[q];
-    v0 = v1 = 0.0;
+    v0 = v1 = w = 0.0;
     pos = kNoSample;
     if (rl != kNoRingLane && i < m.n) {
       const double* r = &B.rec[i].x + 2 * half;
       v0 = r[0];
       v1 = r[1];
       if (half) pos = 2u * B.keys[i] + L.gc[rl];
+      if constexpr (WK != kWeightLean)
+        if (B.w_s && !half) w = B.w_s[i];
     }
   }
   template <uint32_t NS>
-  __device__ __forceinline__ void store(Staged<NS>& S, uint32_t p, uint32_t half) const {
+  __device__ __forceinline__ void store(Staged<NS, WK>& S, uint32_t p, uint32_t half) const {
     if (half) {
       S.z[p] = v0;
       S.g[p] = pos;
     } else {
       S.x[p] = v0;
       S.y[p] = v1;
+      if constexpr (WK != kWeightLean) S.w[p] = w;
     }
   }
 };
 
 // One lane's cell of a square, and the constants of the weights.
-template <bool LEAN>
+template <uint32_t WK>
 struct SquareCell {
+  static constexpr bool LEAN = WK == kWeightLean;
   double npx, npy, npz;
   uint32_t uring, dring, wlo, wwid;
   double h_hi, h_lo, k0h, k1v, e3v;
@@ -484,13 +547,22 @@ struct WeightOperand {
 // takes cell l % 16 and samples 8 (l / 16) .. + 7 (of value block blk), which
 // is the layout of an MFMA operand.  Returns the lanes with a selected pair;
 // guard: those with one within rounding of the radius (kept here).
-template <int DT, bool LEAN, uint32_t NS>
-__device__ __forceinline__ uint64_t weigh_kblock(const MfmaJob& J, SquareCell<LEAN>& Q, const Staged<NS>& S,
-                                                 uint32_t at, uint32_t wl, uint32_t ww, uint32_t cell, uint32_t blk,
-                                                 const double* s_exp, WeightOperand& A, uint64_t& guard) {
-  constexpr bool bf = DT == kDtBf16;
+template <int DT, uint32_t WK, uint32_t NS>
+__device__ __forceinline__ uint64_t weigh_kblock(const MfmaJob& J, SquareCell<WK>& Q, const Staged<NS, WK>& S,
+                                                 const MfmaFrames<WK>& F, uint32_t at, uint32_t wl, uint32_t ww,
+                                                 uint32_t cell, uint32_t blk, const double* s_exp, WeightOperand& A,
+                                                 uint64_t& guard) {
+  constexpr bool bf = DT == kDtBf16, LEAN = WK == kWeightLean;
   uint64_t any = 0;
   guard = 0;
+  double fu[3] = {0.0, 0.0, 0.0}, fv[3] = {0.0, 0.0, 0.0};
+  if constexpr (WK == kWeight2d) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      fu[i] = F.u[i][Q.cb];
+      fv[i] = F.v[i][Q.cb];
+    }
+  }
 #pragma unroll
   for (uint32_t hf = 0; hf < 2; ++hf) {  // four samples at a time
     const uint32_t j0 = at + (__lane_id() >> 4) * 8 + hf * 4;
@@ -508,6 +580,9 @@ __device__ __forceinline__ uint64_t weigh_kblock(const MfmaJob& J, SquareCell<LE
       guard |= sel[e] & __builtin_amdgcn_ballot_w64(!(t[e] < Q.h_lo));
     }
     any |= (sel[0] | sel[1]) | (sel[2] | sel[3]);
+    double qw[4] = {1.0, 1.0, 1.0, 1.0};
+    if constexpr (!LEAN)
+      if (J.B.w_s) lds_read4(&S.w[j0], qw);  // uniform
 #pragma unroll
     for (uint32_t k = 0; k < 2; ++k) {
       const uint32_t jj = hf * 2 + k;
@@ -518,13 +593,22 @@ __device__ __forceinline__ uint64_t weigh_kblock(const MfmaJob& J, SquareCell<LE
       double wt[2] = {0.0, 0.0};
       if constexpr (LEAN) {
         gauss_weight_lean2(t[2 * k], t[2 * k + 1], Q.k0h, Q.k1v, Q.e3v, s_exp, wt);
+      } else if constexpr (WK != kWeightCall) {
+        const double c2[2] = {t[2 * k], t[2 * k + 1]};
+        const double dx[2] = {Q.npx + qx[2 * k], Q.npx + qx[2 * k + 1]};
+        const double dy[2] = {Q.npy + qy[2 * k], Q.npy + qy[2 * k + 1]};
+        const double dz[2] = {Q.npz + qz[2 * k], Q.npz + qz[2 * k + 1]};
+        pair_weights_series<WK>(J.P, c2, dx, dy, dz, fu, fv, s_exp, wt);
+        if (J.B.w_s) {  // uniform
+          wt[0] *= qw[2 * k];
+          wt[1] *= qw[2 * k + 1];
+        }
       } else {
 #pragma unroll
         for (uint32_t e = 0; e < 2; ++e)
           if (__builtin_amdgcn_inverse_ballot_w64(sel[2 * k + e])) {
-            const uint32_t isrc = blk * kVB + jj * 2 + e;
-            wt[e] = pair_weight_any(J.P, J.B, J.kt, t[2 * k + e], s_exp, cell, isrc);
-            if (J.B.w_s) wt[e] *= J.B.w_s[isrc];
+            wt[e] = pair_weight_call(J.P, J.B, J.kt, t[2 * k + e], s_exp, cell, blk * kVB + jj * 2 + e);
+            if (J.B.w_s) wt[e] *= qw[2 * k + e];
           }
       }
       const f32x2_t wf = {__builtin_amdgcn_inverse_ballot_w64(sel[2 * k]) ? (float)wt[0] : 0.f,
@@ -547,11 +631,11 @@ __device__ __forceinline__ uint64_t weigh_kblock(const MfmaJob& J, SquareCell<LE
 // a pair that it rejects is taken out again.  A lean weight is subtracted from
 // the sum, exactly; with the general weights, which may be infinite or NaN by
 // the sample's, the sum starts again from wsum0, its value before the k-block.
-template <int DT, bool LEAN, uint32_t NS>
-__device__ __forceinline__ void guard_kblock(const MfmaJob& J, SquareCell<LEAN>& Q, const Staged<NS>& S, uint32_t at,
-                                             uint32_t wl, uint32_t ww, uint32_t cell, uint32_t blk, double wsum0,
+template <int DT, uint32_t WK, uint32_t NS>
+__device__ __forceinline__ void guard_kblock(const MfmaJob& J, SquareCell<WK>& Q, const Staged<NS, WK>& S,
+                                             uint32_t at, uint32_t wl, uint32_t ww, uint32_t cell, uint32_t blk, double wsum0,
                                              WeightOperand& A) {
-  constexpr bool bf = DT == kDtBf16;
+  constexpr bool bf = DT == kDtBf16, LEAN = WK == kWeightLean;
 #pragma unroll 1
   for (uint32_t e = 0; e < 8; ++e) {
     const uint32_t j = at + (__lane_id() >> 4) * 8 + e;
@@ -623,9 +707,9 @@ __device__ __forceinline__ const char* value_rows(const MfmaJob& J, uint32_t ch_
 
 // One block of 64 cells and up to 16 NB channels (group `group` of them): a
 // wave takes a square of 16 cells, on its own but for the set-up and the
-// stores.  LEAN: GAUSS1D at lean_weight_ok radii without sample weights.
-template <int DT, int NB, bool LEAN>
-__device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint32_t group, MfmaLds& lds,
+// stores.  WK: mfma_weight_kind.
+template <int DT, int NB, uint32_t WK>
+__device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint32_t group, MfmaLds<WK>& lds,
                                           const double* s_exp) {
   constexpr bool bf = DT == kDtBf16;
   const GridParams& P = J.P;
@@ -634,13 +718,15 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
   const hcg_ring_meta m = *B.meta;
   const uint32_t y0 = (tile / J.tiles_x) << (6u - J.tc_shift), x0 = (tile % J.tiles_x) << J.tc_shift;
   MfmaCells& C = lds.s.c;
-  MfmaWave& W = lds.s.w[wave];
+  MfmaWave<WK>& W = lds.s.w[wave];
   const Squares sq(J.tc_shift);
 
   if (wave == 0) {
     bool lv;
     const CellGeom g = block_cell(P, B, m, y0, x0, J.tc_shift, lv);
     put_cell(C, lane, g);
+  } else if (wave == 1) {
+    put_frames(J, lds.s.f, y0, x0);
   }
   __syncthreads();
   const uint32_t cb = sq.cell(wave, lane & 15u);
@@ -648,7 +734,7 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
   const bool live = crow < P.side && ccol < P.side;
   const uint32_t cell = live ? crow * P.side + ccol : 0;
   uint32_t r_begin, r_end;
-  SquareCell<LEAN> Q;
+  SquareCell<WK> Q;
   {
     CellGeom g;
     g.win = C.win[cb];
@@ -679,7 +765,7 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
       tile_sync();
       list_blocks(W.bl, q0, cnt);
       tile_sync();
-      StageRegs st;
+      StageRegs<WK> st;
       st.fetch(B, m, W.bl, 0, lane & 31u, lane >> 5);
       for (uint32_t u = 0; u < nkb; ++u) {
         tile_sync();  // the previous k-block is consumed
@@ -699,7 +785,7 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
         WeightOperand A;
         uint64_t guard;
         const double wsum0 = Q.wsum;
-        const uint64_t any = weigh_kblock<DT>(J, Q, W.st, 0, wl, ww, cell, blk, s_exp, A, guard);
+        const uint64_t any = weigh_kblock<DT>(J, Q, W.st, lds.s.f, 0, wl, ww, cell, blk, s_exp, A, guard);
         if (guard) {  // uniform, rare
           // the sums wait in scratch memory meanwhile (volatile: here and only
           // here), and the channel values are read again: across the call they
@@ -780,13 +866,15 @@ __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint3
 // channel values of two k-blocks are read when the two before are done with,
 // and arrive while weights are evaluated.
 constexpr uint32_t kWideList = 256;
+template <uint32_t WK>
 union MfmaWideLds {
   struct {
     s16x8_t a[2][4][4][2][64];  // [round parity][k-block][square][hi, lo][lane]
     uint32_t any[2][4][4];      // the operand holds a weight
-    Staged<128> st[2];
+    Staged<128, WK> st[2];
     BlockList<kWideList> bl;
     MfmaCells c;
+    MfmaFrames<WK> f;
     double wsum[kWideWaves][16];
     double inv[kMcCols];
     uint32_t total;
@@ -794,8 +882,8 @@ union MfmaWideLds {
   float t[kWideWaves][16 * 64];  // the epilogue's 16 channels x 64 cells of a wave
 };
 
-template <int DT, bool LEAN>
-__device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint32_t group, MfmaWideLds& lds,
+template <int DT, uint32_t WK>
+__device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint32_t group, MfmaWideLds<WK>& lds,
                                           const double* s_exp) {
   constexpr bool bf = DT == kDtBf16;
   const GridParams& P = J.P;
@@ -832,6 +920,7 @@ __device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint3
     const BlockSpan S = cells_span(P, m, g);
     if (lane == 0) L.span = S;
   }
+  if (wave == 6) put_frames(J, lds.s.f, y0, x0);
   __syncthreads();
   const uint32_t cb = sq.cell(mb_own, lane & 15u);
   const uint32_t crow = y0 + (cb >> J.tc_shift), ccol = x0 + (cb & ((1u << J.tc_shift) - 1u));
@@ -839,7 +928,7 @@ __device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint3
   const uint32_t cell = live ? crow * P.side + ccol : 0;
   const uint32_t r_begin = __builtin_amdgcn_readfirstlane(L.span.T.r_begin);
   const uint32_t r_end = __builtin_amdgcn_readfirstlane(L.span.T.r_end);
-  SquareCell<LEAN> Q;
+  SquareCell<WK> Q;
   Q.init(P, C, cb, __builtin_amdgcn_readfirstlane((uint32_t)L.span.simple) != 0);
   const uint32_t ch_base = (group * kWideWaves + wave) * 64u;
   const bool mine = ch_base < J.nchan;  // uniform: the wave has channels
@@ -866,7 +955,7 @@ __device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint3
       __syncthreads();
       // waves 0 to 3 stage the 128 samples of round r (a k-block past the
       // last is neither staged nor weighed)
-      StageRegs st;
+      StageRegs<WK> st;
       const uint32_t ssp = (wave & 1u) * 64 + lane;  // sample of a round
       auto fetch = [&](uint32_t r) {
         if (wave < 4 && 4 * r + (ssp >> 5) < nkb) st.fetch(B, m, L, 4 * r + (ssp >> 5), ssp & 31u, wave >> 1);
@@ -894,7 +983,7 @@ __device__ __forceinline__ void mfma_wide(const MfmaJob& J, uint32_t tile, uint3
           WeightOperand A;
           uint64_t guard;
           const double wsum0 = Q.wsum;
-          any = weigh_kblock<DT>(J, Q, lds.s.st[par], k * 32, wl, ww, cell, blk, s_exp, A, guard);
+          any = weigh_kblock<DT>(J, Q, lds.s.st[par], lds.s.f, k * 32, wl, ww, cell, blk, s_exp, A, guard);
           if (guard) {  // uniform, rare; the sums wait in scratch memory (see mfma_tile)
             volatile float keep[64];
 #pragma unroll
@@ -1026,42 +1115,42 @@ __device__ inline uint32_t block_tile(uint32_t b, uint32_t ntiles, uint32_t tile
 }
 
 // The kernel instances: NB 16-channel blocks per wave (mfma_tile), or 0: mfma_wide.
-constexpr int mfma_waves_per_simd(int nb, bool lean) {
-  return !lean || nb == 0 ? 2 : nb <= 2 ? 4 : nb <= 6 ? 3 : 2;
+constexpr int mfma_waves_per_simd(int nb, uint32_t kind) {
+  return kind != kWeightLean || nb == 0 ? 2 : nb <= 2 ? 4 : nb <= 6 ? 3 : 2;
 }
 constexpr uint32_t mfma_threads(int nb) { return 64 * (nb == 0 ? kWideWaves : (uint32_t)kMcWaves); }
-template <int NB>
+template <int NB, uint32_t WK>
 struct InstanceLds {
-  typedef MfmaLds type;
+  typedef MfmaLds<WK> type;
 };
-template <>
-struct InstanceLds<0> {
-  typedef MfmaWideLds type;
+template <uint32_t WK>
+struct InstanceLds<0, WK> {
+  typedef MfmaWideLds<WK> type;
 };
-template <int DT, int NB, bool LEAN>
+template <int DT, int NB, uint32_t WK>
 __device__ __forceinline__ void mfma_work(const MfmaJob& J, uint32_t tile, uint32_t group) {
-  __shared__ typename InstanceLds<NB>::type lds;
+  __shared__ typename InstanceLds<NB, WK>::type lds;
   __shared__ double s_exp[64];
   if (threadIdx.x < 64) exp_table_load(s_exp);
   if constexpr (NB == 0)
-    mfma_wide<DT, LEAN>(J, tile, group, lds, s_exp);
+    mfma_wide<DT, WK>(J, tile, group, lds, s_exp);
   else
-    mfma_tile<DT, NB, LEAN>(J, tile, group, lds, s_exp);
+    mfma_tile<DT, NB, WK>(J, tile, group, lds, s_exp);
 }
 
 // One job: grid = (tile_blocks, or a run of them from `first` on, channel groups).
-template <int DT, int NB, bool LEAN>
-__global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, LEAN))))
+template <int DT, int NB, uint32_t WK>
+__global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, WK))))
     k_grid_mfma(MfmaJob J, uint32_t first) {
   const uint32_t tile = block_tile(first + blockIdx.x, J.ntiles, J.tiles_x, NB == 0);
   if (tile >= J.ntiles) return;  // uniform
-  mfma_work<DT, NB, LEAN>(J, tile, blockIdx.y);
+  mfma_work<DT, NB, WK>(J, tile, blockIdx.y);
 }
 
 // The jobs of a batch that one instance serves, in one launch: a workgroup
 // finds its job by binary search over the range starts (multiples of 8).
-template <int DT, int NB, bool LEAN>
-__global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, LEAN))))
+template <int DT, int NB, uint32_t WK>
+__global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_simd(NB, WK))))
     k_grid_mfma_batch(const TileRange* __restrict__ ranges, uint32_t nranges, const MfmaJob* __restrict__ jobs,
                       uint32_t first) {
   const uint32_t block = first + blockIdx.x;
@@ -1077,14 +1166,14 @@ __global__ void __launch_bounds__(mfma_threads(NB)) __attribute__((amdgpu_waves_
   const uint32_t lb = block - ranges[lo].first, per = tile_blocks(J.ntiles, J.tiles_x, NB == 0);
   const uint32_t tile = block_tile(lb % per, J.ntiles, J.tiles_x, NB == 0), group = lb / per;
   if (tile >= J.ntiles) return;  // uniform
-  mfma_work<DT, NB, LEAN>(J, tile, group);
+  mfma_work<DT, NB, WK>(J, tile, group);
 }
 
 // The instance of a job: its form (mfma_form) and value type.
-static uint32_t nb_of_instance(uint32_t inst) { return nb_of_form(inst / 2); }
+static uint32_t nb_of_instance(uint32_t inst) { return kFormNb[inst / 2]; }
 bool mfma_uses_plan(uint32_t inst) { return nb_of_instance(inst) == 0; }
 uint32_t mfma_instance(const MfmaJob& J) {
-  return 2 * mfma_form(J.nchan, J.kt == kKtGaussLean && !J.B.w_s) + (J.dtype == HCG_DTYPE_BF16 ? 0u : 1u);
+  return 2 * mfma_form(J.nchan, mfma_weight_kind(J.kt, J.B.w_s != nullptr)) + (J.dtype == HCG_DTYPE_BF16 ? 0u : 1u);
 }
 static uint32_t mfma_groups(const MfmaJob& J, uint32_t inst) {
   const uint32_t nb = nb_of_instance(inst);
@@ -1095,13 +1184,16 @@ uint64_t mfma_blocks(const MfmaJob& J) {
   return (uint64_t)tile_blocks(J.ntiles, J.tiles_x, nb_of_instance(inst) == 0) * mfma_groups(J, inst);
 }
 
-#define HCG_MFMA_PAIR(X, I, NB, LEAN) X(2 * (I), kDtBf16, NB, LEAN) X(2 * (I) + 1, kDtF16, NB, LEAN)
-#define HCG_MFMA_INSTANCES(X)                                                                               \
-  HCG_MFMA_PAIR(X, 0, kNbOf[0], true) HCG_MFMA_PAIR(X, 1, kNbOf[1], true) HCG_MFMA_PAIR(X, 2, kNbOf[2], true) \
-  HCG_MFMA_PAIR(X, 3, kNbOf[3], true) HCG_MFMA_PAIR(X, 4, kNbOf[4], true) HCG_MFMA_PAIR(X, 5, kNbOf[5], true) \
-  HCG_MFMA_PAIR(X, 6, kNbOf[6], true) HCG_MFMA_PAIR(X, 7, kNbOf[7], true)                                     \
-  HCG_MFMA_PAIR(X, kNbs, kNbOf[kGeneral[0]], false) HCG_MFMA_PAIR(X, kNbs + 1, kNbOf[kGeneral[1]], false)     \
-  HCG_MFMA_PAIR(X, kNbs + 2, kNbOf[kGeneral[2]], false)
+#define HCG_MFMA_FORM(X, I)                                \
+  X(2 * (I), kDtBf16, (int)kFormNb[I], kind_of_form(I)) \
+  X(2 * (I) + 1, kDtF16, (int)kFormNb[I], kind_of_form(I))
+#define HCG_MFMA_INSTANCES(X)                                                                              \
+  HCG_MFMA_FORM(X, 0) HCG_MFMA_FORM(X, 1) HCG_MFMA_FORM(X, 2) HCG_MFMA_FORM(X, 3) HCG_MFMA_FORM(X, 4)      \
+  HCG_MFMA_FORM(X, 5) HCG_MFMA_FORM(X, 6) HCG_MFMA_FORM(X, 7) HCG_MFMA_FORM(X, 8) HCG_MFMA_FORM(X, 9)      \
+  HCG_MFMA_FORM(X, 10) HCG_MFMA_FORM(X, 11) HCG_MFMA_FORM(X, 12) HCG_MFMA_FORM(X, 13) HCG_MFMA_FORM(X, 14) \
+  HCG_MFMA_FORM(X, 15) HCG_MFMA_FORM(X, 16) HCG_MFMA_FORM(X, 17) HCG_MFMA_FORM(X, 18) HCG_MFMA_FORM(X, 19) \
+  HCG_MFMA_FORM(X, 20) HCG_MFMA_FORM(X, 21) HCG_MFMA_FORM(X, 22) HCG_MFMA_FORM(X, 23) HCG_MFMA_FORM(X, 24) \
+  HCG_MFMA_FORM(X, 25) HCG_MFMA_FORM(X, 26) HCG_MFMA_FORM(X, 27) HCG_MFMA_FORM(X, 28) HCG_MFMA_FORM(X, 29)
 
 static int launch_mfma_job(const MfmaJob& J, hipStream_t s) {
   const uint32_t inst = mfma_instance(J);
@@ -1111,8 +1203,8 @@ static int launch_mfma_job(const MfmaJob& J, hipStream_t s) {
     HCG_CHECK_LAUNCH("k_mfma_plan");
   }
   launch_runs(tile_blocks(J.ntiles, J.tiles_x, nb == 0), mfma_threads(nb), [&](uint32_t first, uint32_t count) {
-#define HCG_CASE(I, DT, NB, LEAN) \
-  case I: k_grid_mfma<DT, NB, LEAN><<<dim3(count, groups), mfma_threads(NB), 0, s>>>(J, first); break;
+#define HCG_CASE(I, DT, NB, WK) \
+  case I: k_grid_mfma<DT, NB, WK><<<dim3(count, groups), mfma_threads(NB), 0, s>>>(J, first); break;
     switch (inst) { HCG_MFMA_INSTANCES(HCG_CASE) }
 #undef HCG_CASE
   });
@@ -1124,9 +1216,9 @@ int launch_mfma_batch(uint32_t inst, const TileRange* ranges, uint32_t nranges, 
                       hipStream_t s) {
   if (nranges == 0 || blocks == 0) return HCG_OK;
   launch_runs(blocks, mfma_threads(nb_of_instance(inst)), [&](uint32_t first, uint32_t count) {
-#define HCG_CASE(I, DT, NB, LEAN)                                                                             \
+#define HCG_CASE(I, DT, NB, WK)                                                                             \
   case I:                                                                                                     \
-    k_grid_mfma_batch<DT, NB, LEAN><<<count, mfma_threads(NB), 0, s>>>(ranges, nranges, jobs, first); break;
+    k_grid_mfma_batch<DT, NB, WK><<<count, mfma_threads(NB), 0, s>>>(ranges, nranges, jobs, first); break;
     switch (inst) { HCG_MFMA_INSTANCES(HCG_CASE) }
 #undef HCG_CASE
   });

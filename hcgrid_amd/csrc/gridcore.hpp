@@ -411,6 +411,41 @@ inline bool frame_weight_ok(const GridParams& P, uint32_t kernel_type) {
   return kernel_type == HCG_TAPERED_SINC && P.f[0] * d2 <= kSincMaxX2 && P.f[1] * d2 < 60000.0;
 }
 
+// Longer series, for radii up to ~9.9 deg (c2 < kSeriesMaxC2): d^2 / c2 =
+// 4 asin^2(sqrt(c2)/2) / c2 = sum of 2 c2^(n-1) / (n^2 C(2n, n)), and d^2 / sin^2 d,
+// which is that over 1 - c2/4; what is left out is below 1e-16.
+constexpr double kSeriesMaxC2 = 0.03;
+inline bool frame_finite(const GridParams& P) {
+  return fabs(P.f[0]) < 1e300 && fabs(P.f[1]) < 1e300 && fabs(P.f[2]) <= 1.0 && fabs(P.f[3]) <= 1.0;
+}
+template <bool OVER_SIN2>
+__host__ __device__ inline double distance_series(double c2) {
+  constexpr int N = OVER_SIN2 ? 8 : 7;
+  double s[N];  // folded at compile time
+  s[0] = 1.0;
+#pragma unroll
+  for (int n = 1; n < N; ++n) {  // 2 / (m^2 C(2m, m)), m = n + 1, from that of n
+    s[n] = s[n - 1] * (double)(n * n) / (double)((n + 1) * (2 * n + 1) * 2);
+  }
+  if constexpr (OVER_SIN2) {
+#pragma unroll
+    for (int n = 1; n < N; ++n) s[n] += 0.25 * s[n - 1];
+  }
+  double r = s[N - 1];
+#pragma unroll
+  for (int n = N - 2; n >= 0; --n) r = fma(c2, r, s[n]);
+  return r;
+}
+
+// sin(x) / x from x^2 <= 9 kSincMaxX2 by the triple angle: sin 3y = sin y (3 - 4 sin^2 y).
+inline bool sinc_triple_ok(const GridParams& P, double d2) {
+  return P.f[0] * d2 <= 9.0 * kSincMaxX2 && P.f[1] * d2 < 60000.0;
+}
+__device__ inline double sinc_triple(double x2) {
+  const double y2 = x2 * (1.0 / 9.0), s = sinc_series(y2);
+  return s * fma(-4.0 / 3.0 * y2, s * s, 1.0);
+}
+
 // GAUSS2D: radii (below ~0.26 deg) where the shorter series does: a pass of
 // 270k samples onto 300^2 takes 255 us with it and 276 with the longer one.
 inline bool frame_weight_short(const GridParams& P) { return P.c_hi < 2e-5; }

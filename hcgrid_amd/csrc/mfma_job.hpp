@@ -16,17 +16,51 @@ constexpr int kMcWaves = 4;                   // waves per workgroup, 16 cells e
 
 constexpr size_t kPlanBytes = 3600;  // a block's plan (MfmaPlan), as hcg_grid_mfma_workspace_size documents
 
-// The weight form of a job (MfmaJob::kt): the kernel type, or
-// kKtGaussSmall (GAUSS1D whose radius rules out the exponent's asin branch
-// and the exp clamp, gauss_small_radius), or kKtGaussLean (also
+// The weight form of a job (MfmaJob::kt): the kernel type for the general
+// evaluation (which calls asin, atan2, sin and exp), or one of the forms without
+// such calls: kKtGaussSmall (GAUSS1D, gauss_small_radius), kKtGaussLean (also
 // lean_weight_ok: the p.q candidate test and gauss_weight_lean of the tile
-// loop).
+// loop), and for radii below ~9.9 deg, from longer series than the tile loop's,
+// kKtGaussSeries (GAUSS1D), kKtFrame2d (GAUSS2D) and kKtSincSeries
+// (TAPERED_SINC, sinc_triple_ok).
 constexpr uint32_t kKtGaussSmall = HCG_GAUSS1D + 16u;
 constexpr uint32_t kKtGaussLean = HCG_GAUSS1D + 32u;
+constexpr uint32_t kKtGaussSeries = HCG_GAUSS1D + 48u;
+constexpr uint32_t kKtFrame2d = HCG_GAUSS2D + 48u;
+constexpr uint32_t kKtSincSeries = HCG_TAPERED_SINC + 48u;
 
 inline uint32_t mfma_weight_form(const GridParams& P, int kernel_type) {
-  if (kernel_type != HCG_GAUSS1D || !gauss_small_radius(P)) return (uint32_t)kernel_type;
-  return lean_weight_ok(P) ? kKtGaussLean : kKtGaussSmall;
+  if (kernel_type == HCG_GAUSS1D && gauss_small_radius(P)) return lean_weight_ok(P) ? kKtGaussLean : kKtGaussSmall;
+  if (!(P.c_hi < kSeriesMaxC2)) return (uint32_t)kernel_type;
+  if (kernel_type == HCG_GAUSS1D) return kKtGaussSeries;
+  if (kernel_type == HCG_GAUSS2D) return frame_finite(P) ? kKtFrame2d : (uint32_t)kernel_type;
+  return sinc_triple_ok(P, P.c_hi * 1.003) ? kKtSincSeries : (uint32_t)kernel_type;
+}
+
+// How the contraction evaluates a job's weights: the lean weight (no sample
+// weights), from series (one kind for each: merged, their constants alone fill
+// the scalar registers), or by calls.  A call's clobbered registers cost the
+// many-channel kernel 46 spills around it, and the transcendental functions
+// themselves several times a series: 1M samples onto 512^2 with GAUSS2D, 64
+// channels, 6.62 ms by calls and 0.78 by series; 300 channels 12.3 and 1.72.
+enum : uint32_t {
+  kWeightLean = 0,
+  kWeightSmall = 1,   // kKtGaussSmall, and kKtGaussLean with sample weights
+  kWeightSeries = 2,  // kKtGaussSeries
+  kWeight2d = 3,      // kKtFrame2d
+  kWeightSinc = 4,    // kKtSincSeries
+  kWeightCall = 5,
+  kWeightKinds = 6
+};
+inline uint32_t mfma_weight_kind(uint32_t kt, bool weighted) {
+  switch (kt) {
+    case kKtGaussLean: return weighted ? kWeightSmall : kWeightLean;
+    case kKtGaussSmall: return kWeightSmall;
+    case kKtGaussSeries: return kWeightSeries;
+    case kKtFrame2d: return kWeight2d;
+    case kKtSincSeries: return kWeightSinc;
+    default: return kWeightCall;
+  }
 }
 
 // One multi-channel job: geometry, sorted channel values and outputs, with
@@ -48,50 +82,49 @@ struct MfmaJob {
 // batch, contraction jobs are told apart by their kernel instance too
 // (kRouteMfma + mfma_instance).
 enum : uint32_t { kRouteOne4 = 0, kRouteOne1 = 1, kRouteFew = 2, kRouteMfma = 3 };
-constexpr uint32_t kMfmaInstances = 22, kRoutes = kRouteMfma + kMfmaInstances;
+constexpr uint32_t kMfmaInstances = 60, kRoutes = kRouteMfma + kMfmaInstances;
 
 // The contraction kernel's forms: 16-channel blocks per wave (mfma_tile), or
-// 0: mfma_wide.  A wave's registers grow with its channel blocks, so its SIMD
-// holds fewer waves; more than kNarrow blocks (kNarrowGeneral with the general
-// weights) take mfma_wide.  An instance is a form for each value type: first
-// the lean weight's forms, then the general weights', kNbOf[kGeneral[...]].
+// 0: mfma_wide, for each kind of weight.  A wave's registers grow with its
+// channel blocks, so its SIMD holds fewer waves; jobs of more than 16 blocks
+// take mfma_wide.  An instance is a form for each value type.
 constexpr uint32_t kWideWaves = 8;  // waves of a mfma_wide workgroup, 64 channels each
-constexpr uint32_t kNbs = 8, kNbOf[kNbs] = {1, 2, 4, 6, 8, 12, 16, 0};
-constexpr uint32_t kNarrow = 16, kNarrowGeneral = 4;
-constexpr uint32_t kGenerals = 3, kGeneral[kGenerals] = {0, 2, 7};
-static_assert(kMfmaInstances == 2 * (kNbs + kGenerals), "instances");
+constexpr uint32_t kForms = 30, kFormNb[kForms] = {1, 2, 4, 6, 8, 12, 16, 0,        // kWeightLean
+                                                   1, 4, 8, 16, 0, 1, 4, 16, 0,     // Small, Series
+                                                   1, 4, 8, 16, 0, 1, 4, 16, 0,     // 2d, Sinc
+                                                   1, 4, 16, 0};                    // Call
+constexpr uint32_t kFormFirst[kWeightKinds + 1] = {0, 8, 13, 17, 22, 26, kForms};
+static_assert(kMfmaInstances == 2 * kForms, "instances");
 
-// The form of a job (index as instances count): the narrowest that holds its channels.
-constexpr uint32_t mfma_form(uint32_t nchan, bool lean) {
-  const uint32_t blocks = (nchan + 15) / 16;
-  uint32_t i = 0;
-  if (lean) {
-    while (i < kNbs - 1 && kNbOf[i] < blocks) ++i;
-    return i;
-  }
-  while (i < kGenerals - 1 && kNbOf[kGeneral[i]] < blocks) ++i;
-  return kNbs + i;
+// The form of a job: the narrowest of its weight's kind that holds its channels.
+constexpr uint32_t mfma_form(uint32_t nchan, uint32_t kind) {
+  uint32_t i = kFormFirst[kind];
+  while (i + 1 < kFormFirst[kind + 1] && 16 * kFormNb[i] < nchan) ++i;
+  return i;
 }
-constexpr uint32_t nb_of_form(uint32_t form) { return kNbOf[form < kNbs ? form : kGeneral[form - kNbs]]; }
+constexpr uint32_t kind_of_form(uint32_t form) {
+  uint32_t k = 0;
+  while (form >= kFormFirst[k + 1]) ++k;
+  return k;
+}
 
 // A lane reads whole 16-channel blocks of a value block: the rows that the
 // form of a job reads, counted from the value block's first, and those that
 // are there after the first row of the last sample's block (its own and the
 // padding's eight blocks, hcg_channels_padded_len).  Rows past the last channel
 // fill MFMA columns that nothing reads, but they have to be in the buffer.
-constexpr uint64_t value_rows_read(uint32_t nchan, bool lean) {
-  const uint64_t nb = nb_of_form(mfma_form(nchan, lean));
+constexpr uint64_t value_rows_read(uint32_t nchan, uint32_t kind) {
+  const uint64_t nb = kFormNb[mfma_form(nchan, kind)];
   if (nchan == 1) return nb ? (nb - 1) * 16 + 1 : 49;  // (every lane reads its block's first row)
   const uint64_t step = nb ? 16 * nb : 64;
   return (nchan + step - 1) / step * step;
 }
 constexpr uint64_t value_rows_held(uint32_t nchan) { return 9ull * nchan; }
-// (past kNarrow blocks a form reads fewer than 64 rows beyond the last one;
-// a single channel takes the lean weight on the tile loop only)
+// (mfma_wide reads fewer than 64 rows beyond the last channel's)
 constexpr bool value_rows_ok() {
   for (uint32_t c = 1; c <= 1024; ++c)
-    for (uint32_t lean = 0; lean < 2; ++lean)
-      if (value_rows_read(c, lean != 0) > value_rows_held(c)) return false;
+    for (uint32_t kind = 0; kind < kWeightKinds; ++kind)
+      if (value_rows_read(c, kind) > value_rows_held(c)) return false;
   return true;
 }
 static_assert(value_rows_ok(), "a form reads past the padded channel values");

@@ -266,8 +266,7 @@ typedef struct hcg_mfma_shape {
 size_t hcg_grid_mfma_workspace_size(uint32_t side, const hcg_mfma_shape *shape);
 
 /* hcg_grid_mfma with a launch shape (NULL = defaults) and a workspace for
- * the tile plan (NULL = none).  With a workspace and more than 256 channels
- * (64 with weights other than GAUSS1D's at radii of 0.018 to 0.26 deg), a
+ * the tile plan (NULL = none).  With a workspace and more than 256 channels, a
  * first small kernel (one wave per tile, many per CU) computes every tile's
  * ring span, each ring's sorted range and each cell's window and unit vector,
  * and the gridding kernel reads them instead of evaluating them itself; the
