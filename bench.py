@@ -499,9 +499,8 @@ def bench_batch(args, log):
     {128..2048}, channels in {1, 16, 64, 256, 512}, BF16/FP16, sigma in
     {0.015, 0.02, 0.03} deg, Dec in [-60, 80]) gridded by one graph: every
     job's geometry build (keys, sort, records, LUT) and the batched
-    launches over all jobs' tiles.  Block shapes per job class and the launch
-    shape are picked by the autotuner first (untimed).  Compared with the
-    single-channel path applied channel by channel to the same jobs."""
+    launches over all jobs' tiles.  Block shapes per job class are picked by
+    the autotuner first (untimed).  Compared with the single-channel path applied channel by channel to the same jobs."""
     import torch
 
     from hcgrid_amd import autotune, batch, gridder, synth
@@ -534,8 +533,7 @@ def bench_batch(args, log):
              for j in jobs]
     bjobs = tuner.tune_jobs(bjobs, keys)
     waves, chunk = tuner.launch_for(bjobs, "batch")
-    log(f"batch: autotuned {len(tuner.tiles)} job classes and the launch shape in {time.perf_counter() - t1:.1f}s "
-        f"(waves {waves}, chunk {chunk})")
+    log(f"batch: autotuned {len(tuner.tiles)} job classes in {time.perf_counter() - t1:.1f}s")
     b = batch.Batch(bjobs, waves=waves, chunk=chunk)
     stream = torch.cuda.Stream()
     torch.cuda.synchronize()
@@ -729,7 +727,7 @@ def bench_served(args, log, tuner=None):
     request's coordinates and values on the device before submitting it
     (no host-to-device transfer in the latency); results stay in HBM.
     tuner: the batched leg's autotuner (block shape per job class), when
-    that leg ran; the launches run at its tuned waves/chunk."""
+    that leg ran."""
     from hcgrid_amd import serve
 
     waves, chunk = 4, 256

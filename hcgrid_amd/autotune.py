@@ -1,15 +1,13 @@
 """Launch-shape autotuner for the multi-channel gridder.
 
-Two knobs:
-  * per job class, the block shape `tile_cols` (cells per workgroup form a
-    (64 / tile_cols) x tile_cols block of the map; squarer blocks re-read
-    fewer channel values, wider ones cross fewer rings).  The FP32
-    accumulation order of the contraction follows the block shape, so two
-    tile_cols give cubes equal only up to FP32 summation order (both within
-    the stated bound of the FP64 oracle), not bit for bit;
-  * per batch, `waves` and `chunk`, which the kernels accept and no longer
-    use (they choose their waves by the channel count); every result is
-    bit-identical.
+The knob is, per job class, the block shape `tile_cols` (cells per workgroup
+form a (64 / tile_cols) x tile_cols block of the map; squarer blocks re-read
+fewer channel values, wider ones cross fewer rings).  The FP32 accumulation
+order of the contraction follows the block shape, so two tile_cols give cubes
+equal only up to FP32 summation order (both within the stated bound of the
+FP64 oracle), not bit for bit.  A batch's `waves` and `chunk` are accepted by
+the library and have no effect (the kernels choose their waves by the channel
+count): launch_for hands out the defaults, or a pair from an older cache file.
 
 Because the tuner picks tile_cols from timings, two fresh tuning runs can
 pick different shapes and so differ in the last FP32 bits.  Persist the
@@ -18,10 +16,9 @@ choices (`path`) and reuse them to keep results reproducible between runs.
 A job class is (channel bucket, sigma, value type, log2 samples-per-cell
 bucket): jobs in one class have the same support in cells and the same
 balance of FP64 weight work against MFMA work, which is what the block
-shape trades.  The tuner times candidates on the device with events (one-job
-batches on a representative job for tile_cols, the whole batch for waves
-and chunk), keeps the fastest, and caches the choice in memory and
-optionally in a JSON file.
+shape trades.  The tuner times one-job batches on a representative job with
+events, keeps the fastest, and caches the choice in memory and optionally in a
+JSON file.
 """
 from __future__ import annotations
 
@@ -32,7 +29,7 @@ import os
 from . import batch as _batch
 
 TILE_COLS = (8, 16, 32, 64)
-LAUNCH_SHAPES = ((4, 256), (8, 512), (2, 128))
+LAUNCH_SHAPE = (4, 256)  # the library's defaults
 
 
 def chan_bucket(nchan: int) -> int:
@@ -108,19 +105,10 @@ class Autotuner:
         return out
 
     def launch_for(self, jobs: list, key: str) -> tuple[int, int]:
-        """(waves, chunk) for this set of jobs."""
+        """(waves, chunk) for this set of jobs: a stored pair, else the default
+        (nothing is timed, as the kernels do not use them)."""
         if key in self.launch:
             w, c = self.launch[key]
             return int(w), int(c)
-        best, best_ms = LAUNCH_SHAPES[0], float("inf")
-        times = {}
-        for w, c in LAUNCH_SHAPES:
-            b = _batch.Batch(jobs, waves=w, chunk=c)
-            ms = self._time(b.enqueue, 1)
-            b.close()
-            times[(w, c)] = ms
-            if ms < best_ms:
-                best, best_ms = (w, c), ms
-        self.launch[key] = list(best)
-        self.log.append(f"{key}: waves/chunk {best} ({', '.join(f'{k}:{v:.2f}ms' for k, v in times.items())})")
-        return best
+        self.launch[key] = list(LAUNCH_SHAPE)
+        return LAUNCH_SHAPE
