@@ -115,9 +115,9 @@ __global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(4))
 
 // A few-channel job of the multi-channel entry points on the tile path: one
 // wave per tile (few_channel_tile_body).  Two waves per SIMD: with its sums and
-// values of eight channels the sample loop takes 208 registers (a grid pass of
-// 300k samples x 2 onto 2048^2 677 us so, 682 at three waves, 1440 at four,
-// where 113 registers spill; 20k x 8 onto 512^2 50, 63 and 99 us).
+// values of eight channels the sample loop takes some 200 registers (a grid
+// pass of 300k samples x 2 onto 2048^2 655 us so, 732 at three waves, 2156 at
+// four, where it spills; 20k x 8 onto 512^2 48, 68 and 146 us).
 constexpr int kFewWaves = 2;
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kFewWaves)))
     k_grid_tiles_few(GridParams P, GridBuffers B, TileOut O, uint32_t tiles_x, uint32_t tiles_y, uint32_t first) {

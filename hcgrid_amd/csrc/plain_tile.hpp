@@ -934,28 +934,22 @@ __device__ __forceinline__ void grid_tile(const GridParams& P, const GridBuffers
                        (t < t_hi && radius_test_ref(B.xwcs, B.ywcs, B.lon_s, B.lat_s, cell, isrc, P.sphere_radius));
               };
               if constexpr (NC > 0) {
-                const auto add = [&]() {
+                // (zeroed copies of the channels' values would take registers)
+                bool in = true;
+                if (near) {
+                  asm volatile("; guard band" ::);
+                  in = inside();
+                }
+                if (in) {
                   const float wf = (float)wt;
 #pragma unroll
                   for (int c = 0; c < NC; ++c) acc_c[k][c] = fmaf(wf, cv[c], acc_c[k][c]);
                   acc_w[k] += wt;
-                };
-                // (what follows the sums differs, so that the two stay apart:
-                // merged they take a lane mask in the common case, and
-                // zeroed copies of the channels' values take registers: 300k
-                // samples x 2 onto 2048^2 3.66 ms so, 2.65 apart)
-                if (near) {
-                  if (inside()) {
-                    add();
-                    asm volatile("; near the radius" ::);
-                  }
-                } else {
-                  add();
                 }
               } else {
                 // a rejected lane adds zero: one compare and no lane mask in
-                // the common case (the sums apart, as above, cost 6% on 20M
-                // samples; the weight's copy 1.5% on weighted maps)
+                // the common case (sums under a mask, as above, cost 6% on
+                // 20M samples; the weight's copy 1.5% on weighted maps)
                 double vv = qv, ww = qw;
                 if (near) {
                   // (a block of its own, so the branch above stays a scalar one)
