@@ -500,7 +500,8 @@ def bench_batch(args, log):
     {0.015, 0.02, 0.03} deg, Dec in [-60, 80]) gridded by one graph: every
     job's geometry build (keys, sort, records, LUT) and the batched
     launches over all jobs' tiles.  Block shapes per job class are picked by
-    the autotuner first (untimed).  Compared with the single-channel path applied channel by channel to the same jobs."""
+    the autotuner first (untimed).  Compared with the single-channel path
+    applied channel by channel to the same jobs."""
     import torch
 
     from hcgrid_amd import autotune, batch, gridder, synth

@@ -47,47 +47,9 @@ inline void launch_runs(uint64_t blocks, uint32_t threads, F&& launch) {
     launch((uint32_t)first, (uint32_t)(blocks - first < most ? blocks - first : most));
 }
 
-// Lanes of the wave whose 8-bit digit equals this lane's (wave64 ballots).
-__device__ inline uint64_t match_digit8(uint32_t d, bool valid) {
-  uint64_t m = __ballot(valid);
-#pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    const bool bit = (d >> b) & 1u;
-    const uint64_t vote = __ballot(bit);
-    m &= bit ? vote : ~vote;
-  }
-  return m;
-}
-
 __device__ inline uint64_t lanemask_lt() {
   const uint32_t lane = __lane_id();
   return lane ? (~0ull >> (64 - lane)) : 0ull;
-}
-
-// First index in [lo, hi) whose key >= key (hi if none).
-__host__ __device__ inline uint32_t lower_bound_u32(const uint32_t* v, uint32_t lo, uint32_t hi,
-                                                    uint32_t key) {
-  while (lo < hi) {
-    const uint32_t mid = lo + ((hi - lo) >> 1);
-    if (v[mid] < key)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-
-// First index in [lo, hi) whose key > key (hi if none).
-__host__ __device__ inline uint32_t upper_bound_u32(const uint32_t* v, uint32_t lo, uint32_t hi,
-                                                    uint32_t key) {
-  while (lo < hi) {
-    const uint32_t mid = lo + ((hi - lo) >> 1);
-    if (v[mid] <= key)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
 }
 
 }  // namespace hcg

@@ -19,7 +19,8 @@
 // registers, every pair of the 16 x 32 (45% of them selected on rasters of
 // two and more samples per cell).  mfma_tile is a wave per square, without
 // barriers, for up to 256 channels; mfma_wide shares a block's weights over
-// 512 channels through LDS.
+// 512 channels through LDS.  Both come for each kind of weight
+// (mfma_weight_kind).
 //
 // What counts is vector instructions (FP64 weights), then the latency of the
 // LDS reads and weight chains at two to four waves per SIMD.  Before, weights
@@ -27,11 +28,11 @@
 // filled by lane = cell, 44% of the lanes on selected pairs) between four
 // workgroup barriers per 128-512 samples, one wave contracting while the
 // rest waited on small jobs.  A pass before and now: 195k samples x 3
-// channels onto 500^2 911 -> 194 us; 482k x 67 onto 511^2 1316 -> 495 us;
-// 300k x 16 onto 2048^2 3337 -> 1395 us; 1.2M x 64 onto 512^2 (new
-// coordinates) 2697 -> 1511 us; 2M x 1024 onto 1024^2 9526 -> 8716 us (this
-// kernel 7.40 -> 6.64 ms: 1.39e9 vector and 2.0e8 MFMA instructions, 64% of
-// the wave cycles waiting at two waves per SIMD).
+// channels onto 500^2 911 -> 190 us; 482k x 67 onto 511^2 1316 -> 413 us;
+// 300k x 16 onto 2048^2 3337 -> 1370 us; 1.2M x 64 onto 512^2 (new
+// coordinates) 2697 -> 1522 us; 2M x 1024 onto 1024^2 9526 -> 8200 us (this
+// kernel 7.40 -> 6.0 ms: 1.34e9 vector and 1.9e8 MFMA instructions at two
+// waves per SIMD).
 //
 // Selection, FP64 distance and weight follow the single-channel kernel
 // exactly; only the products with channel values run in BF16/FP16.
@@ -707,7 +708,7 @@ __device__ __forceinline__ const char* value_rows(const MfmaJob& J, uint32_t ch_
 
 // One block of 64 cells and up to 16 NB channels (group `group` of them): a
 // wave takes a square of 16 cells, on its own but for the set-up and the
-// stores.  WK: mfma_weight_kind.
+// stores.  WK: the kind of weight (mfma_weight_kind).
 template <int DT, int NB, uint32_t WK>
 __device__ __forceinline__ void mfma_tile(const MfmaJob& J, uint32_t tile, uint32_t group, MfmaLds<WK>& lds,
                                           const double* s_exp) {

@@ -7,8 +7,9 @@
 //   sorted samples with lpix_r(a) <= key <= rpix_r(a) (whole ring when the
 //   anchor colatitude is <= 20 or >= 160 deg, gridding.cu:341-356),
 //   great-circle distance from the cell itself < sphere_radius.
-// Accumulation order per cell is the reference's: ring ascending, sorted
-// index ascending, FP64.
+// Sums are FP64.  The order is the reference's (ring ascending, sorted index
+// ascending) within each of a cell's partial sums: four lane phases, in each of
+// the ring streams that share a tile of a small map (plain_tile.hpp).
 //
 // What differs from the reference's arithmetic (not its selection):
 //  * ring windows use the per-ring cos/sin table built with the LUT instead

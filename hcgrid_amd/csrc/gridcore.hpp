@@ -140,16 +140,16 @@ __device__ inline Window window_of(const GridParams& P, uint32_t firstring, uint
 // start_int - 1 wrap, HCGrid/gridding.cu:326, 363-367); HCG_SELECT_DISC grids them.
 __device__ inline bool skips_first_ring(const GridParams& P) { return P.selection != HCG_SELECT_DISC; }
 
-// lpix/rpix of ring r (HCGrid/gridding.cu:336-360).  Returns false where the
-// reference would `continue` without advancing (an endless loop there); the
-// ring is skipped here instead.  ang2pix(theta_r, phi) == loc2pix(cos theta_r, ...).
-// The longitude edges of a compat window do not depend on the ring:
-// compat_edges gives them once, ring_window_at takes them.
+// The longitude edges of a compat window, which do not depend on the ring.
 __device__ inline void compat_edges(const GridParams& P, const Window& w, double& tl, double& tr) {
   tl = fmodulo4((w.phi - P.disc_size) * kInvHalfPi);
   tr = fmodulo4((w.phi + P.disc_size) * kInvHalfPi);
 }
 
+// lpix/rpix of ring r (HCGrid/gridding.cu:336-360), tl and tr the window's edges
+// (compat_edges).  Returns false where the reference would `continue` without
+// advancing (an endless loop there); the ring is skipped here instead.
+// ang2pix(theta_r, phi) == loc2pix(cos theta_r, ...).
 __device__ inline bool ring_window_at(const Hpx32& hx, const Window& w, double tl, double tr, uint32_t ring,
                                       double rz, double rs, uint32_t& lpix, uint32_t& rpix) {
   uint32_t sp, npr;
@@ -188,20 +188,15 @@ __device__ inline bool ring_window_at(const Hpx32& hx, const Window& w, double t
 
 // The reference's radius test (HCGrid/helpers.cu:128-130, gridding.cu:381-386)
 // for a pair inside the guard band.
-__device__ __forceinline__ bool radius_test_inline(const double* xwcs, const double* ywcs, const double* lon_s,
-                                                   const double* lat_s, uint32_t cell, uint32_t i, double radius) {
+[[maybe_unused]] static __device__ __noinline__ bool radius_test_ref(const double* xwcs, const double* ywcs,
+                                                                     const double* lon_s, const double* lat_s,
+                                                                     uint32_t cell, uint32_t i, double radius) {
   const double l1 = xwcs[cell] * kDeg2Rad, b1 = ywcs[cell] * kDeg2Rad;
   const double l2 = lon_s[i] * kDeg2Rad, b2 = lat_s[i] * kDeg2Rad;
   const double a = sin((b1 - b2) / 2.);
   const double c = sin((l1 - l2) / 2.);
   const double d = 2 * asin(sqrt(a * a + cos(b1) * cos(b2) * (c * c))) * kRad2Deg;
   return d < radius;
-}
-
-[[maybe_unused]] static __device__ __noinline__ bool radius_test_ref(const double* xwcs, const double* ywcs,
-                                                                     const double* lon_s, const double* lat_s,
-                                                                     uint32_t cell, uint32_t i, double radius) {
-  return radius_test_inline(xwcs, ywcs, lon_s, lat_s, cell, i, radius);
 }
 
 [[maybe_unused]] static __device__ __noinline__ double asin2_direct(double h) {
@@ -232,17 +227,13 @@ __device__ inline double gauss_exponent_series(const GridParams& P, double c2) {
   return c2 * fma(c2, fma(c2, fma(c2, P.k3, P.k2), P.k1), P.k0);
 }
 
-// True when every selected pair (c2 < c_hi) takes the series branch and its
-// scaled exponent stays above exp_scaled_neg's clamp (host side).
-// 16-bit values (BF16 or FP16) to and from FP32, round to nearest even.
-__device__ inline uint16_t round16(float f, bool bf) {
-  return bf ? __builtin_bit_cast(uint16_t, (__bf16)f) : __builtin_bit_cast(uint16_t, (_Float16)f);
-}
-
+// A 16-bit value (BF16 or FP16) in FP32.
 __device__ inline float widen16(uint16_t h, bool bf) {
   return bf ? (float)__builtin_bit_cast(__bf16, h) : (float)__builtin_bit_cast(_Float16, h);
 }
 
+// True when every selected pair (c2 < c_hi) takes the series branch and its
+// scaled exponent stays above exp_scaled_neg's clamp (host side).
 inline bool gauss_small_radius(const GridParams& P) {
   if (!(P.c_hi < 4e-4)) return false;
   const double y = P.c_hi * (P.k0 + P.c_hi * (P.k1 + P.c_hi * (P.k2 + P.c_hi * P.k3)));
@@ -493,37 +484,6 @@ template <int KT>
 }
 
 // ---- wave-level helpers ----
-
-// 64-way search over keys[lo, hi): first index whose key >= K (UPPER=false) or
-// > K (UPPER=true).  Wave-uniform inputs and result.
-template <bool UPPER>
-__device__ inline uint32_t wave_search(const uint32_t* __restrict__ keys, uint32_t lo, uint32_t hi, uint32_t K) {
-  const uint32_t lane = __lane_id();
-  while (hi - lo > 64) {
-    const uint32_t step = (hi - lo + 63) / 64;
-    const uint32_t p = lo + lane * step;
-    const bool inr = p < hi;
-    const uint32_t kv = inr ? keys[p] : 0xFFFFFFFFu;
-    const bool ge = inr ? (UPPER ? kv > K : kv >= K) : true;
-    const uint64_t m = __ballot(ge);
-    if (m == 0) {  // all 64 probes in range and below K: the answer is past the last probe
-      lo = lo + 63 * step + 1;
-      continue;
-    }
-    const uint32_t f = (uint32_t)__ffsll((unsigned long long)m) - 1;
-    const uint32_t pf = lo + f * step;
-    if (f == 0) return lo;
-    const uint32_t nlo = lo + (f - 1) * step + 1;
-    hi = pf < hi ? pf : hi;
-    lo = nlo;
-  }
-  const uint32_t p = lo + lane;
-  const bool inr = p < hi;
-  const uint32_t kv = inr ? keys[p] : 0u;
-  const bool ge = inr && (UPPER ? kv > K : kv >= K);
-  const uint64_t m = __ballot(ge);
-  return m ? lo + (uint32_t)__ffsll((unsigned long long)m) - 1 : hi;
-}
 
 // Wave reductions by DPP (row shifts by 1, 2, 4, 8, then the row broadcasts:
 // lane 63 holds the result), returned wave-uniform.  A lane whose source is

@@ -26,8 +26,8 @@
 // evaluation are nearly all selected: with lane = cell and one band per lane
 // 44% of the lane slots did selected pairs on the 20M-sample raster (rows
 // outside a ring's reach and the window's corners outside the disc idled
-// through the weight): 1.97e9 vector instructions and 4.40 ms then, 1.34e9
-// and 3.42 ms now.  On sparse maps the per-ring chain of searches, loads and
+// through the weight): 1.97e9 vector instructions and 4.40 ms then, 1.39e9
+// and 3.49 ms now.  On sparse maps the per-ring chain of searches, loads and
 // window arithmetic is what counts (160k samples onto 1024^2: 199 us).
 //
 // The selection, distance and weight are the ones described in
@@ -112,9 +112,10 @@ inline uint32_t tile_count_of(uint32_t side) { return tile_cols_of(side) * ((sid
 // One-channel jobs of the multi-channel entry points (hcg_grid_mfma*, batch
 // jobs) that take the FP64 tile path instead of the MFMA contraction:
 // GAUSS1D, no per-sample weights, a radius small enough for the three-term
-// weight series.  With one channel the FP64 weight is all the work, and
-// the tile loop evaluates it several times faster than the MFMA kernel's
-// weight stage; the result is also closer to FP64 (unrounded weights).
+// weight series.  The result is closer to FP64 (unrounded weights), and with
+// one channel the weight is all the work: here and in the contraction 1M
+// samples onto 512^2 227 and 304 us, 300k onto 2048^2 631 and 934, 5k onto 20^2
+// 68 and 79; 2M onto 128^2, on few tiles, 1374 and 1090.
 inline bool one_channel_tiles(const GridParams& P, uint32_t kernel_type, bool weighted, uint32_t nchan) {
   return nchan == 1 && kernel_type == HCG_GAUSS1D && !weighted && gauss_tiny_radius(P);
 }
@@ -124,8 +125,7 @@ inline bool one_channel_tiles(const GridParams& P, uint32_t kernel_type, bool we
 // kOneChannelMinTiles tiles (four per SIMD of the 256-CU chip) split each
 // tile's rings over kOneChannelStreams waves, ring r to stream
 // (r - first ring) % streams; larger maps take one wave per tile.  (A
-// 5M-sample 128^2 map, 256 tiles: 25 ms on one wave per tile, against 15
-// ms on the MFMA kernel, which spreads a block's weights over its waves.)
+// 5M-sample 128^2 map, 256 tiles, took 25 ms on one wave per tile.)
 constexpr uint32_t kOneChannelMinTiles = 4096;
 constexpr uint32_t kOneChannelStreams = 4;
 inline uint32_t one_channel_streams(uint32_t side) {
@@ -136,13 +136,13 @@ inline uint32_t one_channel_streams(uint32_t side) {
 // sample per kFewCellsPerSample cells, otherwise as one_channel_tiles, at
 // dot_distance_ok radii (their tile loop tests candidates on p.q), on maps
 // of at least kOneChannelMinTiles tiles) also take the tile loop: FP64
-// weights, FP32 accumulation per channel, one wave per tile at several
-// waves per SIMD.  On sparse maps the MFMA kernel's fixed chain of barriers
-// and global round trips per 64-cell block outweighs the per-pair work:
-// 300k samples x 2..8 channels onto 2048^2 (0.07 samples per cell) took
-// 1.96-2.10 ms here against 2.20-2.23 ms there.  With 16 channels, or at
-// 0.6-13 samples per cell, the MFMA kernel is the faster one (3M x 16 onto
-// 2048^2: 6.98 against 8.35 ms; 3.4M x 2 onto 512^2: 3.31 against 4.23 ms).
+// weights, FP32 accumulation per channel, one wave per tile.  On sparse maps a
+// set-up per 64 cells and no value blocks outweigh the matrix products: 300k
+// samples x 2 onto 2048^2 (0.07 samples per cell) 655 us here and 935 in the
+// contraction, x 8 692 and 947; 400k x 8 onto 2048^2 (0.095) 775 and 994; 20k x
+// 8 onto 512^2 48 and 65.  On denser maps the contraction is the faster one
+// (195k x 3 onto 500^2: 190 us a pass, and 382 with this loop before it had
+// its registers).
 constexpr int kFewChannels = 8;
 constexpr uint32_t kFewCellsPerSample = 10;
 constexpr uint32_t kFewCap = 128;  // staged samples per round

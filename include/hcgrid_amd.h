@@ -428,6 +428,8 @@ int hcg_batch_create_in(uint32_t njobs, const hcg_batch_job *jobs, uint32_t wave
  * equal hcg_grid_mfma_shaped's with the same tile_cols, bit for bit. */
 int hcg_batch_enqueue(hcg_batch *b, void *stream);
 
+/* nitems and blocks: the gridding launches' workgroups; waves and chunk as given
+ * (or their defaults). */
 typedef struct hcg_batch_stats {
     uint32_t njobs, nitems, blocks, waves, chunk, reserved;
     size_t device_bytes;
