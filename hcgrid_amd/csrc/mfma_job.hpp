@@ -150,6 +150,19 @@ int launch_batch_tiles(uint32_t route, const TileRange* ranges, uint32_t nranges
 uint32_t mfma_instance(const MfmaJob& J);
 bool mfma_uses_plan(uint32_t instance);
 uint64_t mfma_blocks(const MfmaJob& J);
+// One launch of an instance (launch_form), and the instances of mfma_gauss.hip
+// and mfma_gauss2d_sinc.hip.
+struct MfmaLaunch {
+  const MfmaJob* job;
+  uint32_t groups;
+  const TileRange* ranges;
+  uint32_t nranges;
+  const MfmaJob* jobs;
+  uint32_t first, count;
+  hipStream_t stream;
+};
+void launch_gauss_forms(uint32_t instance, const MfmaLaunch& L);
+void launch_gauss2d_sinc_forms(uint32_t instance, const MfmaLaunch& L);
 // Launches one instance's workgroups.
 int launch_mfma_batch(uint32_t instance, const TileRange* ranges, uint32_t nranges, uint32_t blocks,
                       const MfmaJob* jobs, hipStream_t s);
